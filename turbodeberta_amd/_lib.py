@@ -72,6 +72,7 @@ class VarlenArgs(C.Structure):
 
 _lock = threading.Lock()
 _lib = None
+_host = None
 
 
 def load() -> C.CDLL:
@@ -105,6 +106,23 @@ def load() -> C.CDLL:
             raise RuntimeError(f"libtdb_attn.so has ABI {lib.tdb_version()}, this package expects {ABI_VERSION}")
         _lib = lib
     return _lib
+
+
+def host():
+    """The operators' native front (_host.so), bound to the loaded library.  Its functions return None for a call
+    they do not take."""
+    global _host
+    if _host is None:
+        import torch  # noqa: F401  (the module links PyTorch's libraries)
+        lib = load()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise RuntimeError(f"{PKG}/_host.so is missing or does not load ({e}): build it with "
+                               "`python -m turbodeberta_amd._build`") from e
+        module.bind(C.cast(lib.tdb_attn_fwd_fixed, C.c_void_p).value, C.cast(lib.tdb_attn_fwd_varlen, C.c_void_p).value)
+        _host = module
+    return _host
 
 
 def check(rc: int) -> None:

@@ -46,6 +46,8 @@ def delta_lut(device: torch.device, max_len: int, position_buckets: int, max_rel
             table = torch.from_numpy(_lib.delta_table(size, int(position_buckets), int(max_relative_distance)))
             hit = (table.to(device), size - 1)
             _lut_cache[key] = hit
+            if device.type == "cuda":
+                _lib.host().add_lut(hit[0], size, int(position_buckets), int(max_relative_distance))
     return hit
 
 

@@ -129,6 +129,10 @@ def flash_attention_with_disentangled(q, k, v, q_pos, k_pos, causal=False, sm_sc
 
     Returns ``o`` with the shape and dtype of ``q``.  Forward only: backward raises RuntimeError.
     """
+    out = _lib.host().fixed(q, k, v, q_pos, k_pos, causal, sm_scale, position_buckets, max_relative_distance,
+                            pos_key_layer, pos_query_layer, seqlens_k, force_generic)
+    if out is not None:
+        return out
     return FlashAttentionDisentangled.apply(q, k, v, q_pos, k_pos, causal, sm_scale, position_buckets,
                                             max_relative_distance, pos_key_layer, pos_query_layer,
                                             seqlens_k, force_generic)

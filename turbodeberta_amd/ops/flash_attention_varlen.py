@@ -135,6 +135,12 @@ def flash_attention_with_disentangled_varlen(q, k, v, q_pos, k_pos, cu_seqlens_q
     ``zero_output`` (see ``prepare``).  Relative positions are in-sequence offsets
     (ops/flash_attention_varlen.py:70,118); each key is masked by its own sequence's length.
     No host synchronisation is made unless ``check_cu_seqlens`` asks for one.  Returns ``o [total_tokens, H, D]``; forward only."""
+    if not check_cu_seqlens:
+        out = _lib.host().varlen(q, k, v, q_pos, k_pos, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, causal,
+                                 sm_scale, position_buckets, max_relative_distance, pos_key_layer, pos_query_layer,
+                                 force_generic, zero_output)
+        if out is not None:
+            return out
     return FlashAttentionDisentangled.apply(q, k, v, q_pos, k_pos, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
                                             max_seqlen_k, causal, sm_scale, position_buckets,
                                             max_relative_distance, pos_key_layer, pos_query_layer, force_generic,
