@@ -1,0 +1,372 @@
+// Matrix-core disentangled-attention forward for float32, head_dim 64 (gfx950, wave64, MFMA 16x16x4 f32).
+//
+// float32 is the type checkpoints load in, and its 1e-4 bar leaves no room for split or reduced operands: products and
+// sums are float32 FMAs, on the matrix cores (152 TFLOP/s measured for a large product; the packed vector forms that
+// would reach that rate are not used here).
+//
+// What bounds it: the matrix pipe.  A 16 x 16 x 64 tile product takes 16 MFMAs = 512 clk, sixteen times a bf16 one, so
+// everything else is chosen to be simple rather than cheap: operands go straight from global memory to registers (a
+// fragment is four 16-byte loads whose lanes cover 64 contiguous bytes of 16 rows), the two position terms are shifted
+// through a wave's own LDS scratch with plain 4-byte reads, and no wave waits for another until the end.
+//
+// Measured (vector-ALU kernel before): 2 x 128 x 12 heads 84 -> 8.9 us; 8 x 12 heads, lengths 96..384, 660 -> 68 us; 8 x 512
+// full 160 us = 81 TFLOP/s without credit for the half-used outer tiles, 101 with (matrix pipe busy 65 % of the time; what is
+// left is the start and end of a workgroup, a tenth, and L2 latency that two waves per SIMD do not quite cover).
+//
+// One workgroup = QT*16 query rows of one (sequence, head); its four waves share out the KEYS (blocks of two
+// 16-key tiles, in turn) and merge their partial softmax sums through LDS at the end.  Splitting the keys rather than the
+// queries gives a 2 x 128 x 12 head call 768 waves of work instead of 96.  QT = 2 spends 1.25x the products the
+// formulation cannot do without (a 16-wide position tile serves 16 + 16 query-key diagonals, and the outer ones of a
+// block are only half used), QT = 1 1.375x but twice the workgroups: see tdb_launch_f32 for the rule.
+//
+// Relative positions come in 16-wide tiles as well: tile e covers r = 16e .. 16e+15, and the (query tile a, key tile b)
+// pair needs r = 16(a-b)-15 .. 16(a-b)+15, i.e. tiles a-b-1 and a-b.  A block of QT query tiles and two key tiles needs
+// QT+2 position tiles; each of their table rows K_r[delta(r)], Q_r[delta(r)] is loaded once per block and contracted
+// with the query tiles (c2p) and the key tiles (p2c) that reach it.
+//   c2p  C'^T[r, i] = K_r[delta(r)].Q_i   lane = query, registers = 4 positions -> scratch C[query][r]
+//   p2c  P'^T[r, j] = Q_r[delta(r)].K_j   lane = key,   registers = 4 positions -> scratch P[key][r]
+// The score tile S^T[j, i] (lane = query, registers = 4 keys) then starts from C[i][i-j] + P[j][i-j].
+// With strips the two starting values are read from the caller's arrays instead.
+// (Same definition as the other kernels: modeling_deberta_v2.py:243, :317-324, :337-343.)
+#include <type_traits>
+
+#include "tdb_internal.h"
+
+namespace {
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+constexpr int WAVES = 4;
+constexpr int D = 64;
+constexpr int KT = 2;                       // key tiles of 16 per block
+constexpr int CS = 16 * (KT + 1) + 4;       // row stride of the c2p scratch (floats): [query][48 positions]
+constexpr int PS(int qt) { return 16 * (qt + 1) + 4; }
+constexpr int scratch_floats(int qt) { return qt * 16 * CS + KT * 16 * PS(qt); }      // per wave
+// the merge needs QT * 1024 floats of partial sums per wave, and 2 * QT * 16 of maxima and denominators
+constexpr int wave_floats(int qt) { return scratch_floats(qt) > qt * (1024 + 32) ? scratch_floats(qt) : qt * (1024 + 32); }
+
+__device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// Lanes of one wave exchange data through LDS: DS instructions of a wave execute in order, so only the compiler has to
+// be kept from moving accesses across.
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Value of the three lanes that share (l & 15), folded: lanes l ^ 16 and l ^ 32.
+__device__ __forceinline__ float fold_max(float x) {
+    x = fmaxf(x, __shfl_xor(x, 16));
+    return fmaxf(x, __shfl_xor(x, 32));
+}
+// exp(x) for x <= 0 to about one unit in the last place: the hardware's base-2 exponential of the rounded x log2(e),
+// corrected to first order by what the rounding (and log2(e)'s own) left out.  A third of the instructions of expf, whose
+// range handling the softmax does not need; arguments below -1e4 (masked keys, the first block's old maximum) give 0.
+__device__ __forceinline__ float exp_neg(float x) {
+    x = fmaxf(x, -1e4f);
+    const float h = x * 1.44269502f;                                              // float(log2 e)
+    const float e = fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269502f, -h));            // + the rest of log2 e
+    const float y = __builtin_amdgcn_exp2f(h);
+    return fmaf(y, e * 0.693147182f, y);
+}
+__device__ __forceinline__ float fold_sum(float x) {
+    x += __shfl_xor(x, 16);
+    return x + __shfl_xor(x, 32);
+}
+
+// Fragment of 16 rows x 64: lane (row = l & 15, g = l >> 4) holds columns 16t + 4g .. +3, t = 0..3.  Both operands of a
+// product use this order, so MFMA (t, e) contracts columns {16t + 4g + e}: any order of the sum is a valid one.
+__device__ __forceinline__ void load_frag(f32x4 (&f)[4], const float* row, int g) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) f[t] = *reinterpret_cast<const f32x4*>(row + 16 * t + 4 * g);
+}
+
+template <int QT, bool STRIP, bool C2P, bool P2C>
+__global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_kernel(const TdbKernelParams p, const int tiles_x) {
+    extern __shared__ __attribute__((aligned(16))) float smem_f[];
+    constexpr int PST = PS(QT);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+    const int c = l & 15, g = l >> 4;       // column (or row) of a tile, group of four rows
+    float* const sC = smem_f + wave * wave_floats(QT);
+    float* const sP = sC + QT * 16 * CS;
+
+    // Block ids go round-robin over the 8 XCDs: four neighbouring query tiles, which read the same keys and values,
+    // are kept on one of them.  The heads of a tile group follow each other (and not the tile groups of a head), so
+    // that every XCD gets its share of every sequence, however their lengths differ.
+    const int slot = blockIdx.x >> 3;
+    const int group = (slot >> 2) * 8 + (blockIdx.x & 7), h = group % p.H, tile = group / p.H * 4 + (slot & 3);
+    int b, row0, len;
+    int64_t tok0;
+    if (tile >= tiles_x || !tdb_locate_tile_sorted(p, QT * 16, tile, b, row0, len, tok0)) return;
+    b = __builtin_amdgcn_readfirstlane(b), row0 = __builtin_amdgcn_readfirstlane(row0), len = __builtin_amdgcn_readfirstlane(len);
+
+    auto base = [&](const void* ptr, int64_t sb, int64_t sh, int64_t sl) {
+        return static_cast<const float*>(ptr) + (p.varlen ? tok0 * sl : int64_t(b) * sb) + int64_t(h) * sh;
+    };
+    float* const O = const_cast<float*>(base(p.o, p.os_b, p.os_h, p.os_l));
+    const int rows_here = min(QT * 16, (p.varlen ? len : p.L) - row0);
+    if (row0 >= len) {                      // padded query rows only (fixed layout): zeros
+        for (int idx = threadIdx.x; idx < rows_here * (D / 4); idx += WAVES * 64)
+            *reinterpret_cast<f32x4*>(O + int64_t(row0 + idx / (D / 4)) * p.os_l + idx % (D / 4) * 4) = f32x4{0.f, 0.f, 0.f, 0.f};
+        return;
+    }
+    const float* const Q = base(p.q, p.qs_b, p.qs_h, p.qs_l);
+    const float* const K = base(p.k, p.ks_b, p.ks_h, p.ks_l);
+    const float* const V = base(p.v, p.vs_b, p.vs_h, p.vs_l);
+    const float* const C = STRIP ? base(p.c2p, p.c2s_b, p.c2s_h, p.c2s_l) : static_cast<const float*>(p.pk) + int64_t(h) * p.pks_h;
+    const float* const P = STRIP ? base(p.p2c, p.p2s_b, p.p2s_h, p.p2s_l) : static_cast<const float*>(p.pq) + int64_t(h) * p.pqs_h;
+    const int lut_max = 2 * p.lut_half;
+    auto delta_of = [&](int r) { return p.lut[min(max(r + p.lut_half, 0), lut_max)]; };
+
+    // This wave's key tiles: blocks of KT, dealt to the waves in turn (the position rows of neighbouring blocks overlap
+    // by half, and waves that work on neighbours at the same time find them in L1), or single tiles where there are few.
+    const int ntiles = (len + 15) >> 4, per = (ntiles + WAVES - 1) / WAVES;
+    const bool few = per < KT;
+    const int first = wave * (few ? 1 : KT), last = few ? min(first + 1, ntiles) : ntiles, stride = WAVES * KT;
+
+    // Table rows of position tile x of the block that starts at key tile bt: r = row0 - 16 bt + 16 (x - 2) + c.
+    int dl[QT + 2];
+    auto read_deltas = [&](int bt) {
+#pragma unroll
+        for (int x = 0; x < QT + 2; ++x) dl[x] = delta_of(row0 - 16 * bt + 16 * (x - 2) + c);
+    };
+    if (!STRIP && (C2P || P2C) && first < last) read_deltas(first);
+
+    f32x4 qf[QT][4];
+#pragma unroll
+    for (int a = 0; a < QT; ++a) load_frag(qf[a], Q + int64_t(min(row0 + 16 * a + c, len - 1)) * p.qs_l, g);
+
+    f32x4 oacc[QT][4];                      // [query tile][u]: row m of tile u is d = 4m + u
+    float m_run[QT], l_run[QT];             // l_run: this lane's keys only
+#pragma unroll
+    for (int a = 0; a < QT; ++a) {
+        m_run[a] = -INFINITY, l_run[a] = 0.f;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) oacc[a][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+
+    // Operands are requested one use ahead: a fragment of position rows while the one before it is contracted, the
+    // values under the score products, the next block's keys and first position rows under the softmax.
+    f32x4 kf[KT][4], pf[2][4];              // keys; position rows of this phase and the next
+    auto load_keys = [&](int bt) {
+#pragma unroll
+        for (int bi = 0; bi < KT; ++bi) load_frag(kf[bi], K + int64_t(min(16 * (bt + bi) + c, len - 1)) * p.ks_l, g);
+    };
+    // phases of a block: position tile x = ph / TERMS, one term after the other (c2p first)
+    constexpr int TERMS = int(C2P) + int(P2C), PHASES = STRIP ? 0 : TERMS * (QT + 2);
+    auto load_pos = [&](int ph) {
+        const int x = ph / (TERMS > 0 ? TERMS : 1);
+        if (C2P && (!P2C || ph % 2 == 0)) load_frag(pf[ph & 1], C + int64_t(dl[x]) * p.pks_r, g);
+        else load_frag(pf[ph & 1], P + int64_t(dl[x]) * p.pqs_r, g);
+    };
+    // Nothing moves across: left alone, the scheduler sinks every load to just before its use (one exposed L2 round
+    // trip per 16 bytes: 190 us instead of 138 at batch 8 x 512).
+    auto issued = [] { __builtin_amdgcn_sched_barrier(0); };
+    if (first < last) {
+        load_keys(first);
+        if (PHASES) load_pos(0);
+    }
+    for (int bt = first; bt < last; bt += stride) {
+        const bool two = bt + 1 < last;     // whether the block's second key tile exists
+        f32x4 s[QT][KT];
+#pragma unroll
+        for (int a = 0; a < QT; ++a)
+#pragma unroll
+            for (int bi = 0; bi < KT; ++bi) s[a][bi] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+        if (STRIP) {
+#pragma unroll
+            for (int a = 0; a < QT; ++a)
+#pragma unroll
+                for (int bi = 0; bi < KT; ++bi)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        const int i = min(row0 + 16 * a + c, len - 1), j = min(16 * (bt + bi) + 4 * g + t, len - 1);
+                        const int d = delta_of(i - j);
+                        if (C2P) s[a][bi][t] += C[int64_t(i) * p.c2s_l + d];
+                        if (P2C) s[a][bi][t] += P[int64_t(j) * p.p2s_l + d];
+                    }
+        } else if (C2P || P2C) {
+            // c2p: query tile a reaches position tiles a .. a+2; p2c: key tile bi reaches 1-bi .. QT+1-bi
+#pragma unroll
+            for (int ph = 0; ph < PHASES; ++ph) {
+                const int x = ph / TERMS;
+                if (ph + 1 < PHASES) load_pos(ph + 1);
+                issued();
+                const f32x4(&f)[4] = pf[ph & 1];
+                if (C2P && (!P2C || ph % 2 == 0)) {
+                    f32x4 acc[QT];
+#pragma unroll
+                    for (int a = 0; a < QT; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int te = 0; te < 16; ++te)
+#pragma unroll
+                        for (int a = 0; a < QT; ++a)
+                            if (x >= a && x <= a + 2) acc[a] = mfma(f[te >> 2][te & 3], qf[a][te >> 2][te & 3], acc[a]);
+#pragma unroll
+                    for (int a = 0; a < QT; ++a)
+                        if (x >= a && x <= a + 2) *reinterpret_cast<f32x4*>(&sC[(16 * a + c) * CS + 16 * (x - a) + 4 * g]) = acc[a];
+                } else {
+                    f32x4 acc[KT];
+#pragma unroll
+                    for (int bi = 0; bi < KT; ++bi) acc[bi] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int te = 0; te < 16; ++te)
+#pragma unroll
+                        for (int bi = 0; bi < KT; ++bi)
+                            if (x >= 1 - bi && x <= QT + 1 - bi) acc[bi] = mfma(f[te >> 2][te & 3], kf[bi][te >> 2][te & 3], acc[bi]);
+#pragma unroll
+                    for (int bi = 0; bi < KT; ++bi)
+                        if (x >= 1 - bi && x <= QT + 1 - bi)
+                            *reinterpret_cast<f32x4*>(&sP[(16 * bi + c) * PST + 16 * (x + bi - 1) + 4 * g]) = acc[bi];
+                }
+            }
+            if (bt + stride < last) read_deltas(bt + stride);
+            wave_fence();
+            // query 16a + c, key 16bi + jl: position i - j sits at 32 - 16 bi + c - jl of C's row and at 16 (a + 1) + c - jl of P's
+#pragma unroll
+            for (int bi = 0; bi < KT; ++bi)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const int jl = 4 * g + t;
+#pragma unroll
+                    for (int a = 0; a < QT; ++a) {
+                        float x = 0.f;
+                        if (C2P) x = sC[(16 * a + c) * CS + 32 - 16 * bi + c - jl];
+                        if (P2C) x += sP[(16 * bi + jl) * PST + 16 * (a + 1) + c - jl];
+                        s[a][bi][t] = x;
+                    }
+                }
+            wave_fence();
+        }
+        f32x4 vf[KT][4];                    // V[key 4g + t][4c .. 4c+3]
+#pragma unroll
+        for (int bi = 0; bi < KT; ++bi)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) vf[bi][t] = *reinterpret_cast<const f32x4*>(V + int64_t(min(16 * (bt + bi) + 4 * g + t, len - 1)) * p.vs_l + 4 * c);
+        issued();
+#pragma unroll
+        for (int te = 0; te < 16; ++te)
+#pragma unroll
+            for (int a = 0; a < QT; ++a) s[a][0] = mfma(kf[0][te >> 2][te & 3], qf[a][te >> 2][te & 3], s[a][0]);
+        if (two) {
+#pragma unroll
+            for (int te = 0; te < 16; ++te)
+#pragma unroll
+                for (int a = 0; a < QT; ++a) s[a][1] = mfma(kf[1][te >> 2][te & 3], qf[a][te >> 2][te & 3], s[a][1]);
+        }
+        if (bt + stride < last) {
+            load_keys(bt + stride);
+            if (PHASES) load_pos(0);
+        }
+        issued();
+        // streaming softmax: this lane has keys 16 bi + 4g + t of query c
+#pragma unroll
+        for (int a = 0; a < QT; ++a) {
+            float mx = -INFINITY;
+#pragma unroll
+            for (int bi = 0; bi < KT; ++bi)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const bool in = (bi == 0 || two) && 16 * (bt + bi) + 4 * g + t < len;
+                    s[a][bi][t] = in ? s[a][bi][t] * p.scale : -INFINITY;
+                    mx = fmaxf(mx, s[a][bi][t]);
+                }
+            const float mn = fmaxf(m_run[a], fold_max(mx));     // finite: the block's first key exists
+            const float alpha = exp_neg(m_run[a] - mn);            // (0 on the first block)
+            float sum = 0.f;
+#pragma unroll
+            for (int bi = 0; bi < KT; ++bi)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    s[a][bi][t] = exp_neg(s[a][bi][t] - mn);
+                    sum += s[a][bi][t];
+                }
+            l_run[a] = l_run[a] * alpha + sum;
+            m_run[a] = mn;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) oacc[a][u] *= alpha;
+        }
+        // O^T[d, q] += V^T P^T: MFMA t contracts keys 4g + t, whose probabilities the lane already holds
+        auto pv = [&](int bi) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int a = 0; a < QT; ++a)
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) oacc[a][u] = mfma(vf[bi][t][u], s[a][bi][t], oacc[a][u]);
+        };
+        pv(0);
+        if (two) pv(1);
+    }
+
+    // Merge of the four waves: partial sums [QT][4][64 lanes] x 16 B, then maxima and denominators of the queries.
+    float* const mine = smem_f + wave * wave_floats(QT);
+    wave_fence();                           // (the scratch above is this wave's own)
+#pragma unroll
+    for (int a = 0; a < QT; ++a) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)         // lane (c, g): d = 16g + 4t + u of query c
+            *reinterpret_cast<f32x4*>(&mine[((a * 4 + t) * 64 + l) * 4]) = f32x4{oacc[a][0][t], oacc[a][1][t], oacc[a][2][t], oacc[a][3][t]};
+        const float l_all = fold_sum(l_run[a]);
+        if (g == 0) {
+            mine[QT * 1024 + a * 32 + c] = m_run[a];
+            mine[QT * 1024 + a * 32 + 16 + c] = l_all;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < QT; ++a) {
+        float f[WAVES], m = -INFINITY, den = 0.f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) m = fmaxf(m, smem_f[w * wave_floats(QT) + QT * 1024 + a * 32 + c]);
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            f[w] = exp_neg(smem_f[w * wave_floats(QT) + QT * 1024 + a * 32 + c] - m);      // (0 for a wave without keys)
+            den += f[w] * smem_f[w * wave_floats(QT) + QT * 1024 + a * 32 + 16 + c];
+        }
+        const int row = row0 + 16 * a + c;
+        const float inv = row < len ? 1.f / den : 0.f;
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4*>(&smem_f[w * wave_floats(QT) + ((a * 4 + wave) * 64 + l) * 4]) * f[w];
+        if (row >= len) sum = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (row < row0 + rows_here) *reinterpret_cast<f32x4*>(O + int64_t(row) * p.os_l + 16 * g + 4 * wave) = sum * inv;
+    }
+}
+
+}  // namespace
+
+bool tdb_f32_supported(const TdbKernelParams& p, int dtype) {
+    return dtype == TDB_F32 && p.D == D && !((p.c2p || p.p2c) && (p.pk || p.pq));
+}
+
+hipError_t tdb_launch_f32(const TdbKernelParams& p, hipStream_t stream) {
+    auto tiles_of = [&](int rows) { return p.varlen ? p.total / rows + p.B : p.B * ((p.L + rows - 1) / rows); };
+    // 32 query rows per workgroup need a tenth fewer products than 16 and half the operand traffic (8 x 512: 160 us against
+    // 200), as long as there are enough workgroups to give every CU its two (2 x 512, 384 of them: 56 us either way).
+    const bool wide = int64_t(tiles_of(32)) * p.H >= 512;
+    const bool strip = p.c2p || p.p2c;
+    const int tiles = tiles_of(wide ? 32 : 16);
+    const int64_t blocks = (int64_t((tiles + 3) / 4) * p.H + 7) / 8 * 32;      // groups of 4 tiles, rounded up to 8 XCDs
+    if (blocks > INT32_MAX) return hipErrorInvalidValue;
+    const dim3 grid{unsigned(blocks)}, block(WAVES * 64);
+    const size_t smem = sizeof(float) * WAVES * wave_floats(wide ? 2 : 1);
+    const bool c2p = strip ? p.c2p != nullptr : p.pk != nullptr, p2c = strip ? p.p2c != nullptr : p.pq != nullptr;
+    auto launch = [&](auto qt, auto s, auto c, auto x) {
+        hipLaunchKernelGGL((attn_f32_kernel<decltype(qt)::value, decltype(s)::value, decltype(c)::value, decltype(x)::value>), grid, block, smem, stream, p, tiles);
+    };
+    using std::bool_constant;
+    auto terms = [&](auto qt) {
+        if (strip && c2p && p2c) launch(qt, bool_constant<true>{}, bool_constant<true>{}, bool_constant<true>{});
+        else if (strip && c2p) launch(qt, bool_constant<true>{}, bool_constant<true>{}, bool_constant<false>{});
+        else if (strip) launch(qt, bool_constant<true>{}, bool_constant<false>{}, bool_constant<true>{});
+        else if (c2p && p2c) launch(qt, bool_constant<false>{}, bool_constant<true>{}, bool_constant<true>{});
+        else if (c2p) launch(qt, bool_constant<false>{}, bool_constant<true>{}, bool_constant<false>{});
+        else if (p2c) launch(qt, bool_constant<false>{}, bool_constant<false>{}, bool_constant<true>{});
+        else launch(qt, bool_constant<false>{}, bool_constant<false>{}, bool_constant<false>{});
+    };
+    if (wide) terms(std::integral_constant<int, 2>{});
+    else terms(std::integral_constant<int, 1>{});
+    return hipGetLastError();
+}

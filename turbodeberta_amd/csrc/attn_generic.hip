@@ -1,7 +1,7 @@
 // Generic disentangled-attention forward: fp32 arithmetic on the vector ALUs for any element
 // type, any head_dim that is a multiple of 8 up to 256, fused tables or precomputed strips.
-// It is the path for fp32 inputs (the 1e-4 parity case) and for shapes the matrix-core kernel
-// does not take.  One wave owns 4 query rows; lanes run over 64 keys at a time.
+// It is the path for what the matrix-core kernels do not take: a head_dim other than 64, and calls
+// that mix a table with a strip.  One wave owns 4 query rows; lanes run over 64 keys at a time.
 //
 //   S[i,j] = scale * ( Q_i.K_j + Q_i.K_r[delta] + K_j.Q_r[delta] ),  delta = lut[i - j + lut_half]
 // as in Hugging Face's DisentangledSelfAttention (modeling_deberta_v2.py:243, :317-324, :337-343),

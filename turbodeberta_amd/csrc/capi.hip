@@ -91,6 +91,8 @@ int dispatch(const TdbKernelParams& kp, int dtype, int flags, void* stream) {
     hipError_t e;
     if (!(flags & TDB_FLAG_FORCE_GENERIC) && tdb_mfma_supported(kp, dtype))
         e = tdb_launch_mfma(kp, dtype, s);
+    else if (!(flags & TDB_FLAG_FORCE_GENERIC) && tdb_f32_supported(kp, dtype))
+        e = tdb_launch_f32(kp, s);
     else
         e = tdb_launch_generic(kp, dtype, s);
     if (e != hipSuccess) return fail(TDB_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));

@@ -36,11 +36,14 @@ struct TdbKernelParams {
 constexpr int TDB_GENERIC_TILE = 16;
 constexpr int TDB_MFMA_TILE = 128;
 
-// true when the matrix-core kernel can take this launch
+// true when the float32 matrix-core kernel can take this launch
+bool tdb_f32_supported(const TdbKernelParams& p, int dtype);
+// true when the 16-bit matrix-core kernel can take this launch
 bool tdb_mfma_supported(const TdbKernelParams& p, int dtype);
 
 // launchers; return hipError_t of the launch
 hipError_t tdb_launch_generic(const TdbKernelParams& p, int dtype, hipStream_t stream);
+hipError_t tdb_launch_f32(const TdbKernelParams& p, hipStream_t stream);
 hipError_t tdb_launch_mfma(const TdbKernelParams& p, int dtype, hipStream_t stream);
 // Cap on the persistent workgroups of a launch (multiple of 8, 0 = none); returns the cap in force.
 int tdb_mfma_set_workgroup_limit(int workgroups);
@@ -94,4 +97,62 @@ __device__ __forceinline__ bool tdb_locate_tile(const TdbKernelParams& p, int ti
         t -= chunk_tiles;
     }
     return false;
+}
+
+// The same map with the sequences taken in order of decreasing length, for up to 64 sequences of different lengths
+// (packed, or a fixed layout with lengths; whole tiles of padding come last): workgroups start in block order, so the
+// long ones start first and the short ones fill the gaps at the end.  A rank per lane (its sequence against every
+// other), one push of the tile counts to their rank, a prefix sum and a ballot; all inside the wave.
+__device__ __forceinline__ bool tdb_locate_tile_sorted(const TdbKernelParams& p, int tile_rows, int block,
+                                                       int& b, int& row0, int& len, int64_t& tok0) {
+    if (p.B > 64 || (!p.varlen && !p.seqlens)) return tdb_locate_tile(p, tile_rows, block, b, row0, len, tok0);
+    const int lane = threadIdx.x & 63;
+    int s = 0, n = 0;
+    if (lane < p.B) {
+        if (p.varlen) {
+            s = p.cu_seqlens[lane];
+            const int e = p.cu_seqlens[lane + 1];
+            n = e - s;
+            if (s < 0 || n < 0 || e > p.total) n = 0;   // malformed entry: no tiles
+            n = min(n, p.L);
+        } else {
+            n = min(max(p.seqlens[lane], 0), p.L);
+        }
+    }
+    int rank = lane >= p.B ? lane : 0;
+    for (int o = 0; o < p.B; ++o) {
+        const int other = __builtin_amdgcn_readlane(n, o);
+        if (lane < p.B) rank += (other > n || (other == n && o < lane)) ? 1 : 0;
+    }
+    const int nt = (n + tile_rows - 1) / tile_rows;
+    auto pick = [&](int count, int t, int& ln, int& within) {   // lane that owns element t of the lanes' counts
+        int incl = count;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int up = __shfl_up(incl, d);
+            if (lane >= d) incl += up;
+        }
+        const unsigned long long owners = __builtin_amdgcn_ballot_w64(incl > t);
+        if (owners == 0) {
+            within = t - __builtin_amdgcn_readlane(incl, 63);   // (what is left of t beyond all counts)
+            return false;
+        }
+        ln = __builtin_amdgcn_readfirstlane(__builtin_ctzll(owners));
+        within = t - (__builtin_amdgcn_readlane(incl, ln) - __builtin_amdgcn_readlane(count, ln));
+        return true;
+    };
+    int ln = 0, within = 0, first = 0;
+    if (pick(__builtin_amdgcn_ds_permute(rank * 4, nt), block, ln, within)) {
+        ln = __builtin_amdgcn_readlane(__builtin_amdgcn_ds_permute(rank * 4, lane), ln);
+    } else {
+        if (p.varlen) return false;
+        const int all = (p.L + tile_rows - 1) / tile_rows;
+        if (!pick(lane < p.B ? all - nt : 0, within, ln, within)) return false;
+        first = __builtin_amdgcn_readlane(nt, ln);
+    }
+    b = ln;
+    row0 = (first + within) * tile_rows;
+    len = __builtin_amdgcn_readlane(n, ln);
+    tok0 = p.varlen ? __builtin_amdgcn_readlane(s, ln) : 0;
+    return true;
 }
