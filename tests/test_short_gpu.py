@@ -1,0 +1,68 @@
+"""The 16-bit kernel for short sequences (up to 128 tokens) at the edges of its units (32 query rows a wave, 64 keys a
+step), against the vector-ALU kernel and bit for bit against the persistent kernel, which a longer maximum selects."""
+import math
+
+import pytest
+import torch
+
+from helpers import assert_close_bf16, make_inputs
+from turbodeberta_amd.ops.flash_attention import flash_attention_with_disentangled
+from turbodeberta_amd.ops.flash_attention_varlen import flash_attention_with_disentangled_varlen
+
+pytestmark = pytest.mark.gpu
+SCALE = 1.0 / math.sqrt(192)
+
+
+def _packed(lens, dtype, terms=("c2p", "p2c"), H=3, seed=0):
+    cu = torch.cat([torch.zeros(1, dtype=torch.long), torch.tensor(lens).cumsum(0)]).int().cuda()
+    d = {n: t.cuda() for n, t in make_inputs(seed, 1, H, max(1, sum(lens)), 64, 256, 512, dtype).items()}
+    q, k, v = (d[n][0].transpose(0, 1).contiguous() for n in "qkv")
+
+    def run(longest, **kw):
+        return flash_attention_with_disentangled_varlen(q, k, v, None, None, cu, cu, longest, longest, False, SCALE, 256, 512,
+                                                        pos_key_layer=d["pk"] if "c2p" in terms else None,
+                                                        pos_query_layer=d["pq"] if "p2c" in terms else None, **kw)
+    return run
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("L", [1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128])
+def test_fixed_edges(L, dtype):
+    d = {n: t.cuda() for n, t in make_inputs(L, 2, 3, L, 64, 256, 512, dtype).items()}
+    got, ref = (flash_attention_with_disentangled(d["q"], d["k"], d["v"], None, None, False, SCALE, 256, 512, pos_key_layer=d["pk"],
+                                                  pos_query_layer=d["pq"], force_generic=f) for f in (False, True))
+    assert_close_bf16(got, ref, f"L={L}")
+
+
+@pytest.mark.parametrize("terms", [("c2p", "p2c"), ("c2p",), ("p2c",), ()])
+@pytest.mark.parametrize("lens", [[1], [30, 2, 33, 64], [16, 40] * 32, [5, 0, 96, 31, 70] * 20, [128, 1, 65, 100] * 25, [3, 9, 17] * 60],
+                         ids=["one", "four", "64_with_single_tiles", "100", "100_to_128", "180_tiny"])
+def test_packed_same_bits_as_the_persistent_kernel(lens, terms):
+    run = _packed(lens, torch.bfloat16, terms)
+    got = run(max(lens))
+    assert torch.equal(got, run(129))
+    assert_close_bf16(got, run(max(lens), force_generic=True), str(terms))
+
+
+@pytest.mark.parametrize("B,L", [(3, 50), (64, 64), (90, 128), (1, 128)])
+def test_lengths_and_padding(B, L):
+    d = {n: t.cuda() for n, t in make_inputs(B, B, 4, L, 64, 256, 512, torch.bfloat16).items()}
+    lens = torch.randint(0, L + 1, (B,), generator=torch.Generator().manual_seed(B)).int()
+    lens[0] = 0 if B > 1 else 40
+    got, ref = (flash_attention_with_disentangled(d["q"], d["k"], d["v"], None, None, False, SCALE, 256, 512, pos_key_layer=d["pk"],
+                                                  pos_query_layer=d["pq"], seqlens_k=lens.cuda(), force_generic=f) for f in (False, True))
+    assert_close_bf16(got, ref, f"{B} x {L}")
+    assert all(not got[b, :, n:].any() for b, n in enumerate(lens.tolist()))
+
+
+def test_rows_follow_their_own_maximum():
+    # scores that grow along the keys raise the running maximum of some rows only: same bits in both kernels
+    d = {n: t.cuda() for n, t in make_inputs(1, 2, 3, 128, 64, 256, 512, torch.bfloat16).items()}
+    d["k"] *= torch.linspace(0.1, 12, 128, device="cuda")[None, None, :, None]
+    d["q"] *= torch.linspace(0.1, 3, 128, device="cuda")[None, None, :, None]
+    pos = dict(pos_key_layer=d["pk"], pos_query_layer=d["pq"])
+    got = flash_attention_with_disentangled(d["q"], d["k"], d["v"], None, None, False, SCALE, 256, 512, **pos)
+    wide = [torch.cat([d[n], d[n][:, :, :1]], 2) for n in "qkv"]                   # one row more, masked by its length
+    lens = torch.tensor([128, 128], dtype=torch.int32, device="cuda")
+    ref = flash_attention_with_disentangled(*wide, None, None, False, SCALE, 256, 512, seqlens_k=lens, **pos)
+    assert torch.equal(got, ref[:, :, :128])

@@ -145,6 +145,7 @@ __device__ __forceinline__ void phase_barrier() {
 // into vector lanes and reloaded in the step loops) and several hundred scalar instructions per tile.
 template <bool HAS_C2P, bool HAS_P2C, int DT, bool FARZ, bool VARLEN, bool STRIP = false>
 __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelParams p, const int nblocks) {
+#pragma clang fp contract(off)              // (products and sums are fused only where it says so: attn_short.hip has to give the same bits)
     static_assert(!(STRIP && FARZ), "the strip instances have no far steps");
     using E = Elem<DT>;
     using ET = typename E::T;
@@ -1143,18 +1144,20 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
             both_halves(mx, own_or_partner, partner_or_own);
             mx = fmaxf(own_or_partner, partner_or_own) + cadd;
         }
-        // The running maximum is only raised (and the accumulators rescaled) when some row of the wave exceeds it
-        // by more than 2^8; until then probabilities of this step may be as large as 256, which bf16 and the fp32
-        // sums carry exactly as well.  (First step: m_run = -inf always triggers, alpha = 0.)
+        // The running maximum of a row is only raised (and its accumulators rescaled) when the row exceeds it by more than
+        // 2^8; until then probabilities of this step may be as large as 256, which bf16 and the fp32 sums carry exactly
+        // as well.  (First step: m_run = -inf always triggers, alpha = 0.)  The rows of a wave decide separately, so that
+        // a row's result does not depend on its neighbours in the tile (the kernel for short sequences has others).
         const float m_new = fmaxf(m_run, mx);          // finite: key 64s < len is never masked
-        if (__builtin_amdgcn_ballot_w64((m_new - m_run) * c_exp > 8.f) != 0) {
-            const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * c_exp);
+        const bool raise = (m_new - m_run) * c_exp > 8.f;
+        if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+            const float alpha = raise ? __builtin_amdgcn_exp2f((m_run - m_new) * c_exp) : 1.f;
             l_run *= alpha;
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) o_acc[t][e] *= alpha;
-            m_run = m_new;
+            m_run = raise ? m_new : m_run;
         }
         const float mc = (m_run - cadd) * c_exp;
         float psum = 0.f;

@@ -89,7 +89,9 @@ void fill_pos(TdbKernelParams& kp, const tdb_pos_args& ps) {
 int dispatch(const TdbKernelParams& kp, int dtype, int flags, void* stream) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     hipError_t e;
-    if (!(flags & TDB_FLAG_FORCE_GENERIC) && tdb_mfma_supported(kp, dtype))
+    if (!(flags & TDB_FLAG_FORCE_GENERIC) && tdb_short_supported(kp, dtype))
+        e = tdb_launch_short(kp, dtype, s);
+    else if (!(flags & TDB_FLAG_FORCE_GENERIC) && tdb_mfma_supported(kp, dtype))
         e = tdb_launch_mfma(kp, dtype, s);
     else if (!(flags & TDB_FLAG_FORCE_GENERIC) && tdb_f32_supported(kp, dtype))
         e = tdb_launch_f32(kp, s);

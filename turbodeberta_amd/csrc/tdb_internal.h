@@ -35,14 +35,19 @@ struct TdbKernelParams {
 // tile heights (query rows per workgroup)
 constexpr int TDB_GENERIC_TILE = 16;
 constexpr int TDB_MFMA_TILE = 128;
+constexpr int TDB_SHORT_TILE = 32;     // per wave
 
 // true when the float32 matrix-core kernel can take this launch
 bool tdb_f32_supported(const TdbKernelParams& p, int dtype);
 // true when the 16-bit matrix-core kernel can take this launch
 bool tdb_mfma_supported(const TdbKernelParams& p, int dtype);
 
+// true when the 16-bit kernel for short sequences can take this launch
+bool tdb_short_supported(const TdbKernelParams& p, int dtype);
+
 // launchers; return hipError_t of the launch
 hipError_t tdb_launch_generic(const TdbKernelParams& p, int dtype, hipStream_t stream);
+hipError_t tdb_launch_short(const TdbKernelParams& p, int dtype, hipStream_t stream);
 hipError_t tdb_launch_f32(const TdbKernelParams& p, hipStream_t stream);
 hipError_t tdb_launch_mfma(const TdbKernelParams& p, int dtype, hipStream_t stream);
 // Cap on the persistent workgroups of a launch (multiple of 8, 0 = none); returns the cap in force.
