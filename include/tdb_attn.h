@@ -42,6 +42,8 @@ extern "C" {
 
 /* bits of the `flags` field */
 #define TDB_FLAG_FORCE_GENERIC 1  /* run the vector-ALU kernel even where the matrix-core kernel applies */
+#define TDB_FLAG_ZERO_UNCOVERED 2 /* packed calls: rows of o that belong to no sequence (or lie beyond max_seqlen) are
+                                     written as zeros; without it they are left as they are */
 
 /*
  * Position inputs shared by both entry points.  Two modes, chosen per term:

@@ -66,3 +66,23 @@ def test_rows_follow_their_own_maximum():
     lens = torch.tensor([128, 128], dtype=torch.int32, device="cuda")
     ref = flash_attention_with_disentangled(*wide, None, None, False, SCALE, 256, 512, seqlens_k=lens, **pos)
     assert torch.equal(got, ref[:, :, :128])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("cu,longest", [([0, 20, 50], 30), ([3, 20, 50], 30), ([0, 20, 50], 12), ([0, 200, 230], 200), ([0, 200, 205], 150),
+                                        ([5] + list(range(5, 230, 3)), 3), ([0], 4)])
+def test_rows_outside_every_sequence_are_zeros(cu, longest, dtype):
+    T = 260
+    d = {n: t.cuda() for n, t in make_inputs(9, 1, 3, T, 64, 256, 512, dtype).items()}
+    q, k, v = (d[n][0].transpose(0, 1).contiguous() for n in "qkv")
+    c = torch.tensor(cu, dtype=torch.int32, device="cuda")
+    junk = torch.full((64 << 20,), float("nan"), device="cuda")           # what a fresh allocation finds
+    del junk
+    run = lambda **kw: flash_attention_with_disentangled_varlen(q, k, v, None, None, c, c, longest, longest, False, SCALE, 256, 512,
+                                                                pos_key_layer=d["pk"], pos_query_layer=d["pq"], **kw)
+    out, ref = run(), run(force_generic=True)
+    inside = torch.zeros(T, dtype=torch.bool)
+    for a, b in zip(cu, cu[1:]):
+        inside[a:min(b, a + longest)] = True
+    assert not out[~inside.cuda()].any() and not ref[~inside.cuda()].any()
+    assert_close_bf16(out, ref)

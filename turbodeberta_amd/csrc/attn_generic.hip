@@ -207,7 +207,16 @@ __global__ __launch_bounds__(WAVES * 64) void attn_generic_kernel(const TdbKerne
     }
 }
 
+__global__ __launch_bounds__(64) void zero_gaps_kernel(const TdbKernelParams p, const int elem) {
+    tdb_fill_gaps(p.gap_cu, p.gap_B, p.L, p.total, static_cast<char*>(p.o), p.os_l * elem, p.os_h * elem, p.H, p.D * elem, blockIdx.x, gridDim.x);
+}
+
 }  // namespace
+
+hipError_t tdb_zero_gaps(const TdbKernelParams& p, int dtype, hipStream_t stream) {
+    hipLaunchKernelGGL(zero_gaps_kernel, dim3(256), dim3(64), 0, stream, p, dtype == TDB_F32 ? 4 : 2);
+    return hipGetLastError();
+}
 
 hipError_t tdb_launch_generic(const TdbKernelParams& p, int dtype, hipStream_t stream) {
     const int tiles = p.varlen ? p.total / TDB_GENERIC_TILE + p.B

@@ -253,6 +253,8 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
             sm.seq_pre[l] = cnt;
         }
     }
+    if (VARLEN && p.gap_cu && wave == 7)
+        tdb_fill_gaps(p.gap_cu, p.gap_B, p.L, p.total, static_cast<char*>(p.o), p.os_l * 2, p.os_h * 2, p.H, 2 * D, blockIdx.x, gridDim.x);
     // fixed layout: tile_id -> (sequence, first row, valid length); same map as tdb_locate_tile
     auto locate = [&](int tile_id, int& bb, int& r0, int& ln, int64_t& t0) {
         const int tiles = (p.L + BM - 1) / BM;
@@ -1348,6 +1350,7 @@ hipError_t tdb_launch_mfma(const TdbKernelParams& whole, int dtype, hipStream_t 
         const int parts = (whole.B + 63) / 64, per = (whole.B + parts - 1) / parts;
         for (int first = 0; first < whole.B; first += per) {
             TdbKernelParams part = whole;
+            if (first > 0) part.gap_cu = nullptr;
             if (whole.cu_seqlens) {
                 part.cu_seqlens = whole.cu_seqlens + first;
             } else {                      // a padded batch dealt like packed sequences (below): the part starts `first` sequences in

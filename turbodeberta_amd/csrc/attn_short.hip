@@ -120,6 +120,7 @@ struct ShortArgs {
     int32_t T, tshift;                      // units of a sequence: tiles 0 .. T-1 of 2^tshift numbers
     int32_t waves;                          // per workgroup
     int32_t single;                         // every unit has a wave of its own
+    int32_t gaps;                           // packed: zeros for the rows outside every sequence
 };
 enum { FIXED = 0, LENGTHS = 1, PACKED = 2 };
 
@@ -258,6 +259,9 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void attn_short_kernel(const ShortA
             }
         __syncthreads();
     }
+
+    if (MODE == PACKED && p.gaps && wave == p.waves - 1)
+        tdb_fill_gaps(p.bounds, p.B, p.L, p.total, p.o, p.ol, p.oh, gridDim.x, 2 * D, wg * gridDim.x + h, gridDim.x * per_head);
 
     const float c_exp = p.c_exp;
     const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -532,6 +536,7 @@ hipError_t tdb_launch_short(const TdbKernelParams& p, int dtype, hipStream_t str
     const int per_head = std::min(p.B, std::max(1, cus / p.H));
     const int units = (p.B + per_head - 1) / per_head << a.tshift;
     const int waves = std::min(MAX_WAVES, std::max(std::max(4, 2 * a.T), units));
+    a.gaps = p.gap_cu != nullptr;
     a.waves = waves, a.single = units <= waves;
     const size_t smem = 16 + (int(c2p) + int(p2c)) * size_t(2 * UQ * a.T * RS * 2) + size_t(waves) * SCRATCH;
     void* args[] = {&a};

@@ -88,15 +88,16 @@ void fill_pos(TdbKernelParams& kp, const tdb_pos_args& ps) {
 
 int dispatch(const TdbKernelParams& kp, int dtype, int flags, void* stream) {
     hipStream_t s = static_cast<hipStream_t>(stream);
-    hipError_t e;
-    if (!(flags & TDB_FLAG_FORCE_GENERIC) && tdb_short_supported(kp, dtype))
+    hipError_t e = hipSuccess;
+    const bool any = !(flags & TDB_FLAG_FORCE_GENERIC);
+    if (any && tdb_short_supported(kp, dtype)) {
         e = tdb_launch_short(kp, dtype, s);
-    else if (!(flags & TDB_FLAG_FORCE_GENERIC) && tdb_mfma_supported(kp, dtype))
+    } else if (any && tdb_mfma_supported(kp, dtype)) {
         e = tdb_launch_mfma(kp, dtype, s);
-    else if (!(flags & TDB_FLAG_FORCE_GENERIC) && tdb_f32_supported(kp, dtype))
-        e = tdb_launch_f32(kp, s);
-    else
-        e = tdb_launch_generic(kp, dtype, s);
+    } else {
+        if (kp.gap_cu) e = tdb_zero_gaps(kp, dtype, s);     // (the other kernels do this themselves)
+        if (e == hipSuccess) e = any && tdb_f32_supported(kp, dtype) ? tdb_launch_f32(kp, s) : tdb_launch_generic(kp, dtype, s);
+    }
     if (e != hipSuccess) return fail(TDB_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
     return TDB_OK;
 }
@@ -223,6 +224,7 @@ int tdb_attn_fwd_varlen(const tdb_varlen_args* a, void* stream) {
     kp.B = a->batch; kp.H = a->heads; kp.D = a->head_dim; kp.L = a->max_seqlen;
     kp.total = a->total_tokens;
     kp.varlen = 1;
+    if (a->flags & TDB_FLAG_ZERO_UNCOVERED) kp.gap_cu = a->cu_seqlens, kp.gap_B = a->batch;
     kp.scale = a->sm_scale;
     fill_pos(kp, a->pos);
     return dispatch(kp, a->dtype, a->flags, stream);

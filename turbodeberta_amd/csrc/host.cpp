@@ -262,10 +262,10 @@ PyObject* py_varlen(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         if (!as_scale(args[10], D, a.sm_scale) || !fill_pos(a.pos, c, H, D, a.max_seqlen)) Py_RETURN_NONE;
         at::Tensor o;
         if (!output_like(q, o)) Py_RETURN_NONE;
-        if (zero) o.zero_();
+        if (zero && cu->size(0) == 1) o.zero_();       // (no sequence: nothing is launched)
         a.dtype = dtype_code(q.scalar_type());
         a.batch = int32_t(cu->size(0) - 1), a.heads = int32_t(H), a.head_dim = int32_t(D), a.total_tokens = int32_t(T);
-        a.flags = generic ? TDB_FLAG_FORCE_GENERIC : 0;
+        a.flags = (generic ? TDB_FLAG_FORCE_GENERIC : 0) | (zero ? TDB_FLAG_ZERO_UNCOVERED : 0);
         a.q = q.data_ptr(), a.k = k.data_ptr(), a.v = v.data_ptr(), a.o = o.data_ptr();
         a.q_stride_t = q.stride(0), a.q_stride_h = q.stride(1);
         a.k_stride_t = k.stride(0), a.k_stride_h = k.stride(1);

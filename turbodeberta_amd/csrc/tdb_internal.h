@@ -18,6 +18,8 @@ struct TdbKernelParams {
     int64_t os_b, os_h, os_l;
     const int32_t* seqlens;     // fixed: [B] valid lengths or nullptr
     const int32_t* cu_seqlens;  // packed: [B+1] or nullptr
+    const int32_t* gap_cu;      // packed: the call's whole cu_seqlens if rows outside every sequence are to be zeroed, or nullptr
+    int32_t gap_B;              // and its batch
     int32_t B, H, D, L;         // L: padded length (fixed) / max_seqlen (packed)
     int32_t total;              // packed: token count
     int32_t varlen;
@@ -47,6 +49,7 @@ bool tdb_short_supported(const TdbKernelParams& p, int dtype);
 
 // launchers; return hipError_t of the launch
 hipError_t tdb_launch_generic(const TdbKernelParams& p, int dtype, hipStream_t stream);
+hipError_t tdb_zero_gaps(const TdbKernelParams& p, int dtype, hipStream_t stream);     // a launch of its own
 hipError_t tdb_launch_short(const TdbKernelParams& p, int dtype, hipStream_t stream);
 hipError_t tdb_launch_f32(const TdbKernelParams& p, hipStream_t stream);
 hipError_t tdb_launch_mfma(const TdbKernelParams& p, int dtype, hipStream_t stream);
@@ -160,4 +163,32 @@ __device__ __forceinline__ bool tdb_locate_tile_sorted(const TdbKernelParams& p,
     len = __builtin_amdgcn_readlane(n, ln);
     tok0 = p.varlen ? __builtin_amdgcn_readlane(s, ln) : 0;
     return true;
+}
+
+// Zeros for the rows of a packed output that belong to no sequence: in front of, between and behind them, and what
+// max_seqlen cuts off.  One wave of each of `workers` workgroups runs this beside the attention itself (a fill of the whole
+// output by a launch of its own took 12 us in front of a 91 us call).  Packings without gaps, all but a few, end after one
+// look at the boundaries, 64 at a time.
+__device__ __forceinline__ void tdb_fill_gaps(const int32_t* cu, int B, int L, int total, char* o, int64_t row_bytes,
+                                              int64_t head_bytes, int heads, int head_dim_bytes, int worker, int workers) {
+    const int lane = threadIdx.x & 63;
+    bool exact = true;
+    for (int b0 = 0; b0 < B; b0 += 64) {
+        const int b = min(b0 + lane, B - 1);
+        const int lo = cu[b], hi = cu[b + 1];
+        exact = exact && lo >= 0 && hi >= lo && hi <= total && hi - lo <= L && (b > 0 || lo == 0) && (b < B - 1 || hi == total);
+    }
+    if (__builtin_amdgcn_ballot_w64(!exact) == 0) return;
+    for (int row = worker; row < total; row += workers) {
+        bool mine = false;
+        for (int b0 = 0; b0 < B; b0 += 64) {
+            const int b = min(b0 + lane, B - 1);
+            const int lo = cu[b], hi = cu[b + 1];
+            mine = mine || (lo >= 0 && hi >= lo && hi <= total && row >= lo && row < lo + min(hi - lo, L));
+        }
+        if (__builtin_amdgcn_ballot_w64(mine) != 0) continue;
+        const int per_head = head_dim_bytes / 16;
+        for (int idx = lane; idx < heads * per_head; idx += 64)
+            *reinterpret_cast<uint4*>(o + row * row_bytes + (idx / per_head) * head_bytes + (idx % per_head) * 16) = uint4{0, 0, 0, 0};
+    }
 }
