@@ -1,0 +1,116 @@
+"""The native encoder loop against the same model's modules: token counts at the edges of its 16-row tiles and on both sides
+of its own products, packed and full batches, and what makes it step aside."""
+import copy
+
+import pytest
+import torch
+from transformers import DebertaV2Config
+
+from turbodeberta_amd import _lib
+from turbodeberta_amd.model import FlashDebertaV2Model, _native_plan
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(dtype, hidden=128, heads=2, layers=2, inner=256):
+    torch.manual_seed(0)
+    cfg = DebertaV2Config(vocab_size=500, hidden_size=hidden, num_hidden_layers=layers, num_attention_heads=heads, intermediate_size=inner,
+                          max_position_embeddings=512, type_vocab_size=0, relative_attention=True, position_buckets=256,
+                          max_relative_positions=512, share_att_key=True, pos_att_type=["c2p", "p2c"], norm_rel_ebd="layer_norm",
+                          position_biased_input=False, layer_norm_eps=1e-7, initializer_range=0.1)
+    model = FlashDebertaV2Model(cfg)
+    with torch.no_grad():
+        for n, p in model.named_parameters():
+            if n.endswith("bias"):
+                p.normal_(std=0.1)
+    return model.to(device="cuda", dtype=dtype).eval()
+
+
+def _ids(lens, L):
+    ids = torch.randint(1, 500, (len(lens), L), generator=torch.Generator().manual_seed(L))
+    for b, n in enumerate(lens):
+        ids[b, n:] = 0
+    return ids.cuda(), (ids != 0).long().cuda()
+
+
+def _both(model, ids, mask):
+    with torch.no_grad():
+        fast = model._forward_native(ids, mask)
+        model.encoder.pack_sequences = False
+        slow = model(input_ids=ids, attention_mask=mask).last_hidden_state
+        model.encoder.pack_sequences = True
+        assert fast is not None
+    return fast, slow
+
+
+TOL = {torch.float32: 1e-5, torch.bfloat16: 2e-2, torch.float16: 3e-3}
+
+
+def _check(fast, slow, mask, dtype):
+    v = mask.bool()
+    a, b = fast[v].double(), slow[v].double()
+    assert ((a - b).norm() / b.norm()).item() <= TOL[dtype]
+    assert not fast[~v].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("lens,L", [([1], 1), ([15], 15), ([17], 17), ([48], 48), ([64], 64), ([65], 65), ([97], 97), ([128], 128), ([129], 129),
+                                    ([100, 3, 40], 100), ([256, 256], 256), ([200, 300, 13], 300)])
+def test_equals_the_modules(lens, L, dtype):
+    ids, mask = _ids(lens, L)
+    _check(*_both(_model(dtype), ids, mask), mask, dtype)
+
+
+@pytest.mark.parametrize("hidden,heads,inner", [(768, 12, 3072), (1024, 16, 4096), (64, 1, 96), (1536, 24, 128)])
+@pytest.mark.parametrize("lens,L", [([40], 40), ([300, 310, 20], 310)])
+def test_widths(hidden, heads, inner, lens, L):
+    ids, mask = _ids(lens, L)
+    _check(*_both(_model(torch.bfloat16, hidden, heads, 1, inner), ids, mask), mask, torch.bfloat16)
+
+
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32, torch.bool, torch.float32, torch.bfloat16])
+def test_mask_scan(dtype):
+    lens = torch.randint(0, 90, (70,), generator=torch.Generator().manual_seed(1)).int()
+    mask = (torch.arange(90)[None] < lens[:, None]).to(dtype).cuda()
+    got, cu, ok, total, ones = _lib.host().scan_mask(mask)
+    assert ok and ones and total == int(lens.sum()) and torch.equal(got.cpu(), lens)
+    assert torch.equal(cu.cpu(), torch.cat([torch.zeros(1, dtype=torch.int64), lens.cumsum(0)]).int())
+    holes = mask.clone()
+    holes[3] = 0
+    holes[3, 5] = 1
+    assert not _lib.host().scan_mask(holes)[2]
+    if dtype != torch.bool:
+        assert not _lib.host().scan_mask(mask * 2)[4]
+
+
+def test_steps_aside_and_comes_back():
+    model = _model(torch.bfloat16)
+    ids, mask = _ids([30, 7], 30)
+    dense = model.encoder.layer[1].output.dense
+    with torch.no_grad():
+        assert model._forward_native(ids, mask) is not None
+        plan = _native_plan(model)
+        assert _native_plan(model) is plan
+        hook = dense.register_forward_hook(lambda m, i, o: o)
+        assert _native_plan(model) is None
+        hook.remove()
+        assert _native_plan(model) is not None
+        model.encoder.layer[0].output.dropout.train()
+        assert _native_plan(model) is None
+        model.eval()
+        first = model._forward_native(ids, mask)
+        dense.weight.mul_(1.5)
+        second = model._forward_native(ids, mask)
+        assert not torch.equal(first, second)
+        _check(*_both(model, ids, mask), mask, torch.bfloat16)
+        dense.forward = lambda x: x
+        assert _native_plan(model) is None
+        del dense.forward
+        model.encoder.layer[1].output.dense = torch.nn.Linear(256, 128).to("cuda", torch.bfloat16).eval()
+        _check(*_both(model, ids, mask), mask, torch.bfloat16)
+        assert model._forward_native(ids, mask * 2) is None                    # the embeddings are scaled by such a mask
+        with torch.autocast("cuda", torch.bfloat16):
+            assert model._forward_native(ids, mask) is None
+        twin = copy.deepcopy(model)
+        assert torch.equal(twin._forward_native(ids, mask), model._forward_native(ids, mask))
+    assert model._forward_native(ids, mask) is None                            # gradients on

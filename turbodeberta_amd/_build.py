@@ -13,7 +13,7 @@ ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 LIB_PATH = os.path.join(PKG, "libtdb_attn.so")
 HOST_PATH = os.path.join(PKG, "_host.so")
-SOURCES = ("capi.hip", "attn_generic.hip", "attn_f32.hip", "attn_short.hip", "attn_mfma.hip")
+SOURCES = ("capi.hip", "attn_generic.hip", "attn_f32.hip", "attn_short.hip", "encoder.hip", "attn_mfma.hip")
 
 # packed-fp32 VALU forms are switched off for every device compile
 HIPCC_FLAGS = [
@@ -50,12 +50,12 @@ def _compile_host() -> str:
     cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wno-attributes",
            "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            *(f for d in include_paths() + [sysconfig.get_paths()["include"]] for f in ("-isystem", d)),
-           "-isystem", os.path.join(rocm, "include"), "-I", os.path.join(ROOT, "include"),
-           os.path.join(CSRC, "host.cpp"), "-o", tmp, "-L", os.path.join(os.path.dirname(torch.__file__), "lib"),
+           "-isystem", os.path.join(rocm, "include"), "-I", os.path.join(ROOT, "include"), "-I", CSRC,
+           *(os.path.join(CSRC, f) for f in ("host.cpp", "host_encoder.cpp")), "-o", tmp, "-L", os.path.join(os.path.dirname(torch.__file__), "lib"),
            "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        raise RuntimeError(f"g++ failed on host.cpp:\n{res.stderr[-4000:]}")
+        raise RuntimeError(f"g++ failed on the host module:\n{res.stderr[-4000:]}")
     os.replace(tmp, HOST_PATH)
     return HOST_PATH
 

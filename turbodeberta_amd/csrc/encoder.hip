@@ -1,0 +1,440 @@
+// The kernels around attention in an encoder layer: embeddings, residual + LayerNorm, products with few rows, mask scan,
+// unpacking.  Large products stay with the library; what is here is bound by memory traffic or by latency:
+//   * residual + LayerNorm in one pass, a wave per row with the row in registers: three arrays of traffic instead of five.
+//   * products with at most 128 rows (a single text): the library takes 8-10 us for 48 x 768 x 768 where the weights are
+//     read in well under one.  Here a workgroup takes 16 output columns and its waves share out the contraction, so that all
+//     of the weight matrix is requested at once; sums of the waves meet in LDS.  Where the output has too few columns to
+//     fill the chip (hidden-sized ones), the contraction is split over workgroups as well, and the residual + LayerNorm
+//     that follows adds the parts up in a fixed order.
+#include <type_traits>
+
+#include "tdb_encoder.h"
+#include "tdb_internal.h"
+
+namespace {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+template <int DT>
+struct Elem;
+template <>
+struct Elem<TDB_BF16> {
+    using T = __bf16;
+    using X8 = bf16x8;
+    static __device__ __forceinline__ f32x4 mfma(X8 a, X8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+};
+template <>
+struct Elem<TDB_F16> {
+    using T = _Float16;
+    using X8 = f16x8;
+    static __device__ __forceinline__ f32x4 mfma(X8 a, X8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+};
+template <>
+struct Elem<TDB_F32> {
+    using T = float;
+};
+
+constexpr int MAX_SPLITS = 8;
+
+// eight consecutive elements as float32, and back
+template <int DT>
+__device__ __forceinline__ void load8(const void* p, int64_t at, float (&v)[8]) {
+    using T = typename Elem<DT>::T;
+    typedef __attribute__((ext_vector_type(8))) T T8;
+    const T8 x = *reinterpret_cast<const T8*>(static_cast<const T*>(p) + at);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = float(x[i]);
+}
+template <int DT>
+__device__ __forceinline__ void store8(void* p, int64_t at, const float (&v)[8]) {
+    using T = typename Elem<DT>::T;
+    typedef __attribute__((ext_vector_type(8))) T T8;
+    T8 x;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = T(v[i]);
+    *reinterpret_cast<T8*>(static_cast<T*>(p) + at) = x;
+}
+
+// Rows of activations, in element offsets of chunk `chunk` (eight columns) of row t.  mt = 0: row after row.  mt > 0, used
+// between the kernels of a short call: in the order in which the products load them -- 32 columns x 16 rows after another,
+// mt of them per 32 columns --, so that a load instruction covers 1 KB in one piece.  (In row order its 64 lanes touch 16 rows,
+// consecutive lanes different ones, and it occupies the CU's load path for 54 clk instead of 16: 48 x 3072 x 768 6.1 us.)
+__device__ __forceinline__ int64_t row_at(int t, int chunk, int hidden, int mt) {
+    return mt == 0 ? int64_t(t) * hidden + chunk * 8 : int64_t((((chunk >> 2) * mt + (t >> 4)) * 64 + (chunk & 3) * 16 + (t & 15)) * 8);
+}
+
+__device__ __forceinline__ float wave_sum(float x) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+    return x;
+}
+
+// LayerNorm of a row held by a wave: lane l has the chunks of eight l, l + 64, ...; chunks past the row hold zeros.
+// (The caller loads the scale and shift with the row: behind the sums they would be another round trip.)
+template <int DT, int CH>
+__device__ __forceinline__ void load_affine(float (&w)[CH][8], float (&b)[CH][8], int chunks, const void* gamma, const void* beta) {
+    const int l = threadIdx.x & 63;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const int el = min(l + 64 * c, chunks - 1) * 8;
+        load8<DT>(gamma, el, w[c]);
+        load8<DT>(beta, el, b[c]);
+    }
+}
+template <int DT, int CH>
+__device__ __forceinline__ void norm_row(float (&v)[CH][8], const float (&w)[CH][8], const float (&b)[CH][8], int chunks, int hidden, float eps,
+                                         void* out, int t, int mt) {
+    const int l = threadIdx.x & 63;
+    float sum = 0.f;
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sum += v[c][i];
+    const float mean = wave_sum(sum) / float(hidden);
+    float sq = 0.f;
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+        if (l + 64 * c < chunks) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float d = v[c][i] - mean;
+                sq += d * d;
+            }
+        }
+    const float rstd = rsqrtf(wave_sum(sq) / float(hidden) + eps);
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+        if (l + 64 * c < chunks) {
+            float y[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) y[i] = (v[c][i] - mean) * rstd * w[c][i] + b[c][i];
+            store8<DT>(out, row_at(t, l + 64 * c, hidden, mt), y);
+        }
+}
+
+template <int DT, int CH>
+__global__ __launch_bounds__(256) void embed_kernel(const void* ids, int ids64, const void* table, int64_t vocab, const void* gamma,
+                                                    const void* beta, float eps, const int32_t* cu, int B, int L, int T, int hidden,
+                                                    int mt, void* out) {
+    const int t = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63, chunks = hidden / 8;
+    if (t >= T) return;
+    int64_t at = t;
+    if (cu) {                               // packed token t: the sequence b with cu[b] <= t < cu[b+1]
+        int lo = 0, hi = B;
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (cu[mid] <= t) lo = mid;
+            else hi = mid;
+        }
+        at = int64_t(lo) * L + (t - cu[lo]);
+    }
+    const int64_t id = ids64 ? static_cast<const int64_t*>(ids)[at] : static_cast<const int32_t*>(ids)[at];
+    const bool ok = id >= 0 && id < vocab;
+    float v[CH][8], w[CH][8], b[CH][8];
+    load_affine<DT, CH>(w, b, chunks, gamma, beta);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[c][i] = 0.f;
+        if (l + 64 * c < chunks) {
+            if (ok) load8<DT>(table, id * hidden + (l + 64 * c) * 8, v[c]);
+            else v[c][0] = __builtin_nanf("");          // an id outside the table: the row says so
+        }
+    }
+    norm_row<DT, CH>(v, w, b, chunks, hidden, eps, out, t, mt);
+}
+
+template <int DT, int CH, bool PARTS>
+__global__ __launch_bounds__(256) void add_norm_kernel(const void* x, int splits, const void* bias, const void* residual, const void* gamma,
+                                                       const void* beta, float eps, int T, int hidden, int mt_in, int mt_out, void* out) {
+    const int t = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63, chunks = hidden / 8;
+    if (t >= T) return;
+    const int64_t at = int64_t(t) * hidden;
+    float v[CH][8], w[CH][8], b[CH][8];
+    load_affine<DT, CH>(w, b, chunks, gamma, beta);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[c][i] = 0.f;
+        const int el = (l + 64 * c) * 8;
+        if (l + 64 * c < chunks) {
+            float r[8];
+            load8<DT>(residual, row_at(t, l + 64 * c, hidden, mt_in), r);
+            if (PARTS) {
+                float y[MAX_SPLITS][8], add[8];             // all requested before the first is added; past the last: it again
+#pragma unroll
+                for (int s = 0; s < MAX_SPLITS; ++s) load8<TDB_F32>(x, int64_t(min(s, splits - 1)) * T * hidden + at + el, y[s]);
+                load8<DT>(bias, el, add);
+#pragma unroll
+                for (int s = 0; s < MAX_SPLITS; ++s)
+                    if (s < splits) {
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) v[c][i] += y[s][i];
+                    }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[c][i] += add[i];
+            } else {
+                load8<DT>(x, at + el, v[c]);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[c][i] += r[i];
+        }
+    }
+    norm_row<DT, CH>(v, w, b, chunks, hidden, eps, out, t, mt_out);
+}
+
+// One workgroup: 16 columns of the output, a share of the contraction given by blockIdx.y and, inside it, by the wave.
+// MT: token tiles of 16, the block of them given by blockIdx.z.  Lane (c, g) has 16 bytes of weight row n0 + c and of token row 16 m + c: columns 32 k + 8 g .. +7.
+// IN / OUT: x / y in the order of row_at with mt tiles in all.
+template <int DT, int MT, bool IN, bool OUT, bool GELU, bool PART>
+__global__ __launch_bounds__(512) void small_gemm_kernel(const void* xv, const void* wv, const void* bias, void* y, int M, int N, int K, int mt, int splits) {
+    using E = Elem<DT>;
+    using X8 = typename E::X8;
+    using T = typename E::T;
+    extern __shared__ __attribute__((aligned(16))) float red[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6, l = threadIdx.x & 63;
+    const int c = l & 15, g = l >> 4, n0 = blockIdx.x * 16, steps = K / 32, tile0 = blockIdx.z * MT;
+    const int parts = splits * waves, part = blockIdx.y * waves + wave;
+    const int k0 = steps * part / parts, k1 = steps * (part + 1) / parts;
+    const T* const w = static_cast<const T*>(wv) + int64_t(n0 + c) * K + 8 * g;
+    const T* x[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) x[m] = static_cast<const T*>(xv) + (IN ? (tile0 + m) * 512 + l * 8 : min(16 * (tile0 + m) + c, M - 1) * K + 8 * g);
+    typedef __attribute__((ext_vector_type(4))) T T4;
+    const int col = n0 + 4 * g;             // (of every element this thread sums up below)
+    T4 b4;
+    if (!PART) b4 = *reinterpret_cast<const T4*>(static_cast<const T*>(bias) + col);
+    f32x4 acc[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto run = [&](int k, auto count) {     // `count` steps from k: all requested before the first is used
+        constexpr int U = decltype(count)::value;
+        X8 a[U], b[U][MT];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            a[u] = *reinterpret_cast<const X8*>(w + 32 * (k + u));
+#pragma unroll
+            for (int m = 0; m < MT; ++m) b[u][m] = *reinterpret_cast<const X8*>(x[m] + (k + u) * (IN ? mt * 512 : 32));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[m] = E::mfma(a[u], b[u][m], acc[m]);
+    };
+    int k = k0;
+    for (; k + 3 <= k1; k += 3) run(k, std::integral_constant<int, 3>{});
+    if (k + 2 == k1) run(k, std::integral_constant<int, 2>{});
+    else if (k + 1 == k1) run(k, std::integral_constant<int, 1>{});
+#pragma unroll
+    for (int m = 0; m < MT; ++m) *reinterpret_cast<f32x4*>(&red[((wave * MT + m) * 64 + l) * 4]) = acc[m];
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < MT * 64; idx += blockDim.x) {
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+        for (int v = 0; v < waves; ++v) sum += *reinterpret_cast<const f32x4*>(&red[(v * MT * 64 + idx) * 4]);
+        const int row = 16 * (tile0 + (idx >> 6)) + (idx & 15);
+        if (row >= M) continue;
+        if (PART) {
+            *reinterpret_cast<f32x4*>(static_cast<float*>(y) + (int64_t(blockIdx.y) * M + row) * N + col) = sum;
+        } else {
+            T4 out;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float v = sum[i] + float(b4[i]);
+                if (GELU) v = 0.5f * v * (1.f + erff(v * 0.70710678f));
+                out[i] = T(v);
+            }
+            *reinterpret_cast<T4*>(static_cast<T*>(y) + row_at(row, col >> 3, N, OUT ? mt : 0) + (col & 7)) = out;
+        }
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ void scan_row(const T* row, int64_t stride, int L, int& count, int& last, bool& ones) {
+    const int l = threadIdx.x & 63;
+    for (int i = l; i < L; i += 64) {
+        const T x = row[i * stride];
+        if (x != T(0)) {
+            ++count;
+            last = i + 1;
+            ones = ones && x == T(1);
+        }
+    }
+}
+
+__global__ __launch_bounds__(1024) void scan_mask_kernel(const void* mask, int type, int64_t sb, int64_t sl, int B, int L, int32_t* lens,
+                                                         int32_t* cu, int32_t* flags, int ticket) {
+    __shared__ int s_len[TDB_SCAN_MAX_BATCH], s_ok, s_ones;
+    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
+    if (threadIdx.x == 0) s_ok = s_ones = 1;
+    __syncthreads();
+    for (int b = wave; b < B; b += 16) {
+        int count = 0, last = 0;
+        bool ones = true;
+        switch (type) {
+            case TDB_MASK_I64: scan_row(static_cast<const int64_t*>(mask) + b * sb, sl, L, count, last, ones); break;
+            case TDB_MASK_I32: scan_row(static_cast<const int32_t*>(mask) + b * sb, sl, L, count, last, ones); break;
+            case TDB_MASK_U8: scan_row(static_cast<const uint8_t*>(mask) + b * sb, sl, L, count, last, ones); break;
+            case TDB_F32: scan_row(static_cast<const float*>(mask) + b * sb, sl, L, count, last, ones); break;
+            case TDB_BF16: scan_row(static_cast<const __bf16*>(mask) + b * sb, sl, L, count, last, ones); break;
+            default: scan_row(static_cast<const _Float16*>(mask) + b * sb, sl, L, count, last, ones); break;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            count += __shfl_xor(count, o);
+            last = max(last, __shfl_xor(last, o));
+        }
+        const bool all_ones = __builtin_amdgcn_ballot_w64(!ones) == 0;
+        if (l == 0) {
+            s_len[b] = count;
+            if (last != count) s_ok = 0;    // (every writer writes the same)
+            if (!all_ones) s_ones = 0;
+        }
+    }
+    __syncthreads();
+    if (wave == 0) {
+        int before = 0;
+        for (int b0 = 0; b0 < B; b0 += 64) {
+            const int n = b0 + l < B ? s_len[b0 + l] : 0;
+            int incl = n;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int up = __shfl_up(incl, d);
+                if (l >= d) incl += up;
+            }
+            if (b0 + l < B) {
+                lens[b0 + l] = n;
+                cu[b0 + l + 1] = before + incl;
+            }
+            before += __shfl(incl, 63);
+        }
+        if (l == 0) {
+            cu[0] = 0;
+            flags[0] = s_ok;
+            flags[1] = before;
+            flags[2] = s_ones;
+            __threadfence_system();
+            __hip_atomic_store(flags + 3, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void unpack_kernel(const uint4* x, const int32_t* cu, int rows, int L, int chunks, uint4* out) {
+    const int r = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+    if (r >= rows) return;
+    const int b = r / L, i = r - b * L, lo = cu[b];
+    const bool in = i < cu[b + 1] - lo;
+    for (int c = l; c < chunks; c += 64) out[int64_t(r) * chunks + c] = in ? x[int64_t(lo + i) * chunks + c] : uint4{0, 0, 0, 0};
+}
+
+// hidden up to 4096 in chunks of eight, CH of them per lane
+template <typename F>
+void with_chunks(int hidden, F f) {
+    if (hidden <= 512) f(std::integral_constant<int, 1>{});
+    else if (hidden <= 1024) f(std::integral_constant<int, 2>{});
+    else if (hidden <= 2048) f(std::integral_constant<int, 4>{});
+    else f(std::integral_constant<int, 8>{});
+}
+template <typename F>
+void with_type(int dtype, F f) {
+    if (dtype == TDB_F32) f(std::integral_constant<int, TDB_F32>{});
+    else if (dtype == TDB_BF16) f(std::integral_constant<int, TDB_BF16>{});
+    else f(std::integral_constant<int, TDB_F16>{});
+}
+
+// Up to here a layer's four products take less on this kernel than the library's host side alone takes for them (19 us each).
+constexpr int SMALL_ROWS = 512;
+
+bool hidden_ok(int hidden) { return hidden > 0 && hidden % 8 == 0 && hidden <= 4096; }
+
+}  // namespace
+
+extern "C" {
+
+int tdb_enc_scan_mask(const void* mask, int type, int64_t stride_b, int64_t stride_l, int B, int L, int32_t* lens, int32_t* cu, int32_t* flags,
+                      int ticket, void* stream) {
+    if (B < 1 || B > TDB_SCAN_MAX_BATCH || L < 1) return int(hipErrorInvalidValue);
+    hipLaunchKernelGGL(scan_mask_kernel, dim3(1), dim3(1024), 0, static_cast<hipStream_t>(stream), mask, type, stride_b, stride_l, B, L, lens, cu, flags, ticket);
+    return int(hipGetLastError());
+}
+
+int tdb_enc_embed(const void* ids, int ids64, const void* table, int64_t vocab, const void* gamma, const void* beta, float eps, const int32_t* cu,
+                  int B, int L, int T, int hidden, int dtype, int mt, void* out, void* stream) {
+    if (!hidden_ok(hidden) || T < 1) return int(hipErrorInvalidValue);
+    with_type(dtype, [&](auto dt) {
+        with_chunks(hidden, [&](auto ch) {
+            hipLaunchKernelGGL((embed_kernel<decltype(dt)::value, decltype(ch)::value>), dim3((T + 3) / 4), dim3(256), 0, static_cast<hipStream_t>(stream),
+                               ids, ids64, table, vocab, gamma, beta, eps, cu, B, L, T, hidden, mt, out);
+        });
+    });
+    return int(hipGetLastError());
+}
+
+int tdb_enc_add_norm(const void* x, int splits, const void* bias, const void* residual, const void* gamma, const void* beta, float eps, int T,
+                     int hidden, int dtype, int mt_in, int mt_out, void* out, void* stream) {
+    if (!hidden_ok(hidden) || T < 1 || splits < 0 || splits > MAX_SPLITS) return int(hipErrorInvalidValue);
+    with_type(dtype, [&](auto dt) {
+        with_chunks(hidden, [&](auto ch) {
+            constexpr int DT = decltype(dt)::value, CH = decltype(ch)::value;
+            const dim3 grid((T + 3) / 4), block(256);
+            hipStream_t s = static_cast<hipStream_t>(stream);
+            if (splits > 0) hipLaunchKernelGGL((add_norm_kernel<DT, CH, true>), grid, block, 0, s, x, splits, bias, residual, gamma, beta, eps, T, hidden, mt_in, mt_out, out);
+            else hipLaunchKernelGGL((add_norm_kernel<DT, CH, false>), grid, block, 0, s, x, 0, bias, residual, gamma, beta, eps, T, hidden, mt_in, mt_out, out);
+        });
+    });
+    return int(hipGetLastError());
+}
+
+int tdb_enc_small_tiles(int M, int N, int K, int dtype) {
+    if ((dtype != TDB_BF16 && dtype != TDB_F16) || M < 1 || M > SMALL_ROWS || N < 1 || N % 32 || K < 1 || K % 32) return 0;
+    const int mt = (M + 15) / 16;
+    return mt <= 4 ? mt : mt <= 6 ? 6 : (mt + 7) / 8 * 8;
+}
+
+int tdb_enc_small_gemm(const void* x, const void* w, const void* bias, int flags, int splits, int M, int N, int K, int dtype, void* y, void* stream) {
+    const int tiles = tdb_enc_small_tiles(M, N, K, dtype);
+    if (tiles == 0 || splits < 0 || splits > MAX_SPLITS) return int(hipErrorInvalidValue);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    bool known = true;
+    auto launch = [&](auto dt, auto mt) {
+        constexpr int DT = decltype(dt)::value, MT = decltype(mt)::value;
+        const int waves = MT > 4 ? 4 : 8;
+        const dim3 grid(N / 16, splits > 0 ? splits : 1, (tiles + MT - 1) / MT), block(waves * 64);
+        const size_t smem = size_t(waves) * MT * 1024;
+        const int shape = splits > 0 ? 8 : 0;
+        switch (shape | flags) {            // the four products of a layer
+            case TDB_ENC_IN: hipLaunchKernelGGL((small_gemm_kernel<DT, MT, true, false, false, false>), grid, block, smem, s, x, w, bias, y, M, N, K, tiles, 1); break;
+            case 8: hipLaunchKernelGGL((small_gemm_kernel<DT, MT, false, false, false, true>), grid, block, smem, s, x, w, bias, y, M, N, K, tiles, splits); break;
+            case TDB_ENC_IN | TDB_ENC_OUT | TDB_ENC_GELU:
+                hipLaunchKernelGGL((small_gemm_kernel<DT, MT, true, true, true, false>), grid, block, smem, s, x, w, bias, y, M, N, K, tiles, 1);
+                break;
+            case 8 | TDB_ENC_IN: hipLaunchKernelGGL((small_gemm_kernel<DT, MT, true, false, false, true>), grid, block, smem, s, x, w, bias, y, M, N, K, tiles, splits); break;
+            default: known = false;
+        }
+    };
+    auto rows = [&](auto dt) {
+        switch (tiles) {
+            case 1: launch(dt, std::integral_constant<int, 1>{}); break;
+            case 2: launch(dt, std::integral_constant<int, 2>{}); break;
+            case 3: launch(dt, std::integral_constant<int, 3>{}); break;
+            case 4: launch(dt, std::integral_constant<int, 4>{}); break;
+            case 6: launch(dt, std::integral_constant<int, 6>{}); break;
+            default: launch(dt, std::integral_constant<int, 8>{});
+        }
+    };
+    if (dtype == TDB_BF16) rows(std::integral_constant<int, TDB_BF16>{});
+    else rows(std::integral_constant<int, TDB_F16>{});
+    return known ? int(hipGetLastError()) : int(hipErrorInvalidValue);
+}
+
+int tdb_enc_unpack(const void* x, const int32_t* cu, int B, int L, int hidden, int dtype, void* out, void* stream) {
+    const int bytes = hidden * (dtype == TDB_F32 ? 4 : 2);
+    if (bytes % 16 || B < 1 || L < 1) return int(hipErrorInvalidValue);
+    hipLaunchKernelGGL(unpack_kernel, dim3((B * L + 3) / 4), dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<const uint4*>(x), cu, B * L, L,
+                       bytes / 16, static_cast<uint4*>(out));
+    return int(hipGetLastError());
+}
+
+}  // extern "C"

@@ -22,6 +22,7 @@
 #include <cstring>
 #include <vector>
 
+#include "host.h"
 #include "tdb_attn.h"
 
 namespace {
@@ -129,21 +130,28 @@ bool inputs_ok(const Common& c, int dims) {
     return true;
 }
 
+// span and delta table of sequences up to max_len; false where no such table has been handed over
+bool fill_delta(tdb_pos_args& pos, int64_t buckets, int64_t max_rel, int64_t max_len, int device) {
+    const int64_t span = buckets > 0 ? buckets : max_rel;
+    if (span < 1) return false;
+    int64_t size = 512;
+    while (size < max_len) size *= 2;
+    for (const Lut& l : luts())
+        if (l.device == device && l.size == size && l.buckets == buckets && l.max_rel == max_rel) {
+            pos.span = int32_t(span);
+            pos.lut_half = int32_t(size - 1);
+            pos.delta_lut = static_cast<const int32_t*>(l.table.data_ptr());
+            return true;
+        }
+    return false;
+}
+
 bool fill_pos(tdb_pos_args& pos, const Common& c, int64_t heads, int64_t head_dim, int64_t max_len) {
     const at::Tensor& q = *c.q;
     if ((c.q_pos && c.pk) || (c.k_pos && c.pq)) return false;
     if (!c.q_pos && !c.k_pos && !c.pk && !c.pq) return true;
-    const int64_t span = c.buckets > 0 ? c.buckets : c.max_rel;
-    if (span < 1) return false;
-    int64_t size = 512;
-    while (size < max_len) size *= 2;
-    const Lut* lut = nullptr;
-    for (const Lut& l : luts())
-        if (l.device == q.device().index() && l.size == size && l.buckets == c.buckets && l.max_rel == c.max_rel) lut = &l;
-    if (!lut) return false;
-    pos.span = int32_t(span);
-    pos.lut_half = int32_t(size - 1);
-    pos.delta_lut = static_cast<const int32_t*>(lut->table.data_ptr());
+    if (!fill_delta(pos, c.buckets, c.max_rel, max_len, q.device().index())) return false;
+    const int64_t span = pos.span;
     for (int n = 0; n < 2; ++n) {
         const at::Tensor* t = n ? c.pq : c.pk;
         if (!t) continue;
@@ -313,4 +321,22 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, kMethods};
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&kModule); }
+int (*tdb_host_fixed())(const tdb_fixed_args*, void*) { return g_fixed; }
+int (*tdb_host_varlen())(const tdb_varlen_args*, void*) { return g_varlen; }
+
+bool tdb_host_fill_tables(tdb_pos_args& pos, const at::Tensor* pk, const at::Tensor* pq, int64_t buckets, int64_t max_rel, int64_t max_len, int device) {
+    if (!pk && !pq) return true;
+    if (!fill_delta(pos, buckets, max_rel, max_len, device)) return false;
+    if (pk) pos.pos_key = pk->data_ptr(), pos.pos_key_stride_h = pk->stride(-3), pos.pos_key_stride_r = pk->stride(-2);
+    if (pq) pos.pos_query = pq->data_ptr(), pos.pos_query_stride_h = pq->stride(-3), pos.pos_query_stride_r = pq->stride(-2);
+    return true;
+}
+
+PyMODINIT_FUNC PyInit__host(void) {
+    PyObject* m = PyModule_Create(&kModule);
+    if (m && !tdb_host_add_encoder(m)) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

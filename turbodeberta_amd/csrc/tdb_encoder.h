@@ -1,0 +1,46 @@
+// Launchers of the kernels around attention in an encoder layer (encoder.hip), called by the native encoder loop (host.cpp).
+// All return a hipError_t as int and take a hipStream_t; nothing here allocates or synchronises.
+#pragma once
+#include <stdint.h>
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+// Element types as in tdb_attn.h; masks additionally: 3 = int64, 4 = int32, 5 = one byte.
+enum { TDB_MASK_I64 = 3, TDB_MASK_I32 = 4, TDB_MASK_U8 = 5 };
+enum { TDB_SCAN_MAX_BATCH = 1024 };
+
+// lens[b] = number of nonzero entries of row b, cu = their running sum from 0; flags[0] = 1 if every row has its nonzero
+// entries first, flags[1] = sum of lens, flags[2] = 1 if every nonzero entry is 1; then flags[3] = ticket.  `flags` may be
+// pinned host memory.
+int tdb_enc_scan_mask(const void* mask, int type, int64_t stride_b, int64_t stride_l, int B, int L, int32_t* lens, int32_t* cu,
+                      int32_t* flags, int ticket, void* stream);
+
+// Order of activation rows: mt = 0 row after row; mt > 0 (tdb_enc_small_tiles) the order in which the small products load
+// them, 16 mt rows of room.
+
+// out[t] = LayerNorm(table[ids of token t]); cu != NULL: token t of the packed batch, cu == NULL: ids in order.
+int tdb_enc_embed(const void* ids, int ids64, const void* table, int64_t vocab, const void* gamma, const void* beta, float eps,
+                  const int32_t* cu, int B, int L, int T, int hidden, int dtype, int mt, void* out, void* stream);
+
+// out = LayerNorm(x + residual); x: [T, hidden] of `dtype`, or (splits > 0, at most 8) [splits, T, hidden] float32 partial sums
+// to which `bias` is added.  mt_in: order of the residual, mt_out: of the output.
+int tdb_enc_add_norm(const void* x, int splits, const void* bias, const void* residual, const void* gamma, const void* beta, float eps,
+                     int T, int hidden, int dtype, int mt_in, int mt_out, void* out, void* stream);
+
+// Products with few rows, 16-bit: y[M, N] = x[M, K] w[N, K]^T + bias, or (splits > 0, at most 8) float32 partial sums
+// [splits, M, N] without bias.  flags: x in the small products' order, y too, GELU (the erf form) applied.  Four combinations
+// exist: IN; splits; IN | OUT | GELU; IN with splits.
+enum { TDB_ENC_IN = 1, TDB_ENC_OUT = 2, TDB_ENC_GELU = 4 };
+int tdb_enc_small_gemm(const void* x, const void* w, const void* bias, int flags, int splits, int M, int N, int K, int dtype, void* y,
+                       void* stream);
+// 16-row tiles (mt) of a product that the above takes, else 0
+int tdb_enc_small_tiles(int M, int N, int K, int dtype);
+
+// out[b, l] = x[cu[b] + l] for l < cu[b+1] - cu[b], zeros elsewhere
+int tdb_enc_unpack(const void* x, const int32_t* cu, int B, int L, int hidden, int dtype, void* out, void* stream);
+
+#ifdef __cplusplus
+}
+#endif

@@ -30,24 +30,32 @@ What differs from the reference glue (model.py:34-186):
 from __future__ import annotations
 
 import math
+import weakref
 from typing import Optional
 
 import torch
 from torch import nn
+from transformers.activations import GELUActivation
 from transformers.modeling_outputs import BaseModelOutput
 from transformers.models.deberta_v2.modeling_deberta_v2 import (
     DebertaV2Attention,
+    DebertaV2Embeddings,
     DebertaV2Encoder,
     DebertaV2ForMaskedLM,
     DebertaV2ForMultipleChoice,
     DebertaV2ForQuestionAnswering,
     DebertaV2ForSequenceClassification,
     DebertaV2ForTokenClassification,
+    DebertaV2Intermediate,
     DebertaV2Layer,
     DebertaV2Model,
+    DebertaV2Output,
+    DebertaV2SelfOutput,
     DisentangledSelfAttention,
 )
 
+from . import _lib
+from .ops._launch import delta_lut
 from .ops.flash_attention import flash_attention_with_disentangled
 from .ops.flash_attention_varlen import flash_attention_with_disentangled_varlen
 from .padding import index_first_axis, key_padding_mask, pad_input
@@ -69,12 +77,13 @@ def _version_of(t):
 
 
 class _MaskInfo:
-    """What the fused paths need to know about an attention mask: ``lengths`` int32 ``[B]`` on the device and
-    ``total``, the number of valid tokens (a host int; ``None`` when the caller declared the lengths without it)."""
-    __slots__ = ("lengths", "total")
+    """What the fused paths need to know about an attention mask: ``lengths`` int32 ``[B]`` on the device,
+    ``total``, the number of valid tokens (a host int; ``None`` when the caller declared the lengths without it), the
+    running sum ``cu`` of the lengths (or None: not computed yet) and whether every nonzero entry is 1 (None: unknown)."""
+    __slots__ = ("lengths", "total", "cu", "ones")
 
-    def __init__(self, lengths, total):
-        self.lengths, self.total = lengths, total
+    def __init__(self, lengths, total, cu=None, ones=None):
+        self.lengths, self.total, self.cu, self.ones = lengths, total, cu, ones
 
 
 def _mask_info(attention_mask):
@@ -90,22 +99,27 @@ def _mask_info(attention_mask):
     cached = getattr(attention_mask, "_tdb_info", None)
     if cached is not None and cached[0] == version:
         return cached[1]
-    valid = key_padding_mask(attention_mask) != 0                               # [B, L]
-    L = valid.shape[-1]
-    lengths = valid.sum(dim=-1, dtype=torch.int32)
-    ok = (valid == (torch.arange(L, device=valid.device)[None, :] < lengths[:, None])).all()
-    if attention_mask.dim() == 4 and attention_mask.shape[1] > 1:
-        ok = ok & ((attention_mask != 0) == (attention_mask[:, :1] != 0)).all()      # one length per sequence: no per-head masks
-    if attention_mask.dim() > 2 and attention_mask.shape[-2] == L and L > 1:
-        full = attention_mask if attention_mask.dim() == 3 else attention_mask[:, 0]
-        ok = ok & ((full != 0) == (valid[:, :, None] & valid[:, None, :])).all()
-    ok_host, total = torch.stack([ok.to(torch.int64), lengths.sum(dtype=torch.int64)]).tolist()   # the one synchronisation
+    scan = _lib.host().scan_mask(attention_mask) if attention_mask.is_cuda and attention_mask.dim() == 2 else None
+    if scan is not None:                                             # one kernel, one synchronisation
+        lengths, cu, ok_host, total, ones = scan
+    else:
+        cu = ones = None
+        valid = key_padding_mask(attention_mask) != 0                               # [B, L]
+        L = valid.shape[-1]
+        lengths = valid.sum(dim=-1, dtype=torch.int32)
+        ok = (valid == (torch.arange(L, device=valid.device)[None, :] < lengths[:, None])).all()
+        if attention_mask.dim() == 4 and attention_mask.shape[1] > 1:
+            ok = ok & ((attention_mask != 0) == (attention_mask[:, :1] != 0)).all()      # one length per sequence: no per-head masks
+        if attention_mask.dim() > 2 and attention_mask.shape[-2] == L and L > 1:
+            full = attention_mask if attention_mask.dim() == 3 else attention_mask[:, 0]
+            ok = ok & ((full != 0) == (valid[:, :, None] & valid[:, None, :])).all()
+        ok_host, total = torch.stack([ok.to(torch.int64), lengths.sum(dtype=torch.int64)]).tolist()   # the one synchronisation
     if not ok_host:
         raise ValueError("attention_mask must be right padded (valid tokens first, no holes) and, if 3-D or 4-D, the "
                          "outer product of a key-padding mask with itself (or one broadcast row of it), equal for all "
                          "heads: the fused attention takes per-sequence lengths.  Use the eager Hugging Face modules for "
                          "other masks.")
-    info = _MaskInfo(lengths, int(total))
+    info = _MaskInfo(lengths, int(total), cu, ones)
     try:
         attention_mask._tdb_info = (version, info)
     except AttributeError:      # tensor subclasses without a __dict__
@@ -120,19 +134,26 @@ def declare_right_padded(attention_mask, lengths, total=None):
     synchronises with the host: a forward on such a mask can be captured into a HIP graph.  ``total`` (a host int, the
     sum of the lengths) additionally lets the encoder pack the batch; without it the encoder keeps the padded layout,
     because the packed token count sizes host-side allocations.  Nothing is verified: wrong lengths give wrong
-    attention.  Returns the mask."""
+    attention.  (The mask's entries are taken to be 0 and 1.)  Returns the mask."""
     if lengths.dtype != torch.int32 or lengths.dim() != 1 or lengths.shape[0] != attention_mask.shape[0]:
         raise ValueError("lengths must be an int32 tensor with one entry per sequence of the mask")
     if lengths.device != attention_mask.device:
         raise ValueError("lengths must live on the mask's device")
-    attention_mask._tdb_info = (_version_of(attention_mask), _MaskInfo(lengths, None if total is None else int(total)))
+    attention_mask._tdb_info = (_version_of(attention_mask), _MaskInfo(lengths, None if total is None else int(total), ones=True))
     return attention_mask
+
+
+def _boundaries(info):
+    """int32 ``[B+1]`` running sum of the lengths, with a leading 0."""
+    if info.cu is None:
+        info.cu = torch.nn.functional.pad(torch.cumsum(info.lengths, dim=0, dtype=torch.int32), (1, 0))
+    return info.cu
 
 
 def _packing_of(info, batch, seqlen, device):
     """``(indices, cu_seqlens)`` of a verified right-padded batch without a further synchronisation: positions of the
     valid tokens in the flattened ``[B*L]`` batch, int32 boundaries with a leading 0."""
-    cu = torch.nn.functional.pad(torch.cumsum(info.lengths, dim=0, dtype=torch.int32), (1, 0))
+    cu = _boundaries(info)
     seq = torch.repeat_interleave(torch.arange(batch, device=device), info.lengths.long(), output_size=info.total)
     indices = torch.arange(info.total, device=device) - cu[:-1].long()[seq] + seq * seqlen
     return indices, cu
@@ -356,6 +377,78 @@ class FlashDebertaV2Encoder(DebertaV2Encoder):
         return BaseModelOutput(last_hidden_state=output_states, hidden_states=all_hidden_states, attentions=None)
 
 
+# Plans of the native encoder loop, by model (kept outside the modules: a plan can be neither copied nor pickled).  False: the
+# model's structure is not one the loop knows.
+_PLANS = weakref.WeakKeyDictionary()
+
+
+def _native_plan(model):
+    """The plan of ``model`` for the native loop from token ids to the last hidden state (csrc/host_encoder.cpp), or None:
+    the plan of an earlier call if the module tree is still what it was, else a new one."""
+    host = _lib.host()
+    plan = _PLANS.get(model)
+    if plan is False or torch.nn.modules.module._has_any_global_hook():
+        return None
+    if plan is not None and host.plan_ok(plan, model):
+        return plan
+    if not _known_structure(model):
+        _PLANS[model] = False
+        return None
+    _PLANS.pop(model, None)
+    if not host.tree_ready(model):               # a module in training mode, a hook, a forward of its own, ...
+        return None
+    emb, enc = model.embeddings, model.encoder
+    table = emb.word_embeddings.weight
+    rel = enc.get_rel_embedding()
+    layers = []
+    for layer in enc.layer:
+        att, so, mid, out = layer.attention.self, layer.attention.output, layer.intermediate.dense, layer.output
+        wqkv, bqkv = att._fused_qkv()
+        pos_key, pos_query, scale, buckets, max_rel = att._position_terms(rel, table.dtype, True)
+        layers.append((wqkv, bqkv, pos_key, pos_query, so.dense.weight, so.dense.bias, so.LayerNorm.weight, so.LayerNorm.bias,
+                       mid.weight, mid.bias, out.dense.weight, out.dense.bias, out.LayerNorm.weight, out.LayerNorm.bias,
+                       float(so.LayerNorm.eps), float(out.LayerNorm.eps)))
+    tensors = [t for l in layers for t in l[:14] if t is not None] + [table, emb.LayerNorm.weight, emb.LayerNorm.bias]
+    if any(t.dtype != table.dtype or t.device != table.device or not (t.is_contiguous() or t.dim() == 3) for t in tensors):
+        return None
+    plan = host.make_plan(model, layers, (table, emb.LayerNorm.weight, emb.LayerNorm.bias, float(emb.LayerNorm.eps)),
+                          att.num_attention_heads, att.attention_head_size, scale, buckets, max_rel)
+    if plan is not None:
+        _PLANS[model] = plan
+    return plan
+
+
+def _known_structure(model):
+    """Whether the modules below ``model`` compute what the native loop computes: stock DeBERTa-v2/v3 layers with the fused
+    attention, exact GELU, no convolution, embeddings that are a table and a LayerNorm."""
+    emb, enc = model.embeddings, model.encoder
+    plain = lambda m, *names: all(type(getattr(m, n)) is nn.Linear and getattr(m, n).bias is not None for n in names)
+    norm = lambda m: type(m) is nn.LayerNorm and m.weight is not None and m.bias is not None
+    if not (type(emb) is DebertaV2Embeddings and type(emb.word_embeddings) is nn.Embedding and emb.word_embeddings.max_norm is None
+            and not emb.position_biased_input and emb.token_type_embeddings is None and emb.embed_proj is None and norm(emb.LayerNorm)
+            and type(enc) is FlashDebertaV2Encoder and enc.conv is None and len(enc.layer) > 0):
+        return False
+    hidden = emb.word_embeddings.weight.shape[1]
+    if hidden % 8 or hidden > 4096 or emb.word_embeddings.weight.dtype not in (torch.float32, torch.bfloat16, torch.float16):
+        return False
+    first = enc.layer[0].attention.self
+    for layer in enc.layer:
+        if not (type(layer) in (DebertaV2Layer, FlashDebertaV2Layer) and type(layer.attention) in (DebertaV2Attention, FlashDebertaV2Attention)
+                and type(layer.attention.self) is FlashDisentangledSelfAttention and type(layer.attention.output) is DebertaV2SelfOutput
+                and type(layer.intermediate) is DebertaV2Intermediate and type(layer.output) is DebertaV2Output
+                and type(layer.intermediate.intermediate_act_fn) is GELUActivation
+                and layer.intermediate.intermediate_act_fn.act is nn.functional.gelu):
+            return False
+        att = layer.attention.self
+        if not (plain(att, "query_proj", "key_proj", "value_proj") and plain(layer.attention.output, "dense") and plain(layer.output, "dense")
+                and plain(layer.intermediate, "dense") and norm(layer.attention.output.LayerNorm) and norm(layer.output.LayerNorm)
+                and att.num_attention_heads * att.attention_head_size == hidden == layer.output.dense.out_features
+                and layer.intermediate.dense.out_features == enc.layer[0].intermediate.dense.out_features
+                and (att.num_attention_heads, att.pos_att_type, att.relative_attention) == (first.num_attention_heads, first.pos_att_type, first.relative_attention)):
+            return False
+    return True
+
+
 class FlashDebertaV2Model(DebertaV2Model):
     def __init__(self, config):
         super().__init__(config)
@@ -383,6 +476,10 @@ class FlashDebertaV2Model(DebertaV2Model):
         given = input_ids if input_ids is not None else inputs_embeds[..., 0]
         if input_ids is not None:
             self.warn_if_padding_and_no_attention_mask(input_ids, attention_mask)
+            if not output_attentions:
+                last = self._forward_native(input_ids, attention_mask)
+                if last is not None:
+                    return BaseModelOutput(last_hidden_state=last, hidden_states=None, attentions=None) if return_dict else (last,)
         if attention_mask is None:
             attention_mask = torch.ones(given.shape, device=given.device)
         if token_type_ids is None:
@@ -395,6 +492,32 @@ class FlashDebertaV2Model(DebertaV2Model):
         if not return_dict:
             return (sequence_output,) + tuple(encoded[2:])
         return BaseModelOutput(last_hidden_state=sequence_output, hidden_states=None, attentions=encoded.attentions)
+
+
+    def _forward_native(self, input_ids, attention_mask):
+        """The last hidden state through the native loop, or None where the modules have to be run: with gradients, in
+        training mode, under autocast or a compiler, with hooks, for masks other than 2-D ones of zeros and ones.  As in the
+        packed encoder, padded positions come back as zeros."""
+        if (self.training or torch.is_grad_enabled() or not input_ids.is_cuda or input_ids.dim() != 2 or not input_ids.numel()
+                or not getattr(self.encoder, "pack_sequences", False) or torch.is_autocast_enabled() or torch.compiler.is_compiling()):
+            return None
+        B, L = input_ids.shape
+        if attention_mask is not None and (attention_mask.shape != input_ids.shape or not attention_mask.is_cuda):
+            return None
+        plan = _native_plan(self)
+        if plan is None:
+            return None
+        cu, total = None, B * L
+        if attention_mask is not None:
+            info = _mask_info(attention_mask)                        # the one host synchronisation
+            if not info.total or not info.ones:
+                return None
+            if info.total < B * L:
+                cu, total = _boundaries(info), info.total
+        enc = self.encoder
+        if enc.relative_attention:
+            delta_lut(input_ids.device, L, enc.layer[0].attention.self.position_buckets, enc.layer[0].attention.self.max_relative_positions)
+        return _lib.host().encode(plan, input_ids, cu, total)
 
 
 class _FusedHead:
