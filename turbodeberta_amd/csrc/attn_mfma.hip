@@ -84,9 +84,10 @@ struct Smem {
     uint16_t qr[WIN * RS];
     uint16_t c[BM * CRS];               // c2p ring: row 32w + n belongs to query row0 + 4n + w, slot = key mod 192
     uint16_t p[BN * PS];
-    int seq_n[64], seq_lo[64];          // valid length and first token of the first 64 sequences
-    int srt_seq[64];                    // packed: the sequences in order of decreasing length (ties: lower index first)
-    int64_t seq_pre[64];                // packed: inclusive prefix sum, in that order, of the sequences' tile counts (all heads)
+    int seq_n[64];                      // valid length of the first 64 sequences
+    __attribute__((aligned(16))) int seq_pre[64];                    // packed: inclusive prefix sum of the sequences' tile counts (all heads), in order of
+                                        // decreasing length (ties: lower index first)
+    __attribute__((aligned(16))) int srt_seq[64][4];                 // packed, in that order: sequence, valid length, first token, tiles before it
     int deal_round[NTHREADS / 64];      // packed: how many tiles this workgroup has taken so far, one copy per wave
 };
 
@@ -193,12 +194,6 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
     // up reads nothing from global memory for batches of up to 64 sequences and keeps no register between lookups.
     // Every wave writes the same values (lane l: sequence l) and reads them back itself: no barrier is needed.
     auto lds_int = [&](const int* q) { return __builtin_amdgcn_readfirstlane(*q); };
-    auto lds_i64 = [&](const int64_t* q) {
-        const int64_t v = *q;
-        const int lo = __builtin_amdgcn_readfirstlane(int(uint32_t(uint64_t(v))));
-        const int hi = __builtin_amdgcn_readfirstlane(int(uint32_t(uint64_t(v) >> 32)));
-        return int64_t((uint64_t(uint32_t(hi)) << 32) | uint32_t(lo));
-    };
     auto tiles_of = [](int n) { return (n + BM - 1) / BM; };
     // Packed launches (at most 64 sequences: the launcher splits larger batches) deal their tiles by cost instead of
     // the strided walk of the fixed layout: a tile costs about 3 key steps plus one per 64 keys of its sequence, so
@@ -231,26 +226,32 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
         }
         sm.seq_n[l] = n;
         if (VARLEN) {                     // (the fixed layout's walk needs the lengths only)
-            sm.seq_lo[l] = lo;
-            // Rank of this lane's sequence by decreasing length (ties: lower index first); the sequence and the tile
-            // count (all heads) that belong at rank l travel to lane l inside the wave, and the tile counts become an
-            // inclusive prefix sum in that order.  (All eight waves write the same final values into the shared
-            // arrays and each reads back what it wrote itself; nothing intermediate goes through them -- a second
-            // wave could be anywhere in this sequence.)
-            int rank = 0;
-            for (int b2 = 0; b2 < 64; ++b2) {
-                const int n2 = sm.seq_n[b2];
-                rank += (n2 > n || (n2 == n && b2 < l)) ? 1 : 0;
+            // Rank of this lane's sequence by decreasing length (ties: lower index first): one compare and one add with
+            // carry for each sequence, whose key comes straight out of its lane's register.  (Reading the lengths back from
+            // LDS, 64 of them whatever the batch, with 64-bit prefix sums through the LDS queue, cost 2.3 us of every packed or
+            // padded launch.)
+            const int key = n * 64 + 63 - l;
+            int rank = l < p.B ? 0 : l;
+            for (int b2 = 0; b2 < p.B; ++b2) {
+                const int key2 = __builtin_amdgcn_readlane(key, b2);
+                if (l < p.B) rank += key2 > key ? 1 : 0;
             }
-            const int seq_here = __builtin_amdgcn_ds_permute(rank * 4, l);
-            int64_t cnt = int64_t(__builtin_amdgcn_ds_permute(rank * 4, tiles_of(n))) * p.H;
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const int64_t up = __shfl_up(cnt, d);
-                if (l >= d) cnt += up;
-            }
-            sm.srt_seq[l] = seq_here;
-            sm.seq_pre[l] = cnt;
+            // Tile counts in that order, and their running sum: shifts inside rows of 16 lanes, then the rows' totals.
+            const int count = __builtin_amdgcn_ds_permute(rank * 4, tiles_of(n) * p.H);
+            int pre = count;
+            pre += __builtin_amdgcn_update_dpp(0, pre, 0x111 /* row_shr:1 */, 0xf, 0xf, false);
+            pre += __builtin_amdgcn_update_dpp(0, pre, 0x112, 0xf, 0xf, false);
+            pre += __builtin_amdgcn_update_dpp(0, pre, 0x114, 0xf, 0xf, false);
+            pre += __builtin_amdgcn_update_dpp(0, pre, 0x118, 0xf, 0xf, false);
+            pre += __builtin_amdgcn_update_dpp(0, pre, 0x142 /* row_bcast:15 */, 0xa, 0xf, false);
+            pre += __builtin_amdgcn_update_dpp(0, pre, 0x143 /* row_bcast:31 */, 0xc, 0xf, false);
+            // (All eight waves write the same final values and each reads back what it wrote itself: no barrier is needed.)
+            sm.seq_pre[l] = pre;
+            sm.srt_seq[l][3] = pre - count;
+            int* const mine = sm.srt_seq[rank];
+            mine[0] = l;
+            mine[1] = n;
+            mine[2] = lo;
         }
     }
     if (VARLEN && p.gap_cu && wave == 7)
@@ -271,20 +272,21 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
         t.tok0 = 0;
         return t;
     };
-    // Tile j of this workgroup in the back-and-forth deal (gridDim.x is a multiple of 8).
+    // Tile j of this workgroup in the back-and-forth deal (gridDim.x is a multiple of 8): the rank that owns it, then that
+    // rank's sequence in one read.
     auto dealt_tile = [&](int j) {
-        const int64_t G = gridDim.x, g = int64_t(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-        const int64_t k = int64_t(j) * G + ((j & 1) ? G - 1 - g : g);
+        const int G = gridDim.x, g = int(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+        const int k = j * G + ((j & 1) ? G - 1 - g : g);
         Tile t = no_tile();
-        if (k >= lds_i64(&sm.seq_pre[63])) return t;
         const unsigned long long owners = __builtin_amdgcn_ballot_w64(sm.seq_pre[l] > k);
-        const int r = __builtin_amdgcn_readfirstlane(__builtin_ctzll(owners));
-        t.b = lds_int(&sm.srt_seq[r]);
-        t.len = lds_int(&sm.seq_n[t.b]);
-        t.tok0 = lds_int(&sm.seq_lo[t.b]);
+        if (owners == 0) return t;
+        const int4 seq = *reinterpret_cast<const int4*>(sm.srt_seq[__builtin_amdgcn_readfirstlane(__builtin_ctzll(owners))]);
+        t.b = __builtin_amdgcn_readfirstlane(seq.x);
+        t.len = __builtin_amdgcn_readfirstlane(seq.y);
+        t.tok0 = __builtin_amdgcn_readfirstlane(seq.z);
         const int per_head = tiles_of(t.len);
-        if (owners == 0 || per_head <= 0) return no_tile();
-        const int within = int(k - (lds_i64(&sm.seq_pre[r]) - int64_t(per_head) * p.H));
+        if (per_head <= 0) return no_tile();
+        const int within = k - __builtin_amdgcn_readfirstlane(seq.w);
         t.head = within / per_head;
         t.row0 = (within - t.head * per_head) * BM;
         t.vb = (within >= 0 && t.head < p.H) ? 0 : -1;     // (always true for a consistent prefix: no tile rather than a stray address)
@@ -350,7 +352,7 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
         return delta_of(b) == delta_of(b + WIN - 2);
     };
 
-    if (VARLEN && p.seqlens) {
+    if (VARLEN && p.seqlens && __builtin_amdgcn_ballot_w64(l < p.B && tiles_of(sm.seq_n[l]) < tiles_of(p.L)) != 0) {
         // The deal only lists tiles with valid query rows; tiles that hold padded rows alone get their zeros here,
         // shared out over the workgroups (every thread fills its share of a tile's rows).
         const int per_seq = (p.L + BM - 1) / BM;
@@ -419,15 +421,21 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
 
     // Q^T fragments of query block w: B operand of S^T = K.Q^T (score wave) and of C'^T = K_r'.Q^T (position wave)
     X8 qb[4];
+    // (Buffer loads here and in the stages below: rows past the end of the sequence read as zeros, with no lane predicated off
+    // and a 32-bit offset instead of a 64-bit address per row -- what opens a tile is bound by its instructions, too.)
+    auto rows_of = [&](const uint16_t* base, int rows, int stride_b) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, rows > 0 ? (rows - 1) * stride_b + 128 : 0, RSRC_FLAGS);
+    };
     auto load_q = [&](X8 (&dst)[4], const Tile& t) {
-        const uint16_t* Qt = static_cast<const uint16_t*>(p.q) + (packed_rows ? t.tok0 * p.qs_l : int64_t(t.b) * p.qs_b) + int64_t(t.head) * p.qs_h;
-        const int qrow = t.row0 + 4 * il + w;
+        const uint16_t* Qt = static_cast<const uint16_t*>(p.q) + (packed_rows ? t.tok0 * p.qs_l : int64_t(t.b) * p.qs_b) + int64_t(t.head) * p.qs_h +
+                             int64_t(t.row0) * p.qs_l;
+        const int qs_b = int(p.qs_l) * 2;
+        const __amdgpu_buffer_rsrc_t rsrc = rows_of(Qt, t.vb >= 0 ? t.len - t.row0 : 0, qs_b);
+        int lane = l;                     // opaque, here and below: offsets are redone where they are used instead of
+        asm volatile("" : "+v"(lane));    // occupying a register through the key steps
+        const int off = (4 * (lane & 31) + w) * qs_b + 16 * (lane >> 5);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            u32x4 x = {0, 0, 0, 0};
-            if (t.vb >= 0 && qrow < t.len) x = *reinterpret_cast<const u32x4*>(Qt + int64_t(qrow) * p.qs_l + 16 * c + 8 * hh);
-            dst[c] = __builtin_bit_cast(X8, x);
-        }
+        for (int c = 0; c < 4; ++c) dst[c] = __builtin_bit_cast(X8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off + 32 * c, 0, 0));
     };
     load_q(qb, cur);
 
@@ -438,25 +446,31 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
     int dl_cold[3][2] = {{0, 0}, {0, 0}, {0, 0}};   // position waves: delta of the new window rows of steps 1 to 3
     {
         const int row = tid >> 3, ch = tid & 7;     // rows 0..63
+        const int ks_b = int(p.ks_l) * 2, pks_b = int(p.pks_r) * 2, pqs_b = int(p.pqs_r) * 2;
         int dl[WIN / 64] = {0, 0, 0};
         if (HAS_POS && !STRIP) {
+            const __amdgpu_buffer_rsrc_t lut = __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(p.lut), 0, (lut_max + 1) * 4, RSRC_FLAGS);
+            const int at = (row0 - (BN - 1) + p.lut_half) * 4;
 #pragma unroll
-            for (int n = 0; n < WIN / 64; ++n) dl[n] = delta_of(row0 - (BN - 1) + row + 64 * n);
+            for (int n = 0; n < WIN / 64; ++n) dl[n] = __builtin_amdgcn_raw_buffer_load_b32(lut, at + 4 * row + 256 * n, 0, 0);
             if (!score_role) {
 #pragma unroll
                 for (int s1 = 0; s1 < 3; ++s1)
 #pragma unroll
                     for (int n = 0; n < 2; ++n)
-                        dl_cold[s1][n] = delta_of(row0 - BN * (s1 + 1) - (BN - 1) + ((tid - 256) >> 3) + 32 * n);
+                        dl_cold[s1][n] = __builtin_amdgcn_raw_buffer_load_b32(lut, at - 256 * (s1 + 1) + 4 * ((tid - 256) >> 3) + 128 * n, 0, 0);
             }
         }
-        const u32x4 k0 = *reinterpret_cast<const u32x4*>(K + int64_t(min(row, len - 1)) * p.ks_l + ch * 8);
-        const u32x4 k1 = *reinterpret_cast<const u32x4*>(K + int64_t(min(BN + row, len - 1)) * p.ks_l + ch * 8);
+        const __amdgpu_buffer_rsrc_t kt = rows_of(K, len, ks_b);
+        const u32x4 k0 = __builtin_amdgcn_raw_buffer_load_b128(kt, row * ks_b + ch * 16, 0, 0);
+        const u32x4 k1 = __builtin_amdgcn_raw_buffer_load_b128(kt, (BN + row) * ks_b + ch * 16, 0, 0);
         u32x4 wk[WIN / 64], wq[WIN / 64];
+        const __amdgpu_buffer_rsrc_t tk = rows_of(HAS_C2P && !STRIP ? PK : K, HAS_C2P && !STRIP ? 2 * p.span : 0, pks_b);
+        const __amdgpu_buffer_rsrc_t tq = rows_of(HAS_P2C && !STRIP ? PQ : K, HAS_P2C && !STRIP ? 2 * p.span : 0, pqs_b);
 #pragma unroll
         for (int n = 0; n < WIN / 64; ++n) {
-            if (HAS_C2P && !STRIP) wk[n] = *reinterpret_cast<const u32x4*>(PK + int64_t(dl[n]) * p.pks_r + ch * 8);
-            if (HAS_P2C && !STRIP) wq[n] = *reinterpret_cast<const u32x4*>(PQ + int64_t(dl[n]) * p.pqs_r + ch * 8);
+            if (HAS_C2P && !STRIP) wk[n] = __builtin_amdgcn_raw_buffer_load_b128(tk, __umul24(dl[n], pks_b) + ch * 16, 0, 0);
+            if (HAS_P2C && !STRIP) wq[n] = __builtin_amdgcn_raw_buffer_load_b128(tq, __umul24(dl[n], pqs_b) + ch * 16, 0, 0);
         }
         *reinterpret_cast<u32x4*>(&sm.k[0][row * RS + ch * 8]) = k0;
         *reinterpret_cast<u32x4*>(&sm.k[1][row * RS + ch * 8]) = k1;
@@ -620,8 +634,8 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
         auto fetch = [&]() {                   // the 64 new window rows of a step (dl_next)
 #pragma unroll
             for (int n = 0; n < 2; ++n) {
-                if (HAS_C2P) pre_kr[n] = __builtin_amdgcn_raw_buffer_load_b128(pk_rsrc, dl_next[n] * pks_b + sch * 16, 0, 0);
-                if (HAS_P2C) pre_qr[n] = __builtin_amdgcn_raw_buffer_load_b128(pq_rsrc, dl_next[n] * pqs_b + sch * 16, 0, 0);
+                if (HAS_C2P) pre_kr[n] = __builtin_amdgcn_raw_buffer_load_b128(pk_rsrc, __umul24(dl_next[n], pks_b) + sch * 16, 0, 0);
+                if (HAS_P2C) pre_qr[n] = __builtin_amdgcn_raw_buffer_load_b128(pq_rsrc, __umul24(dl_next[n], pqs_b) + sch * 16, 0, 0);
             }
         };
         // delta of the 64 new window rows of key step s: relative positions row0 - 64s - 63 + srow (+ 32).  Read through
@@ -791,14 +805,14 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
 #pragma unroll
             for (int s1 = 0; s1 < 3; ++s1) dl_step[s1][0] = dl_step[s1][1] = 0;
             if (HAS_POS && t.vb >= 0) {
-                int sr = srow;            // opaque: keeps a dozen precomputed row offsets out of long-lived registers
-                asm volatile("" : "+v"(sr));
+                int at = srow4 + (t.row0 - (BN - 1) + p.lut_half) * 4;
+                asm volatile("" : "+v"(at));
 #pragma unroll
-                for (int n = 0; n < WIN / 32; ++n) dl_win[n] = delta_of(t.row0 - (BN - 1) + sr + 32 * n);
+                for (int n = 0; n < WIN / 32; ++n) dl_win[n] = __builtin_amdgcn_raw_buffer_load_b32(lut_rsrc, at + 128 * n, 0, 0);
 #pragma unroll
                 for (int s1 = 0; s1 < 3; ++s1)
 #pragma unroll
-                    for (int n = 0; n < 2; ++n) dl_step[s1][n] = delta_of(t.row0 - BN * (s1 + 1) - (BN - 1) + sr + 32 * n);
+                    for (int n = 0; n < 2; ++n) dl_step[s1][n] = __builtin_amdgcn_raw_buffer_load_b32(lut_rsrc, at - 256 * (s1 + 1) + 128 * n, 0, 0);
             }
         };
         auto read_stage = [&](const Tile& t) {
@@ -809,13 +823,17 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
 #pragma unroll
             for (int n = 0; n < WIN / 32; ++n) st_wk[n] = st_wq[n] = none;
             if (t.vb >= 0) {
+                const __amdgpu_buffer_rsrc_t kt = rows_of(Kt, t.len, int(p.ks_l) * 2);
+                const __amdgpu_buffer_rsrc_t tk = rows_of(HAS_C2P ? PKt : Kt, HAS_C2P ? 2 * p.span : 0, pks_b), tq = rows_of(HAS_P2C ? PQt : Kt, HAS_P2C ? 2 * p.span : 0, pqs_b);
+                int lane = stid;
+                asm volatile("" : "+v"(lane));
+                const int chb = (lane & 7) * 16, koff = (lane >> 3) * int(p.ks_l) * 2 + chb;
 #pragma unroll
-                for (int n = 0; n < 4; ++n)
-                    st_k[n] = *reinterpret_cast<const u32x4*>(Kt + int64_t(min(srow + 32 * n, t.len - 1)) * p.ks_l + sch * 8);
+                for (int n = 0; n < 4; ++n) st_k[n] = __builtin_amdgcn_raw_buffer_load_b128(kt, koff + 64 * n * int(p.ks_l), 0, 0);
 #pragma unroll
                 for (int n = 0; n < WIN / 32; ++n) {
-                    if (HAS_C2P) st_wk[n] = *reinterpret_cast<const u32x4*>(PKt + int64_t(dl_win[n]) * p.pks_r + sch * 8);
-                    if (HAS_P2C) st_wq[n] = *reinterpret_cast<const u32x4*>(PQt + int64_t(dl_win[n]) * p.pqs_r + sch * 8);
+                    if (HAS_C2P) st_wk[n] = __builtin_amdgcn_raw_buffer_load_b128(tk, __umul24(dl_win[n], pks_b) + chb, 0, 0);
+                    if (HAS_P2C) st_wq[n] = __builtin_amdgcn_raw_buffer_load_b128(tq, __umul24(dl_win[n], pqs_b) + chb, 0, 0);
                 }
             }
         };
@@ -1316,8 +1334,10 @@ bool tdb_mfma_supported(const TdbKernelParams& p, int dtype) {
     if (p.c2p && (rows * p.c2s_l * 2 + int64_t(4) * p.span >= lim || p.c2s_l < 0)) return false;
     if (p.p2c && (rows * p.p2s_l * 2 + int64_t(4) * p.span >= lim || p.p2s_l < 0)) return false;
     if (rows * p.ks_l * 2 >= lim || rows * p.vs_l * 2 >= lim) return false;
-    if (p.pk && int64_t(2) * p.span * p.pks_r * 2 >= lim) return false;
-    if (p.pq && int64_t(2) * p.span * p.pqs_r * 2 >= lim) return false;
+    if (rows * p.qs_l * 2 >= lim) return false;
+    // (a table row's offset is a 24-bit product)
+    if (p.pk && (int64_t(2) * p.span * p.pks_r * 2 >= lim || p.pks_r * 2 >= int64_t(1) << 24)) return false;
+    if (p.pq && (int64_t(2) * p.span * p.pqs_r * 2 >= lim || p.pqs_r * 2 >= int64_t(1) << 24)) return false;
     return true;
 }
 
