@@ -1,6 +1,7 @@
 """The native encoder loop against the same model's modules: token counts at the edges of its 16-row tiles and on both sides
 of its own products, packed and full batches, and what makes it step aside."""
 import copy
+import ctypes as C
 
 import pytest
 import torch
@@ -114,3 +115,35 @@ def test_steps_aside_and_comes_back():
         twin = copy.deepcopy(model)
         assert torch.equal(twin._forward_native(ids, mask), model._forward_native(ids, mask))
     assert model._forward_native(ids, mask) is None                            # gradients on
+
+
+@pytest.mark.parametrize("dtype,code", [(torch.bfloat16, 1), (torch.float16, 2)])
+@pytest.mark.parametrize("tile", range(7))
+def test_product_tiles(tile, dtype, code):
+    """Every tile of the products (0: the one the kernel chooses) where it ends inside the output, and with fewer steps of the
+    contraction than it has stages, whole and in parts."""
+    lib, ptr = _lib.load(), lambda t: C.c_void_p(t.data_ptr())
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for M, N, K in [(1, 8, 64), (33, 72, 128), (127, 136, 192), (130, 264, 448), (513, 520, 832)]:
+        g = torch.Generator(device="cuda").manual_seed(M)
+        x = torch.randn(M, K, device="cuda", generator=g).to(dtype)
+        w, b = (torch.randn(N, K, device="cuda", generator=g) / K ** 0.5).to(dtype), torch.randn(N, device="cuda", generator=g).to(dtype)
+        y, parts = torch.full((M, N), 7., device="cuda", dtype=dtype), torch.full((2, M, N), 7., device="cuda")
+        ref = x.double() @ w.double().t()
+        run = lambda flags, splits, out: lib.tdb_enc_gemm(ptr(x), ptr(w), ptr(b), flags | tile << 8, splits, M, N, K, code, ptr(out), stream)
+        eps = torch.finfo(dtype).eps
+        assert run(0, 1, y) == 0
+        torch.testing.assert_close(y.double(), ref + b.double(), rtol=eps, atol=eps)
+        assert run(4, 1, y) == 0
+        torch.testing.assert_close(y.double(), torch.nn.functional.gelu(ref + b.double()), rtol=eps, atol=eps)
+        if K > 64:
+            assert run(0, 2, parts) == 0
+            torch.testing.assert_close(parts.double().sum(0), ref, rtol=1e-5, atol=1e-5)
+
+
+def test_product_limits():
+    lib = _lib.load()
+    for M, N, K, dtype in [(16, 8, 96, 1), (16, 12, 64, 1), (0, 8, 64, 1), (16, 8, 64, 0), (1 << 16, 8, 1 << 15, 1)]:
+        assert lib.tdb_enc_gemm_splits(M, N, K, dtype) == 0
+        assert lib.tdb_enc_gemm(None, None, None, 0, 1, M, N, K, dtype, None, None) != 0
+    assert lib.tdb_enc_gemm(None, None, None, 0, 2, 16, 8, 64, 1, None, None) != 0       # more parts than steps

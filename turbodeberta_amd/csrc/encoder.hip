@@ -1,7 +1,7 @@
 // The kernels around attention in an encoder layer: embeddings, residual + LayerNorm, products with few rows, mask scan,
-// unpacking.  Large products stay with the library; what is here is bound by memory traffic or by latency:
+// unpacking.  Products with more rows are in gemm.hip; what is here is bound by memory traffic or by latency:
 //   * residual + LayerNorm in one pass, a wave per row with the row in registers: three arrays of traffic instead of five.
-//   * products with at most 128 rows (a single text): the library takes 8-10 us for 48 x 768 x 768 where the weights are
+//   * products with at most 64 rows (a single text): the library takes 8-10 us for 48 x 768 x 768 where the weights are
 //     read in well under one.  Here a workgroup takes 16 output columns and its waves share out the contraction, so that all
 //     of the weight matrix is requested at once; sums of the waves meet in LDS.  Where the output has too few columns to
 //     fill the chip (hidden-sized ones), the contraction is split over workgroups as well, and the residual + LayerNorm
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(256) void embed_kernel(const void* ids, int ids64, 
     norm_row<DT, CH>(v, w, b, chunks, hidden, eps, out, t, mt);
 }
 
-template <int DT, int CH, bool PARTS>
+template <int DT, int CH, int PARTS>      // PARTS: 0, or the most partial sums
 __global__ __launch_bounds__(256) void add_norm_kernel(const void* x, int splits, const void* bias, const void* residual, const void* gamma,
                                                        const void* beta, float eps, int T, int hidden, int mt_in, int mt_out, void* out) {
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63, chunks = hidden / 8;
@@ -162,13 +162,13 @@ __global__ __launch_bounds__(256) void add_norm_kernel(const void* x, int splits
         if (l + 64 * c < chunks) {
             float r[8];
             load8<DT>(residual, row_at(t, l + 64 * c, hidden, mt_in), r);
-            if (PARTS) {
-                float y[MAX_SPLITS][8], add[8];             // all requested before the first is added; past the last: it again
+            if constexpr (PARTS > 0) {
+                float y[PARTS][8], add[8];             // all requested before the first is added; past the last: it again
 #pragma unroll
-                for (int s = 0; s < MAX_SPLITS; ++s) load8<TDB_F32>(x, int64_t(min(s, splits - 1)) * T * hidden + at + el, y[s]);
+                for (int s = 0; s < PARTS; ++s) load8<TDB_F32>(x, int64_t(min(s, splits - 1)) * T * hidden + at + el, y[s]);
                 load8<DT>(bias, el, add);
 #pragma unroll
-                for (int s = 0; s < MAX_SPLITS; ++s)
+                for (int s = 0; s < PARTS; ++s)
                     if (s < splits) {
 #pragma unroll
                         for (int i = 0; i < 8; ++i) v[c][i] += y[s][i];
@@ -186,22 +186,22 @@ __global__ __launch_bounds__(256) void add_norm_kernel(const void* x, int splits
 }
 
 // One workgroup: 16 columns of the output, a share of the contraction given by blockIdx.y and, inside it, by the wave.
-// MT: token tiles of 16, the block of them given by blockIdx.z.  Lane (c, g) has 16 bytes of weight row n0 + c and of token row 16 m + c: columns 32 k + 8 g .. +7.
-// IN / OUT: x / y in the order of row_at with mt tiles in all.
+// MT: token tiles of 16.  Lane (c, g) has 16 bytes of weight row n0 + c and of token row 16 m + c: columns 32 k + 8 g .. +7.
+// IN / OUT: x / y in the order of row_at.
 template <int DT, int MT, bool IN, bool OUT, bool GELU, bool PART>
-__global__ __launch_bounds__(512) void small_gemm_kernel(const void* xv, const void* wv, const void* bias, void* y, int M, int N, int K, int mt, int splits) {
+__global__ __launch_bounds__(512) void small_gemm_kernel(const void* xv, const void* wv, const void* bias, void* y, int M, int N, int K, int splits) {
     using E = Elem<DT>;
     using X8 = typename E::X8;
     using T = typename E::T;
     extern __shared__ __attribute__((aligned(16))) float red[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6, l = threadIdx.x & 63;
-    const int c = l & 15, g = l >> 4, n0 = blockIdx.x * 16, steps = K / 32, tile0 = blockIdx.z * MT;
+    const int c = l & 15, g = l >> 4, n0 = blockIdx.x * 16, steps = K / 32;
     const int parts = splits * waves, part = blockIdx.y * waves + wave;
     const int k0 = steps * part / parts, k1 = steps * (part + 1) / parts;
     const T* const w = static_cast<const T*>(wv) + int64_t(n0 + c) * K + 8 * g;
     const T* x[MT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) x[m] = static_cast<const T*>(xv) + (IN ? (tile0 + m) * 512 + l * 8 : min(16 * (tile0 + m) + c, M - 1) * K + 8 * g);
+    for (int m = 0; m < MT; ++m) x[m] = static_cast<const T*>(xv) + (IN ? m * 512 + l * 8 : min(16 * m + c, M - 1) * K + 8 * g);
     typedef __attribute__((ext_vector_type(4))) T T4;
     const int col = n0 + 4 * g;             // (of every element this thread sums up below)
     T4 b4;
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(512) void small_gemm_kernel(const void* xv, const v
         for (int u = 0; u < U; ++u) {
             a[u] = *reinterpret_cast<const X8*>(w + 32 * (k + u));
 #pragma unroll
-            for (int m = 0; m < MT; ++m) b[u][m] = *reinterpret_cast<const X8*>(x[m] + (k + u) * (IN ? mt * 512 : 32));
+            for (int m = 0; m < MT; ++m) b[u][m] = *reinterpret_cast<const X8*>(x[m] + (k + u) * (IN ? MT * 512 : 32));
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(512) void small_gemm_kernel(const void* xv, const v
     for (int idx = threadIdx.x; idx < MT * 64; idx += blockDim.x) {
         f32x4 sum = {0.f, 0.f, 0.f, 0.f};
         for (int v = 0; v < waves; ++v) sum += *reinterpret_cast<const f32x4*>(&red[(v * MT * 64 + idx) * 4]);
-        const int row = 16 * (tile0 + (idx >> 6)) + (idx & 15);
+        const int row = 16 * (idx >> 6) + (idx & 15);
         if (row >= M) continue;
         if (PART) {
             *reinterpret_cast<f32x4*>(static_cast<float*>(y) + (int64_t(blockIdx.y) * M + row) * N + col) = sum;
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(512) void small_gemm_kernel(const void* xv, const v
                 if (GELU) v = 0.5f * v * (1.f + erff(v * 0.70710678f));
                 out[i] = T(v);
             }
-            *reinterpret_cast<T4*>(static_cast<T*>(y) + row_at(row, col >> 3, N, OUT ? mt : 0) + (col & 7)) = out;
+            *reinterpret_cast<T4*>(static_cast<T*>(y) + row_at(row, col >> 3, N, OUT ? MT : 0) + (col & 7)) = out;
         }
     }
 }
@@ -344,8 +344,9 @@ void with_type(int dtype, F f) {
     else f(std::integral_constant<int, TDB_F16>{});
 }
 
-// Up to here a layer's four products take less on this kernel than the library's host side alone takes for them (19 us each).
-constexpr int SMALL_ROWS = 512;
+// Up to here a layer's four products take less here than in the tiles of gemm.hip (768 wide: 16.5 against 18.5 us at 64 rows,
+// 20.2 against 19.1 at 80).
+constexpr int SMALL_ROWS = 64;
 
 bool hidden_ok(int hidden) { return hidden > 0 && hidden % 8 == 0 && hidden <= 4096; }
 
@@ -380,8 +381,11 @@ int tdb_enc_add_norm(const void* x, int splits, const void* bias, const void* re
             constexpr int DT = decltype(dt)::value, CH = decltype(ch)::value;
             const dim3 grid((T + 3) / 4), block(256);
             hipStream_t s = static_cast<hipStream_t>(stream);
-            if (splits > 0) hipLaunchKernelGGL((add_norm_kernel<DT, CH, true>), grid, block, 0, s, x, splits, bias, residual, gamma, beta, eps, T, hidden, mt_in, mt_out, out);
-            else hipLaunchKernelGGL((add_norm_kernel<DT, CH, false>), grid, block, 0, s, x, 0, bias, residual, gamma, beta, eps, T, hidden, mt_in, mt_out, out);
+            auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, x, splits, bias, residual, gamma, beta, eps, T, hidden, mt_in, mt_out, out); };
+            if (splits == 0) go(add_norm_kernel<DT, CH, 0>);
+            else if (splits <= 2) go(add_norm_kernel<DT, CH, 2>);
+            else if (splits <= 4) go(add_norm_kernel<DT, CH, 4>);
+            else go(add_norm_kernel<DT, CH, MAX_SPLITS>);
         });
     });
     return int(hipGetLastError());
@@ -389,8 +393,7 @@ int tdb_enc_add_norm(const void* x, int splits, const void* bias, const void* re
 
 int tdb_enc_small_tiles(int M, int N, int K, int dtype) {
     if ((dtype != TDB_BF16 && dtype != TDB_F16) || M < 1 || M > SMALL_ROWS || N < 1 || N % 32 || K < 1 || K % 32) return 0;
-    const int mt = (M + 15) / 16;
-    return mt <= 4 ? mt : mt <= 6 ? 6 : (mt + 7) / 8 * 8;
+    return (M + 15) / 16;
 }
 
 int tdb_enc_small_gemm(const void* x, const void* w, const void* bias, int flags, int splits, int M, int N, int K, int dtype, void* y, void* stream) {
@@ -400,17 +403,17 @@ int tdb_enc_small_gemm(const void* x, const void* w, const void* bias, int flags
     bool known = true;
     auto launch = [&](auto dt, auto mt) {
         constexpr int DT = decltype(dt)::value, MT = decltype(mt)::value;
-        const int waves = MT > 4 ? 4 : 8;
-        const dim3 grid(N / 16, splits > 0 ? splits : 1, (tiles + MT - 1) / MT), block(waves * 64);
+        constexpr int waves = 8;
+        const dim3 grid(N / 16, splits > 0 ? splits : 1), block(waves * 64);
         const size_t smem = size_t(waves) * MT * 1024;
         const int shape = splits > 0 ? 8 : 0;
         switch (shape | flags) {            // the four products of a layer
-            case TDB_ENC_IN: hipLaunchKernelGGL((small_gemm_kernel<DT, MT, true, false, false, false>), grid, block, smem, s, x, w, bias, y, M, N, K, tiles, 1); break;
-            case 8: hipLaunchKernelGGL((small_gemm_kernel<DT, MT, false, false, false, true>), grid, block, smem, s, x, w, bias, y, M, N, K, tiles, splits); break;
+            case TDB_ENC_IN: hipLaunchKernelGGL((small_gemm_kernel<DT, MT, true, false, false, false>), grid, block, smem, s, x, w, bias, y, M, N, K, 1); break;
+            case 8: hipLaunchKernelGGL((small_gemm_kernel<DT, MT, false, false, false, true>), grid, block, smem, s, x, w, bias, y, M, N, K, splits); break;
             case TDB_ENC_IN | TDB_ENC_OUT | TDB_ENC_GELU:
-                hipLaunchKernelGGL((small_gemm_kernel<DT, MT, true, true, true, false>), grid, block, smem, s, x, w, bias, y, M, N, K, tiles, 1);
+                hipLaunchKernelGGL((small_gemm_kernel<DT, MT, true, true, true, false>), grid, block, smem, s, x, w, bias, y, M, N, K, 1);
                 break;
-            case 8 | TDB_ENC_IN: hipLaunchKernelGGL((small_gemm_kernel<DT, MT, true, false, false, true>), grid, block, smem, s, x, w, bias, y, M, N, K, tiles, splits); break;
+            case 8 | TDB_ENC_IN: hipLaunchKernelGGL((small_gemm_kernel<DT, MT, true, false, false, true>), grid, block, smem, s, x, w, bias, y, M, N, K, splits); break;
             default: known = false;
         }
     };
@@ -419,9 +422,7 @@ int tdb_enc_small_gemm(const void* x, const void* w, const void* bias, int flags
             case 1: launch(dt, std::integral_constant<int, 1>{}); break;
             case 2: launch(dt, std::integral_constant<int, 2>{}); break;
             case 3: launch(dt, std::integral_constant<int, 3>{}); break;
-            case 4: launch(dt, std::integral_constant<int, 4>{}); break;
-            case 6: launch(dt, std::integral_constant<int, 6>{}); break;
-            default: launch(dt, std::integral_constant<int, 8>{});
+            default: launch(dt, std::integral_constant<int, 4>{});
         }
     };
     if (dtype == TDB_BF16) rows(std::integral_constant<int, TDB_BF16>{});

@@ -35,7 +35,9 @@ struct Enc {
     decltype(&tdb_enc_small_gemm) small_gemm;
     decltype(&tdb_enc_small_tiles) small_tiles;
     decltype(&tdb_enc_unpack) unpack;
-} g_enc = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    decltype(&tdb_enc_gemm) gemm;
+    decltype(&tdb_enc_gemm_splits) gemm_splits;
+} g_enc = {};
 
 struct Decref {
     void operator()(PyObject* o) const { Py_XDECREF(o); }
@@ -217,23 +219,27 @@ at::Tensor encode(const Plan& p, const at::Tensor& ids, const at::Tensor* cu, in
     const bool small = tiles[0] && tiles[1] && tiles[2];
     const int mt = small ? tiles[0] : 0;    // (the same for all three)
     const int64_t rows = small ? 16 * mt : T;
-    // Contractions with hidden-sized outputs are split so that about one workgroup per CU comes of it.
-    const int splits = small ? int(std::max<int64_t>(1, std::min<int64_t>(8, 256 * 16 / (hidden * ((mt + 7) / 8))))) : 0;
+    // Contractions with hidden-sized outputs are split where the output alone gives the CUs too little to do; the add + norm
+    // behind them adds the parts up.  (Few rows: about one workgroup per CU.)
+    const int few = int(std::max<int64_t>(1, std::min<int64_t>(8, 256 * 16 / hidden)));
+    const int splits_o = small ? few : g_enc.gemm_splits(int(T), int(hidden), int(hidden), dt);
+    const int splits_f = small ? few : g_enc.gemm_splits(int(T), int(hidden), int(inner), dt);
+    const bool own = !small && splits_o && splits_f && g_enc.gemm_splits(int(T), int(3 * hidden), int(hidden), dt) && g_enc.gemm_splits(int(T), int(inner), int(hidden), dt);
     at::Tensor x = empty({rows, hidden}, type), y = empty({rows, hidden}, type), attended = empty({T, hidden}, type);
     at::Tensor last = small ? empty({T, hidden}, type) : x;             // the last layer's output, row after row
-    at::Tensor qkv, ff, part;
-    if (small) {
-        qkv = empty({T, 3 * hidden}, type), ff = empty({rows, inner}, type);
-        part = empty({splits, T, hidden}, at::kFloat);
-    }
+    at::Tensor qkv, ff, part, proj;
+    if (small || own) qkv = empty({T, 3 * hidden}, type), ff = empty({rows, inner}, type);
+    if (small || (own && std::max(splits_o, splits_f) > 1)) part = empty({std::max(splits_o, splits_f), T, hidden}, at::kFloat);
+    if (own && std::min(splits_o, splits_f) == 1) proj = empty({T, hidden}, type);
     must(g_enc.embed(ids.data_ptr(), ids.scalar_type() == at::kLong, p.emb.data_ptr(), p.emb.size(0), p.emb_g.data_ptr(), p.emb_b.data_ptr(),
                      float(p.emb_eps), bounds, int(B), int(L), int(T), int(hidden), dt, mt, x.data_ptr(), s));
     auto ptr = [](const at::Tensor& t) { return t.data_ptr(); };
-    auto norm = [&](const at::Tensor& d, const at::Tensor& bias, const at::Tensor& res, const at::Tensor& g, const at::Tensor& b, double eps, at::Tensor& out, int mt_out) {
+    auto norm = [&](const at::Tensor& d, int splits, const at::Tensor& bias, const at::Tensor& res, const at::Tensor& g, const at::Tensor& b, double eps, at::Tensor& out, int mt_out) {
         must(g_enc.add_norm(ptr(d), splits, ptr(bias), ptr(res), ptr(g), ptr(b), float(eps), int(T), int(hidden), dt, mt, mt_out, ptr(out), s));
     };
     for (const Layer& w : p.layers) {
         if (small) must(g_enc.small_gemm(ptr(x), ptr(w.wqkv), ptr(w.bqkv), TDB_ENC_IN, 0, int(T), int(3 * hidden), int(hidden), dt, ptr(qkv), s));
+        else if (own) must(g_enc.gemm(ptr(x), ptr(w.wqkv), ptr(w.bqkv), 0, 1, int(T), int(3 * hidden), int(hidden), dt, ptr(qkv), s));
         else qkv = at::addmm(w.bqkv, x, w.wqkv.t());
         tdb_pos_args pos;
         memset(&pos, 0, sizeof(pos));
@@ -267,16 +273,25 @@ at::Tensor encode(const Plan& p, const at::Tensor& ids, const at::Tensor* cu, in
         at::Tensor& out = &w == &p.layers.back() ? last : x;
         const int mt_out = &w == &p.layers.back() ? 0 : mt;
         if (small) {
-            must(g_enc.small_gemm(ptr(attended), ptr(w.wo), nullptr, 0, splits, int(T), int(hidden), int(hidden), dt, ptr(part), s));
-            norm(part, w.bo, x, w.g1, w.b1, w.eps1, y, mt);
+            must(g_enc.small_gemm(ptr(attended), ptr(w.wo), nullptr, 0, few, int(T), int(hidden), int(hidden), dt, ptr(part), s));
+            norm(part, few, w.bo, x, w.g1, w.b1, w.eps1, y, mt);
             must(g_enc.small_gemm(ptr(y), ptr(w.wi), ptr(w.bi), TDB_ENC_IN | TDB_ENC_OUT | TDB_ENC_GELU, 0, int(T), int(inner), int(hidden), dt, ptr(ff), s));
-            must(g_enc.small_gemm(ptr(ff), ptr(w.wf), nullptr, TDB_ENC_IN, splits, int(T), int(hidden), int(inner), dt, ptr(part), s));
-            norm(part, w.bf, y, w.g2, w.b2, w.eps2, out, mt_out);
+            must(g_enc.small_gemm(ptr(ff), ptr(w.wf), nullptr, TDB_ENC_IN, few, int(T), int(hidden), int(inner), dt, ptr(part), s));
+            norm(part, few, w.bf, y, w.g2, w.b2, w.eps2, out, mt_out);
+        } else if (own) {
+            auto product = [&](const at::Tensor& in, const at::Tensor& weight, const at::Tensor& bias, int splits, int64_t k) {
+                at::Tensor& d = splits > 1 ? part : proj;
+                must(g_enc.gemm(ptr(in), ptr(weight), ptr(bias), 0, splits, int(T), int(hidden), int(k), dt, ptr(d), s));
+                return d;
+            };
+            norm(product(attended, w.wo, w.bo, splits_o, hidden), splits_o > 1 ? splits_o : 0, w.bo, x, w.g1, w.b1, w.eps1, y, 0);
+            must(g_enc.gemm(ptr(y), ptr(w.wi), ptr(w.bi), TDB_ENC_GELU, 1, int(T), int(inner), int(hidden), dt, ptr(ff), s));
+            norm(product(ff, w.wf, w.bf, splits_f, inner), splits_f > 1 ? splits_f : 0, w.bf, y, w.g2, w.b2, w.eps2, out, 0);
         } else {
-            norm(at::addmm(w.bo, attended, w.wo.t()), w.bo, x, w.g1, w.b1, w.eps1, y, 0);
+            norm(at::addmm(w.bo, attended, w.wo.t()), 0, w.bo, x, w.g1, w.b1, w.eps1, y, 0);
             at::Tensor f = at::addmm(w.bi, y, w.wi.t());
             at::gelu_(f);
-            norm(at::addmm(w.bf, f, w.wf.t()), w.bf, y, w.g2, w.b2, w.eps2, out, 0);
+            norm(at::addmm(w.bf, f, w.wf.t()), 0, w.bf, y, w.g2, w.b2, w.eps2, out, 0);
         }
     }
     if (!cu) return last.view({B, L, hidden});
@@ -399,14 +414,16 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // bind_encoder(addresses of the tdb_enc_* functions in the order of Enc)
 PyObject* py_bind_encoder(PyObject*, PyObject* args) {
-    unsigned long long f[6];
-    if (!PyArg_ParseTuple(args, "KKKKKK", f, f + 1, f + 2, f + 3, f + 4, f + 5)) return nullptr;
+    unsigned long long f[8];
+    if (!PyArg_ParseTuple(args, "KKKKKKKK", f, f + 1, f + 2, f + 3, f + 4, f + 5, f + 6, f + 7)) return nullptr;
     g_enc.scan_mask = reinterpret_cast<decltype(g_enc.scan_mask)>(f[0]);
     g_enc.embed = reinterpret_cast<decltype(g_enc.embed)>(f[1]);
     g_enc.add_norm = reinterpret_cast<decltype(g_enc.add_norm)>(f[2]);
     g_enc.small_gemm = reinterpret_cast<decltype(g_enc.small_gemm)>(f[3]);
     g_enc.small_tiles = reinterpret_cast<decltype(g_enc.small_tiles)>(f[4]);
     g_enc.unpack = reinterpret_cast<decltype(g_enc.unpack)>(f[5]);
+    g_enc.gemm = reinterpret_cast<decltype(g_enc.gemm)>(f[6]);
+    g_enc.gemm_splits = reinterpret_cast<decltype(g_enc.gemm_splits)>(f[7]);
     Py_RETURN_NONE;
 }
 

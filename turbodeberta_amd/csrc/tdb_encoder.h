@@ -38,6 +38,15 @@ int tdb_enc_small_gemm(const void* x, const void* w, const void* bias, int flags
 // 16-row tiles (mt) of a product that the above takes, else 0
 int tdb_enc_small_tiles(int M, int N, int K, int dtype);
 
+// Products of any size, 16-bit, rows in order: y[M, N] = x[M, K] w[N, K]^T + bias (flags: 0 or TDB_ENC_GELU), or (splits > 1)
+// float32 partial sums [splits, M, N] without bias.  K a multiple of 64, N of 8; pointers 16-byte aligned.
+// flags >> TDB_ENC_TILE_SHIFT: 1 + the number of a tile, for tests; 0: the kernel's choice.
+enum { TDB_ENC_TILE_SHIFT = 8 };
+int tdb_enc_gemm(const void* x, const void* w, const void* bias, int flags, int splits, int M, int N, int K, int dtype, void* y,
+                 void* stream);
+// the number of partial sums that is best for a product whose reader adds them up; 0: a product that the above does not take
+int tdb_enc_gemm_splits(int M, int N, int K, int dtype);
+
 // out[b, l] = x[cu[b] + l] for l < cu[b+1] - cu[b], zeros elsewhere
 int tdb_enc_unpack(const void* x, const int32_t* cu, int B, int L, int hidden, int dtype, void* out, void* stream);
 

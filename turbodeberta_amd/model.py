@@ -409,7 +409,7 @@ def _native_plan(model):
                        mid.weight, mid.bias, out.dense.weight, out.dense.bias, out.LayerNorm.weight, out.LayerNorm.bias,
                        float(so.LayerNorm.eps), float(out.LayerNorm.eps)))
     tensors = [t for l in layers for t in l[:14] if t is not None] + [table, emb.LayerNorm.weight, emb.LayerNorm.bias]
-    if any(t.dtype != table.dtype or t.device != table.device or not (t.is_contiguous() or t.dim() == 3) for t in tensors):
+    if any(t.dtype != table.dtype or t.device != table.device or t.data_ptr() % 16 or not (t.is_contiguous() or t.dim() == 3) for t in tensors):
         return None
     plan = host.make_plan(model, layers, (table, emb.LayerNorm.weight, emb.LayerNorm.bias, float(emb.LayerNorm.eps)),
                           att.num_attention_heads, att.attention_head_size, scale, buckets, max_rel)
