@@ -86,3 +86,26 @@ def test_rows_outside_every_sequence_are_zeros(cu, longest, dtype):
         inside[a:min(b, a + longest)] = True
     assert not out[~inside.cuda()].any() and not ref[~inside.cuda()].any()
     assert_close_bf16(out, ref)
+
+
+@pytest.mark.parametrize("terms", [("c2p", "p2c"), ("c2p",), ("p2c",)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,L,buckets", [(2, 1, 256), (3, 32, 256), (2, 33, 16), (70, 65, 256), (2, 96, 16), (40, 128, 256)])
+def test_strips(B, L, buckets, dtype, terms):
+    """Strips of random values, packed, full and padded: against the vector-ALU kernel, and packed bit for bit against the
+    persistent kernel."""
+    d = {n: t.cuda() for n, t in make_inputs(L, B, 3, L, 64, 256, 512, dtype).items()}
+    g = torch.Generator(device="cuda").manual_seed(L)
+    strip = [torch.randn(B, 3, L, 2 * buckets, device="cuda", generator=g).to(dtype) if t in terms else None for t in ("c2p", "p2c")]
+    lens = torch.randint(0, L + 1, (B,), generator=torch.Generator().manual_seed(B)).int()
+    lens[0] = L
+    for kw in ({}, {"seqlens_k": lens.cuda()}):
+        got, ref = (flash_attention_with_disentangled(d["q"], d["k"], d["v"], *strip, False, SCALE, buckets, 512, force_generic=f, **kw) for f in (False, True))
+        assert_close_bf16(got, ref, f"{B} x {L}")
+    rows = lambda t: torch.cat([t[b, :, :n].transpose(0, 1) for b, n in enumerate(lens.tolist())]).contiguous() if t is not None else None
+    cu = torch.cat([torch.zeros(1, dtype=torch.long), lens.cumsum(0)]).int().cuda()
+    a, b = (flash_attention_with_disentangled_varlen(*(rows(d[n]) for n in "qkv"), *(rows(s) for s in strip), cu, cu, n, n, False, SCALE, buckets, 512)
+            for n in (L, 129))
+    assert torch.equal(a, b)
+    assert all(torch.equal(a[cu[i]:cu[i + 1]].transpose(0, 1), got_b) for i, got_b in
+               ((i, flash_attention_with_disentangled(d["q"], d["k"], d["v"], *strip, False, SCALE, buckets, 512, seqlens_k=lens.cuda())[i, :, :lens[i]]) for i in (0, B - 1)))

@@ -23,6 +23,11 @@
 //   c2p  C'^T[r, i] = K_r'[r].Q_i, lane = query -> scratch C[query][r], 8-byte stores; element (i, j) is C[i][i - j]
 //   p2c  P'^T[r, j] = Q_r'[r].K_j, lane = key   -> scratch P[key][r];                  element (i, j) is P[j][i - j]
 // The shifts read dwords and pick the halves with a byte permute whose selector depends on the lane's parity.
+//
+// STRIP: the caller has the position terms as strips (c2p[i][delta], p2c[j][delta]).  The persistent kernel's position waves
+// move them in tiles of 128; here the wave gathers the 2 x 32 x 64 elements of its step itself, into registers, a step or unit
+// ahead -- four waves a workgroup for their sake.  Measured (12 heads, bf16), persistent kernel before: 1 x 16 10.4 -> 4.8 us,
+// 30 x 64 12.3 -> 6.7, 8 x 100 10.5 -> 9.3, 32 x 96 18.4 -> 15.4, 32 x 128 18.8 -> 18.3.  Bound: the 64 gathers of a step.
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -48,6 +53,7 @@ constexpr int UQ = TDB_SHORT_TILE;      // query rows of a unit
 constexpr int BN = 64;                  // keys per step
 constexpr int MAX_T = 4;                // query tiles of the longest sequence
 constexpr int MAX_WAVES = 8;            // two per SIMD
+constexpr int STRIP_WAVES = 4;          // of the strip instances, which hold the gathered elements of a step in registers
 constexpr int RS = 72;                  // LDS row stride of 16-bit rows of 64 (144 B: conflict-free 16-byte reads)
 constexpr int CS = 100;                 // row stride of C[32 queries][96 positions]: 8-byte stores of 16 lanes on distinct banks
 constexpr int PS = 68;                  // row stride of P[64 keys][64 positions]
@@ -114,7 +120,9 @@ struct ShortArgs {
     const char *pk, *pq;
     const int32_t *lut, *bounds;            // bounds: lengths or cu_seqlens
     uint32_t qb, qh, ql, kb, kh, kl, vb, vh, vl, ob, oh, ol;      // batch (packed: token), head, row
-    uint32_t pkh, pkr, pqh, pqr;
+    uint32_t pkh, pkr, pqh, pqr;            // tables: head, row; strips: head, row of pk / pq ...
+    uint32_t pkb, pqb;                      // ... and batch (packed: token)
+    int32_t span;
     int32_t B, L, total, lut_half;
     float c_exp;                            // scale * log2(e): softmax in base 2
     int32_t T, tshift;                      // units of a sequence: tiles 0 .. T-1 of 2^tshift numbers
@@ -124,8 +132,8 @@ struct ShortArgs {
 };
 enum { FIXED = 0, LENGTHS = 1, PACKED = 2 };
 
-template <bool C2P, bool P2C, int DT, int MODE>
-__global__ __launch_bounds__(MAX_WAVES * 64) void attn_short_kernel(const ShortArgs p) {
+template <bool C2P, bool P2C, int DT, int MODE, bool STRIP>
+__global__ __launch_bounds__((STRIP ? STRIP_WAVES : MAX_WAVES) * 64) void attn_short_kernel(const ShortArgs p) {
 #pragma clang fp contract(off)              // (a product and a sum are fused here and there where the persistent kernel's are)
     using E = Elem<DT>;
     using X8 = typename E::X8;
@@ -134,11 +142,12 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void attn_short_kernel(const ShortA
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
     const int h = blockIdx.x, wg = blockIdx.y, per_head = gridDim.y;
     const int rows = 2 * UQ * p.T;          // relative positions -32T .. 32T - 1
-    // LDS: counter, tables, the waves' scratch
+    // LDS: counter, tables (strips: their columns, for positions from 64 before the first), the waves' scratch
     int* const counter = reinterpret_cast<int*>(smem_s);
     uint16_t* const sKr = reinterpret_cast<uint16_t*>(smem_s + 16);
     uint16_t* const sQr = sKr + (C2P ? rows * RS : 0);
-    uint16_t* const scratch = sQr + (P2C ? rows * RS : 0) + wave * (SCRATCH / 2);
+    int* const sD = reinterpret_cast<int*>(smem_s + 16);
+    uint16_t* const scratch = (STRIP ? sKr + 2 * (BN + rows) : sQr + (P2C ? rows * RS : 0)) + wave * (SCRATCH / 2);
 
     if (!p.single) {
         if (tid == 0) *counter = p.waves;           // (the waves' first units are their own numbers)
@@ -221,10 +230,41 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void attn_short_kernel(const ShortA
         }
     };
 
+    // Strips: the elements that a step needs, as 16-bit loads.  c2p: lane = key, query row0 + t; a load reads neighbouring
+    // columns of one row, and the scratch turns them.  p2c: lane = query, the keys that the lane's accumulator has; a load reads
+    // neighbouring columns of two rows.  Rows past the sequence read as zeros.
+    uint16_t cv[STRIP && C2P ? UQ : 1], pv[STRIP && P2C ? 2 : 1][16];
+    auto gather = [&](const Unit& u, int k0) {
+        const bool two = u.len > k0 + 32;
+        const int first = u.row0 - k0 + UQ * p.T + BN;      // sD index of row0 - k0
+        if (STRIP && P2C) {
+            const char* const base = p.pq + uint64_t(h) * p.pqh + uint64_t(u.at) * p.pqb;
+            const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, (u.len - 1) * p.pqr + 4 * p.span, 0x00020000);
+            const int* const d = sD + first + (l & 31) - 4 * (l >> 5) - 63;
+            const uint32_t row = 4 * (l >> 5) * p.pqr;
+#pragma unroll
+            for (int jt = 0; jt < 2; ++jt)
+                if (jt == 0 || two) {
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const int key = 32 * jt + 8 * (e >> 2) + (e & 3);
+                        pv[jt][e] = uint16_t(__builtin_amdgcn_raw_buffer_load_b16(rsrc, row + (k0 + key) * p.pqr + d[63 - key], 0, 0));
+                    }
+                }
+        }
+        if (STRIP && C2P) {
+            const char* const base = p.pk + uint64_t(h) * p.pkh + uint64_t(u.at) * p.pkb;
+            const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, (u.len - 1) * p.pkr + 4 * p.span, 0x00020000);
+            const int* const d = sD + first - l;
+#pragma unroll
+            for (int t = 0; t < UQ; ++t) cv[t] = uint16_t(__builtin_amdgcn_raw_buffer_load_b16(rsrc, (u.row0 + t) * p.pkr + d[t], 0, 0));
+        }
+    };
+
     // Table rows: every delta value first, then the first unit's rows, then every table row (thread: chunk tid & 7 of rows
     // (tid >> 3) + n 8 p.waves; the launcher brings enough waves for four passes).  No branches around the loads, or each
     // would wait for the last; what lies past the delta table reads as row 0.
-    constexpr int N = C2P || P2C ? 4 : 0;
+    constexpr int N = !STRIP && (C2P || P2C) ? 4 : 0;
     const int per_pass = 8 * p.waves;
     int d[4];
     {
@@ -232,6 +272,11 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void attn_short_kernel(const ShortA
         const int off = ((tid >> 3) - UQ * p.T + p.lut_half) * 4;
 #pragma unroll
         for (int n = 0; n < N; ++n) d[n] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, off + n * per_pass * 4, 0, 0);
+    }
+    if (STRIP) {
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(p.lut), 0, (2 * p.lut_half + 1) * 4, 0x00020000);
+        for (int i = tid; i < BN + rows; i += 64 * p.waves)
+            sD[i] = 2 * __builtin_amdgcn_raw_buffer_load_b32(rsrc, (i - BN - UQ * p.T + p.lut_half) * 4, 0, 0);
     }
     Unit cur = take(wave);
     if (cur.seq >= 0) {
@@ -258,6 +303,10 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void attn_short_kernel(const ShortA
                 if (P2C) *reinterpret_cast<u32x4*>(sQr + el + n * per_pass * RS) = wq[n];
             }
         __syncthreads();
+    }
+    if (STRIP) {
+        __syncthreads();
+        if (cur.seq >= 0) gather(cur, 0);
     }
 
     if (MODE == PACKED && p.gaps && wave == p.waves - 1)
@@ -307,7 +356,13 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void attn_short_kernel(const ShortA
                     *reinterpret_cast<u32x2*>(at + 8 * a) = u32x2{pack2<E>(acc[4 * a], acc[4 * a + 1]), pack2<E>(acc[4 * a + 2], acc[4 * a + 3])};
             };
             f32x16 s[2] = {zero16, zero16};
-            if (P2C) {
+            if (STRIP && P2C) {
+#pragma unroll
+                for (int jt = 0; jt < JT; ++jt)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) s[jt][e] = E::pick(pv[jt][e], E::PICK[0]);
+            }
+            if (!STRIP && P2C) {
                 asm volatile("" : "+v"(il), "+v"(hh));
 #pragma unroll
                 for (int jt = 0; jt < JT; ++jt)
@@ -335,6 +390,19 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void attn_short_kernel(const ShortA
                 for (int jt = 0; jt < JT; ++jt) s[jt] = E::mfma(kf[jt][c], qf[c], s[jt]);
             if (C2P) {                      // (after the score products, which read no scratch)
                 asm volatile("" : "+v"(il), "+v"(hh));
+                uint32_t w[JT][8];
+                if (STRIP) {
+#pragma unroll
+                    for (int t = 0; t < UQ; ++t) scratch[t * PS + l] = cv[t];
+                    wave_fence();
+#pragma unroll
+                    for (int jt = 0; jt < JT; ++jt)
+#pragma unroll
+                        for (int a = 0; a < 4; ++a) {
+                            const u32x2 x = *reinterpret_cast<const u32x2*>(scratch + il * PS + 32 * jt + 8 * a + 4 * hh);
+                            w[jt][2 * a] = x[0], w[jt][2 * a + 1] = x[1];
+                        }
+                } else {
 #pragma unroll
                 for (int y = TWO ? 0 : 1; y < 3; ++y) put(scratch + il * CS + 32 * y + 4 * hh, chain(sKr + (prow + 32 * y) * RS, qf));
                 wave_fence();
@@ -343,7 +411,6 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void attn_short_kernel(const ShortA
                 // two byte permutes per group of four and no unpacking.
                 const uint32_t swap = (il & 1) ? 0x01000302u : 0x03020504u;       // (x0 is even where il is odd)
                 const auto* at = TDB_LDS(const uint32_t, scratch) + il * (CS / 2) + ((61 + il) >> 1) - 2 * hh;
-                uint32_t w[JT][8];
 #pragma unroll
                 for (int jt = 0; jt < JT; ++jt)
 #pragma unroll
@@ -352,6 +419,7 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void attn_short_kernel(const ShortA
                         w[jt][2 * a] = __builtin_amdgcn_perm(d2, d1, swap);
                         w[jt][2 * a + 1] = __builtin_amdgcn_perm(d1, d0, swap);
                     }
+                }
 #pragma unroll
                 for (int c2 = 0; c2 < 2; ++c2) {
                     X8 one;                 // row il: key 16 c2 + 8 (e >> 2) + 4 hh + (e & 3)
@@ -373,6 +441,10 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void attn_short_kernel(const ShortA
                 load_k(nxt, 0);
                 load_q(nxt);
                 load_v(nxt, 0);
+            }
+            if (STRIP) {
+                if (k0 + 32 * JT < len) gather(cur, k0 + BN);
+                else if (nxt.seq >= 0) gather(nxt, 0);
             }
             wave_fence();
             X8 vf[2][2][2];                 // V^T through the transposing read: [key tile][16 keys][dim tile]
@@ -471,28 +543,28 @@ __global__ __launch_bounds__(MAX_WAVES * 64) void attn_short_kernel(const ShortA
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mutex;
-bool g_attr_set[kMaxDevices][24] = {{false}};
+bool g_attr_set[kMaxDevices][48] = {{false}};
 int g_cus[kMaxDevices] = {0};
 
-template <int DT, int MODE>
+template <int DT, int MODE, bool STRIP>
 const void* kernel_of(bool c2p, bool p2c) {
-    return c2p ? (p2c ? reinterpret_cast<const void*>(&attn_short_kernel<true, true, DT, MODE>) : reinterpret_cast<const void*>(&attn_short_kernel<true, false, DT, MODE>))
-               : (p2c ? reinterpret_cast<const void*>(&attn_short_kernel<false, true, DT, MODE>) : reinterpret_cast<const void*>(&attn_short_kernel<false, false, DT, MODE>));
+    return c2p ? (p2c ? reinterpret_cast<const void*>(&attn_short_kernel<true, true, DT, MODE, STRIP>) : reinterpret_cast<const void*>(&attn_short_kernel<true, false, DT, MODE, STRIP>))
+               : (p2c ? reinterpret_cast<const void*>(&attn_short_kernel<false, true, DT, MODE, STRIP>) : reinterpret_cast<const void*>(&attn_short_kernel<false, false, DT, MODE, false>));
 }
-template <int DT>
+template <int DT, bool STRIP>
 const void* kernel_of(bool c2p, bool p2c, int mode) {
-    return mode == FIXED ? kernel_of<DT, FIXED>(c2p, p2c) : mode == LENGTHS ? kernel_of<DT, LENGTHS>(c2p, p2c) : kernel_of<DT, PACKED>(c2p, p2c);
+    return mode == FIXED ? kernel_of<DT, FIXED, STRIP>(c2p, p2c) : mode == LENGTHS ? kernel_of<DT, LENGTHS, STRIP>(c2p, p2c) : kernel_of<DT, PACKED, STRIP>(c2p, p2c);
 }
 
 }  // namespace
 
 bool tdb_short_supported(const TdbKernelParams& p, int dtype) {
-    if ((dtype != TDB_BF16 && dtype != TDB_F16) || p.D != D || p.c2p || p.p2c || p.L > UQ * MAX_T) return false;
+    if ((dtype != TDB_BF16 && dtype != TDB_F16) || p.D != D || p.L > UQ * MAX_T || ((p.pk || p.pq) && (p.c2p || p.p2c))) return false;
     // byte strides in 32 bits, byte offsets inside a sequence and inside a head's table in 31
-    const int64_t lim = int64_t(1) << 31, outer[] = {p.qs_b, p.qs_h, p.ks_b, p.ks_h, p.vs_b, p.vs_h, p.os_b, p.os_h, p.pks_h, p.pqs_h};
+    const int64_t lim = int64_t(1) << 31, outer[] = {p.qs_b, p.qs_h, p.ks_b, p.ks_h, p.vs_b, p.vs_h, p.os_b, p.os_h, p.pks_h, p.pqs_h, p.c2s_b, p.c2s_h, p.p2s_b, p.p2s_h};
     for (int64_t s : outer)
         if (s >= lim) return false;
-    for (int64_t s : {p.qs_l, p.ks_l, p.vs_l, p.os_l})
+    for (int64_t s : {p.qs_l, p.ks_l, p.vs_l, p.os_l, p.c2s_l, p.p2s_l})
         if (s * 2 * (UQ * MAX_T) >= lim) return false;
     return int64_t(2) * p.span * p.pks_r * 2 < lim && int64_t(2) * p.span * p.pqs_r * 2 < lim && 2 * int64_t(p.lut_half) + 1 < lim / 4;
 }
@@ -502,29 +574,32 @@ hipError_t tdb_launch_short(const TdbKernelParams& p, int dtype, hipStream_t str
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
-    const bool c2p = p.pk != nullptr, p2c = p.pq != nullptr;
+    const bool strip = p.c2p || p.p2c, c2p = p.pk || p.c2p, p2c = p.pq || p.p2c;
     const int mode = p.varlen ? PACKED : p.seqlens ? LENGTHS : FIXED;
     ShortArgs a;
     a.q = static_cast<const char*>(p.q), a.k = static_cast<const char*>(p.k), a.v = static_cast<const char*>(p.v), a.o = static_cast<char*>(p.o);
-    a.pk = static_cast<const char*>(p.pk), a.pq = static_cast<const char*>(p.pq);
+    a.pk = static_cast<const char*>(strip ? p.c2p : p.pk), a.pq = static_cast<const char*>(strip ? p.p2c : p.pq);
     a.lut = p.lut, a.bounds = p.varlen ? p.cu_seqlens : p.seqlens;
     auto bytes = [](int64_t s) { return uint32_t(2 * s); };
     a.qb = bytes(p.varlen ? p.qs_l : p.qs_b), a.qh = bytes(p.qs_h), a.ql = bytes(p.qs_l);
     a.kb = bytes(p.varlen ? p.ks_l : p.ks_b), a.kh = bytes(p.ks_h), a.kl = bytes(p.ks_l);
     a.vb = bytes(p.varlen ? p.vs_l : p.vs_b), a.vh = bytes(p.vs_h), a.vl = bytes(p.vs_l);
     a.ob = bytes(p.varlen ? p.os_l : p.os_b), a.oh = bytes(p.os_h), a.ol = bytes(p.os_l);
-    a.pkh = bytes(p.pks_h), a.pkr = bytes(p.pks_r), a.pqh = bytes(p.pqs_h), a.pqr = bytes(p.pqs_r);
+    a.pkh = bytes(strip ? p.c2s_h : p.pks_h), a.pkr = bytes(strip ? p.c2s_l : p.pks_r);
+    a.pqh = bytes(strip ? p.p2s_h : p.pqs_h), a.pqr = bytes(strip ? p.p2s_l : p.pqs_r);
+    a.pkb = bytes(p.varlen ? p.c2s_l : p.c2s_b), a.pqb = bytes(p.varlen ? p.p2s_l : p.p2s_b), a.span = p.span;
     a.B = p.B, a.L = p.L, a.total = p.total, a.lut_half = p.lut_half;
     a.c_exp = p.scale * 1.4426950408889634f;
     a.T = (p.L + UQ - 1) / UQ;
     a.tshift = a.T > 2 ? 2 : a.T - 1;
-    const void* fn = dtype == TDB_F16 ? kernel_of<TDB_F16>(c2p, p2c, mode) : kernel_of<TDB_BF16>(c2p, p2c, mode);
+    const void* fn = dtype == TDB_F16 ? (strip ? kernel_of<TDB_F16, true>(c2p, p2c, mode) : kernel_of<TDB_F16, false>(c2p, p2c, mode))
+                                      : (strip ? kernel_of<TDB_BF16, true>(c2p, p2c, mode) : kernel_of<TDB_BF16, false>(c2p, p2c, mode));
     int cus = 0;
     {
         std::lock_guard<std::mutex> lock(g_mutex);
         if (g_cus[dev] == 0 && (hipDeviceGetAttribute(&g_cus[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || g_cus[dev] < 1)) g_cus[dev] = 1;
         cus = g_cus[dev];
-        bool& set = g_attr_set[dev][mode * 8 + (dtype == TDB_F16 ? 4 : 0) + (c2p ? 2 : 0) + (p2c ? 1 : 0)];
+        bool& set = g_attr_set[dev][(strip ? 24 : 0) + mode * 8 + (dtype == TDB_F16 ? 4 : 0) + (c2p ? 2 : 0) + (p2c ? 1 : 0)];
         if (!set) {
             e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
             if (e != hipSuccess) return e;
@@ -535,10 +610,10 @@ hipError_t tdb_launch_short(const TdbKernelParams& p, int dtype, hipStream_t str
     // four passes.  (T = 4: 8 waves and the tables fill 147 KB of LDS.)
     const int per_head = std::min(p.B, std::max(1, cus / p.H));
     const int units = (p.B + per_head - 1) / per_head << a.tshift;
-    const int waves = std::min(MAX_WAVES, std::max(std::max(4, 2 * a.T), units));
+    const int waves = std::min(strip ? STRIP_WAVES : MAX_WAVES, std::max(std::max(4, 2 * a.T), units));
     a.gaps = p.gap_cu != nullptr;
     a.waves = waves, a.single = units <= waves;
-    const size_t smem = 16 + (int(c2p) + int(p2c)) * size_t(2 * UQ * a.T * RS * 2) + size_t(waves) * SCRATCH;
+    const size_t smem = 16 + (strip ? (BN + 2 * UQ * a.T) * sizeof(int) : (int(c2p) + int(p2c)) * size_t(2 * UQ * a.T * RS * 2)) + size_t(waves) * SCRATCH;
     void* args[] = {&a};
     return hipLaunchKernel(fn, dim3(unsigned(p.H), unsigned(per_head)), dim3(waves * 64), args, smem, stream);
 }
