@@ -70,3 +70,11 @@ def test_packed(B):
                                                          pos_key_layer=d["pk"], pos_query_layer=d["pq"], force_generic=f)
                 for f in (False, True))
     assert_close_fp32(got, ref, f"B={B}")
+
+
+@pytest.mark.parametrize("terms", [("c2p", "p2c"), ("c2p",), ("p2c",), ()])
+@pytest.mark.parametrize("B,L", [(2, 1), (2, 16), (2, 33), (2, 64), (90, 17), (90, 64)])
+def test_single_key_tiles(B, L, terms):
+    """Up to 64 tokens a wave has one key tile; both query tile heights."""
+    d = {n: t.cuda() for n, t in make_inputs(L, B, 6, L, 64, 256, 512).items()}
+    assert_close_fp32(*_both(d, terms), what=f"{B} x {L} {terms}")

@@ -9,7 +9,7 @@
 // fragment is four 16-byte loads whose lanes cover 64 contiguous bytes of 16 rows), the two position terms are shifted
 // through a wave's own LDS scratch with plain 4-byte reads, and no wave waits for another until the end.
 //
-// Measured (vector-ALU kernel before): 2 x 128 x 12 heads 84 -> 8.9 us; 8 x 12 heads, lengths 96..384, 660 -> 68 us; 8 x 512
+// Measured (vector-ALU kernel before): 1 x 20 x 12 heads 24 -> 5.6 us; 2 x 128 84 -> 8.9; 8 x 12 heads, lengths 96..384, 660 -> 68 us; 8 x 512
 // full 160 us = 81 TFLOP/s without credit for the half-used outer tiles, 101 with (matrix pipe busy 65 % of the time; what is
 // left is the start and end of a workgroup, a tenth, and L2 latency that two waves per SIMD do not quite cover).
 //
@@ -20,8 +20,8 @@
 // block are only half used), QT = 1 1.375x but twice the workgroups: see tdb_launch_f32 for the rule.
 //
 // Relative positions come in 16-wide tiles as well: tile e covers r = 16e .. 16e+15, and the (query tile a, key tile b)
-// pair needs r = 16(a-b)-15 .. 16(a-b)+15, i.e. tiles a-b-1 and a-b.  A block of QT query tiles and two key tiles needs
-// QT+2 position tiles; each of their table rows K_r[delta(r)], Q_r[delta(r)] is loaded once per block and contracted
+// pair needs r = 16(a-b)-15 .. 16(a-b)+15, i.e. tiles a-b-1 and a-b.  A block of QT query tiles and KT key tiles needs
+// QT+KT position tiles; each of their table rows K_r[delta(r)], Q_r[delta(r)] is loaded once per block and contracted
 // with the query tiles (c2p) and the key tiles (p2c) that reach it.
 //   c2p  C'^T[r, i] = K_r[delta(r)].Q_i   lane = query, registers = 4 positions -> scratch C[query][r]
 //   p2c  P'^T[r, j] = Q_r[delta(r)].K_j   lane = key,   registers = 4 positions -> scratch P[key][r]
@@ -38,12 +38,11 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 constexpr int WAVES = 4;
 constexpr int D = 64;
-constexpr int KT = 2;                       // key tiles of 16 per block
-constexpr int CS = 16 * (KT + 1) + 4;       // row stride of the c2p scratch (floats): [query][48 positions]
-constexpr int PS(int qt) { return 16 * (qt + 1) + 4; }
-constexpr int scratch_floats(int qt) { return qt * 16 * CS + KT * 16 * PS(qt); }      // per wave
+constexpr int GAP_WGS = 64;                 // workgroups that look for packed rows outside every sequence
+constexpr int pos_stride(int n) { return 16 * (n + 1) + 4; }     // floats of a scratch row: n + 1 position tiles
+constexpr int scratch_floats(int qt, int kt) { return qt * 16 * pos_stride(kt) + kt * 16 * pos_stride(qt); }      // per wave
 // the merge needs QT * 1024 floats of partial sums per wave, and 2 * QT * 16 of maxima and denominators
-constexpr int wave_floats(int qt) { return scratch_floats(qt) > qt * (1024 + 32) ? scratch_floats(qt) : qt * (1024 + 32); }
+constexpr int wave_floats(int qt, int kt) { return scratch_floats(qt, kt) > qt * (1024 + 32) ? scratch_floats(qt, kt) : qt * (1024 + 32); }
 
 __device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
@@ -81,14 +80,21 @@ __device__ __forceinline__ void load_frag(f32x4 (&f)[4], const float* row, int g
     for (int t = 0; t < 4; ++t) f[t] = *reinterpret_cast<const f32x4*>(row + 16 * t + 4 * g);
 }
 
-template <int QT, bool STRIP, bool C2P, bool P2C>
+// KT: key tiles of 16 per block.
+template <int QT, int KT, bool STRIP, bool C2P, bool P2C>
 __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_kernel(const TdbKernelParams p, const int tiles_x) {
     extern __shared__ __attribute__((aligned(16))) float smem_f[];
-    constexpr int PST = PS(QT);
+    constexpr int CST = pos_stride(KT), PST = pos_stride(QT), WAVE = wave_floats(QT, KT);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
     const int c = l & 15, g = l >> 4;       // column (or row) of a tile, group of four rows
-    float* const sC = smem_f + wave * wave_floats(QT);
-    float* const sP = sC + QT * 16 * CS;
+    float* const sC = smem_f + wave * WAVE;
+    float* const sP = sC + QT * 16 * CST;
+
+    if (p.gap_cu && blockIdx.x + GAP_WGS >= gridDim.x) {
+        const int worker = (blockIdx.x + GAP_WGS - gridDim.x) * WAVES + wave;
+        tdb_fill_gaps(p.gap_cu, p.gap_B, p.L, p.total, static_cast<char*>(p.o), p.os_l * 4, p.os_h * 4, p.H, 4 * D, worker, GAP_WGS * WAVES);
+        return;
+    }
 
     // Block ids go round-robin over the 8 XCDs: four neighbouring query tiles, which read the same keys and values,
     // are kept on one of them.  The heads of a tile group follow each other (and not the tile groups of a head), so
@@ -121,14 +127,14 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
     // This wave's key tiles: blocks of KT, dealt to the waves in turn (the position rows of neighbouring blocks overlap
     // by half, and waves that work on neighbours at the same time find them in L1), or single tiles where there are few.
     const int ntiles = (len + 15) >> 4, per = (ntiles + WAVES - 1) / WAVES;
-    const bool few = per < KT;
+    const bool few = KT > 1 && per < KT;
     const int first = wave * (few ? 1 : KT), last = few ? min(first + 1, ntiles) : ntiles, stride = WAVES * KT;
 
-    // Table rows of position tile x of the block that starts at key tile bt: r = row0 - 16 bt + 16 (x - 2) + c.
-    int dl[QT + 2];
+    // Table rows of position tile x of the block that starts at key tile bt: r = row0 - 16 bt + 16 (x - KT) + c.
+    int dl[QT + KT];
     auto read_deltas = [&](int bt) {
 #pragma unroll
-        for (int x = 0; x < QT + 2; ++x) dl[x] = delta_of(row0 - 16 * bt + 16 * (x - 2) + c);
+        for (int x = 0; x < QT + KT; ++x) dl[x] = delta_of(row0 - 16 * bt + 16 * (x - KT) + c);
     };
     if (!STRIP && (C2P || P2C) && first < last) read_deltas(first);
 
@@ -153,7 +159,7 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
         for (int bi = 0; bi < KT; ++bi) load_frag(kf[bi], K + int64_t(min(16 * (bt + bi) + c, len - 1)) * p.ks_l, g);
     };
     // phases of a block: position tile x = ph / TERMS, one term after the other (c2p first)
-    constexpr int TERMS = int(C2P) + int(P2C), PHASES = STRIP ? 0 : TERMS * (QT + 2);
+    constexpr int TERMS = int(C2P) + int(P2C), PHASES = STRIP ? 0 : TERMS * (QT + KT);
     auto load_pos = [&](int ph) {
         const int x = ph / (TERMS > 0 ? TERMS : 1);
         if (C2P && (!P2C || ph % 2 == 0)) load_frag(pf[ph & 1], C + int64_t(dl[x]) * p.pks_r, g);
@@ -167,7 +173,7 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
         if (PHASES) load_pos(0);
     }
     for (int bt = first; bt < last; bt += stride) {
-        const bool two = bt + 1 < last;     // whether the block's second key tile exists
+        const bool two = KT > 1 && bt + 1 < last;     // whether the block's second key tile exists
         f32x4 s[QT][KT];
 #pragma unroll
         for (int a = 0; a < QT; ++a)
@@ -187,7 +193,8 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
                         if (P2C) s[a][bi][t] += P[int64_t(j) * p.p2s_l + d];
                     }
         } else if (C2P || P2C) {
-            // c2p: query tile a reaches position tiles a .. a+2; p2c: key tile bi reaches 1-bi .. QT+1-bi
+            // c2p: query tile a reaches position tiles a .. a+KT; p2c: key tile bi reaches KT-1-bi .. QT+KT-1-bi.
+            // (A product with a single tile is summed in two halves: a dependent MFMA waits longer than the pipe is busy.)
 #pragma unroll
             for (int ph = 0; ph < PHASES; ++ph) {
                 const int x = ph / TERMS;
@@ -195,35 +202,42 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
                 issued();
                 const f32x4(&f)[4] = pf[ph & 1];
                 if (C2P && (!P2C || ph % 2 == 0)) {
-                    f32x4 acc[QT];
+                    constexpr int HALVES = QT * KT == 1 ? 2 : 1;
+                    f32x4 acc[QT][HALVES];
 #pragma unroll
-                    for (int a = 0; a < QT; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    for (int a = 0; a < QT; ++a)
+#pragma unroll
+                        for (int n = 0; n < HALVES; ++n) acc[a][n] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int te = 0; te < 16; ++te)
 #pragma unroll
                         for (int a = 0; a < QT; ++a)
-                            if (x >= a && x <= a + 2) acc[a] = mfma(f[te >> 2][te & 3], qf[a][te >> 2][te & 3], acc[a]);
+                            if (x >= a && x <= a + KT) acc[a][te % HALVES] = mfma(f[te >> 2][te & 3], qf[a][te >> 2][te & 3], acc[a][te % HALVES]);
 #pragma unroll
                     for (int a = 0; a < QT; ++a)
-                        if (x >= a && x <= a + 2) *reinterpret_cast<f32x4*>(&sC[(16 * a + c) * CS + 16 * (x - a) + 4 * g]) = acc[a];
+                        if (x >= a && x <= a + KT)
+                            *reinterpret_cast<f32x4*>(&sC[(16 * a + c) * CST + 16 * (x - a) + 4 * g]) = HALVES > 1 ? acc[a][0] + acc[a][HALVES - 1] : acc[a][0];
                 } else {
-                    f32x4 acc[KT];
+                    constexpr int HALVES = KT == 1 ? 2 : 1;
+                    f32x4 acc[KT][HALVES];
 #pragma unroll
-                    for (int bi = 0; bi < KT; ++bi) acc[bi] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    for (int bi = 0; bi < KT; ++bi)
+#pragma unroll
+                        for (int n = 0; n < HALVES; ++n) acc[bi][n] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int te = 0; te < 16; ++te)
 #pragma unroll
                         for (int bi = 0; bi < KT; ++bi)
-                            if (x >= 1 - bi && x <= QT + 1 - bi) acc[bi] = mfma(f[te >> 2][te & 3], kf[bi][te >> 2][te & 3], acc[bi]);
+                            if (x >= KT - 1 - bi && x <= QT + KT - 1 - bi) acc[bi][te % HALVES] = mfma(f[te >> 2][te & 3], kf[bi][te >> 2][te & 3], acc[bi][te % HALVES]);
 #pragma unroll
                     for (int bi = 0; bi < KT; ++bi)
-                        if (x >= 1 - bi && x <= QT + 1 - bi)
-                            *reinterpret_cast<f32x4*>(&sP[(16 * bi + c) * PST + 16 * (x + bi - 1) + 4 * g]) = acc[bi];
+                        if (x >= KT - 1 - bi && x <= QT + KT - 1 - bi)
+                            *reinterpret_cast<f32x4*>(&sP[(16 * bi + c) * PST + 16 * (x + bi - (KT - 1)) + 4 * g]) = HALVES > 1 ? acc[bi][0] + acc[bi][HALVES - 1] : acc[bi][0];
                 }
             }
             if (bt + stride < last) read_deltas(bt + stride);
             wave_fence();
-            // query 16a + c, key 16bi + jl: position i - j sits at 32 - 16 bi + c - jl of C's row and at 16 (a + 1) + c - jl of P's
+            // query 16a + c, key 16bi + jl: position i - j sits at 16 (KT - bi) + c - jl of C's row and at 16 (a + 1) + c - jl of P's
 #pragma unroll
             for (int bi = 0; bi < KT; ++bi)
 #pragma unroll
@@ -232,7 +246,7 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
 #pragma unroll
                     for (int a = 0; a < QT; ++a) {
                         float x = 0.f;
-                        if (C2P) x = sC[(16 * a + c) * CS + 32 - 16 * bi + c - jl];
+                        if (C2P) x = sC[(16 * a + c) * CST + 16 * (KT - bi) + c - jl];
                         if (P2C) x += sP[(16 * bi + jl) * PST + 16 * (a + 1) + c - jl];
                         s[a][bi][t] = x;
                     }
@@ -245,16 +259,20 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
 #pragma unroll
             for (int t = 0; t < 4; ++t) vf[bi][t] = *reinterpret_cast<const f32x4*>(V + int64_t(min(16 * (bt + bi) + 4 * g + t, len - 1)) * p.vs_l + 4 * c);
         issued();
-#pragma unroll
-        for (int te = 0; te < 16; ++te)
-#pragma unroll
-            for (int a = 0; a < QT; ++a) s[a][0] = mfma(kf[0][te >> 2][te & 3], qf[a][te >> 2][te & 3], s[a][0]);
-        if (two) {
+        auto score = [&](int bi) {
+            constexpr int HALVES = QT * KT == 1 ? 2 : 1;
+            f32x4 rest = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int te = 0; te < 16; ++te)
 #pragma unroll
-                for (int a = 0; a < QT; ++a) s[a][1] = mfma(kf[1][te >> 2][te & 3], qf[a][te >> 2][te & 3], s[a][1]);
-        }
+                for (int a = 0; a < QT; ++a) {
+                    f32x4& sum = te % HALVES ? rest : s[a][bi];
+                    sum = mfma(kf[bi][te >> 2][te & 3], qf[a][te >> 2][te & 3], sum);
+                }
+            if (HALVES > 1) s[0][0] += rest;
+        };
+        score(0);
+        if (two) score(KT - 1);
         if (bt + stride < last) {
             load_keys(bt + stride);
             if (PHASES) load_pos(0);
@@ -297,11 +315,11 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
                     for (int u = 0; u < 4; ++u) oacc[a][u] = mfma(vf[bi][t][u], s[a][bi][t], oacc[a][u]);
         };
         pv(0);
-        if (two) pv(1);
+        if (two) pv(KT - 1);
     }
 
     // Merge of the four waves: partial sums [QT][4][64 lanes] x 16 B, then maxima and denominators of the queries.
-    float* const mine = smem_f + wave * wave_floats(QT);
+    float* const mine = smem_f + wave * WAVE;
     wave_fence();                           // (the scratch above is this wave's own)
 #pragma unroll
     for (int a = 0; a < QT; ++a) {
@@ -319,17 +337,17 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
     for (int a = 0; a < QT; ++a) {
         float f[WAVES], m = -INFINITY, den = 0.f;
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) m = fmaxf(m, smem_f[w * wave_floats(QT) + QT * 1024 + a * 32 + c]);
+        for (int w = 0; w < WAVES; ++w) m = fmaxf(m, smem_f[w * WAVE + QT * 1024 + a * 32 + c]);
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) {
-            f[w] = exp_neg(smem_f[w * wave_floats(QT) + QT * 1024 + a * 32 + c] - m);      // (0 for a wave without keys)
-            den += f[w] * smem_f[w * wave_floats(QT) + QT * 1024 + a * 32 + 16 + c];
+            f[w] = exp_neg(smem_f[w * WAVE + QT * 1024 + a * 32 + c] - m);      // (0 for a wave without keys)
+            den += f[w] * smem_f[w * WAVE + QT * 1024 + a * 32 + 16 + c];
         }
         const int row = row0 + 16 * a + c;
         const float inv = row < len ? 1.f / den : 0.f;
         f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4*>(&smem_f[w * wave_floats(QT) + ((a * 4 + wave) * 64 + l) * 4]) * f[w];
+        for (int w = 0; w < WAVES; ++w) sum += *reinterpret_cast<const f32x4*>(&smem_f[w * WAVE + ((a * 4 + wave) * 64 + l) * 4]) * f[w];
         if (row >= len) sum = f32x4{0.f, 0.f, 0.f, 0.f};
         if (row < row0 + rows_here) *reinterpret_cast<f32x4*>(O + int64_t(row) * p.os_l + 16 * g + 4 * wave) = sum * inv;
     }
@@ -348,25 +366,30 @@ hipError_t tdb_launch_f32(const TdbKernelParams& p, hipStream_t stream) {
     const bool wide = int64_t(tiles_of(32)) * p.H >= 512;
     const bool strip = p.c2p || p.p2c;
     const int tiles = tiles_of(wide ? 32 : 16);
-    const int64_t blocks = (int64_t((tiles + 3) / 4) * p.H + 7) / 8 * 32;      // groups of 4 tiles, rounded up to 8 XCDs
+    const int64_t blocks = (int64_t((tiles + 3) / 4) * p.H + 7) / 8 * 32 + (p.gap_cu ? GAP_WGS : 0);      // groups of 4 tiles, rounded up to 8 XCDs
     if (blocks > INT32_MAX) return hipErrorInvalidValue;
+    // Up to 64 tokens a wave has a single key tile: blocks of two would spend a third of their loads and products on a
+    // second one that is not there (1 x 64 8.2 -> 6.8 us).
+    const bool single = p.L <= 16 * WAVES;
     const dim3 grid{unsigned(blocks)}, block(WAVES * 64);
-    const size_t smem = sizeof(float) * WAVES * wave_floats(wide ? 2 : 1);
+    const size_t smem = sizeof(float) * WAVES * wave_floats(wide ? 2 : 1, single ? 1 : 2);
     const bool c2p = strip ? p.c2p != nullptr : p.pk != nullptr, p2c = strip ? p.p2c != nullptr : p.pq != nullptr;
-    auto launch = [&](auto qt, auto s, auto c, auto x) {
-        hipLaunchKernelGGL((attn_f32_kernel<decltype(qt)::value, decltype(s)::value, decltype(c)::value, decltype(x)::value>), grid, block, smem, stream, p, tiles);
+    auto launch = [&](auto qt, auto kt, auto s, auto c, auto x) {
+        hipLaunchKernelGGL((attn_f32_kernel<decltype(qt)::value, decltype(kt)::value, decltype(s)::value, decltype(c)::value, decltype(x)::value>), grid, block, smem, stream, p, tiles);
     };
     using std::bool_constant;
-    auto terms = [&](auto qt) {
-        if (strip && c2p && p2c) launch(qt, bool_constant<true>{}, bool_constant<true>{}, bool_constant<true>{});
-        else if (strip && c2p) launch(qt, bool_constant<true>{}, bool_constant<true>{}, bool_constant<false>{});
-        else if (strip) launch(qt, bool_constant<true>{}, bool_constant<false>{}, bool_constant<true>{});
-        else if (c2p && p2c) launch(qt, bool_constant<false>{}, bool_constant<true>{}, bool_constant<true>{});
-        else if (c2p) launch(qt, bool_constant<false>{}, bool_constant<true>{}, bool_constant<false>{});
-        else if (p2c) launch(qt, bool_constant<false>{}, bool_constant<false>{}, bool_constant<true>{});
-        else launch(qt, bool_constant<false>{}, bool_constant<false>{}, bool_constant<false>{});
+    auto terms = [&](auto qt, auto kt) {
+        if (strip && c2p && p2c) launch(qt, kt, bool_constant<true>{}, bool_constant<true>{}, bool_constant<true>{});
+        else if (strip && c2p) launch(qt, kt, bool_constant<true>{}, bool_constant<true>{}, bool_constant<false>{});
+        else if (strip) launch(qt, kt, bool_constant<true>{}, bool_constant<false>{}, bool_constant<true>{});
+        else if (c2p && p2c) launch(qt, kt, bool_constant<false>{}, bool_constant<true>{}, bool_constant<true>{});
+        else if (c2p) launch(qt, kt, bool_constant<false>{}, bool_constant<true>{}, bool_constant<false>{});
+        else if (p2c) launch(qt, kt, bool_constant<false>{}, bool_constant<false>{}, bool_constant<true>{});
+        else launch(qt, kt, bool_constant<false>{}, bool_constant<false>{}, bool_constant<false>{});
     };
-    if (wide) terms(std::integral_constant<int, 2>{});
-    else terms(std::integral_constant<int, 1>{});
+    constexpr std::integral_constant<int, 1> one;
+    constexpr std::integral_constant<int, 2> two;
+    if (wide) single ? terms(two, one) : terms(two, two);
+    else single ? terms(one, one) : terms(one, two);
     return hipGetLastError();
 }

@@ -94,9 +94,11 @@ int dispatch(const TdbKernelParams& kp, int dtype, int flags, void* stream) {
         e = tdb_launch_short(kp, dtype, s);
     } else if (any && tdb_mfma_supported(kp, dtype)) {
         e = tdb_launch_mfma(kp, dtype, s);
+    } else if (any && tdb_f32_supported(kp, dtype)) {
+        e = tdb_launch_f32(kp, s);
     } else {
         if (kp.gap_cu) e = tdb_zero_gaps(kp, dtype, s);     // (the other kernels do this themselves)
-        if (e == hipSuccess) e = any && tdb_f32_supported(kp, dtype) ? tdb_launch_f32(kp, s) : tdb_launch_generic(kp, dtype, s);
+        if (e == hipSuccess) e = tdb_launch_generic(kp, dtype, s);
     }
     if (e != hipSuccess) return fail(TDB_ERR_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
     return TDB_OK;
