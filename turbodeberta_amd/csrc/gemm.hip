@@ -49,21 +49,6 @@ struct GemmArgs {
 
 constexpr int BK = 64;                      // 128 bytes of a row: whole cache lines
 
-// v Phi(v) as v / (1 + 2^-(v r(v^2))), r a polynomial fitted here to the logarithm of Phi(v) / Phi(-v): relative error 4e-6
-// where the result exceeds 1e-6 in size, absolute 1e-8 |v| below, far inside the rounding of the 16-bit result.  11 plain
-// instructions and two quarter-rate ones per element; erff takes about 40.
-__device__ __forceinline__ float gelu(float v) {
-    const float u = v * v;
-    float r = 4.8300428e-9f;
-    r = fmaf(r, u, -3.6335534e-7f);
-    r = fmaf(r, u, 1.0997374e-5f);
-    r = fmaf(r, u, -1.5498421e-4f);
-    r = fmaf(r, u, -1.1572413e-4f);
-    r = fmaf(r, u, 0.10487763f);
-    r = fmaf(r, u, 2.3021847f);
-    return v * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-(v * r)));
-}
-
 // 64 lanes x 16 bytes from base + off (per lane) to 1 KB of LDS at `lds` (nothing else in this file uses m0)
 __device__ __forceinline__ void load_lds(uint32_t lds, const void* base, uint32_t off) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
@@ -254,7 +239,7 @@ __global__ __launch_bounds__(WM* WN * 64, 2) void gemm_kernel(GemmArgs p) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     float v = acc[i][j][4 * g + e] + float(bias[j][g][e]);
-                    if (GELU) v = gelu(v);
+                    if (GELU) v = tdb_gelu(v);
                     out[e] = T(v);
                 }
                 *reinterpret_cast<T4*>(mine + (l & 31) * STRIDE + (j * 32 + 8 * g + 4 * h) * 2) = out;

@@ -165,6 +165,21 @@ __device__ __forceinline__ bool tdb_locate_tile_sorted(const TdbKernelParams& p,
     return true;
 }
 
+// v Phi(v) as v / (1 + 2^-(v r(v^2))), r a polynomial fitted here to the logarithm of Phi(v) / Phi(-v): relative error 4e-6
+// where the result exceeds 1e-6 in size, absolute 1e-8 |v| below, far inside the rounding of the 16-bit result.  11 plain
+// instructions and two quarter-rate ones per element; erff takes about 40.
+__device__ __forceinline__ float tdb_gelu(float v) {
+    const float u = v * v;
+    float r = 4.8300428e-9f;
+    r = fmaf(r, u, -3.6335534e-7f);
+    r = fmaf(r, u, 1.0997374e-5f);
+    r = fmaf(r, u, -1.5498421e-4f);
+    r = fmaf(r, u, -1.1572413e-4f);
+    r = fmaf(r, u, 0.10487763f);
+    r = fmaf(r, u, 2.3021847f);
+    return v * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-(v * r)));
+}
+
 // Zeros for the rows of a packed output that belong to no sequence: in front of, between and behind them, and what
 // max_seqlen cuts off.  One wave of each of `workers` workgroups runs this beside the attention itself (a fill of the whole
 // output by a launch of its own took 12 us in front of a 91 us call).  Packings without gaps, all but a few, end after one
