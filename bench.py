@@ -12,9 +12,8 @@ A "step" is one attention forward over one batch of synthetic DeBERTa-v3-base at
   strips  the reference's own call signature -- c2p / p2c strips [B, H, L, 2*span] computed by the caller -- on the
           matrix-core kernel: batch 8 x seq 256 and batch 32 x seq 512, bf16, priced against HBM (the strips are
           most of the bytes)   (`strips`)
-  generic the vector-ALU kernel that serves float32 inputs and what the matrix-core kernel does not take: the
-          attention of the config-1 layer (batch 2 x seq 128, float32), and the batch 8 x seq 256 strip call forced
-          onto it for comparison   (`generic`)
+  generic the attention of the config-1 layer in float32 (batch 2 x seq 128, MFMA 16x16x4), and the batch 8 x seq 256
+          strip call forced onto the vector-ALU kernel for comparison   (`generic`)
 
 Prints ONE JSON line.  `value` is algorithmic attention TFLOP/s of the fixed workload over the timed
 region; FLOPs per sequence of valid length l and per head:  4*l*l*d (QK^T + PV) + 4*l*W*d (c2p + p2c),
@@ -48,7 +47,7 @@ BUCKETS, MAX_REL, SPAN = 256, 512, 256
 PEAK_BF16_TFLOPS = 2500.0       # MI355X dense bf16 MFMA, AMD public spec
 PEAK_HBM_GBS = 8000.0
 METRIC = "attn TFLOP/s + tokens/s, DeBERTa-v3-base b32xL512 bf16, fixed and varlen"
-PEAK_FP32_VALU_TFLOPS = 157.3   # MI355X vector fp32, AMD public spec (what the generic kernel is priced against)
+PEAK_FP32_TFLOPS = 157.3        # MI355X fp32, vector and matrix alike, AMD public spec
 # HBM bytes per launch are not measured by this script: they come from `rocprofv3 --pmc FETCH_SIZE` / `--pmc WRITE_SIZE`
 # runs of it, each counter scaled by what it reads for a plain 512 MiB device copy.  The figures, the commands, the
 # commit and a digest of the kernel source they were taken at are recorded in the files named here; `roofline.traffic`
@@ -482,8 +481,9 @@ def main():
         notes = {"config1_fp32": "attention of the config-1 layer: batch 2 x seq 128, 12 heads x 64, float32, fused tables",
                  "strips_bf16_forced": "strip-taking signature, batch 8 x seq 256, bf16, forced onto the vector-ALU kernel "
                                        "(without the flag it runs on the matrix cores: `strips.b8xL256`)"}
+        kernels = {"config1_fp32": ("attn_f32_kernel", "mfma"), "strips_bf16_forced": ("attn_generic_kernel", "valu")}
         extra["generic"] = {name: {"workload": notes[name],
-                                   **measure(pl, ln, name, "attn_generic_kernel", peak=PEAK_FP32_VALU_TFLOPS, bound="valu")}
+                                   **measure(pl, ln, name, kernels[name][0], peak=PEAK_FP32_TFLOPS, bound=kernels[name][1])}
                             for name, (pl, ln) in build_generic(dev).items()}
     head = res_fixed or res_var or extra.get("long") or next(iter((extra.get("strips") or extra["generic"]).values()))
     out.update({"value": head["value"], "ms_per_step": head["ms_per_step"], "tokens_per_s": head["tokens_per_s"],
