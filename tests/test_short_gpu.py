@@ -1,4 +1,4 @@
-"""The 16-bit kernel for short sequences (up to 128 tokens) at the edges of its units (32 query rows a wave, 64 keys a
+"""The 16-bit kernel for short sequences (up to 128 tokens, 160 in large launches) at the edges of its units (32 query rows a wave, 64 keys a
 step), against the vector-ALU kernel and bit for bit against the persistent kernel, which a longer maximum selects."""
 import math
 
@@ -40,7 +40,7 @@ def test_fixed_edges(L, dtype):
 def test_packed_same_bits_as_the_persistent_kernel(lens, terms):
     run = _packed(lens, torch.bfloat16, terms)
     got = run(max(lens))
-    assert torch.equal(got, run(129))
+    assert torch.equal(got, run(161))
     assert_close_bf16(got, run(max(lens), force_generic=True), str(terms))
 
 
@@ -105,7 +105,25 @@ def test_strips(B, L, buckets, dtype, terms):
     rows = lambda t: torch.cat([t[b, :, :n].transpose(0, 1) for b, n in enumerate(lens.tolist())]).contiguous() if t is not None else None
     cu = torch.cat([torch.zeros(1, dtype=torch.long), lens.cumsum(0)]).int().cuda()
     a, b = (flash_attention_with_disentangled_varlen(*(rows(d[n]) for n in "qkv"), *(rows(s) for s in strip), cu, cu, n, n, False, SCALE, buckets, 512)
-            for n in (L, 129))
+            for n in (L, 161))
     assert torch.equal(a, b)
     assert all(torch.equal(a[cu[i]:cu[i + 1]].transpose(0, 1), got_b) for i, got_b in
                ((i, flash_attention_with_disentangled(d["q"], d["k"], d["v"], *strip, False, SCALE, buckets, 512, seqlens_k=lens.cuda())[i, :, :lens[i]]) for i in (0, B - 1)))
+
+
+@pytest.mark.parametrize("terms", [("c2p", "p2c"), ("c2p",), ("p2c",)])
+@pytest.mark.parametrize("lens", [[129] * 70, [160] * 64, [160, 5, 129, 96, 0, 33] * 50], ids=["129", "160", "mixed"])
+def test_five_query_tiles(lens, terms):
+    run = _packed(lens, torch.bfloat16, terms)
+    got = run(max(lens))
+    assert torch.equal(got, run(161))
+    assert_close_bf16(got, run(max(lens), force_generic=True), str(terms))
+
+
+@pytest.mark.parametrize("B,L,ragged", [(50, 129, False), (50, 160, False), (110, 160, True)])
+def test_five_query_tiles_fixed(B, L, ragged):
+    d = {n: t.cuda() for n, t in make_inputs(B, B, 3, L, 64, 256, 512, torch.float16).items()}
+    lens = torch.randint(0, L + 1, (B,), generator=torch.Generator().manual_seed(B)).int().cuda() if ragged else None
+    got, ref = (flash_attention_with_disentangled(d["q"], d["k"], d["v"], None, None, False, SCALE, 256, 512, pos_key_layer=d["pk"],
+                                                  pos_query_layer=d["pq"], seqlens_k=lens, force_generic=f) for f in (False, True))
+    assert_close_bf16(got, ref, f"{B} x {L}")

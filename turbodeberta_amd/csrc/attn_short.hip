@@ -5,7 +5,7 @@
 // for the one it runs: 300 sequences of 4 to 96 tokens x 12 heads took 118 us where their bytes take 19.
 // Here a WAVE owns 32 query rows of one (sequence, head) and nothing else in the workgroup waits for it:
 //   * a workgroup belongs to one head and keeps that head's table rows K_r[delta(r)], Q_r[delta(r)] for EVERY relative
-//     position the launch can meet (2 * 32 T of them, T = ceil(max length / 32) <= 4) in LDS, loaded once;
+//     position the launch can meet (2 * 32 T of them, T = ceil(max length / 32) <= 5) in LDS, loaded once;
 //   * its waves take (sequence, query tile) units from a counter in LDS -- units differ in cost --, all tiles of a
 //     sequence going to one workgroup, so that its keys and values come from HBM once;
 //   * keys, position products and values pass through one scratch area of the wave, one after the other.
@@ -13,7 +13,8 @@
 // 128 x 96 42 -> 28, 128 x 128 43 -> 37; packed 64 of 4..32 tokens 21 -> 9, 64 of 32..128 28.6 -> 21.9, 300 of 4..96
 // 120 -> 40 (of which 6 are the zero fill of the output).  What bounds it now: a small call, the instructions and memory
 // round trips in front of its one step; a large one, LDS instructions (some 700 clk per CU and wave step) under two waves
-// per SIMD.  128 tokens are the limit because the tables of 256 relative positions and eight waves' scratch fill the LDS.
+// per SIMD.  160 tokens are the limit because the tables of 320 relative positions and seven waves' scratch fill the LDS; many_tiles
+// below says from where they pay.
 // The arithmetic is the persistent kernel's, operation for operation (64 keys per softmax step; MFMA chains over the same
 // columns in the same order; position products rounded to the element type, p2c as the initial accumulator, c2p added
 // after the score products): a sequence gives the same bits in whichever launch it travels.
@@ -51,7 +52,7 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 constexpr int D = 64;
 constexpr int UQ = TDB_SHORT_TILE;      // query rows of a unit
 constexpr int BN = 64;                  // keys per step
-constexpr int MAX_T = 4;                // query tiles of the longest sequence
+constexpr int MAX_T = 5;                // query tiles of the longest sequence
 constexpr int MAX_WAVES = 8;            // two per SIMD
 constexpr int STRIP_WAVES = 4;          // of the strip instances, which hold the gathered elements of a step in registers
 constexpr int RS = 72;                  // LDS row stride of 16-bit rows of 64 (144 B: conflict-free 16-byte reads)
@@ -258,17 +259,18 @@ __global__ __launch_bounds__((STRIP ? STRIP_WAVES : MAX_WAVES) * 64) void attn_s
     };
 
     // Table rows: every delta value first, then the first unit's rows, then every table row (thread: chunk tid & 7 of rows
-    // (tid >> 3) + n 8 p.waves; the launcher brings enough waves for four passes).  No branches around the loads, or each
+    // (tid >> 3) + n 8 p.waves; up to four query tiles the launcher brings enough waves for four passes).  No branches around the loads, or each
     // would wait for the last; what lies past the delta table reads as row 0.
     constexpr int N = !STRIP && (C2P || P2C) ? 4 : 0;
     const int per_pass = 8 * p.waves;
     int d[4];
-    {
+    auto read_deltas = [&](int first) {
         const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(p.lut), 0, (2 * p.lut_half + 1) * 4, 0x00020000);
-        const int off = ((tid >> 3) - UQ * p.T + p.lut_half) * 4;
+        const int off = (first + (tid >> 3) - UQ * p.T + p.lut_half) * 4;
 #pragma unroll
         for (int n = 0; n < N; ++n) d[n] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, off + n * per_pass * 4, 0, 0);
-    }
+    };
+    read_deltas(0);
     if (STRIP) {
         const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(p.lut), 0, (2 * p.lut_half + 1) * 4, 0x00020000);
         for (int i = tid; i < BN + rows; i += 64 * p.waves)
@@ -282,22 +284,27 @@ __global__ __launch_bounds__((STRIP ? STRIP_WAVES : MAX_WAVES) * 64) void attn_s
     }
     __builtin_amdgcn_sched_barrier(0);      // (left alone, the scheduler sinks every load to its use)
     if (N) {
-        u32x4 wk[4], wq[4];
         const uint32_t ch = (tid & 7) * 16;
         const char *const pk = p.pk + uint64_t(h) * p.pkh, *const pq = p.pq + uint64_t(h) * p.pqh;
+        for (int first = 0;;) {
+            u32x4 wk[4], wq[4];
 #pragma unroll
-        for (int n = 0; n < N; ++n) {
-            if (C2P) wk[n] = *reinterpret_cast<const u32x4*>(pk + (uint32_t(d[n]) * p.pkr + ch));
-            if (P2C) wq[n] = *reinterpret_cast<const u32x4*>(pq + (uint32_t(d[n]) * p.pqr + ch));
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        const int el = (tid >> 3) * RS + (tid & 7) * 8;
-#pragma unroll
-        for (int n = 0; n < N; ++n)
-            if ((tid >> 3) + n * per_pass < rows) {
-                if (C2P) *reinterpret_cast<u32x4*>(sKr + el + n * per_pass * RS) = wk[n];
-                if (P2C) *reinterpret_cast<u32x4*>(sQr + el + n * per_pass * RS) = wq[n];
+            for (int n = 0; n < N; ++n) {
+                if (C2P) wk[n] = *reinterpret_cast<const u32x4*>(pk + (uint32_t(d[n]) * p.pkr + ch));
+                if (P2C) wq[n] = *reinterpret_cast<const u32x4*>(pq + (uint32_t(d[n]) * p.pqr + ch));
             }
+            __builtin_amdgcn_sched_barrier(0);
+            const int row = first + (tid >> 3), el = row * RS + (tid & 7) * 8;
+#pragma unroll
+            for (int n = 0; n < N; ++n)
+                if (row + n * per_pass < rows) {
+                    if (C2P) *reinterpret_cast<u32x4*>(sKr + el + n * per_pass * RS) = wk[n];
+                    if (P2C) *reinterpret_cast<u32x4*>(sQr + el + n * per_pass * RS) = wq[n];
+                }
+            first += 4 * per_pass;
+            if (first >= rows) break;       // (five query tiles take a second turn)
+            read_deltas(first);
+        }
         __syncthreads();
     }
     if (STRIP) {
@@ -602,8 +609,21 @@ const void* kernel_of(bool c2p, bool p2c, int mode) {
 
 }  // namespace
 
+// Above 128 tokens the persistent kernel has two tiles of 128 rows per sequence, each two key steps dearer than its three; one
+// round of tiles over the CUs is still quicker than three steps of a wave here (8 x 160: 11.5 against 13.7 us), two are not
+// (11 x 160 18.1 against 13.8, packed 150 of 10..160, three launches there, 73.9 against 43.9).  Where the lengths differ a tile
+// is half as many steps and the line lies higher (packed 32 of 30..140: 17 either way).  Strips stay there (4 x 140 12.6 against
+// 18.2: their gathers are shared out over four waves).
+static bool many_tiles(const TdbKernelParams& p) {
+    if (p.c2p || p.p2c) return false;
+    const int64_t BH = int64_t(p.B) * p.H;
+    if (p.varlen ? 10 * int64_t(p.total) > 9 * int64_t(p.B) * p.L : !p.seqlens) return 2 * BH > 256;
+    return (p.varlen ? int64_t(p.H) * (p.total / 128) + BH / 2 : BH * 3 / 2) > 448;
+}
+
 bool tdb_short_supported(const TdbKernelParams& p, int dtype) {
     if ((dtype != TDB_BF16 && dtype != TDB_F16) || p.D != D || p.L > UQ * MAX_T || ((p.pk || p.pq) && (p.c2p || p.p2c))) return false;
+    if (p.L > 128 && !many_tiles(p)) return false;
     // byte strides in 32 bits, byte offsets inside a sequence and inside a head's table in 31
     const int64_t lim = int64_t(1) << 31, outer[] = {p.qs_b, p.qs_h, p.ks_b, p.ks_h, p.vs_b, p.vs_h, p.os_b, p.os_h, p.pks_h, p.pqs_h, p.c2s_b, p.c2s_h, p.p2s_b, p.p2s_h};
     for (int64_t s : outer)
@@ -635,7 +655,7 @@ hipError_t tdb_launch_short(const TdbKernelParams& p, int dtype, hipStream_t str
     a.B = p.B, a.L = p.L, a.total = p.total, a.lut_half = p.lut_half;
     a.c_exp = p.scale * 1.4426950408889634f;
     a.T = (p.L + UQ - 1) / UQ;
-    a.tshift = a.T > 2 ? 2 : a.T - 1;
+    a.tshift = a.T > 4 ? 3 : a.T > 2 ? 2 : a.T - 1;
     const void* fn = dtype == TDB_F16 ? (strip ? kernel_of<TDB_F16, true>(c2p, p2c, mode) : kernel_of<TDB_F16, false>(c2p, p2c, mode))
                                       : (strip ? kernel_of<TDB_BF16, true>(c2p, p2c, mode) : kernel_of<TDB_BF16, false>(c2p, p2c, mode));
     int cus = 0;
@@ -654,7 +674,7 @@ hipError_t tdb_launch_short(const TdbKernelParams& p, int dtype, hipStream_t str
     // four passes.  (T = 4: 8 waves and the tables fill 147 KB of LDS.)
     const int per_head = std::min(p.B, std::max(1, cus / p.H));
     const int units = (p.B + per_head - 1) / per_head << a.tshift;
-    const int waves = std::min(strip ? STRIP_WAVES : MAX_WAVES, std::max(std::max(4, 2 * a.T), units));
+    const int waves = std::min(strip ? STRIP_WAVES : a.T > 4 ? MAX_WAVES - 1 : MAX_WAVES, std::max(std::max(4, 2 * a.T), units));
     a.gaps = p.gap_cu != nullptr;
     a.waves = waves, a.single = units <= waves;
     const size_t smem = 16 + (strip ? (BN + 2 * UQ * a.T) * sizeof(int) : (int(c2p) + int(p2c)) * size_t(2 * UQ * a.T * RS * 2)) + size_t(waves) * SCRATCH;
