@@ -117,6 +117,30 @@ def test_steps_aside_and_comes_back():
     assert model._forward_native(ids, mask) is None                            # gradients on
 
 
+class _LastHidden(torch.nn.Module):
+    def __init__(self, model):
+        super().__init__()
+        self.model = model
+
+    def forward(self, ids, mask):
+        return self.model(input_ids=ids, attention_mask=mask).last_hidden_state
+
+
+@pytest.mark.parametrize("lens", [[30, 7, 12], [30, 30, 30]])
+def test_traced_model_replays_on_other_inputs(lens):
+    model = _model(torch.float32)
+    run = _LastHidden(model).eval()
+    with torch.no_grad():
+        example = _ids(lens, 30)
+        run(*example)
+        traced = torch.jit.trace(run, example, check_trace=False)
+        for other in ([30, 7, 12], [3, 30, 29], [1, 1, 1]):
+            ids, mask = _ids(other, 30)
+            ids = torch.where(ids > 0, 500 - ids, 0)
+            got, v = traced(ids, mask), mask.bool()
+            torch.testing.assert_close(got[v], _both(model, ids, mask)[1][v], rtol=1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("dtype,code", [(torch.bfloat16, 1), (torch.float16, 2)])
 @pytest.mark.parametrize("tile", range(7))
 def test_product_tiles(tile, dtype, code):

@@ -73,3 +73,28 @@ def test_calls_left_to_the_python_path(odd):
     elif odd == "empty":
         a[:3] = [t[:0] for t in a[:3]]
     assert _lib.host().fixed(*a) is None
+
+
+@pytest.mark.parametrize("form", ["tables", "lengths", "strips", "packed"])
+def test_traced_operators_replay_on_other_inputs(form):
+    """A trace holds the call and not its result."""
+    def call(q, k, v, pk, pq, n):
+        if form == "packed":
+            rows = lambda t: t[0].transpose(0, 1)
+            return fv.flash_attention_with_disentangled_varlen(rows(q), rows(k), rows(v), None, None, n, n, 70, 70, False, SCALE, 256, 512,
+                                                               pos_key_layer=pk, pos_query_layer=pq)
+        strips, tables = (None, None), dict(pos_key_layer=pk, pos_query_layer=pq)
+        if form == "strips":
+            strips, tables = (torch.matmul(x, t.transpose(-1, -2).contiguous()) for x, t in ((q, pk), (k, pq))), {}
+        return fa.flash_attention_with_disentangled(q, k, v, *strips, False, SCALE, 256, 512, seqlens_k=n if form == "lengths" else None, **tables)
+
+    def inputs(seed, split):
+        d, _ = _call(seed)
+        n = [0, split, 70] if form == "packed" else [70, split]
+        return d["q"], d["k"], d["v"], d["pk"], d["pq"], torch.tensor(n, dtype=torch.int32, device="cuda")
+
+    call(*inputs(0, 30))                        # (the front takes the call from here on: it has its position table)
+    traced = torch.jit.trace(call, inputs(0, 30), check_trace=False)
+    for seed, split in [(1, 30), (2, 9)]:
+        a = inputs(seed, split)
+        assert torch.equal(traced(*a), call(*a))

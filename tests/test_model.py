@@ -136,6 +136,22 @@ def test_declared_masks_are_not_inspected():
             declare_right_padded(holes, bad)
 
 
+def test_traced_masks_are_measured_in_every_replay():
+    """Lengths, boundaries and packing follow the replay's mask, also where the example has been measured before."""
+    from turbodeberta_amd.model import _boundaries, _mask_info, _packing_of
+    example, other = torch.tensor([[1, 1, 1, 0], [1, 1, 0, 0]]), torch.tensor([[1, 0, 0, 0], [1, 1, 1, 1]])
+    _boundaries(_mask_info(example))
+
+    def measure(mask):
+        info = _mask_info(mask)
+        return info.lengths, *_packing_of(info, 2, 4, mask.device)
+
+    traced = torch.jit.trace(measure, (example,), check_trace=False)
+    lengths, indices, cu = traced(other)
+    assert lengths.tolist() == [1, 4] and cu.tolist() == [0, 1, 5] and indices.tolist() == [0, 4, 5, 6, 7]
+    assert _mask_info(example).lengths.tolist() == [3, 2]
+
+
 def test_model_passes_the_hidden_state_wish_as_an_argument():
     """The model tells the encoder per call (not through module state) whether the layers' outputs are wanted."""
     m = FlashDebertaV2Model(_tiny()).eval()

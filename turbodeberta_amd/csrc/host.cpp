@@ -4,13 +4,14 @@
 // What bounds a small call is the host: packing ~60 fields through ctypes, torch.autograd.Function and the Python
 // checks took 23 us per call where the kernel takes 8 (batch 1, 29 tokens).  Here the same call costs the output's
 // allocation and the launch.  Anything out of the ordinary -- a wrong shape or type, a tensor that needs a copy, a
-// gradient to record, another device than the current one, a tensor subclass -- returns None, and the caller takes
-// the Python path (ops/*.py: prepare), which copies, switches the device, or raises the error.
+// gradient to record, another device than the current one, a tensor subclass, a tracer or dispatch mode -- returns None,
+// and the caller takes the Python path (ops/*.py: prepare), which copies, switches the device, or raises the error.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
 #include <ATen/ATen.h>
 #include <ATen/ExpandUtils.h>
+#include <ATen/TracerMode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/GradMode.h>
 #include <c10/hip/HIPFunctions.h>
@@ -204,7 +205,7 @@ PyObject* finish(int rc, at::Tensor&& o) {
 // fixed(q, k, v, q_pos, k_pos, causal, sm_scale, position_buckets, max_relative_distance, pos_key_layer,
 //       pos_query_layer, seqlens_k, force_generic)
 PyObject* py_fixed(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-    if (nargs != 13 || !g_fixed || c10::impl::dispatch_mode_enabled()) Py_RETURN_NONE;
+    if (nargs != 13 || !g_fixed || tdb_host_observed()) Py_RETURN_NONE;
     try {
         bool ok = true, causal, generic;
         Common c;
@@ -246,7 +247,7 @@ PyObject* py_fixed(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 // varlen(q, k, v, q_pos, k_pos, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, causal, sm_scale,
 //        position_buckets, max_relative_distance, pos_key_layer, pos_query_layer, force_generic, zero_output)
 PyObject* py_varlen(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-    if (nargs != 17 || !g_varlen || c10::impl::dispatch_mode_enabled()) Py_RETURN_NONE;
+    if (nargs != 17 || !g_varlen || tdb_host_observed()) Py_RETURN_NONE;
     try {
         bool ok = true, causal, generic, zero;
         Common c;
@@ -310,7 +311,11 @@ PyObject* py_add_lut(PyObject*, PyObject* args) {
     Py_RETURN_NONE;
 }
 
+// observed(): see tdb_host_observed
+PyObject* py_observed(PyObject*, PyObject*) { return PyBool_FromLong(tdb_host_observed()); }
+
 PyMethodDef kMethods[] = {
+    {"observed", py_observed, METH_NOARGS, nullptr},
     {"bind", py_bind, METH_VARARGS, nullptr},
     {"add_lut", py_add_lut, METH_VARARGS, nullptr},
     {"fixed", reinterpret_cast<PyCFunction>(py_fixed), METH_FASTCALL, nullptr},
@@ -323,6 +328,8 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, kMethods};
 
 int (*tdb_host_fixed())(const tdb_fixed_args*, void*) { return g_fixed; }
 int (*tdb_host_varlen())(const tdb_varlen_args*, void*) { return g_varlen; }
+
+bool tdb_host_observed() { return c10::impl::dispatch_mode_enabled() || at::tracer::impl::is_dispatch_enabled(); }
 
 bool tdb_host_fill_tables(tdb_pos_args& pos, const at::Tensor* pk, const at::Tensor* pq, int64_t buckets, int64_t max_rel, int64_t max_len, int device) {
     if (!pk && !pq) return true;

@@ -14,4 +14,8 @@ int (*tdb_host_varlen())(const tdb_varlen_args*, void*);
 // for this length is at hand.  No tables: nothing is filled.
 bool tdb_host_fill_tables(tdb_pos_args& pos, const at::Tensor* pk, const at::Tensor* pq, int64_t buckets, int64_t max_rel, int64_t max_len, int device);
 
+// Whether somebody records the operations of this thread (a tracer, a dispatch mode): a result made here would be a constant
+// to a tracer and nothing at all to a mode.
+bool tdb_host_observed();
+
 bool tdb_host_add_encoder(PyObject* module);

@@ -355,7 +355,7 @@ PyObject* py_plan_ok(PyObject*, PyObject* const* args, Py_ssize_t n) {
 // scan_mask(mask [B, L]) -> (lengths, cu_seqlens, right_padded, total, ones), or None for a mask it does not take.  Waits for the GPU.
 PyObject* py_scan_mask(PyObject*, PyObject* const* args, Py_ssize_t n) {
     TDB_TRY
-    if (n != 1 || !THPVariable_CheckExact(args[0])) Py_RETURN_NONE;
+    if (n != 1 || tdb_host_observed() || !THPVariable_CheckExact(args[0])) Py_RETURN_NONE;
     const at::Tensor& m = THPVariable_Unpack(args[0]);
     const int type = m.is_cuda() ? mask_type(m.scalar_type()) : -1;
     if (type < 0 || m.dim() != 2 || m.size(0) < 1 || m.size(0) > TDB_SCAN_MAX_BATCH || m.size(1) < 1 || m.size(1) > INT32_MAX ||
@@ -396,7 +396,7 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     TDB_TRY
     Plan* p = n == 4 ? plan_of(args[0]) : nullptr;
     if (!p) return nullptr;
-    if (!THPVariable_CheckExact(args[1]) || c10::GradMode::is_enabled()) Py_RETURN_NONE;
+    if (tdb_host_observed() || !THPVariable_CheckExact(args[1]) || c10::GradMode::is_enabled()) Py_RETURN_NONE;
     const at::Tensor& ids = THPVariable_Unpack(args[1]);
     const at::Tensor* cu = args[2] == Py_None ? nullptr : &THPVariable_Unpack(args[2]);
     const int64_t T = PyLong_AsLongLong(args[3]);

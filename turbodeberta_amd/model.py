@@ -79,11 +79,12 @@ def _version_of(t):
 class _MaskInfo:
     """What the fused paths need to know about an attention mask: ``lengths`` int32 ``[B]`` on the device,
     ``total``, the number of valid tokens (a host int; ``None`` when the caller declared the lengths without it), the
-    running sum ``cu`` of the lengths (or None: not computed yet) and whether every nonzero entry is 1 (None: unknown)."""
-    __slots__ = ("lengths", "total", "cu", "ones")
+    running sum ``cu`` of the lengths (or None: not computed yet), whether every nonzero entry is 1 (None: unknown) and
+    whether the caller declared all this."""
+    __slots__ = ("lengths", "total", "cu", "ones", "declared")
 
-    def __init__(self, lengths, total, cu=None, ones=None):
-        self.lengths, self.total, self.cu, self.ones = lengths, total, cu, ones
+    def __init__(self, lengths, total, cu=None, ones=None, declared=False):
+        self.lengths, self.total, self.cu, self.ones, self.declared = lengths, total, cu, ones, declared
 
 
 def _mask_info(attention_mask):
@@ -94,10 +95,12 @@ def _mask_info(attention_mask):
     same for every head; other shapes raise ``ValueError`` in ``key_padding_mask``.  The check costs one host synchronisation per mask object;
     the result is attached to the tensor, so the layers of an encoder, which all receive the same mask object
     (modeling_deberta_v2.py:651-660), share it.  (A mask without a modification counter -- an inference tensor --
-    is trusted not to be modified in place between calls.)"""
+    is trusted not to be modified in place between calls.)  Under ``torch.jit.trace`` nothing is attached or taken from an
+    earlier call: to the tracer such lengths are constants, and a replay on another mask would go by the first one's."""
     version = _version_of(attention_mask)
+    tracing = torch.jit.is_tracing()
     cached = getattr(attention_mask, "_tdb_info", None)
-    if cached is not None and cached[0] == version:
+    if cached is not None and cached[0] == version and (cached[1].declared or not tracing):
         return cached[1]
     scan = _lib.host().scan_mask(attention_mask) if attention_mask.is_cuda and attention_mask.dim() == 2 else None
     if scan is not None:                                             # one kernel, one synchronisation
@@ -120,6 +123,8 @@ def _mask_info(attention_mask):
                          "heads: the fused attention takes per-sequence lengths.  Use the eager Hugging Face modules for "
                          "other masks.")
     info = _MaskInfo(lengths, int(total), cu, ones)
+    if tracing:
+        return info
     try:
         attention_mask._tdb_info = (version, info)
     except AttributeError:      # tensor subclasses without a __dict__
@@ -139,21 +144,28 @@ def declare_right_padded(attention_mask, lengths, total=None):
         raise ValueError("lengths must be an int32 tensor with one entry per sequence of the mask")
     if lengths.device != attention_mask.device:
         raise ValueError("lengths must live on the mask's device")
-    attention_mask._tdb_info = (_version_of(attention_mask), _MaskInfo(lengths, None if total is None else int(total), ones=True))
+    attention_mask._tdb_info = (_version_of(attention_mask), _MaskInfo(lengths, None if total is None else int(total), ones=True, declared=True))
     return attention_mask
 
 
 def _boundaries(info):
     """int32 ``[B+1]`` running sum of the lengths, with a leading 0."""
-    if info.cu is None:
-        info.cu = torch.nn.functional.pad(torch.cumsum(info.lengths, dim=0, dtype=torch.int32), (1, 0))
-    return info.cu
+    if info.cu is not None and not torch.jit.is_tracing():
+        return info.cu
+    cu = torch.nn.functional.pad(torch.cumsum(info.lengths, dim=0, dtype=torch.int32), (1, 0))
+    if not torch.jit.is_tracing():
+        info.cu = cu
+    return cu
 
 
 def _packing_of(info, batch, seqlen, device):
     """``(indices, cu_seqlens)`` of a verified right-padded batch without a further synchronisation: positions of the
-    valid tokens in the flattened ``[B*L]`` batch, int32 boundaries with a leading 0."""
+    valid tokens in the flattened ``[B*L]`` batch, int32 boundaries with a leading 0.  (Under ``torch.jit.trace`` their
+    number is found again in every replay.)"""
     cu = _boundaries(info)
+    if torch.jit.is_tracing():
+        valid = torch.arange(seqlen, device=device)[None, :] < info.lengths[:, None]
+        return torch.nonzero(valid.flatten()).flatten(), cu
     seq = torch.repeat_interleave(torch.arange(batch, device=device), info.lengths.long(), output_size=info.total)
     indices = torch.arange(info.total, device=device) - cu[:-1].long()[seq] + seq * seqlen
     return indices, cu
@@ -496,10 +508,11 @@ class FlashDebertaV2Model(DebertaV2Model):
 
     def _forward_native(self, input_ids, attention_mask):
         """The last hidden state through the native loop, or None where the modules have to be run: with gradients, in
-        training mode, under autocast or a compiler, with hooks, for masks other than 2-D ones of zeros and ones.  As in the
-        packed encoder, padded positions come back as zeros."""
+        training mode, under autocast, a compiler, a tracer or a dispatch mode, with hooks, for masks other than 2-D ones of
+        zeros and ones.  As in the packed encoder, padded positions come back as zeros."""
         if (self.training or torch.is_grad_enabled() or not input_ids.is_cuda or input_ids.dim() != 2 or not input_ids.numel()
-                or not getattr(self.encoder, "pack_sequences", False) or torch.is_autocast_enabled() or torch.compiler.is_compiling()):
+                or not getattr(self.encoder, "pack_sequences", False) or torch.is_autocast_enabled() or torch.compiler.is_compiling()
+                or _lib.host().observed()):
             return None
         B, L = input_ids.shape
         if attention_mask is not None and (attention_mask.shape != input_ids.shape or not attention_mask.is_cuda):
