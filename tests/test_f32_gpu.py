@@ -30,6 +30,45 @@ def test_tile_edges(B, H, L):
         assert_close_fp32(got, oracle_fixed(cpu, 256, 512), f"L={L} oracle")
 
 
+NAN, INF = float("nan"), float("inf")
+
+
+@pytest.mark.parametrize("where", ["query", "key", "value", "last_value", "c2p_row", "p2c_row", "score", "low_scores", "padding"])
+@pytest.mark.parametrize("B,H,L", [(2, 2, 50), (2, 2, 130), (33, 16, 77)])
+def test_nan_and_infinity_reach_what_they_belong_to(where, B, H, L):
+    """As in the definition: a key that is NaN leaves no query of its sequence a number, a position row that is NaN none that
+    meets it, a value its own columns; scores of -infinity (a whole block of them too) weigh nothing; padding is not read."""
+    d = make_inputs(5, B, H, L, 64, 256, 512)
+    lens = None
+    if where == "query":
+        d["q"][1, 0, 3, 7] = NAN
+    elif where == "key":
+        d["k"][1, 1, L - 1, 0] = NAN
+    elif where == "value":
+        d["v"][0, 1, 5, 9] = NAN
+    elif where == "last_value":
+        d["v"][0, 0, L - 1, 2], d["v"][1, 1, L - 1, 63] = INF, -INF
+    elif where == "c2p_row":
+        d["pk"][1, 256 + 20, 4] = NAN
+    elif where == "p2c_row":
+        d["pq"][0, 256 - 30, 60] = NAN
+    elif where == "score":
+        d["q"][0, 0, 2] = d["k"][0, 0, 4] = 3e19
+    elif where == "low_scores":
+        d["q"], d["pk"], d["pq"] = d["q"].abs(), d["pk"] * 0, d["pq"] * 0
+        d["k"][:, :, :L - 9] = d["k"][0, 1] = -3e38             # (0, 1): no key left, NaN
+    elif where == "padding":
+        lens = torch.full((B,), L - 20, dtype=torch.int32)
+        d["lengths"] = lens
+    ref = oracle_fixed(d, 256, 512)
+    if where == "padding":
+        for n in "qkv":
+            d[n][:, :, L - 20:] = NAN
+    got = _both({n: t.cuda() for n, t in d.items()}, lens=None if lens is None else lens.cuda())[0].cpu()
+    assert torch.equal(got.isnan(), ref.isnan()) and ref.isnan().any() == (where not in ("last_value", "padding"))
+    torch.testing.assert_close(got, ref, rtol=1e-4, atol=1e-4, equal_nan=True)
+
+
 @pytest.mark.parametrize("terms", [("c2p",), ("p2c",), ()])
 @pytest.mark.parametrize("B,H", [(1, 2), (40, 16)])
 def test_term_subsets(terms, B, H):

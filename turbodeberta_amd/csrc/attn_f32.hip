@@ -28,6 +28,7 @@
 // The score tile S^T[j, i] (lane = query, registers = 4 keys) then starts from C[i][i-j] + P[j][i-j].
 // With strips the two starting values are read from the caller's arrays instead.
 // (Same definition as the other kernels: modeling_deberta_v2.py:243, :317-324, :337-343.)
+#include <cfloat>
 #include <type_traits>
 
 #include "tdb_internal.h"
@@ -60,9 +61,10 @@ __device__ __forceinline__ float fold_max(float x) {
 }
 // exp(x) for x <= 0 to about one unit in the last place: the hardware's base-2 exponential of the rounded x log2(e),
 // corrected to first order by what the rounding (and log2(e)'s own) left out.  A third of the instructions of expf, whose
-// range handling the softmax does not need; arguments below -1e4 (masked keys, the first block's old maximum) give 0.
+// range handling the softmax does not need; arguments below -1e4 (masked keys, the first block's old maximum) give 0, NaN
+// gives NaN (fmaxf would make a 0 of it, and of a key that is none a finite answer).
 __device__ __forceinline__ float exp_neg(float x) {
-    x = fmaxf(x, -1e4f);
+    x = __builtin_elementwise_maximum(x, -1e4f);
     const float h = x * 1.44269502f;                                              // float(log2 e)
     const float e = fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269502f, -h));            // + the rest of log2 e
     const float y = __builtin_amdgcn_exp2f(h);
@@ -146,7 +148,7 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
     float m_run[QT], l_run[QT];             // l_run: this lane's keys only
 #pragma unroll
     for (int a = 0; a < QT; ++a) {
-        m_run[a] = -INFINITY, l_run[a] = 0.f;
+        m_run[a] = -FLT_MAX, l_run[a] = 0.f;        // finite: a block whose scores are all -inf leaves no NaN behind
 #pragma unroll
         for (int u = 0; u < 4; ++u) oacc[a][u] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
@@ -278,6 +280,14 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
             if (PHASES) load_pos(0);
         }
         issued();
+        // Values past the end are zeros, not the last row again: that may be infinite, and its probability there is 0.
+        if (16 * (bt + KT) > len) {
+#pragma unroll
+            for (int bi = 0; bi < KT; ++bi)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    if (16 * (bt + bi) + 4 * g + t >= len) vf[bi][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
         // streaming softmax: this lane has keys 16 bi + 4g + t of query c
 #pragma unroll
         for (int a = 0; a < QT; ++a) {
@@ -288,9 +298,9 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
                 for (int t = 0; t < 4; ++t) {
                     const bool in = (bi == 0 || two) && 16 * (bt + bi) + 4 * g + t < len;
                     s[a][bi][t] = in ? s[a][bi][t] * p.scale : -INFINITY;
-                    mx = fmaxf(mx, s[a][bi][t]);
+                    mx = fmaxf(mx, s[a][bi][t]);        // (NaN scores pass it by and meet exp_neg)
                 }
-            const float mn = fmaxf(m_run[a], fold_max(mx));     // finite: the block's first key exists
+            const float mn = fmaxf(m_run[a], fold_max(mx));
             const float alpha = exp_neg(m_run[a] - mn);            // (0 on the first block)
             float sum = 0.f;
 #pragma unroll
@@ -335,7 +345,7 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
     __syncthreads();
 #pragma unroll
     for (int a = 0; a < QT; ++a) {
-        float f[WAVES], m = -INFINITY, den = 0.f;
+        float f[WAVES], m = -FLT_MAX, den = 0.f;
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) m = fmaxf(m, smem_f[w * WAVE + QT * 1024 + a * 32 + c]);
 #pragma unroll
