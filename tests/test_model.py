@@ -5,6 +5,8 @@ reduction, packing round trips, loud failure without a GPU.  GPU part: a two-lay
 the golden last hidden state written by Hugging Face's eager model, the eager fallback for
 ``output_attentions``, and a bf16 encoder against Hugging Face eager run on the same device."""
 import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -173,6 +175,49 @@ def test_model_passes_the_hidden_state_wish_as_an_argument():
     assert not any(k.startswith("_tdb_all") for k in vars(m.encoder))
     with pytest.raises(ValueError, match="exactly one"):
         m(input_ids=ids, inputs_embeds=torch.zeros(2, 3, 4))
+
+
+class _Twice(torch.nn.Module):
+    def forward(self, x):
+        return 2 * x
+
+
+@pytest.mark.parametrize("place", ["embeddings", "encoder.layer.0.attention.output", "encoder.layer.1.output"])
+def test_native_plan_leaves_foreign_dropouts_to_the_modules(place):
+    from turbodeberta_amd.model import _native_plan
+    with torch.no_grad():
+        assert _native_plan(FlashDebertaV2Model(_tiny()).eval()) is not None
+        m = FlashDebertaV2Model(_tiny()).eval()
+        m.get_submodule(place).dropout = _Twice().eval()
+        assert _native_plan(m) is None
+
+
+def test_native_plan_knows_methods_replaced_before_the_import():
+    code = ("import torch; f = torch.nn.LayerNorm.forward; torch.nn.LayerNorm.forward = lambda self, x: f(self, x) + 1\n"
+            "from turbodeberta_amd.model import _stock_methods; assert not _stock_methods()")
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+
+
+@pytest.mark.parametrize("cls", ["Linear", "LayerNorm", "Dropout", "DebertaV2SelfOutput", "DebertaV2Layer", "DebertaV2Embeddings", "FlashDebertaV2Encoder",
+                                 "FlashDisentangledSelfAttention"])
+@pytest.mark.parametrize("method", ["forward", "__call__", "forward_packed"])
+def test_native_plan_ends_where_a_method_is_replaced_on_its_class(cls, method, monkeypatch):
+    """With a plan at hand and without; it is back when the method is."""
+    import transformers.models.deberta_v2.modeling_deberta_v2 as hf
+    from turbodeberta_amd import model as ours
+    owner = next(getattr(m, cls) for m in (ours, hf, torch.nn) if hasattr(m, cls))
+    if not hasattr(owner, method):
+        pytest.skip("no such method")
+    m = patch_model(DebertaV2Model(_tiny()).eval())
+    with torch.no_grad():
+        plan = ours._native_plan(m)
+        assert plan is not None and ours._native_plan(m) is plan
+        before = getattr(owner, method)
+        monkeypatch.setattr(owner, method, lambda *a, **k: before(*a, **k))
+        assert ours._native_plan(m) is None
+        assert ours._native_plan(FlashDebertaV2Model(_tiny()).eval()) is None
+        monkeypatch.undo()
+        assert ours._native_plan(m) is not None
 
 
 # ------------------------------------------------------------------------------------- GPU

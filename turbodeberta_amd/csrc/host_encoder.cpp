@@ -3,8 +3,9 @@
 // What bounds a short request is the host: a 48-token text through 12 layers spent 2.4 ms in Python modules and the
 // dispatch of 158 small kernels where the weights can be read in 38 us.  A *plan* holds what the loop needs of each layer
 // (weights, the concatenated Q/K/V weight, the position tables) together with a snapshot of the module tree; every call
-// first compares the tree with the snapshot -- types, children, parameters and their modification counters, training
-// flags, hooks, replaced forwards -- and a difference makes the caller build a new plan or take the modules as they are.
+// first compares the tree with the snapshot -- types and their methods, children, parameters and their modification
+// counters, training flags, hooks, replaced forwards -- and a difference makes the caller build a new plan or take the
+// modules as they are.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -49,6 +50,8 @@ PyObject* name(const char* s) { return PyUnicode_InternFromString(s); }
 struct Names {
     PyObject *training = name("training"), *forward = name("forward"), *params = name("_parameters"), *modules = name("_modules"),
              *hooks = name("_forward_hooks"), *pre_hooks = name("_forward_pre_hooks");
+    // methods of a module's type that the loop stands in for
+    PyObject* methods[4] = {forward, name("__call__"), name("forward_packed"), name("get_rel_embedding")};
 };
 const Names& names() {
     static const Names* n = new Names;
@@ -75,6 +78,12 @@ struct ModuleRef {
     std::vector<Param> params;
 };
 
+// A type of the tree and what its methods were (null: none of that name).
+struct TypeRef {
+    Owned type;
+    Owned methods[4];
+};
+
 struct Layer {
     at::Tensor wqkv, bqkv, pk, pq, wo, bo, g1, b1, wi, bi, wf, bf, g2, b2;
     double eps1, eps2;
@@ -82,6 +91,7 @@ struct Layer {
 
 struct Plan {
     std::vector<ModuleRef> tree;
+    std::vector<TypeRef> types;
     std::vector<Layer> layers;
     at::Tensor emb, emb_g, emb_b;
     double emb_eps;
@@ -125,8 +135,13 @@ bool module_ok(const ModuleRef& m) {
     return true;
 }
 
+PyTypeObject* as_type(const Owned& o) { return reinterpret_cast<PyTypeObject*>(o.get()); }
+
 bool tree_ok(const Plan& plan, PyObject* root) {
     if (plan.tree.empty() || plan.tree[0].object != root) return false;
+    for (const auto& t : plan.types)
+        for (int i = 0; i < 4; ++i)
+            if (_PyType_Lookup(as_type(t.type), names().methods[i]) != t.methods[i].get()) return false;
     for (const auto& m : plan.tree)         // parents come before their children
         if (!module_ok(m)) return false;
     return true;
@@ -143,6 +158,18 @@ bool snapshot(Plan& plan, PyObject* module) {
     plan.tree.emplace_back();
     plan.tree[at].object = module;
     plan.tree[at].type = Py_TYPE(module);
+    bool known = false;
+    for (const auto& t : plan.types) known = known || as_type(t.type) == Py_TYPE(module);
+    if (!known) {
+        TypeRef t;
+        auto own = [](Owned& to, PyObject* o) {
+            Py_XINCREF(o);
+            to.reset(o);
+        };
+        own(t.type, reinterpret_cast<PyObject*>(Py_TYPE(module)));
+        for (int i = 0; i < 4; ++i) own(t.methods[i], _PyType_Lookup(Py_TYPE(module), n.methods[i]));
+        plan.types.push_back(std::move(t));
+    }
     PyObject *k, *v;
     Py_ssize_t pos = 0;
     while (PyDict_Next(params, &pos, &k, &v)) {

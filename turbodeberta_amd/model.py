@@ -407,7 +407,7 @@ def _native_plan(model):
         _PLANS[model] = False
         return None
     _PLANS.pop(model, None)
-    if not host.tree_ready(model):               # a module in training mode, a hook, a forward of its own, ...
+    if not _stock_methods() or not host.tree_ready(model):  # a module in training mode, a hook, a forward of its own, ...
         return None
     emb, enc = model.embeddings, model.encoder
     table = emb.word_embeddings.weight
@@ -432,12 +432,14 @@ def _native_plan(model):
 
 def _known_structure(model):
     """Whether the modules below ``model`` compute what the native loop computes: stock DeBERTa-v2/v3 layers with the fused
-    attention, exact GELU, no convolution, embeddings that are a table and a LayerNorm."""
+    attention, exact GELU, no convolution, embeddings that are a table and a LayerNorm, and in the places of the dropouts
+    dropouts, which the loop leaves out."""
     emb, enc = model.embeddings, model.encoder
+    dropout = lambda m: type(m.dropout) is nn.Dropout
     plain = lambda m, *names: all(type(getattr(m, n)) is nn.Linear and getattr(m, n).bias is not None for n in names)
     norm = lambda m: type(m) is nn.LayerNorm and m.weight is not None and m.bias is not None
     if not (type(emb) is DebertaV2Embeddings and type(emb.word_embeddings) is nn.Embedding and emb.word_embeddings.max_norm is None
-            and not emb.position_biased_input and emb.token_type_embeddings is None and emb.embed_proj is None and norm(emb.LayerNorm)
+            and not emb.position_biased_input and emb.token_type_embeddings is None and emb.embed_proj is None and norm(emb.LayerNorm) and dropout(emb)
             and type(enc) is FlashDebertaV2Encoder and enc.conv is None and len(enc.layer) > 0):
         return False
     hidden = emb.word_embeddings.weight.shape[1]
@@ -448,6 +450,8 @@ def _known_structure(model):
         if not (type(layer) in (DebertaV2Layer, FlashDebertaV2Layer) and type(layer.attention) in (DebertaV2Attention, FlashDebertaV2Attention)
                 and type(layer.attention.self) is FlashDisentangledSelfAttention and type(layer.attention.output) is DebertaV2SelfOutput
                 and type(layer.intermediate) is DebertaV2Intermediate and type(layer.output) is DebertaV2Output
+                and dropout(layer.attention.self) and dropout(layer.attention.output) and dropout(layer.output)
+                and type(getattr(layer.attention.self, "pos_dropout", None)) in (nn.Dropout, type(None))
                 and type(layer.intermediate.intermediate_act_fn) is GELUActivation
                 and layer.intermediate.intermediate_act_fn.act is nn.functional.gelu):
             return False
@@ -459,6 +463,28 @@ def _known_structure(model):
                 and (att.num_attention_heads, att.pos_att_type, att.relative_attention) == (first.num_attention_heads, first.pos_att_type, first.relative_attention)):
             return False
     return True
+
+
+# The methods that the native loop was written for, as their classes' own files define them; where one has been replaced on
+# its class the modules are run.  (What happens to them later, or on an instance, the snapshot of a plan sees.)
+_LOOP_TYPES = (nn.Linear, nn.LayerNorm, nn.Embedding, nn.Dropout, GELUActivation, DebertaV2Embeddings, DebertaV2Attention, DebertaV2SelfOutput,
+               DebertaV2Intermediate, DebertaV2Output, DebertaV2Layer, FlashDebertaV2Attention, FlashDebertaV2Layer,
+               FlashDisentangledSelfAttention, FlashDebertaV2Encoder)
+
+
+def _own(cls, name):
+    """The class's method of this name (None: it has none), or an object that is nobody's method where another module put
+    it there."""
+    owner = next((c for c in cls.__mro__ if name in vars(c)), None)
+    f = owner and vars(owner)[name]
+    return f if f is None or (f.__module__ == owner.__module__ and not hasattr(f, "__wrapped__")) else object()
+
+
+_STOCK = [(cls, name, _own(cls, name)) for cls in _LOOP_TYPES for name in ("forward", "__call__", "forward_packed", "get_rel_embedding")]
+
+
+def _stock_methods():
+    return all(getattr(cls, name, None) is method for cls, name, method in _STOCK)
 
 
 class FlashDebertaV2Model(DebertaV2Model):
