@@ -4,9 +4,11 @@ CPU part: parameter names equal Hugging Face's (stock checkpoints load), in-plac
 reduction, packing round trips, loud failure without a GPU.  GPU part: a two-layer model against
 the golden last hidden state written by Hugging Face's eager model, the eager fallback for
 ``output_attentions``, and a bf16 encoder against Hugging Face eager run on the same device."""
+import gc
 import os
 import subprocess
 import sys
+import weakref
 
 import numpy as np
 import pytest
@@ -190,6 +192,36 @@ def test_native_plan_leaves_foreign_dropouts_to_the_modules(place):
         m = FlashDebertaV2Model(_tiny()).eval()
         m.get_submodule(place).dropout = _Twice().eval()
         assert _native_plan(m) is None
+
+
+@pytest.mark.parametrize("place,name,value,known", [("encoder.layer.1.output.LayerNorm", "eps", 0.5, True), ("embeddings.LayerNorm", "eps", 0.5, True),
+                                                    ("encoder.layer.0.intermediate.intermediate_act_fn", "act", torch.nn.functional.silu, False),
+                                                    ("encoder.layer.0.attention.self", "position_buckets", 8, False),
+                                                    ("embeddings.word_embeddings", "max_norm", 1.0, False)])
+def test_native_plan_follows_the_attributes_it_was_made_from(place, name, value, known):
+    from turbodeberta_amd.model import _native_plan
+    m = FlashDebertaV2Model(_tiny()).eval()
+    m.note = 0
+    with torch.no_grad():
+        plan = _native_plan(m)
+        m.note = 1                       # the caller's own, on the root
+        m.eval()
+        assert plan is not None and _native_plan(m) is plan
+        setattr(m.get_submodule(place), name, value)
+        new = _native_plan(m)
+        assert new is not plan and (new is not None) == known
+
+
+def test_native_plan_does_not_keep_its_model():
+    from turbodeberta_amd import model as ours
+    m = FlashDebertaV2Model(_tiny()).eval()
+    m.encoder.layer[0].report = lambda: m
+    with torch.no_grad():
+        assert ours._native_plan(m) is not None
+    gone = weakref.ref(m)
+    del m
+    gc.collect()
+    assert gone() is None
 
 
 def test_native_plan_knows_methods_replaced_before_the_import():

@@ -4,8 +4,8 @@
 // dispatch of 158 small kernels where the weights can be read in 38 us.  A *plan* holds what the loop needs of each layer
 // (weights, the concatenated Q/K/V weight, the position tables) together with a snapshot of the module tree; every call
 // first compares the tree with the snapshot -- types and their methods, children, parameters and their modification
-// counters, training flags, hooks, replaced forwards -- and a difference makes the caller build a new plan or take the
-// modules as they are.
+// counters, attributes, training flags, hooks, replaced forwards -- and a difference makes the caller build a new plan or
+// take the modules as they are.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -74,8 +74,14 @@ struct ModuleRef {
         uint32_t version;
         void* data;
     };
+    struct Attr {                           // what else its dictionary holds: sizes, eps, an activation's function, ...
+        Owned key, value;                   // (value: kept alive where it cannot be what keeps the model alive)
+        PyObject* object;
+    };
     std::vector<Child> children;
     std::vector<Param> params;
+    std::vector<Attr> attrs;                // (not of the root, which callers may write to as they like)
+    mutable uint64_t state;                 // of the dictionary when it last was as it should be
 };
 
 // A type of the tree and what its methods were (null: none of that name).
@@ -110,11 +116,41 @@ bool empty_dict(PyObject* dict, PyObject* key) {
     return v && PyDict_Check(v) && PyDict_GET_SIZE(v) == 0;
 }
 
-bool module_ok(const ModuleRef& m) {
+// What a module keeps for itself (its registries, which are looked at one by one, and caches).
+bool is_private(PyObject* key) {
+    return PyUnicode_Check(key) && PyUnicode_READY(key) == 0 && PyUnicode_GET_LENGTH(key) > 0 && PyUnicode_READ_CHAR(key, 0) == '_';
+}
+
+// The other attributes of an instance dictionary, in their order and by identity.
+bool attrs_ok(const ModuleRef& m, PyObject* dict) {
+    size_t n = 0;
+    PyObject *k, *v;
+    Py_ssize_t pos = 0;
+    while (PyDict_Next(dict, &pos, &k, &v)) {
+        if (n < m.attrs.size() && k == m.attrs[n].key.get() && v == m.attrs[n].object) ++n;
+        else if (!is_private(k)) return false;
+    }
+    return n == m.attrs.size();
+}
+
+// A number that no other state of any dictionary has, or 0.
+uint64_t state_of(PyObject* dict) {
+#if PY_VERSION_HEX < 0x030c0000
+    return reinterpret_cast<PyDictObject*>(dict)->ma_version_tag;
+#else
+    return 0;
+#endif
+}
+
+bool module_ok(const ModuleRef& m, bool attrs) {
     const Names& n = names();
     if (Py_TYPE(m.object) != m.type) return false;
     PyObject* d = dict_of(m.object);
-    if (!d || PyDict_GetItem(d, n.training) != Py_False || PyDict_GetItem(d, n.forward)) return false;
+    if (!d) return false;
+    if (!m.state || state_of(d) != m.state) {
+        if (PyDict_GetItem(d, n.training) != Py_False || PyDict_GetItem(d, n.forward) || (attrs && !attrs_ok(m, d))) return false;
+        m.state = state_of(d);
+    }
     if (!empty_dict(d, n.hooks) || !empty_dict(d, n.pre_hooks)) return false;
     PyObject *params = PyDict_GetItem(d, n.params), *modules = PyDict_GetItem(d, n.modules);
     if (!params || !PyDict_Check(params) || PyDict_GET_SIZE(params) != Py_ssize_t(m.params.size())) return false;
@@ -143,12 +179,12 @@ bool tree_ok(const Plan& plan, PyObject* root) {
         for (int i = 0; i < 4; ++i)
             if (_PyType_Lookup(as_type(t.type), names().methods[i]) != t.methods[i].get()) return false;
     for (const auto& m : plan.tree)         // parents come before their children
-        if (!module_ok(m)) return false;
+        if (!module_ok(m, m.object != root)) return false;
     return true;
 }
 
-// Appends `module` and what is below it; false where something cannot be held to account later.
-bool snapshot(Plan& plan, PyObject* module) {
+// Appends `module` and what is below it; false where something cannot be held to account later.  (`whole` false: to find out.)
+bool snapshot(Plan& plan, PyObject* module, bool whole) {
     const Names& n = names();
     PyObject* d = dict_of(module);
     if (!d) return false;
@@ -158,6 +194,7 @@ bool snapshot(Plan& plan, PyObject* module) {
     plan.tree.emplace_back();
     plan.tree[at].object = module;
     plan.tree[at].type = Py_TYPE(module);
+    plan.tree[at].state = 0;
     bool known = false;
     for (const auto& t : plan.types) known = known || as_type(t.type) == Py_TYPE(module);
     if (!known) {
@@ -187,6 +224,21 @@ bool snapshot(Plan& plan, PyObject* module) {
         plan.tree[at].params.push_back(std::move(p));
     }
     pos = 0;
+    const bool attrs = whole && at > 0;
+    if (attrs) plan.tree[at].attrs.reserve(8);
+    while (attrs && PyDict_Next(d, &pos, &k, &v))
+        if (!is_private(k)) {
+            ModuleRef::Attr a;
+            Py_INCREF(k);
+            a.key.reset(k);
+            a.object = v;
+            if (!PyCallable_Check(v) || PyCFunction_Check(v)) {
+                Py_INCREF(v);
+                a.value.reset(v);
+            }
+            plan.tree[at].attrs.push_back(std::move(a));
+        }
+    pos = 0;
     std::vector<PyObject*> below;
     while (PyDict_Next(modules, &pos, &k, &v)) {
         ModuleRef::Child c;
@@ -197,8 +249,8 @@ bool snapshot(Plan& plan, PyObject* module) {
         if (v != Py_None) below.push_back(v);
     }
     for (PyObject* m : below)
-        if (!snapshot(plan, m)) return false;
-    return module_ok(plan.tree[at]);
+        if (!snapshot(plan, m, whole)) return false;
+    return module_ok(plan.tree[at], attrs);
 }
 
 Plan* plan_of(PyObject* o) { return static_cast<Plan*>(PyCapsule_GetPointer(o, kPlan)); }
@@ -357,7 +409,7 @@ PyObject* py_make_plan(PyObject*, PyObject* args) {
         plan->layers.push_back(std::move(w));
     }
     if (PyErr_Occurred()) return nullptr;
-    if (plan->layers.empty() || !snapshot(*plan, root)) Py_RETURN_NONE;
+    if (plan->layers.empty() || !snapshot(*plan, root, true)) Py_RETURN_NONE;
     return PyCapsule_New(plan.release(), kPlan, [](PyObject* c) { delete plan_of(c); });
     TDB_CATCH
 }
@@ -366,7 +418,7 @@ PyObject* py_make_plan(PyObject*, PyObject* args) {
 PyObject* py_tree_ready(PyObject*, PyObject* root) {
     TDB_TRY
     Plan p;
-    return PyBool_FromLong(snapshot(p, root));
+    return PyBool_FromLong(snapshot(p, root, false));
     TDB_CATCH
 }
 

@@ -430,12 +430,16 @@ def _native_plan(model):
     return plan
 
 
+# What the native loop takes to be the same in all attention modules
+_PER_MODEL = ("num_attention_heads", "attention_head_size", "pos_att_type", "relative_attention", "position_buckets", "max_relative_positions")
+
+
 def _known_structure(model):
     """Whether the modules below ``model`` compute what the native loop computes: stock DeBERTa-v2/v3 layers with the fused
     attention, exact GELU, no convolution, embeddings that are a table and a LayerNorm, and in the places of the dropouts
     dropouts, which the loop leaves out."""
     emb, enc = model.embeddings, model.encoder
-    dropout = lambda m: type(m.dropout) is nn.Dropout
+    dropout = lambda m: type(m._modules.get("dropout")) is nn.Dropout
     plain = lambda m, *names: all(type(getattr(m, n)) is nn.Linear and getattr(m, n).bias is not None for n in names)
     norm = lambda m: type(m) is nn.LayerNorm and m.weight is not None and m.bias is not None
     if not (type(emb) is DebertaV2Embeddings and type(emb.word_embeddings) is nn.Embedding and emb.word_embeddings.max_norm is None
@@ -445,22 +449,21 @@ def _known_structure(model):
     hidden = emb.word_embeddings.weight.shape[1]
     if hidden % 8 or hidden > 4096 or emb.word_embeddings.weight.dtype not in (torch.float32, torch.bfloat16, torch.float16):
         return False
-    first = enc.layer[0].attention.self
+    first = None                                 # (attention, feed-forward) of the first layer
     for layer in enc.layer:
-        if not (type(layer) in (DebertaV2Layer, FlashDebertaV2Layer) and type(layer.attention) in (DebertaV2Attention, FlashDebertaV2Attention)
-                and type(layer.attention.self) is FlashDisentangledSelfAttention and type(layer.attention.output) is DebertaV2SelfOutput
-                and type(layer.intermediate) is DebertaV2Intermediate and type(layer.output) is DebertaV2Output
-                and dropout(layer.attention.self) and dropout(layer.attention.output) and dropout(layer.output)
-                and type(getattr(layer.attention.self, "pos_dropout", None)) in (nn.Dropout, type(None))
-                and type(layer.intermediate.intermediate_act_fn) is GELUActivation
-                and layer.intermediate.intermediate_act_fn.act is nn.functional.gelu):
+        if not (type(layer) in (DebertaV2Layer, FlashDebertaV2Layer) and type(layer.attention) in (DebertaV2Attention, FlashDebertaV2Attention)):
             return False
-        att = layer.attention.self
-        if not (plain(att, "query_proj", "key_proj", "value_proj") and plain(layer.attention.output, "dense") and plain(layer.output, "dense")
-                and plain(layer.intermediate, "dense") and norm(layer.attention.output.LayerNorm) and norm(layer.output.LayerNorm)
-                and att.num_attention_heads * att.attention_head_size == hidden == layer.output.dense.out_features
-                and layer.intermediate.dense.out_features == enc.layer[0].intermediate.dense.out_features
-                and (att.num_attention_heads, att.pos_att_type, att.relative_attention) == (first.num_attention_heads, first.pos_att_type, first.relative_attention)):
+        att, so, mid, out = layer.attention.self, layer.attention.output, layer.intermediate, layer.output
+        first = first or (att, mid)
+        if not (type(att) is FlashDisentangledSelfAttention and type(so) is DebertaV2SelfOutput and type(mid) is DebertaV2Intermediate
+                and type(out) is DebertaV2Output and type(mid.intermediate_act_fn) is GELUActivation
+                and mid.intermediate_act_fn.act is nn.functional.gelu
+                and dropout(att) and dropout(so) and dropout(out) and type(att._modules.get("pos_dropout")) in (nn.Dropout, type(None))):
+            return False
+        if not (plain(att, "query_proj", "key_proj", "value_proj") and plain(so, "dense") and plain(out, "dense") and plain(mid, "dense")
+                and norm(so.LayerNorm) and norm(out.LayerNorm) and att.num_attention_heads * att.attention_head_size == hidden == out.dense.out_features
+                and mid.dense.out_features == first[1].dense.out_features
+                and all(getattr(att, n, None) == getattr(first[0], n, None) for n in _PER_MODEL)):
             return False
     return True
 
