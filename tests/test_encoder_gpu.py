@@ -117,6 +117,17 @@ def test_steps_aside_and_comes_back():
     assert model._forward_native(ids, mask) is None                            # gradients on
 
 
+def test_boundaries_it_does_not_take():
+    model, (ids, mask) = _model(torch.bfloat16), _ids([30, 7, 12], 30)
+    with torch.no_grad():
+        model._forward_native(ids, mask)
+        plan, cu = _native_plan(model), torch.tensor([0, 30, 37, 49], dtype=torch.int32, device="cuda")
+        encode = _lib.host().encode
+        assert encode(plan, ids, cu, 49) is not None
+        for bad in (cu.long(), cu.cpu(), cu[:3], cu[None], cu.repeat_interleave(2)[::2], [0, 30, 37, 49]):
+            assert encode(plan, ids, bad, 49) is None
+
+
 class _LastHidden(torch.nn.Module):
     def __init__(self, model):
         super().__init__()

@@ -9,6 +9,7 @@ import os
 import subprocess
 import sys
 import weakref
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -210,6 +211,18 @@ def test_native_plan_follows_the_attributes_it_was_made_from(place, name, value,
         setattr(m.get_submodule(place), name, value)
         new = _native_plan(m)
         assert new is not plan and (new is not None) == known
+
+
+def test_native_loop_leaves_masks_of_another_device_to_the_modules(monkeypatch):
+    from turbodeberta_amd import model as ours
+    m = FlashDebertaV2Model(_tiny()).eval()
+    on = lambda device: SimpleNamespace(is_cuda=True, shape=(2, 3), dim=lambda: 2, numel=lambda: 6, device=torch.device(device))
+    seen = []
+    monkeypatch.setattr(ours, "_native_plan", lambda model: seen.append(model))
+    with torch.no_grad():
+        assert m._forward_native(on("cuda:0"), on("cuda:0")) is None and seen == [m]
+        assert m._forward_native(on("cuda:0"), on("cuda:1")) is None and m._forward_native(on("cuda:0"), on("cpu")) is None
+    assert seen == [m]
 
 
 def test_native_plan_does_not_keep_its_model():

@@ -470,14 +470,20 @@ PyObject* py_scan_mask(PyObject*, PyObject* const* args, Py_ssize_t n) {
     TDB_CATCH
 }
 
-// encode(plan, ids [B, L], cu_seqlens or None, tokens) -> last hidden state, or None for ids it does not take
+// encode(plan, ids [B, L], cu_seqlens or None, tokens) -> last hidden state, or None for ids or boundaries it does not take
 PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     TDB_TRY
     Plan* p = n == 4 ? plan_of(args[0]) : nullptr;
     if (!p) return nullptr;
     if (tdb_host_observed() || !THPVariable_CheckExact(args[1]) || c10::GradMode::is_enabled()) Py_RETURN_NONE;
     const at::Tensor& ids = THPVariable_Unpack(args[1]);
-    const at::Tensor* cu = args[2] == Py_None ? nullptr : &THPVariable_Unpack(args[2]);
+    const at::Tensor* cu = nullptr;
+    if (args[2] != Py_None) {
+        if (!THPVariable_CheckExact(args[2])) Py_RETURN_NONE;
+        cu = &THPVariable_Unpack(args[2]);
+        if (cu->device() != ids.device() || cu->scalar_type() != at::kInt || cu->dim() != 1 || !cu->is_contiguous() || ids.dim() != 2 || cu->size(0) != ids.size(0) + 1)
+            Py_RETURN_NONE;
+    }
     const int64_t T = PyLong_AsLongLong(args[3]);
     if (ids.dim() != 2 || (ids.scalar_type() != at::kLong && ids.scalar_type() != at::kInt) || !ids.is_contiguous() || ids.device() != p->emb.device() ||
         ids.device().index() != c10::hip::current_device() || T < 1 || ids.numel() > INT32_MAX || 3 * T * p->emb.size(1) > INT32_MAX)

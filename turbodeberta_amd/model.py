@@ -544,7 +544,7 @@ class FlashDebertaV2Model(DebertaV2Model):
                 or _lib.host().observed()):
             return None
         B, L = input_ids.shape
-        if attention_mask is not None and (attention_mask.shape != input_ids.shape or not attention_mask.is_cuda):
+        if attention_mask is not None and (attention_mask.shape != input_ids.shape or attention_mask.device != input_ids.device):
             return None
         plan = _native_plan(self)
         if plan is None:
