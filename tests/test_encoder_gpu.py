@@ -5,6 +5,7 @@ import ctypes as C
 
 import pytest
 import torch
+from torch.utils.flop_counter import FlopCounterMode
 from transformers import DebertaV2Config
 
 from turbodeberta_amd import _lib
@@ -112,6 +113,9 @@ def test_steps_aside_and_comes_back():
         assert model._forward_native(ids, mask * 2) is None                    # the embeddings are scaled by such a mask
         with torch.autocast("cuda", torch.bfloat16):
             assert model._forward_native(ids, mask) is None
+        with FlopCounterMode(display=False) as counter:
+            model(input_ids=ids, attention_mask=mask)
+        assert counter.get_total_flops() > 2 * int(mask.sum()) * 2 * (4 * 128 * 128 + 2 * 128 * 256) * 0.9
         twin = copy.deepcopy(model)
         assert torch.equal(twin._forward_native(ids, mask), model._forward_native(ids, mask))
     assert model._forward_native(ids, mask) is None                            # gradients on

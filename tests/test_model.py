@@ -213,16 +213,60 @@ def test_native_plan_follows_the_attributes_it_was_made_from(place, name, value,
         assert new is not plan and (new is not None) == known
 
 
+def _ids_on(device):
+    return SimpleNamespace(is_cuda=True, shape=(2, 3), dim=lambda: 2, numel=lambda: 6, device=torch.device(device))
+
+
 def test_native_loop_leaves_masks_of_another_device_to_the_modules(monkeypatch):
     from turbodeberta_amd import model as ours
-    m = FlashDebertaV2Model(_tiny()).eval()
-    on = lambda device: SimpleNamespace(is_cuda=True, shape=(2, 3), dim=lambda: 2, numel=lambda: 6, device=torch.device(device))
-    seen = []
+    m, on, seen = FlashDebertaV2Model(_tiny()).eval(), _ids_on, []
     monkeypatch.setattr(ours, "_native_plan", lambda model: seen.append(model))
     with torch.no_grad():
         assert m._forward_native(on("cuda:0"), on("cuda:0")) is None and seen == [m]
         assert m._forward_native(on("cuda:0"), on("cuda:1")) is None and m._forward_native(on("cuda:0"), on("cpu")) is None
     assert seen == [m]
+
+
+def test_native_loop_is_off_where_operations_are_watched(monkeypatch):
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from turbodeberta_amd import model as ours
+    class Watch(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    m, ids, seen = FlashDebertaV2Model(_tiny()).eval(), _ids_on("cuda:0"), []
+    monkeypatch.setattr(ours, "_native_plan", lambda model: seen.append(model))
+    with torch.no_grad():
+        for mode in (Watch(), TorchDispatchMode()):
+            with mode:
+                assert m._forward_native(ids, None) is None and not seen
+        with torch.device("cpu"):
+            assert m._forward_native(ids, None) is None and seen
+
+
+@pytest.mark.parametrize("kind", ["tangent", "attribute", "subclass", "transform"])
+def test_native_plan_takes_plain_parameters_only(kind):
+    from torch.autograd import forward_ad
+    from turbodeberta_amd.model import _native_plan
+    m = FlashDebertaV2Model(_tiny()).eval()
+    dense = m.encoder.layer[0].output.dense
+    w = dense.weight.detach()
+    with torch.no_grad(), forward_ad.dual_level():
+        assert _native_plan(m) is not None
+        if kind == "subclass":
+            dense.weight = torch.nn.Parameter(w.as_subclass(type("Marked", (torch.Tensor,), {})))
+            assert _native_plan(m) is None
+        elif kind == "transform":
+            def inside(t):
+                dense._parameters["weight"] = t
+                assert _native_plan(m) is None
+                return t.sum()
+            torch.func.grad(inside)(w)
+        else:
+            del dense.weight
+            dense.weight = forward_ad.make_dual(w, torch.ones_like(w)) if kind == "tangent" else w
+            assert _native_plan(m) is None
 
 
 def test_native_plan_does_not_keep_its_model():

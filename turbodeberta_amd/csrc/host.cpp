@@ -90,15 +90,6 @@ bool rows_ok(const at::Tensor& t) {
     return strides_ok(t.strides(), t.element_size()) && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
 
-// A strided tensor of q's device with nothing to record: no gradient, no tangent, no transform wrapped around it.
-bool plain(const at::Tensor& t, const at::Tensor& q, bool grad) {
-    static const c10::DispatchKeySet wrapped({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
-                                              c10::DispatchKey::Functionalize, c10::DispatchKey::Python, c10::DispatchKey::Batched});
-    if (t.key_set().has_any(wrapped)) return false;
-    if (t.unsafeGetTensorImpl()->autograd_meta() && t._fw_grad(0).defined()) return false;
-    return t.device() == q.device() && t.layout() == at::kStrided && !(grad && t.requires_grad()) && !t.is_neg() && !t.is_conj();
-}
-
 int dtype_code(at::ScalarType t) {
     return t == at::kFloat ? TDB_F32 : t == at::kBFloat16 ? TDB_BF16 : t == at::kHalf ? TDB_F16 : -1;
 }
@@ -127,7 +118,7 @@ bool inputs_ok(const Common& c, int dims) {
     if (!q.is_cuda() || dtype_code(q.scalar_type()) < 0 || k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type()) return false;
     if (q.device().index() != c10::hip::current_device()) return false;
     for (const at::Tensor* t : {c.q, c.k, c.v})
-        if (!plain(*t, q, c.grad) || !rows_ok(*t)) return false;
+        if (!tdb_host_plain(*t, q, c.grad) || !rows_ok(*t)) return false;
     return true;
 }
 
@@ -158,7 +149,7 @@ bool fill_pos(tdb_pos_args& pos, const Common& c, int64_t heads, int64_t head_di
         if (!t) continue;
         const int64_t lead = t->dim() - 3;      // [H, rows, D], or with a leading 1
         if (lead < 0 || lead > 1 || (lead == 1 && t->size(0) != 1) || t->size(lead) != heads || t->size(lead + 1) < 2 * span ||
-            t->size(lead + 2) != head_dim || t->scalar_type() != q.scalar_type() || !plain(*t, q, c.grad) || !rows_ok(*t))
+            t->size(lead + 2) != head_dim || t->scalar_type() != q.scalar_type() || !tdb_host_plain(*t, q, c.grad) || !rows_ok(*t))
             return false;
         if (n) {
             pos.pos_query = t->data_ptr();
@@ -175,7 +166,7 @@ bool fill_pos(tdb_pos_args& pos, const Common& c, int64_t heads, int64_t head_di
         const at::Tensor* t = n ? c.k_pos : c.q_pos;
         if (!t) continue;
         if (t->dim() != outer + 1 || t->sizes().slice(0, outer) != q.sizes().slice(0, outer) || t->size(outer) != 2 * span ||
-            t->stride(outer) != 1 || t->scalar_type() != q.scalar_type() || !plain(*t, q, c.grad))
+            t->stride(outer) != 1 || t->scalar_type() != q.scalar_type() || !tdb_host_plain(*t, q, c.grad))
             return false;
         const int64_t sb = outer == 3 ? t->stride(0) : 0;
         const int64_t sh = t->stride(1), sl = outer == 3 ? t->stride(2) : t->stride(0);
@@ -191,7 +182,7 @@ bool fill_pos(tdb_pos_args& pos, const Common& c, int64_t heads, int64_t head_di
 }
 
 bool int32_vector(const at::Tensor& t, const at::Tensor& q, bool grad) {
-    return t.dim() == 1 && t.scalar_type() == at::kInt && t.is_contiguous() && plain(t, q, grad);
+    return t.dim() == 1 && t.scalar_type() == at::kInt && t.is_contiguous() && tdb_host_plain(t, q, grad);
 }
 
 void* stream_of(const at::Tensor& q) { return c10::hip::getCurrentHIPStream(q.device().index()).stream(); }
@@ -328,6 +319,14 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, kMethods};
 
 int (*tdb_host_fixed())(const tdb_fixed_args*, void*) { return g_fixed; }
 int (*tdb_host_varlen())(const tdb_varlen_args*, void*) { return g_varlen; }
+
+bool tdb_host_plain(const at::Tensor& t, const at::Tensor& q, bool grad) {
+    static const c10::DispatchKeySet wrapped({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                              c10::DispatchKey::Functionalize, c10::DispatchKey::Python, c10::DispatchKey::Batched});
+    if (t.key_set().has_any(wrapped)) return false;
+    if (t.unsafeGetTensorImpl()->autograd_meta() && t._fw_grad(0).defined()) return false;
+    return t.device() == q.device() && t.layout() == at::kStrided && !(grad && t.requires_grad()) && !t.is_neg() && !t.is_conj();
+}
 
 bool tdb_host_observed() { return c10::impl::dispatch_mode_enabled() || at::tracer::impl::is_dispatch_enabled(); }
 

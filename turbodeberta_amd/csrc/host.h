@@ -18,4 +18,8 @@ bool tdb_host_fill_tables(tdb_pos_args& pos, const at::Tensor* pk, const at::Ten
 // to a tracer and nothing at all to a mode.
 bool tdb_host_observed();
 
+// A strided tensor of q's device with nothing to record: no gradient (looked at if `grad`), no tangent, no transform wrapped
+// around it.
+bool tdb_host_plain(const at::Tensor& t, const at::Tensor& q, bool grad);
+
 bool tdb_host_add_encoder(PyObject* module);

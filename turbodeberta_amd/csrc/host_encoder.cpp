@@ -183,8 +183,8 @@ bool tree_ok(const Plan& plan, PyObject* root) {
     return true;
 }
 
-// Appends `module` and what is below it; false where something cannot be held to account later.  (`whole` false: to find out.)
-bool snapshot(Plan& plan, PyObject* module, bool whole) {
+// Appends `module` and what is below it; false where something cannot be held to account later.
+bool snapshot(Plan& plan, PyObject* module) {
     const Names& n = names();
     PyObject* d = dict_of(module);
     if (!d) return false;
@@ -209,24 +209,27 @@ bool snapshot(Plan& plan, PyObject* module, bool whole) {
     }
     PyObject *k, *v;
     Py_ssize_t pos = 0;
+    while (PyDict_Next(d, &pos, &k, &v))
+        if (PyType_HasFeature(Py_TYPE(v), Py_TPFLAGS_HEAPTYPE) && PyType_IsSubtype(Py_TYPE(v), reinterpret_cast<PyTypeObject*>(THPVariableClass)))
+            return false;                   // a weight that is no parameter
+    pos = 0;
     while (PyDict_Next(params, &pos, &k, &v)) {
         ModuleRef::Param p;
         Py_INCREF(k);
         p.key.reset(k);
         p.version = 0, p.data = nullptr;
         if (v != Py_None) {
-            if (!THPVariable_Check(v)) return false;
+            if (!THPVariable_CheckExact(v)) return false;
             p.tensor = THPVariable_Unpack(v);
-            if (p.tensor.is_inference()) return false;      // no modification counter
+            if (!tdb_host_plain(p.tensor, p.tensor, false) || p.tensor.is_inference()) return false;       // (inference: no modification counter)
             p.version = p.tensor._version();
             p.data = p.tensor.data_ptr();
         }
         plan.tree[at].params.push_back(std::move(p));
     }
     pos = 0;
-    const bool attrs = whole && at > 0;
-    if (attrs) plan.tree[at].attrs.reserve(8);
-    while (attrs && PyDict_Next(d, &pos, &k, &v))
+    if (at > 0) plan.tree[at].attrs.reserve(8);
+    while (at > 0 && PyDict_Next(d, &pos, &k, &v))
         if (!is_private(k)) {
             ModuleRef::Attr a;
             Py_INCREF(k);
@@ -249,8 +252,8 @@ bool snapshot(Plan& plan, PyObject* module, bool whole) {
         if (v != Py_None) below.push_back(v);
     }
     for (PyObject* m : below)
-        if (!snapshot(plan, m, whole)) return false;
-    return module_ok(plan.tree[at], attrs);
+        if (!snapshot(plan, m)) return false;
+    return module_ok(plan.tree[at], at > 0);
 }
 
 Plan* plan_of(PyObject* o) { return static_cast<Plan*>(PyCapsule_GetPointer(o, kPlan)); }
@@ -387,15 +390,26 @@ at::Tensor encode(const Plan& p, const at::Tensor& ids, const at::Tensor* cu, in
         return nullptr;                                              \
     }
 
-// make_plan(root, layers, embedding, heads, head_dim, scale, buckets, max_rel): a plan, or None where the tree below `root`
-// cannot be snapshot.  layers: tuples of 14 tensors (query/key/value bias, tables may be None) and two epsilons.
-PyObject* py_make_plan(PyObject*, PyObject* args) {
+// begin_plan(root): a plan that holds the snapshot only, or None where the tree below `root` cannot be held to account (a module
+// in training mode, a hook, a forward of its own, parameters that are not plain or have no modification counter)
+PyObject* py_begin_plan(PyObject*, PyObject* root) {
     TDB_TRY
-    PyObject *root, *layers, *emb;
+    auto plan = std::make_unique<Plan>();
+    if (!snapshot(*plan, root)) Py_RETURN_NONE;
+    return PyCapsule_New(plan.release(), kPlan, [](PyObject* c) { delete plan_of(c); });
+    TDB_CATCH
+}
+
+// complete_plan(plan, root, layers, embedding, heads, head_dim, scale, buckets, max_rel): whether the plan can be used; not where
+// the tree has changed since it was begun.  layers: tuples of 14 tensors (tables may be None) and two epsilons.
+PyObject* py_complete_plan(PyObject*, PyObject* args) {
+    TDB_TRY
+    PyObject *capsule, *root, *layers, *emb;
     long long heads, head_dim, buckets, max_rel;
     double scale;
-    if (!PyArg_ParseTuple(args, "OO!O!LLdLL", &root, &PyList_Type, &layers, &PyTuple_Type, &emb, &heads, &head_dim, &scale, &buckets, &max_rel)) return nullptr;
-    auto plan = std::make_unique<Plan>();
+    if (!PyArg_ParseTuple(args, "OOO!O!LLdLL", &capsule, &root, &PyList_Type, &layers, &PyTuple_Type, &emb, &heads, &head_dim, &scale, &buckets, &max_rel)) return nullptr;
+    Plan* const plan = plan_of(capsule);
+    if (!plan) return nullptr;
     plan->heads = heads, plan->head_dim = head_dim, plan->scale = float(scale), plan->buckets = buckets, plan->max_rel = max_rel;
     if (!get_tensor(emb, 0, plan->emb) || !get_tensor(emb, 1, plan->emb_g) || !get_tensor(emb, 2, plan->emb_b)) return nullptr;
     plan->emb_eps = PyFloat_AsDouble(PyTuple_GetItem(emb, 3));
@@ -409,16 +423,7 @@ PyObject* py_make_plan(PyObject*, PyObject* args) {
         plan->layers.push_back(std::move(w));
     }
     if (PyErr_Occurred()) return nullptr;
-    if (plan->layers.empty() || !snapshot(*plan, root, true)) Py_RETURN_NONE;
-    return PyCapsule_New(plan.release(), kPlan, [](PyObject* c) { delete plan_of(c); });
-    TDB_CATCH
-}
-
-// tree_ready(root): whether a plan could be made now (eval mode everywhere, no hooks, parameters with modification counters)
-PyObject* py_tree_ready(PyObject*, PyObject* root) {
-    TDB_TRY
-    Plan p;
-    return PyBool_FromLong(snapshot(p, root, false));
+    return PyBool_FromLong(!plan->layers.empty() && tree_ok(*plan, root));
     TDB_CATCH
 }
 
@@ -436,6 +441,7 @@ PyObject* py_scan_mask(PyObject*, PyObject* const* args, Py_ssize_t n) {
     TDB_TRY
     if (n != 1 || tdb_host_observed() || !THPVariable_CheckExact(args[0])) Py_RETURN_NONE;
     const at::Tensor& m = THPVariable_Unpack(args[0]);
+    if (!tdb_host_plain(m, m, false)) Py_RETURN_NONE;
     const int type = m.is_cuda() ? mask_type(m.scalar_type()) : -1;
     if (type < 0 || m.dim() != 2 || m.size(0) < 1 || m.size(0) > TDB_SCAN_MAX_BATCH || m.size(1) < 1 || m.size(1) > INT32_MAX ||
         m.device().index() != c10::hip::current_device())
@@ -475,17 +481,18 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     TDB_TRY
     Plan* p = n == 4 ? plan_of(args[0]) : nullptr;
     if (!p) return nullptr;
-    if (tdb_host_observed() || !THPVariable_CheckExact(args[1]) || c10::GradMode::is_enabled()) Py_RETURN_NONE;
+    if (p->layers.empty() || tdb_host_observed() || !THPVariable_CheckExact(args[1]) || c10::GradMode::is_enabled()) Py_RETURN_NONE;
     const at::Tensor& ids = THPVariable_Unpack(args[1]);
+    if (!tdb_host_plain(ids, p->emb, false)) Py_RETURN_NONE;
     const at::Tensor* cu = nullptr;
     if (args[2] != Py_None) {
         if (!THPVariable_CheckExact(args[2])) Py_RETURN_NONE;
         cu = &THPVariable_Unpack(args[2]);
-        if (cu->device() != ids.device() || cu->scalar_type() != at::kInt || cu->dim() != 1 || !cu->is_contiguous() || ids.dim() != 2 || cu->size(0) != ids.size(0) + 1)
+        if (!tdb_host_plain(*cu, ids, false) || cu->scalar_type() != at::kInt || cu->dim() != 1 || !cu->is_contiguous() || ids.dim() != 2 || cu->size(0) != ids.size(0) + 1)
             Py_RETURN_NONE;
     }
     const int64_t T = PyLong_AsLongLong(args[3]);
-    if (ids.dim() != 2 || (ids.scalar_type() != at::kLong && ids.scalar_type() != at::kInt) || !ids.is_contiguous() || ids.device() != p->emb.device() ||
+    if (ids.dim() != 2 || (ids.scalar_type() != at::kLong && ids.scalar_type() != at::kInt) || !ids.is_contiguous() ||
         ids.device().index() != c10::hip::current_device() || T < 1 || ids.numel() > INT32_MAX || 3 * T * p->emb.size(1) > INT32_MAX)
         Py_RETURN_NONE;
     at::Tensor out;
@@ -514,8 +521,8 @@ PyObject* py_bind_encoder(PyObject*, PyObject* args) {
 
 PyMethodDef kMethods[] = {
     {"bind_encoder", py_bind_encoder, METH_VARARGS, nullptr},
-    {"make_plan", py_make_plan, METH_VARARGS, nullptr},
-    {"tree_ready", py_tree_ready, METH_O, nullptr},
+    {"begin_plan", py_begin_plan, METH_O, nullptr},
+    {"complete_plan", py_complete_plan, METH_VARARGS, nullptr},
     {"plan_ok", reinterpret_cast<PyCFunction>(py_plan_ok), METH_FASTCALL, nullptr},
     {"scan_mask", reinterpret_cast<PyCFunction>(py_scan_mask), METH_FASTCALL, nullptr},
     {"encode", reinterpret_cast<PyCFunction>(py_encode), METH_FASTCALL, nullptr},

@@ -35,6 +35,7 @@ from typing import Optional
 
 import torch
 from torch import nn
+from torch.utils._device import DeviceContext
 from transformers.activations import GELUActivation
 from transformers.modeling_outputs import BaseModelOutput
 from transformers.models.deberta_v2.modeling_deberta_v2 import (
@@ -407,7 +408,8 @@ def _native_plan(model):
         _PLANS[model] = False
         return None
     _PLANS.pop(model, None)
-    if not _stock_methods() or not host.tree_ready(model):  # a module in training mode, a hook, a forward of its own, ...
+    plan = host.begin_plan(model) if _stock_methods() else None
+    if plan is None:                             # a module in training mode, a hook, a forward of its own, ...
         return None
     emb, enc = model.embeddings, model.encoder
     table = emb.word_embeddings.weight
@@ -423,10 +425,10 @@ def _native_plan(model):
     tensors = [t for l in layers for t in l[:14] if t is not None] + [table, emb.LayerNorm.weight, emb.LayerNorm.bias]
     if any(t.dtype != table.dtype or t.device != table.device or t.data_ptr() % 16 or not (t.is_contiguous() or t.dim() == 3) for t in tensors):
         return None
-    plan = host.make_plan(model, layers, (table, emb.LayerNorm.weight, emb.LayerNorm.bias, float(emb.LayerNorm.eps)),
-                          att.num_attention_heads, att.attention_head_size, scale, buckets, max_rel)
-    if plan is not None:
-        _PLANS[model] = plan
+    if not host.complete_plan(plan, model, layers, (table, emb.LayerNorm.weight, emb.LayerNorm.bias, float(emb.LayerNorm.eps)),
+                              att.num_attention_heads, att.attention_head_size, scale, buckets, max_rel):
+        return None
+    _PLANS[model] = plan
     return plan
 
 
@@ -490,6 +492,13 @@ def _stock_methods():
     return all(getattr(cls, name, None) is method for cls, name, method in _STOCK)
 
 
+def _observed():
+    """Whether somebody watches the operations of this thread, or changes them: a tracer, a dispatch mode, a function mode
+    other than a default device."""
+    return _lib.host().observed() or any(type(torch._C._get_function_stack_at(i)) is not DeviceContext
+                                         for i in range(torch._C._len_torch_function_stack()))
+
+
 class FlashDebertaV2Model(DebertaV2Model):
     def __init__(self, config):
         super().__init__(config)
@@ -537,11 +546,11 @@ class FlashDebertaV2Model(DebertaV2Model):
 
     def _forward_native(self, input_ids, attention_mask):
         """The last hidden state through the native loop, or None where the modules have to be run: with gradients, in
-        training mode, under autocast, a compiler, a tracer or a dispatch mode, with hooks, for masks other than 2-D ones of
-        zeros and ones.  As in the packed encoder, padded positions come back as zeros."""
+        training mode, under autocast, a compiler, a tracer or a mode that watches the operations, with hooks, for masks other
+        than 2-D ones of zeros and ones.  As in the packed encoder, padded positions come back as zeros."""
         if (self.training or torch.is_grad_enabled() or not input_ids.is_cuda or input_ids.dim() != 2 or not input_ids.numel()
                 or not getattr(self.encoder, "pack_sequences", False) or torch.is_autocast_enabled() or torch.compiler.is_compiling()
-                or _lib.host().observed()):
+                or _observed()):
             return None
         B, L = input_ids.shape
         if attention_mask is not None and (attention_mask.shape != input_ids.shape or attention_mask.device != input_ids.device):
