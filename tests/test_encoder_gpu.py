@@ -2,6 +2,7 @@
 of its own products, packed and full batches, and what makes it step aside."""
 import copy
 import ctypes as C
+import threading
 
 import pytest
 import torch
@@ -83,6 +84,38 @@ def test_mask_scan(dtype):
     assert not _lib.host().scan_mask(holes)[2]
     if dtype != torch.bool:
         assert not _lib.host().scan_mask(mask * 2)[4]
+
+
+def test_mask_scans_of_many_threads():
+    """Threads that come and go leave no pinned memory behind; threads at the same time get their own answers."""
+    masks = [(torch.arange(50)[None] < torch.arange(1, 9)[:, None] + n).long().cuda() for n in range(8)]
+    wrong, start = [], threading.Barrier(8)
+
+    def scan(n, times, wait):
+        if wait:
+            start.wait()
+        with torch.cuda.stream(torch.cuda.Stream() if wait else torch.cuda.current_stream()):
+            for _ in range(times):
+                lens, _, ok, total, _ = _lib.host().scan_mask(masks[n])
+                if not ok or total != 36 + 8 * n or lens.tolist() != list(range(1 + n, 9 + n)):
+                    wrong.append(n)
+
+    def pinned():
+        with open("/proc/self/maps") as f:
+            return sum("/dev/dri/" in line or "/dev/kfd" in line for line in f)
+
+    def run(threads):
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+
+    torch.cuda.synchronize()
+    run([threading.Thread(target=scan, args=(n, 50, True)) for n in range(8)])
+    before = pinned()
+    for _ in range(100):
+        run([threading.Thread(target=scan, args=(0, 1, False))])
+    assert not wrong and pinned() - before < 20
 
 
 def test_steps_aside_and_comes_back():

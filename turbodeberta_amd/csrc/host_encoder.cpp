@@ -436,6 +436,36 @@ PyObject* py_plan_ok(PyObject*, PyObject* const* args, Py_ssize_t n) {
     TDB_CATCH
 }
 
+// Pinned memory for the answers of mask scans: one page of slots for the process, handed out and given back with the GIL held,
+// so that a call has a slot to itself whatever threads and streams there are.  (A slot whose kernel may still write to it,
+// after an error, is not given back.)
+struct Slot {
+    int32_t flags[3], ticket;               // as tdb_enc_scan_mask writes them
+    int32_t pad[12];                        // a cache line
+};
+constexpr int SLOTS = 64;
+struct Slots {
+    std::vector<Slot*> unused;
+    bool ready = false;
+} g_slots;
+
+Slot* take_slot() {
+    if (!g_slots.ready) {
+        void* page = nullptr;
+        if (hipHostMalloc(&page, SLOTS * sizeof(Slot), hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        memset(page, 0, SLOTS * sizeof(Slot));
+        for (int i = 0; i < SLOTS; ++i) g_slots.unused.push_back(static_cast<Slot*>(page) + i);
+        g_slots.ready = true;
+    }
+    if (g_slots.unused.empty()) return nullptr;
+    Slot* s = g_slots.unused.back();
+    g_slots.unused.pop_back();
+    return s;
+}
+
 // scan_mask(mask [B, L]) -> (lengths, cu_seqlens, right_padded, total, ones), or None for a mask it does not take.  Waits for the GPU.
 PyObject* py_scan_mask(PyObject*, PyObject* const* args, Py_ssize_t n) {
     TDB_TRY
@@ -446,22 +476,21 @@ PyObject* py_scan_mask(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (type < 0 || m.dim() != 2 || m.size(0) < 1 || m.size(0) > TDB_SCAN_MAX_BATCH || m.size(1) < 1 || m.size(1) > INT32_MAX ||
         m.device().index() != c10::hip::current_device())
         Py_RETURN_NONE;
-    // The kernel's answer comes back through pinned memory, one buffer per thread for good.  Watching the ticket that it writes
-    // last is some 15 us quicker than waiting for the stream; what takes long (work queued before it) waits for the stream.
-    static thread_local int32_t *flags = nullptr, ticket = 0;
-    if (!flags) {
-        if (hipHostMalloc(reinterpret_cast<void**>(&flags), 64, hipHostMallocPortable) != hipSuccess) Py_RETURN_NONE;
-        memset(flags, 0, 64);
-    }
-    ticket = ticket == INT32_MAX ? 1 : ticket + 1;
     const int64_t B = m.size(0);
     at::Tensor both = at::detail::empty_cuda({2 * B + 1}, at::kInt, m.device(), std::nullopt);
     int32_t* const lens = static_cast<int32_t*>(both.data_ptr());
     hipStream_t s = current_stream(m);
-    must(g_enc.scan_mask(m.data_ptr(), type, m.stride(0), m.stride(1), int(B), int(m.size(1)), lens, lens + B, flags, ticket, s));
+    // Watching the ticket that the kernel writes last is some 15 us quicker than waiting for the stream; what takes long (work
+    // queued before it) waits for the stream.
+    Slot* const slot = take_slot();
+    if (!slot) Py_RETURN_NONE;
+    const int32_t wanted = slot->ticket == INT32_MAX ? 1 : slot->ticket + 1;
+    if (const int rc = g_enc.scan_mask(m.data_ptr(), type, m.stride(0), m.stride(1), int(B), int(m.size(1)), lens, lens + B, reinterpret_cast<int32_t*>(slot), wanted, s)) {
+        g_slots.unused.push_back(slot);     // (not launched)
+        must(rc);
+    }
     hipError_t e = hipSuccess;
-    const int32_t wanted = ticket;
-    int32_t* const seen = flags + 3;
+    int32_t* const seen = &slot->ticket;
     Py_BEGIN_ALLOW_THREADS
     const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(20);
     while (__atomic_load_n(seen, __ATOMIC_ACQUIRE) != wanted)
@@ -471,8 +500,10 @@ PyObject* py_scan_mask(PyObject*, PyObject* const* args, Py_ssize_t n) {
         }
     Py_END_ALLOW_THREADS
     TORCH_CHECK(e == hipSuccess, "attention mask: ", hipGetErrorString(e));
+    const Slot got = *slot;
+    g_slots.unused.push_back(slot);
     return Py_BuildValue("(NNNiN)", THPVariable_Wrap(both.narrow(0, 0, B)), THPVariable_Wrap(both.narrow(0, B, B + 1)),
-                         PyBool_FromLong(flags[0]), int(flags[1]), PyBool_FromLong(flags[2]));
+                         PyBool_FromLong(got.flags[0]), int(got.flags[1]), PyBool_FromLong(got.flags[2]));
     TDB_CATCH
 }
 
