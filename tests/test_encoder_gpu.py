@@ -154,6 +154,27 @@ def test_steps_aside_and_comes_back():
     assert model._forward_native(ids, mask) is None                            # gradients on
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("id_type", [torch.int64, torch.int32])
+@pytest.mark.parametrize("bad", [-1, 500, 2 ** 31 - 1])
+def test_ids_outside_the_vocabulary(bad, id_type, dtype):
+    model, (ids, mask) = _model(dtype), _ids([30, 7, 12], 30)
+    ids = ids.to(id_type)
+    run = lambda mask: model._forward_native(ids, mask)                          # (the modules never see such ids)
+    with torch.no_grad():
+        good = run(mask)
+        ids[1, 7], ids[2, 29] = bad, bad                                        # padding
+        assert torch.equal(run(mask.clone()), good)
+        ids[1, 6] = bad
+        with pytest.raises(IndexError, match="500"):
+            run(mask.clone())
+        out = run(mask)                                                         # measured before: nothing is read back
+        assert out[1, :7].isnan().all() and torch.equal(out[0], good[0]) and torch.equal(out[2], good[2])
+        ids[1, 7] = ids[2, 29] = 5
+        out = run(None)
+        assert out[1].isnan().all() and not out[0].isnan().any() and not out[2].isnan().any()
+
+
 def test_boundaries_it_does_not_take():
     model, (ids, mask) = _model(torch.bfloat16), _ids([30, 7, 12], 30)
     with torch.no_grad():

@@ -251,46 +251,62 @@ __global__ __launch_bounds__(512) void small_gemm_kernel(const void* xv, const v
     }
 }
 
+struct ScanIds {
+    const void* ids;                        // of the row, or nullptr
+    int ids64;
+    int64_t vocab;
+    __device__ __forceinline__ bool in_table(int i) const {
+        if (!ids) return true;
+        const int64_t id = ids64 ? static_cast<const int64_t*>(ids)[i] : static_cast<const int32_t*>(ids)[i];
+        return id >= 0 && id < vocab;
+    }
+};
+
 template <typename T>
-__device__ __forceinline__ void scan_row(const T* row, int64_t stride, int L, int& count, int& last, bool& ones) {
+__device__ __forceinline__ void scan_row(const T* row, int64_t stride, int L, const ScanIds& ids, int& count, int& last, bool& ones, bool& known) {
     const int l = threadIdx.x & 63;
     for (int i = l; i < L; i += 64) {
         const T x = row[i * stride];
+        const bool in = ids.in_table(i);
         if (x != T(0)) {
             ++count;
             last = i + 1;
             ones = ones && x == T(1);
+            known = known && in;
         }
     }
 }
 
-__global__ __launch_bounds__(1024) void scan_mask_kernel(const void* mask, int type, int64_t sb, int64_t sl, int B, int L, int32_t* lens,
-                                                         int32_t* cu, int32_t* flags, int ticket) {
-    __shared__ int s_len[TDB_SCAN_MAX_BATCH], s_ok, s_ones;
+__global__ __launch_bounds__(1024) void scan_mask_kernel(const void* mask, int type, int64_t sb, int64_t sl, int B, int L, ScanIds ids,
+                                                         int32_t* lens, int32_t* cu, int32_t* flags, int ticket) {
+    __shared__ int s_len[TDB_SCAN_MAX_BATCH], s_ok, s_ones, s_known;
     const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
-    if (threadIdx.x == 0) s_ok = s_ones = 1;
+    if (threadIdx.x == 0) s_ok = s_ones = s_known = 1;
     __syncthreads();
     for (int b = wave; b < B; b += 16) {
         int count = 0, last = 0;
-        bool ones = true;
+        bool ones = true, known = true;
+        ScanIds row = ids;
+        if (ids.ids) row.ids = static_cast<const char*>(ids.ids) + int64_t(b) * L * (ids.ids64 ? 8 : 4);
         switch (type) {
-            case TDB_MASK_I64: scan_row(static_cast<const int64_t*>(mask) + b * sb, sl, L, count, last, ones); break;
-            case TDB_MASK_I32: scan_row(static_cast<const int32_t*>(mask) + b * sb, sl, L, count, last, ones); break;
-            case TDB_MASK_U8: scan_row(static_cast<const uint8_t*>(mask) + b * sb, sl, L, count, last, ones); break;
-            case TDB_F32: scan_row(static_cast<const float*>(mask) + b * sb, sl, L, count, last, ones); break;
-            case TDB_BF16: scan_row(static_cast<const __bf16*>(mask) + b * sb, sl, L, count, last, ones); break;
-            default: scan_row(static_cast<const _Float16*>(mask) + b * sb, sl, L, count, last, ones); break;
+            case TDB_MASK_I64: scan_row(static_cast<const int64_t*>(mask) + b * sb, sl, L, row, count, last, ones, known); break;
+            case TDB_MASK_I32: scan_row(static_cast<const int32_t*>(mask) + b * sb, sl, L, row, count, last, ones, known); break;
+            case TDB_MASK_U8: scan_row(static_cast<const uint8_t*>(mask) + b * sb, sl, L, row, count, last, ones, known); break;
+            case TDB_F32: scan_row(static_cast<const float*>(mask) + b * sb, sl, L, row, count, last, ones, known); break;
+            case TDB_BF16: scan_row(static_cast<const __bf16*>(mask) + b * sb, sl, L, row, count, last, ones, known); break;
+            default: scan_row(static_cast<const _Float16*>(mask) + b * sb, sl, L, row, count, last, ones, known); break;
         }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) {
             count += __shfl_xor(count, o);
             last = max(last, __shfl_xor(last, o));
         }
-        const bool all_ones = __builtin_amdgcn_ballot_w64(!ones) == 0;
+        const bool all_ones = __builtin_amdgcn_ballot_w64(!ones) == 0, all_known = __builtin_amdgcn_ballot_w64(!known) == 0;
         if (l == 0) {
             s_len[b] = count;
             if (last != count) s_ok = 0;    // (every writer writes the same)
             if (!all_ones) s_ones = 0;
+            if (!all_known) s_known = 0;
         }
     }
     __syncthreads();
@@ -315,8 +331,9 @@ __global__ __launch_bounds__(1024) void scan_mask_kernel(const void* mask, int t
             flags[0] = s_ok;
             flags[1] = before;
             flags[2] = s_ones;
+            flags[3] = s_known;
             __threadfence_system();
-            __hip_atomic_store(flags + 3, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(flags + 4, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
 }
@@ -354,10 +371,11 @@ bool hidden_ok(int hidden) { return hidden > 0 && hidden % 8 == 0 && hidden <= 4
 
 extern "C" {
 
-int tdb_enc_scan_mask(const void* mask, int type, int64_t stride_b, int64_t stride_l, int B, int L, int32_t* lens, int32_t* cu, int32_t* flags,
-                      int ticket, void* stream) {
+int tdb_enc_scan_mask(const void* mask, int type, int64_t stride_b, int64_t stride_l, int B, int L, const void* ids, int ids64, int64_t vocab,
+                      int32_t* lens, int32_t* cu, int32_t* flags, int ticket, void* stream) {
     if (B < 1 || B > TDB_SCAN_MAX_BATCH || L < 1) return int(hipErrorInvalidValue);
-    hipLaunchKernelGGL(scan_mask_kernel, dim3(1), dim3(1024), 0, static_cast<hipStream_t>(stream), mask, type, stride_b, stride_l, B, L, lens, cu, flags, ticket);
+    hipLaunchKernelGGL(scan_mask_kernel, dim3(1), dim3(1024), 0, static_cast<hipStream_t>(stream), mask, type, stride_b, stride_l, B, L,
+                       ScanIds{ids, ids64, vocab}, lens, cu, flags, ticket);
     return int(hipGetLastError());
 }
 

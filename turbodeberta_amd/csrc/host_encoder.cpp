@@ -436,12 +436,17 @@ PyObject* py_plan_ok(PyObject*, PyObject* const* args, Py_ssize_t n) {
     TDB_CATCH
 }
 
+// Token ids that the kernels can read: [B, L] row after row, of x's device
+bool ids_ok(const at::Tensor& ids, const at::Tensor& x) {
+    return tdb_host_plain(ids, x, false) && ids.dim() == 2 && (ids.scalar_type() == at::kLong || ids.scalar_type() == at::kInt) && ids.is_contiguous();
+}
+
 // Pinned memory for the answers of mask scans: one page of slots for the process, handed out and given back with the GIL held,
 // so that a call has a slot to itself whatever threads and streams there are.  (A slot whose kernel may still write to it,
 // after an error, is not given back.)
 struct Slot {
-    int32_t flags[3], ticket;               // as tdb_enc_scan_mask writes them
-    int32_t pad[12];                        // a cache line
+    int32_t flags[4], ticket;               // as tdb_enc_scan_mask writes them
+    int32_t pad[11];                        // a cache line
 };
 constexpr int SLOTS = 64;
 struct Slots {
@@ -466,16 +471,27 @@ Slot* take_slot() {
     return s;
 }
 
-// scan_mask(mask [B, L]) -> (lengths, cu_seqlens, right_padded, total, ones), or None for a mask it does not take.  Waits for the GPU.
+// scan_mask(mask [B, L]) -> (lengths, cu_seqlens, right_padded, total, ones), or None for a mask it does not take.
+// scan_mask(mask, ids [B, L], vocab) -> the same and whether the ids of the valid tokens lie in [0, vocab) (ids that encode() does
+// not take are not looked at).  Waits for the GPU.
 PyObject* py_scan_mask(PyObject*, PyObject* const* args, Py_ssize_t n) {
     TDB_TRY
-    if (n != 1 || tdb_host_observed() || !THPVariable_CheckExact(args[0])) Py_RETURN_NONE;
+    if ((n != 1 && n != 3) || tdb_host_observed() || !THPVariable_CheckExact(args[0])) Py_RETURN_NONE;
     const at::Tensor& m = THPVariable_Unpack(args[0]);
     if (!tdb_host_plain(m, m, false)) Py_RETURN_NONE;
     const int type = m.is_cuda() ? mask_type(m.scalar_type()) : -1;
     if (type < 0 || m.dim() != 2 || m.size(0) < 1 || m.size(0) > TDB_SCAN_MAX_BATCH || m.size(1) < 1 || m.size(1) > INT32_MAX ||
         m.device().index() != c10::hip::current_device())
         Py_RETURN_NONE;
+    const void* ids = nullptr;
+    int ids64 = 0;
+    int64_t vocab = 0;
+    if (n == 3 && THPVariable_CheckExact(args[1])) {
+        const at::Tensor& t = THPVariable_Unpack(args[1]);
+        vocab = PyLong_AsLongLong(args[2]);
+        if (vocab == -1 && PyErr_Occurred()) return nullptr;
+        if (ids_ok(t, m) && t.sizes() == m.sizes()) ids = t.data_ptr(), ids64 = t.scalar_type() == at::kLong;
+    }
     const int64_t B = m.size(0);
     at::Tensor both = at::detail::empty_cuda({2 * B + 1}, at::kInt, m.device(), std::nullopt);
     int32_t* const lens = static_cast<int32_t*>(both.data_ptr());
@@ -485,7 +501,8 @@ PyObject* py_scan_mask(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Slot* const slot = take_slot();
     if (!slot) Py_RETURN_NONE;
     const int32_t wanted = slot->ticket == INT32_MAX ? 1 : slot->ticket + 1;
-    if (const int rc = g_enc.scan_mask(m.data_ptr(), type, m.stride(0), m.stride(1), int(B), int(m.size(1)), lens, lens + B, reinterpret_cast<int32_t*>(slot), wanted, s)) {
+    if (const int rc = g_enc.scan_mask(m.data_ptr(), type, m.stride(0), m.stride(1), int(B), int(m.size(1)), ids, ids64, vocab, lens, lens + B,
+                                        reinterpret_cast<int32_t*>(slot), wanted, s)) {
         g_slots.unused.push_back(slot);     // (not launched)
         must(rc);
     }
@@ -502,8 +519,10 @@ PyObject* py_scan_mask(PyObject*, PyObject* const* args, Py_ssize_t n) {
     TORCH_CHECK(e == hipSuccess, "attention mask: ", hipGetErrorString(e));
     const Slot got = *slot;
     g_slots.unused.push_back(slot);
-    return Py_BuildValue("(NNNiN)", THPVariable_Wrap(both.narrow(0, 0, B)), THPVariable_Wrap(both.narrow(0, B, B + 1)),
-                         PyBool_FromLong(got.flags[0]), int(got.flags[1]), PyBool_FromLong(got.flags[2]));
+    PyObject *lengths = THPVariable_Wrap(both.narrow(0, 0, B)), *cu = THPVariable_Wrap(both.narrow(0, B, B + 1));
+    PyObject *right_padded = PyBool_FromLong(got.flags[0]), *ones = PyBool_FromLong(got.flags[2]);
+    if (n == 1) return Py_BuildValue("(NNNiN)", lengths, cu, right_padded, int(got.flags[1]), ones);
+    return Py_BuildValue("(NNNiNN)", lengths, cu, right_padded, int(got.flags[1]), ones, PyBool_FromLong(got.flags[3]));
     TDB_CATCH
 }
 
@@ -514,17 +533,16 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (!p) return nullptr;
     if (p->layers.empty() || tdb_host_observed() || !THPVariable_CheckExact(args[1]) || c10::GradMode::is_enabled()) Py_RETURN_NONE;
     const at::Tensor& ids = THPVariable_Unpack(args[1]);
-    if (!tdb_host_plain(ids, p->emb, false)) Py_RETURN_NONE;
+    if (!ids_ok(ids, p->emb)) Py_RETURN_NONE;
     const at::Tensor* cu = nullptr;
     if (args[2] != Py_None) {
         if (!THPVariable_CheckExact(args[2])) Py_RETURN_NONE;
         cu = &THPVariable_Unpack(args[2]);
-        if (!tdb_host_plain(*cu, ids, false) || cu->scalar_type() != at::kInt || cu->dim() != 1 || !cu->is_contiguous() || ids.dim() != 2 || cu->size(0) != ids.size(0) + 1)
+        if (!tdb_host_plain(*cu, ids, false) || cu->scalar_type() != at::kInt || cu->dim() != 1 || !cu->is_contiguous() || cu->size(0) != ids.size(0) + 1)
             Py_RETURN_NONE;
     }
     const int64_t T = PyLong_AsLongLong(args[3]);
-    if (ids.dim() != 2 || (ids.scalar_type() != at::kLong && ids.scalar_type() != at::kInt) || !ids.is_contiguous() ||
-        ids.device().index() != c10::hip::current_device() || T < 1 || ids.numel() > INT32_MAX || 3 * T * p->emb.size(1) > INT32_MAX)
+    if (ids.device().index() != c10::hip::current_device() || T < 1 || ids.numel() > INT32_MAX || 3 * T * p->emb.size(1) > INT32_MAX)
         Py_RETURN_NONE;
     at::Tensor out;
     {

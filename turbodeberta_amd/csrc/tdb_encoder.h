@@ -12,15 +12,16 @@ enum { TDB_MASK_I64 = 3, TDB_MASK_I32 = 4, TDB_MASK_U8 = 5 };
 enum { TDB_SCAN_MAX_BATCH = 1024 };
 
 // lens[b] = number of nonzero entries of row b, cu = their running sum from 0; flags[0] = 1 if every row has its nonzero
-// entries first, flags[1] = sum of lens, flags[2] = 1 if every nonzero entry is 1; then flags[3] = ticket.  `flags` may be
-// pinned host memory.
-int tdb_enc_scan_mask(const void* mask, int type, int64_t stride_b, int64_t stride_l, int B, int L, int32_t* lens, int32_t* cu,
-                      int32_t* flags, int ticket, void* stream);
+// entries first, flags[1] = sum of lens, flags[2] = 1 if every nonzero entry is 1, flags[3] = 1 if the ids at nonzero entries
+// (ids: [B, L] row after row, or NULL: not looked at) lie in [0, vocab); then flags[4] = ticket.  `flags` may be pinned host
+// memory.
+int tdb_enc_scan_mask(const void* mask, int type, int64_t stride_b, int64_t stride_l, int B, int L, const void* ids, int ids64, int64_t vocab,
+                      int32_t* lens, int32_t* cu, int32_t* flags, int ticket, void* stream);
 
 // Order of activation rows: mt = 0 row after row; mt > 0 (tdb_enc_small_tiles) the order in which the small products load
 // them, 16 mt rows of room.
 
-// out[t] = LayerNorm(table[ids of token t]); cu != NULL: token t of the packed batch, cu == NULL: ids in order.
+// out[t] = LayerNorm(table[ids of token t]), NaN for an id outside the table; cu != NULL: token t of the packed batch, cu == NULL: ids in order.
 int tdb_enc_embed(const void* ids, int ids64, const void* table, int64_t vocab, const void* gamma, const void* beta, float eps,
                   const int32_t* cu, int B, int L, int T, int hidden, int dtype, int mt, void* out, void* stream);
 

@@ -88,7 +88,7 @@ class _MaskInfo:
         self.lengths, self.total, self.cu, self.ones, self.declared = lengths, total, cu, ones, declared
 
 
-def _mask_info(attention_mask):
+def _mask_info(attention_mask, ids=None, vocab=0):
     """Valid lengths of a batch whose mask is **right padded** (valid tokens first), verified: the kernels take
     per-sequence lengths, so a mask with holes or left padding cannot be expressed and raises ``ValueError`` instead
     of attending to the wrong tokens.  A 3-D / 4-D mask must be the outer product ``m_i * m_j`` Hugging Face's
@@ -97,15 +97,20 @@ def _mask_info(attention_mask):
     the result is attached to the tensor, so the layers of an encoder, which all receive the same mask object
     (modeling_deberta_v2.py:651-660), share it.  (A mask without a modification counter -- an inference tensor --
     is trusted not to be modified in place between calls.)  Under ``torch.jit.trace`` nothing is attached or taken from an
-    earlier call: to the tracer such lengths are constants, and a replay on another mask would go by the first one's."""
+    earlier call: to the tracer such lengths are constants, and a replay on another mask would go by the first one's.
+
+    With ``ids`` (of the mask's shape), a valid token whose id does not lie in ``[0, vocab)`` raises ``IndexError`` where the
+    mask is measured by the one kernel, which then reads the ids as well."""
     version = _version_of(attention_mask)
     tracing = torch.jit.is_tracing()
     cached = getattr(attention_mask, "_tdb_info", None)
     if cached is not None and cached[0] == version and (cached[1].declared or not tracing):
         return cached[1]
-    scan = _lib.host().scan_mask(attention_mask) if attention_mask.is_cuda and attention_mask.dim() == 2 else None
+    scan = _lib.host().scan_mask(attention_mask, ids, vocab) if attention_mask.is_cuda and attention_mask.dim() == 2 else None
     if scan is not None:                                             # one kernel, one synchronisation
-        lengths, cu, ok_host, total, ones = scan
+        lengths, cu, ok_host, total, ones, known = scan
+        if not known:
+            raise IndexError(f"input_ids: the ids of valid tokens must lie in [0, {vocab})")
     else:
         cu = ones = None
         valid = key_padding_mask(attention_mask) != 0                               # [B, L]
@@ -511,7 +516,12 @@ class FlashDebertaV2Model(DebertaV2Model):
         then uses the last one (modeling_deberta_v2.py:760-768).  When the caller did not ask for the hidden states
         (and no ``z_steps`` pass needs the last but one), the encoder is told so through its ``intermediate_states``
         argument, so that the packed path does not scatter every layer's result back to ``[B, L, hidden]`` for
-        nothing.  Nothing is stored on the modules: concurrent calls on one model do not see each other's flags."""
+        nothing.  Nothing is stored on the modules: concurrent calls on one model do not see each other's flags.
+
+        Ids outside the vocabulary: where the native loop runs and a mask is measured (the first call with a mask object) a
+        valid token's id raises ``IndexError``; without a mask, with one that has been measured before or that the caller has
+        declared, nothing is read back and every token of that id's sequence comes back as NaN.  The other paths are
+        PyTorch's embedding, whose kernel aborts the process."""
         cfg = self.config
         want_hidden = output_hidden_states if output_hidden_states is not None else cfg.output_hidden_states
         if want_hidden or self.z_steps > 1 or kwargs:
@@ -560,7 +570,7 @@ class FlashDebertaV2Model(DebertaV2Model):
             return None
         cu, total = None, B * L
         if attention_mask is not None:
-            info = _mask_info(attention_mask)                        # the one host synchronisation
+            info = _mask_info(attention_mask, input_ids, self.embeddings.word_embeddings.weight.shape[0])    # the one host synchronisation
             if not info.total or not info.ones:
                 return None
             if info.total < B * L:
