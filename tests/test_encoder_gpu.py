@@ -234,6 +234,21 @@ def test_product_tiles(tile, dtype, code):
             torch.testing.assert_close(parts.double().sum(0), ref, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("dtype,code", [(torch.bfloat16, 1), (torch.float16, 2)])
+def test_gelu_over_its_range(dtype, code):
+    """GELU of the products' epilogue, through a product with a unit vector: half a unit in the last place of the result, the
+    fit's 6e-6 and, below -5, its 3e-10."""
+    lib, ptr = _lib.load(), lambda t: C.c_void_p(t.data_ptr())
+    v = torch.cat([torch.linspace(-9, 9, 20001), torch.tensor([0., -20., 20., -6e4, 6e4, float("inf"), -float("inf"), float("nan")])]).to(dtype).cuda()
+    x, w, b = torch.zeros(len(v), 64, dtype=dtype, device="cuda"), torch.zeros(8, 64, dtype=dtype, device="cuda"), torch.zeros(8, dtype=dtype, device="cuda")
+    x[:, 0], w[:, 0] = v, 1
+    y = torch.empty(len(v), 8, dtype=dtype, device="cuda")
+    assert lib.tdb_enc_gemm(ptr(x), ptr(w), ptr(b), 4, 1, len(v), 8, 64, code, ptr(y), C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    ref = torch.nn.functional.gelu(v.double())[:, None].expand(-1, 8)
+    smallest = 2.0 ** -24 if dtype == torch.float16 else 0.0
+    torch.testing.assert_close(y.double(), ref, rtol=torch.finfo(dtype).eps / 2 + 6e-6, atol=smallest / 2 + 3e-10, equal_nan=True)
+
+
 def test_product_limits():
     lib = _lib.load()
     for M, N, K, dtype in [(16, 8, 96, 1), (16, 12, 64, 1), (0, 8, 64, 1), (16, 8, 64, 0), (1 << 16, 8, 1 << 15, 1)]:

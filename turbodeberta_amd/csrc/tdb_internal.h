@@ -165,18 +165,22 @@ __device__ __forceinline__ bool tdb_locate_tile_sorted(const TdbKernelParams& p,
     return true;
 }
 
-// v Phi(v) as v / (1 + 2^-(v r(v^2))), r a polynomial fitted here to the logarithm of Phi(v) / Phi(-v): relative error 4e-6
-// where the result exceeds 1e-6 in size, absolute 1e-8 |v| below, far inside the rounding of the 16-bit result.  11 plain
-// instructions and two quarter-rate ones per element; erff takes about 40.
+// v Phi(v) as v / (1 + 2^-(v r(v^2))), r a polynomial fitted here to the logarithm of Phi(v) / Phi(-v).  Error against 64 bits,
+// evaluated in 32 (in brackets that of v (1 + erf) / 2 in 32 bits, which cancels below): relative 2.4e-6 on [-1, 0] and 3.1e-6
+// (2.6e-6) on [-2.5, 0], 3.6e-6 (4.6e-4) to -4, 4.4e-6 (4.3e-3) to -4.5, 6e-6 (4.7e-2) to -5; below, where the result is under
+// 1.5e-6 in size, 1e-10 absolute to -5.5 and 3e-10 beyond.  v r grows with v throughout, so the result goes to 0 and to v.
+// 13 plain instructions and two quarter-rate ones per element; erff takes about 40.
 __device__ __forceinline__ float tdb_gelu(float v) {
     const float u = v * v;
-    float r = 4.8300428e-9f;
-    r = fmaf(r, u, -3.6335534e-7f);
-    r = fmaf(r, u, 1.0997374e-5f);
-    r = fmaf(r, u, -1.5498421e-4f);
-    r = fmaf(r, u, -1.1572413e-4f);
-    r = fmaf(r, u, 0.10487763f);
-    r = fmaf(r, u, 2.3021847f);
+    float r = 1.8808817e-12f;
+    r = fmaf(r, u, -2.7793998e-10f);
+    r = fmaf(r, u, 1.7831045e-8f);
+    r = fmaf(r, u, -6.4697991e-7f);
+    r = fmaf(r, u, 1.4255226e-5f);
+    r = fmaf(r, u, -1.751849e-4f);
+    r = fmaf(r, u, -5.1022547e-5f);
+    r = fmaf(r, u, 0.10478447f);
+    r = fmaf(r, u, 2.3022261f);
     return v * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-(v * r)));
 }
 
