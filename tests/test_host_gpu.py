@@ -98,3 +98,9 @@ def test_traced_operators_replay_on_other_inputs(form):
     for seed, split in [(1, 30), (2, 9)]:
         a = inputs(seed, split)
         assert torch.equal(traced(*a), call(*a))
+
+
+def test_compute_units_are_the_devices():
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    assert _lib.load().tdb_compute_units(0) == _lib.load().tdb_compute_units(-1) == units
+    assert _lib.load().tdb_enc_small_splits(768) == min(8, units * 16 // 768)

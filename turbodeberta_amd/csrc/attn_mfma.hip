@@ -1349,7 +1349,6 @@ constexpr int kMaxDevices = 64;
 constexpr int FAR_MIN_LEN = 1536;
 constexpr int kInstances = 64;      // 32 for tables (layout, far, type, c2p, p2c), the strip instances above them
 std::mutex g_dev_mutex;
-int g_cus[kMaxDevices] = {0};
 bool g_attr_set[kMaxDevices][kInstances] = {{false}};
 std::atomic<int> g_workgroup_limit{0};       // cap on the persistent workgroups of a launch (multiple of 8), 0 = none
 
@@ -1444,15 +1443,9 @@ hipError_t tdb_launch_mfma(const TdbKernelParams& whole, int dtype, hipStream_t 
 #undef TDB_PICK_T
 #undef TDB_PICK_STRIP
 #undef TDB_PICK
-    int cus = 0;
+    int cus = std::max(tdb_compute_units(dev), 8) / 8 * 8;
     {
         std::lock_guard<std::mutex> lock(g_dev_mutex);
-        if (g_cus[dev] == 0) {
-            int n = 0;
-            if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 8) n = 8;
-            g_cus[dev] = n / 8 * 8;
-        }
-        cus = g_cus[dev];
         if (!g_attr_set[dev][instance]) {
             e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(smem));
             if (e != hipSuccess) return e;

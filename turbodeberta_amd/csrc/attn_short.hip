@@ -595,7 +595,6 @@ __global__ __launch_bounds__((STRIP ? STRIP_WAVES : MAX_WAVES) * 64) void attn_s
 constexpr int kMaxDevices = 64;
 std::mutex g_mutex;
 bool g_attr_set[kMaxDevices][48] = {{false}};
-int g_cus[kMaxDevices] = {0};
 
 template <int DT, int MODE, bool STRIP>
 const void* kernel_of(bool c2p, bool p2c) {
@@ -616,9 +615,9 @@ const void* kernel_of(bool c2p, bool p2c, int mode) {
 // 18.2: their gathers are shared out over four waves).
 static bool many_tiles(const TdbKernelParams& p) {
     if (p.c2p || p.p2c) return false;
-    const int64_t BH = int64_t(p.B) * p.H;
-    if (p.varlen ? 10 * int64_t(p.total) > 9 * int64_t(p.B) * p.L : !p.seqlens) return 2 * BH > 256;
-    return (p.varlen ? int64_t(p.H) * (p.total / 128) + BH / 2 : BH * 3 / 2) > 448;
+    const int64_t BH = int64_t(p.B) * p.H, cus = tdb_compute_units(-1);
+    if (p.varlen ? 10 * int64_t(p.total) > 9 * int64_t(p.B) * p.L : !p.seqlens) return 2 * BH > cus;
+    return (p.varlen ? int64_t(p.H) * (p.total / 128) + BH / 2 : BH * 3 / 2) > cus * 7 / 4;
 }
 
 bool tdb_short_supported(const TdbKernelParams& p, int dtype) {
@@ -658,11 +657,9 @@ hipError_t tdb_launch_short(const TdbKernelParams& p, int dtype, hipStream_t str
     a.tshift = a.T > 4 ? 3 : a.T > 2 ? 2 : a.T - 1;
     const void* fn = dtype == TDB_F16 ? (strip ? kernel_of<TDB_F16, true>(c2p, p2c, mode) : kernel_of<TDB_F16, false>(c2p, p2c, mode))
                                       : (strip ? kernel_of<TDB_BF16, true>(c2p, p2c, mode) : kernel_of<TDB_BF16, false>(c2p, p2c, mode));
-    int cus = 0;
+    const int cus = tdb_compute_units(dev);
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        if (g_cus[dev] == 0 && (hipDeviceGetAttribute(&g_cus[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || g_cus[dev] < 1)) g_cus[dev] = 1;
-        cus = g_cus[dev];
         bool& set = g_attr_set[dev][(strip ? 24 : 0) + mode * 8 + (dtype == TDB_F16 ? 4 : 0) + (c2p ? 2 : 0) + (p2c ? 1 : 0)];
         if (!set) {
             e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);

@@ -1,5 +1,6 @@
 // C-ABI front end of libtdb_attn.so: argument validation (host only, testable without a GPU),
 // the relative-position tables, and the two launch entry points.
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -132,6 +133,24 @@ int32_t bucket_one(int32_t r, int32_t buckets, int32_t max_pos, bool& exact) {
 }  // namespace
 
 extern "C" {
+
+int tdb_compute_units(int device) {
+    constexpr int kDevices = 64, kMI355X = 256;
+    static std::atomic<int> known[kDevices];        // 0: not asked yet (twice does no harm)
+    if (device < 0 && hipGetDevice(&device) != hipSuccess) {
+        (void)hipGetLastError();
+        return kMI355X;
+    }
+    if (device < 0 || device >= kDevices) return kMI355X;
+    int n = known[device].load(std::memory_order_relaxed);
+    if (n > 0) return n;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || n < 1) {
+        (void)hipGetLastError();
+        return kMI355X;
+    }
+    known[device].store(n, std::memory_order_relaxed);
+    return n;
+}
 
 int tdb_version(void) { return TDB_ABI_VERSION; }
 

@@ -6,6 +6,7 @@
 //     of the weight matrix is requested at once; sums of the waves meet in LDS.  Where the output has too few columns to
 //     fill the chip (hidden-sized ones), the contraction is split over workgroups as well, and the residual + LayerNorm
 //     that follows adds the parts up in a fixed order.
+#include <algorithm>
 #include <type_traits>
 
 #include "tdb_encoder.h"
@@ -416,6 +417,9 @@ int tdb_enc_small_tiles(int M, int N, int K, int dtype) {
     if ((dtype != TDB_BF16 && dtype != TDB_F16) || M < 1 || M > SMALL_ROWS || N < 1 || N % 32 || K < 1 || K % 32) return 0;
     return (M + 15) / 16;
 }
+
+// About one workgroup (of 16 columns) per CU.
+int tdb_enc_small_splits(int N) { return std::max(1, std::min(MAX_SPLITS, tdb_compute_units(-1) * 16 / std::max(N, 1))); }
 
 int tdb_enc_small_gemm(const void* x, const void* w, const void* bias, int flags, int splits, int M, int N, int K, int dtype, void* y, void* stream) {
     const int tiles = tdb_enc_small_tiles(M, N, K, dtype);

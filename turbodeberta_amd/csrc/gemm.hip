@@ -267,10 +267,10 @@ constexpr Cost COST[] = {{32, 64, 2.96f, 0.62f, 0.148f, 0.07f},  {64, 64, 2.86f,
 constexpr int TILES = 6;
 constexpr int SPLITS[] = {1, 2, 3, 4, 6, 8};
 
-float cost(int tile, int splits, int M, int N, int K, bool gelu) {
+float cost(int tile, int splits, int M, int N, int K, bool gelu, int cus) {
     const Cost& c = COST[tile];
     const int64_t blocks = int64_t((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * splits;
-    const float steps = float(K / BK) / float(splits), n = float((blocks + 255) / 256), fill = float(blocks) / 256.f;
+    const float steps = float(K / BK) / float(splits), n = float((blocks + cus - 1) / cus), fill = float(blocks) / float(cus);
     // Partial sums are written, and read by the kernel after this one, at some 5 bytes per ns.
     const float parts = splits > 1 ? float(splits * 8 - 4) * float(M) * float(N) / 5e6f : 0.f;
     return c.base + fill * c.round + n * (steps * c.step + (gelu ? c.gelu : 0.f)) + parts;
@@ -282,10 +282,11 @@ struct Choice {
 Choice choose(int M, int N, int K, bool gelu, int splits) {             // splits 0: any
     Choice best{1, 1};
     float least = 1e30f;
+    const int cus = tdb_compute_units(-1);
     for (int t = 0; t < TILES; ++t)
         for (int s : SPLITS) {
             if (splits ? s != splits : s > 1 && s > K / BK / 2) continue;
-            if (const float c = cost(t, s, M, N, K, gelu); c < least) least = c, best = {t, s};
+            if (const float c = cost(t, s, M, N, K, gelu, cus); c < least) least = c, best = {t, s};
         }
     return best;
 }

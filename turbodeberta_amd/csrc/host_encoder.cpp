@@ -35,6 +35,7 @@ struct Enc {
     decltype(&tdb_enc_add_norm) add_norm;
     decltype(&tdb_enc_small_gemm) small_gemm;
     decltype(&tdb_enc_small_tiles) small_tiles;
+    decltype(&tdb_enc_small_splits) small_splits;
     decltype(&tdb_enc_unpack) unpack;
     decltype(&tdb_enc_gemm) gemm;
     decltype(&tdb_enc_gemm_splits) gemm_splits;
@@ -302,8 +303,8 @@ at::Tensor encode(const Plan& p, const at::Tensor& ids, const at::Tensor* cu, in
     const int mt = small ? tiles[0] : 0;    // (the same for all three)
     const int64_t rows = small ? 16 * mt : T;
     // Contractions with hidden-sized outputs are split where the output alone gives the CUs too little to do; the add + norm
-    // behind them adds the parts up.  (Few rows: about one workgroup per CU.)
-    const int few = int(std::max<int64_t>(1, std::min<int64_t>(8, 256 * 16 / hidden)));
+    // behind them adds the parts up.
+    const int few = g_enc.small_splits(int(hidden));
     const int splits_o = small ? few : g_enc.gemm_splits(int(T), int(hidden), int(hidden), dt);
     const int splits_f = small ? few : g_enc.gemm_splits(int(T), int(hidden), int(inner), dt);
     const bool own = !small && splits_o && splits_f && g_enc.gemm_splits(int(T), int(3 * hidden), int(hidden), dt) && g_enc.gemm_splits(int(T), int(inner), int(hidden), dt);
@@ -555,16 +556,17 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // bind_encoder(addresses of the tdb_enc_* functions in the order of Enc)
 PyObject* py_bind_encoder(PyObject*, PyObject* args) {
-    unsigned long long f[8];
-    if (!PyArg_ParseTuple(args, "KKKKKKKK", f, f + 1, f + 2, f + 3, f + 4, f + 5, f + 6, f + 7)) return nullptr;
+    unsigned long long f[9];
+    if (!PyArg_ParseTuple(args, "KKKKKKKKK", f, f + 1, f + 2, f + 3, f + 4, f + 5, f + 6, f + 7, f + 8)) return nullptr;
     g_enc.scan_mask = reinterpret_cast<decltype(g_enc.scan_mask)>(f[0]);
     g_enc.embed = reinterpret_cast<decltype(g_enc.embed)>(f[1]);
     g_enc.add_norm = reinterpret_cast<decltype(g_enc.add_norm)>(f[2]);
     g_enc.small_gemm = reinterpret_cast<decltype(g_enc.small_gemm)>(f[3]);
     g_enc.small_tiles = reinterpret_cast<decltype(g_enc.small_tiles)>(f[4]);
-    g_enc.unpack = reinterpret_cast<decltype(g_enc.unpack)>(f[5]);
-    g_enc.gemm = reinterpret_cast<decltype(g_enc.gemm)>(f[6]);
-    g_enc.gemm_splits = reinterpret_cast<decltype(g_enc.gemm_splits)>(f[7]);
+    g_enc.small_splits = reinterpret_cast<decltype(g_enc.small_splits)>(f[5]);
+    g_enc.unpack = reinterpret_cast<decltype(g_enc.unpack)>(f[6]);
+    g_enc.gemm = reinterpret_cast<decltype(g_enc.gemm)>(f[7]);
+    g_enc.gemm_splits = reinterpret_cast<decltype(g_enc.gemm_splits)>(f[8]);
     Py_RETURN_NONE;
 }
 

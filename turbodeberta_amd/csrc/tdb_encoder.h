@@ -38,6 +38,8 @@ int tdb_enc_small_gemm(const void* x, const void* w, const void* bias, int flags
                        void* stream);
 // 16-row tiles (mt) of a product that the above takes, else 0
 int tdb_enc_small_tiles(int M, int N, int K, int dtype);
+// the number of partial sums of a product with N columns whose reader adds them up
+int tdb_enc_small_splits(int N);
 
 // Products of any size, 16-bit, rows in order: y[M, N] = x[M, K] w[N, K]^T + bias (flags: 0 or TDB_ENC_GELU), or (splits > 1)
 // float32 partial sums [splits, M, N] without bias.  K a multiple of 64, N of 8; pointers 16-byte aligned.

@@ -34,6 +34,9 @@ struct TdbKernelParams {
     int64_t p2s_b, p2s_h, p2s_l;
 };
 
+// Compute units of a device (negative: the current one); 256, an MI355X, where there is none to ask.
+extern "C" int tdb_compute_units(int device);
+
 // tile heights (query rows per workgroup)
 constexpr int TDB_GENERIC_TILE = 16;
 constexpr int TDB_MFMA_TILE = 128;
