@@ -5,7 +5,7 @@ import math
 import pytest
 import torch
 
-from helpers import assert_close_bf16, make_inputs
+from helpers import assert_close_bf16, make_inputs, oracle_fixed
 from turbodeberta_amd.ops.flash_attention import flash_attention_with_disentangled
 from turbodeberta_amd.ops.flash_attention_varlen import flash_attention_with_disentangled_varlen
 
@@ -53,6 +53,46 @@ def test_lengths_and_padding(B, L):
                                                   pos_query_layer=d["pq"], seqlens_k=lens.cuda(), force_generic=f) for f in (False, True))
     assert_close_bf16(got, ref, f"{B} x {L}")
     assert all(not got[b, :, n:].any() for b, n in enumerate(lens.tolist()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("where", ["query", "key", "value", "last_value", "c2p_row", "p2c_row", "padding", "strip"])
+@pytest.mark.parametrize("L", [29, 50, 128])
+def test_nan_and_infinity_reach_what_they_belong_to(where, L, dtype):
+    """As in the definition: a key that is NaN leaves no query of its sequence a number, a position row that is NaN none that
+    meets it, a value its own columns; padding is not read."""
+    nan, inf = float("nan"), float("inf")
+    d, lens, tables, strips = make_inputs(5, 2, 2, L, 64, 256, 512, dtype), None, ("pk", "pq"), [None, None]
+    if where == "query":
+        d["q"][1, 0, 3, 7] = nan
+    elif where == "key":
+        d["k"][1, 1, L - 1, 0] = nan
+    elif where == "value":
+        d["v"][0, 1, 5, 9] = nan
+    elif where == "last_value":
+        d["v"][0, 0, L - 1, 2], d["v"][1, 1, L - 1, 63] = inf, -inf
+    elif where == "c2p_row":
+        d["pk"][1, 256 + 20, 4] = nan
+    elif where == "p2c_row":
+        d["pq"][0, 256 - 20, 60] = nan
+    elif where == "padding":
+        lens = d["lengths"] = torch.full((2,), L - 20, dtype=torch.int32)
+    ref = oracle_fixed(d, 256, 512)
+    if where == "padding":
+        for n in "qkv":
+            d[n][:, :, L - 20:] = nan
+    elif where == "strip":
+        tables, strips = (), [(x.float() @ t.float().transpose(-1, -2)[None]).to(dtype) for x, t in ((d["q"], d["pk"]), (d["k"], d["pq"]))]
+        strips[0][0, 0, 3, 256 + 2] = nan           # query 3 meets it at key 1
+        strips[1][1, 1, 4, 256 - 3] = nan           # key 4 at query 1
+        ref[0, 0, 3] = ref[1, 1, 1] = nan
+    g = lambda t: None if t is None else t.cuda()
+    got = flash_attention_with_disentangled(g(d["q"]), g(d["k"]), g(d["v"]), *map(g, strips), False, SCALE, 256, 512, seqlens_k=g(lens),
+                                            pos_key_layer=g(d["pk"]) if tables else None, pos_query_layer=g(d["pq"]) if tables else None).float().cpu()
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
+    assert ref.isnan().any() == (where not in ("last_value", "padding"))
+    number = ref.isfinite()
+    assert_close_bf16(got[number], ref[number], where)
 
 
 def test_rows_follow_their_own_maximum():
