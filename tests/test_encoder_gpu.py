@@ -211,6 +211,13 @@ def test_ids_outside_the_vocabulary(bad, id_type, dtype):
         assert out[1].isnan().all() and not out[0].isnan().any() and not out[2].isnan().any()
 
 
+def test_refused_heads_raise_the_operators_error():
+    model, (ids, mask) = _model(torch.bfloat16, hidden=72, heads=6, inner=96), _ids([30, 7, 12], 30)
+    for m in (mask, torch.ones_like(mask)):
+        with torch.no_grad(), pytest.raises(ValueError, match="head_dim 12"):
+            model(input_ids=ids, attention_mask=m)
+
+
 def test_boundaries_it_does_not_take():
     model, (ids, mask) = _model(torch.bfloat16), _ids([30, 7, 12], 30)
     with torch.no_grad():

@@ -287,6 +287,7 @@ int mask_type(at::ScalarType t) {
     }
 }
 
+// Undefined where the attention is refused (a head size, a length): the modules raise its message.
 at::Tensor encode(const Plan& p, const at::Tensor& ids, const at::Tensor* cu, int64_t T) {
     const int64_t B = ids.size(0), L = ids.size(1), H = p.heads, D = p.head_dim, hidden = p.emb.size(1);
     const auto type = p.emb.scalar_type();
@@ -352,7 +353,7 @@ at::Tensor encode(const Plan& p, const at::Tensor& ids, const at::Tensor* cu, in
             a.pos = pos;
             rc = tdb_host_fixed()(&a, s);
         }
-        TORCH_CHECK(rc == TDB_OK, "attention launch failed with status ", rc);
+        if (rc != TDB_OK) return at::Tensor();
         at::Tensor& out = &w == &p.layers.back() ? last : x;
         const int mt_out = &w == &p.layers.back() ? 0 : mt;
         if (small) {
@@ -527,7 +528,7 @@ PyObject* py_scan_mask(PyObject*, PyObject* const* args, Py_ssize_t n) {
     TDB_CATCH
 }
 
-// encode(plan, ids [B, L], cu_seqlens or None, tokens) -> last hidden state, or None for ids or boundaries it does not take
+// encode(plan, ids [B, L], cu_seqlens or None, tokens) -> last hidden state, or None for ids, boundaries or heads it does not take
 PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     TDB_TRY
     Plan* p = n == 4 ? plan_of(args[0]) : nullptr;
@@ -550,6 +551,7 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
         at::AutoDispatchBelowADInplaceOrView below;
         out = encode(*p, ids, cu, T);
     }
+    if (!out.defined()) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(out));
     TDB_CATCH
 }
