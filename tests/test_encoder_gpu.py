@@ -12,7 +12,7 @@ from transformers.models.deberta_v2.modeling_deberta_v2 import DebertaV2Model
 
 from golden_inputs import fill_params
 from turbodeberta_amd import _lib
-from turbodeberta_amd.model import FlashDebertaV2Model, _native_plan, patch_model
+from turbodeberta_amd.model import FlashDebertaV2Model, _native_plan, declare_right_padded, patch_model
 
 pytestmark = pytest.mark.gpu
 
@@ -209,6 +209,43 @@ def test_ids_outside_the_vocabulary(bad, id_type, dtype):
         ids[1, 7] = ids[2, 29] = 5
         out = run(None)
         assert out[1].isnan().all() and not out[0].isnan().any() and not out[2].isnan().any()
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_nothing_computed_under_capture_is_kept(packed):
+    """A forward captured before any eager one: the eager ones after it do not find what only a replay computes."""
+    model, warm = _model(torch.bfloat16), _model(torch.bfloat16)
+    ids, mask = _ids([30, 7, 12] if packed else [30, 30, 30], 30)
+    fresh = lambda: declare_right_padded(mask.clone(), mask.sum(-1, dtype=torch.int32), int(mask.sum())) if packed else None
+    with torch.no_grad():
+        want = warm._forward_native(ids, fresh())                  # (kernels and position tables are there from here on)
+        declared, graph = fresh(), torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            out = model._forward_native(ids, declared)
+        assert out is not None
+        junk = torch.full((1 << 24,), float("nan"), device="cuda")
+        assert torch.equal(model._forward_native(ids, declared), want)
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            assert torch.equal(out, want) and torch.equal(model._forward_native(ids, declared), want)
+        del junk
+
+
+def test_a_plan_serves_other_streams():
+    model, twin = _model(torch.bfloat16), _model(torch.bfloat16)
+    ids, mask = _ids([30, 7, 12], 30)
+    side = torch.cuda.Stream()
+    with torch.no_grad():
+        want = twin._forward_native(ids, None)
+        torch.cuda.synchronize()
+        torch.cuda._sleep(20_000_000)                              # the first call's weights are concatenated behind this
+        first = model._forward_native(ids, None)
+        with torch.cuda.stream(side):
+            second = model._forward_native(ids, None)
+        torch.cuda.synchronize()
+    assert torch.equal(first, want) and torch.equal(second, want)
 
 
 def test_refused_heads_raise_the_operators_error():

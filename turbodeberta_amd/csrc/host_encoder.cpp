@@ -12,6 +12,7 @@
 #include <ATen/ATen.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/GradMode.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
@@ -546,6 +547,8 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int64_t T = PyLong_AsLongLong(args[3]);
     if (ids.device().index() != c10::hip::current_device() || T < 1 || ids.numel() > INT32_MAX || 3 * T * p->emb.size(1) > INT32_MAX)
         Py_RETURN_NONE;
+    // (the boundaries may have been made on another stream and belong to the mask, whose owner does not know of them)
+    if (cu) c10::hip::HIPCachingAllocator::recordStream(cu->storage().data_ptr(), c10::hip::getCurrentHIPStream(ids.device().index()));
     at::Tensor out;
     {
         at::AutoDispatchBelowADInplaceOrView below;

@@ -77,15 +77,21 @@ def _version_of(t):
         return None
 
 
+def _lasting(t):
+    """Whether what is computed now from ``t`` may be kept for later calls: under graph capture it holds nothing before the
+    graph is replayed."""
+    return not (t.is_cuda and torch.cuda.is_current_stream_capturing())
+
+
 class _MaskInfo:
     """What the fused paths need to know about an attention mask: ``lengths`` int32 ``[B]`` on the device,
     ``total``, the number of valid tokens (a host int; ``None`` when the caller declared the lengths without it), the
-    running sum ``cu`` of the lengths (or None: not computed yet), whether every nonzero entry is 1 (None: unknown) and
-    whether the caller declared all this."""
-    __slots__ = ("lengths", "total", "cu", "ones", "declared")
+    running sum ``cu`` of the lengths (or None: not computed yet), the ``stream`` on which that sum has been queued (None: it
+    is there), whether every nonzero entry is 1 (None: unknown) and whether the caller declared all this."""
+    __slots__ = ("lengths", "total", "cu", "ones", "declared", "stream")
 
     def __init__(self, lengths, total, cu=None, ones=None, declared=False):
-        self.lengths, self.total, self.cu, self.ones, self.declared = lengths, total, cu, ones, declared
+        self.lengths, self.total, self.cu, self.ones, self.declared, self.stream = lengths, total, cu, ones, declared, None
 
 
 def _mask_info(attention_mask, ids=None, vocab=0):
@@ -155,12 +161,14 @@ def declare_right_padded(attention_mask, lengths, total=None):
 
 
 def _boundaries(info):
-    """int32 ``[B+1]`` running sum of the lengths, with a leading 0."""
-    if info.cu is not None and not torch.jit.is_tracing():
+    """int32 ``[B+1]`` running sum of the lengths, with a leading 0.  Kept for later calls on the same stream."""
+    n, tracing = info.lengths, torch.jit.is_tracing()
+    stream = torch.cuda.current_stream(n.device).cuda_stream if n.is_cuda else None
+    if info.cu is not None and not tracing and info.stream in (None, stream):
         return info.cu
-    cu = torch.nn.functional.pad(torch.cumsum(info.lengths, dim=0, dtype=torch.int32), (1, 0))
-    if not torch.jit.is_tracing():
-        info.cu = cu
+    cu = torch.nn.functional.pad(torch.cumsum(n, dim=0, dtype=torch.int32), (1, 0))
+    if not tracing and _lasting(n):
+        info.cu, info.stream = cu, stream
     return cu
 
 
@@ -282,7 +290,8 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         if cached is None or cached[0] != key:
             rel = rel_embeddings[0:2 * self.pos_ebd_size]                # dropout is the identity in eval mode
             cached = (key, self._project_tables(rel))
-            self.__dict__["_tdb_tables"] = cached
+            if _lasting(rel):
+                self.__dict__["_tdb_tables"] = cached
         return cached[1]
 
     def _fused_qkv(self):
@@ -296,7 +305,8 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
             if b is None and any(m.bias is not None for m in mods):
                 b = torch.cat([m.bias if m.bias is not None else m.weight.new_zeros(m.weight.shape[0]) for m in mods])
             cached = (key, (w, b))
-            self.__dict__["_tdb_qkv"] = cached
+            if _lasting(w):
+                self.__dict__["_tdb_qkv"] = cached
         return cached[1]
 
 
@@ -349,7 +359,8 @@ class FlashDebertaV2Encoder(DebertaV2Encoder):
                 rel = rel.detach()           # a tensor of its own to carry the tag (shares the storage)
             rel._tdb_source = key
             cached = (key, rel)
-            self.__dict__["_tdb_rel"] = cached
+            if _lasting(rel):
+                self.__dict__["_tdb_rel"] = cached
         return cached[1]
 
     def forward(self, hidden_states, attention_mask, output_hidden_states=True, output_attentions=False,
@@ -433,7 +444,10 @@ def _native_plan(model):
     if not host.complete_plan(plan, model, layers, (table, emb.LayerNorm.weight, emb.LayerNorm.bias, float(emb.LayerNorm.eps)),
                               att.num_attention_heads, att.attention_head_size, scale, buckets, max_rel):
         return None
-    _PLANS[model] = plan
+    if _lasting(table):
+        if table.is_cuda:
+            torch.cuda.current_stream(table.device).synchronize()    # later calls may come on other streams
+        _PLANS[model] = plan
     return plan
 
 
