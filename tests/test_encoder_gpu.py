@@ -248,6 +248,17 @@ def test_a_plan_serves_other_streams():
     assert torch.equal(first, want) and torch.equal(second, want)
 
 
+@pytest.mark.parametrize("lengths,total", [([30, 7, 12], 60), ([30, 7, 12], 20), ([60, -9, 70], 80)])
+def test_declared_lengths_that_do_not_fit(lengths, total):
+    """Nobody verifies them and the results mean nothing; every access stays inside."""
+    model, (ids, mask) = _model(torch.bfloat16), _ids([30, 7, 12], 30)
+    with torch.no_grad():
+        want = model._forward_native(ids, mask)
+        wrong = declare_right_padded(mask.clone(), torch.tensor(lengths, dtype=torch.int32, device="cuda"), total)
+        assert model._forward_native(ids, wrong).shape == want.shape
+        assert torch.equal(model._forward_native(ids, mask.clone()), want)
+
+
 def test_refused_heads_raise_the_operators_error():
     model, (ids, mask) = _model(torch.bfloat16, hidden=72, heads=6, inner=96), _ids([30, 7, 12], 30)
     for m in (mask, torch.ones_like(mask)):

@@ -141,6 +141,18 @@ def test_declared_masks_are_not_inspected():
             declare_right_padded(holes, bad)
 
 
+@pytest.mark.parametrize("lengths,total", [([3, 0, 4, 1], 8), ([4, 4, 4, 4], 16), ([0, 0, 1, 0], 1), ([3, 0, 4, 1], 5), ([3, 0, 4, 1], 12), ([9, -2, 4, 1], 12)])
+def test_packing_stays_inside_the_batch(lengths, total):
+    """Positions of the valid tokens; with lengths that do not fit (nobody verifies a declared mask) whatever, but inside."""
+    from turbodeberta_amd.model import _mask_info, _packing_of, declare_right_padded
+    n = torch.tensor(lengths, dtype=torch.int32)
+    info = _mask_info(declare_right_padded(torch.ones(4, 4), n, total=total))
+    indices, cu = _packing_of(info, 4, 4, n.device)
+    assert len(indices) == total and indices.min() >= 0 and indices.max() < 16 and cu.tolist() == [0, *n.cumsum(0).tolist()]
+    if total == sum(lengths) and min(lengths) >= 0 and max(lengths) <= 4:
+        assert indices.tolist() == [4 * b + i for b, m in enumerate(lengths) for i in range(m)]
+
+
 def test_traced_masks_are_measured_in_every_replay():
     """Lengths, boundaries and packing follow the replay's mask, also where the example has been measured before."""
     from turbodeberta_amd.model import _boundaries, _mask_info, _packing_of

@@ -129,7 +129,7 @@ __global__ __launch_bounds__(256) void embed_kernel(const void* ids, int ids64, 
             if (cu[mid] <= t) lo = mid;
             else hi = mid;
         }
-        at = int64_t(lo) * L + (t - cu[lo]);
+        at = min(max(int64_t(lo) * L + (t - cu[lo]), int64_t(0)), int64_t(B) * L - 1);     // (a caller's boundaries may not fit)
     }
     const int64_t id = ids64 ? static_cast<const int64_t*>(ids)[at] : static_cast<const int32_t*>(ids)[at];
     const bool ok = id >= 0 && id < vocab;
@@ -339,11 +339,11 @@ __global__ __launch_bounds__(1024) void scan_mask_kernel(const void* mask, int t
     }
 }
 
-__global__ __launch_bounds__(256) void unpack_kernel(const uint4* x, const int32_t* cu, int rows, int L, int chunks, uint4* out) {
+__global__ __launch_bounds__(256) void unpack_kernel(const uint4* x, const int32_t* cu, int rows, int L, int T, int chunks, uint4* out) {
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
     if (r >= rows) return;
     const int b = r / L, i = r - b * L, lo = cu[b];
-    const bool in = i < cu[b + 1] - lo;
+    const bool in = i < cu[b + 1] - lo && lo >= 0 && lo < T - i;
     for (int c = l; c < chunks; c += 64) out[int64_t(r) * chunks + c] = in ? x[int64_t(lo + i) * chunks + c] : uint4{0, 0, 0, 0};
 }
 
@@ -455,10 +455,10 @@ int tdb_enc_small_gemm(const void* x, const void* w, const void* bias, int flags
     return known ? int(hipGetLastError()) : int(hipErrorInvalidValue);
 }
 
-int tdb_enc_unpack(const void* x, const int32_t* cu, int B, int L, int hidden, int dtype, void* out, void* stream) {
+int tdb_enc_unpack(const void* x, const int32_t* cu, int B, int L, int T, int hidden, int dtype, void* out, void* stream) {
     const int bytes = hidden * (dtype == TDB_F32 ? 4 : 2);
     if (bytes % 16 || B < 1 || L < 1) return int(hipErrorInvalidValue);
-    hipLaunchKernelGGL(unpack_kernel, dim3((B * L + 3) / 4), dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<const uint4*>(x), cu, B * L, L,
+    hipLaunchKernelGGL(unpack_kernel, dim3((B * L + 3) / 4), dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<const uint4*>(x), cu, B * L, L, T,
                        bytes / 16, static_cast<uint4*>(out));
     return int(hipGetLastError());
 }

@@ -381,7 +381,7 @@ at::Tensor encode(const Plan& p, const at::Tensor& ids, const at::Tensor* cu, in
     }
     if (!cu) return last.view({B, L, hidden});
     at::Tensor out = empty({B, L, hidden}, type);
-    must(g_enc.unpack(ptr(last), bounds, int(B), int(L), int(hidden), dt, ptr(out), s));
+    must(g_enc.unpack(ptr(last), bounds, int(B), int(L), int(T), int(hidden), dt, ptr(out), s));
     return out;
 }
 

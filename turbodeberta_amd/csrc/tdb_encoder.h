@@ -50,8 +50,8 @@ int tdb_enc_gemm(const void* x, const void* w, const void* bias, int flags, int 
 // the number of partial sums that is best for a product whose reader adds them up; 0: a product that the above does not take
 int tdb_enc_gemm_splits(int M, int N, int K, int dtype);
 
-// out[b, l] = x[cu[b] + l] for l < cu[b+1] - cu[b], zeros elsewhere
-int tdb_enc_unpack(const void* x, const int32_t* cu, int B, int L, int hidden, int dtype, void* out, void* stream);
+// out[b, l] = x[cu[b] + l] for l < cu[b+1] - cu[b], zeros elsewhere (and for what does not lie in the T rows of x)
+int tdb_enc_unpack(const void* x, const int32_t* cu, int B, int L, int T, int hidden, int dtype, void* out, void* stream);
 
 #ifdef __cplusplus
 }

@@ -150,8 +150,8 @@ def declare_right_padded(attention_mask, lengths, total=None):
     ``_mask_info`` caches its own findings, so every fused module that receives this mask object uses them and none
     synchronises with the host: a forward on such a mask can be captured into a HIP graph.  ``total`` (a host int, the
     sum of the lengths) additionally lets the encoder pack the batch; without it the encoder keeps the padded layout,
-    because the packed token count sizes host-side allocations.  Nothing is verified: wrong lengths give wrong
-    attention.  (The mask's entries are taken to be 0 and 1.)  Returns the mask."""
+    because the packed token count sizes host-side allocations.  Nothing is verified: wrong lengths, or a total that is
+    not their sum, give wrong results.  (The mask's entries are taken to be 0 and 1.)  Returns the mask."""
     if lengths.dtype != torch.int32 or lengths.dim() != 1 or lengths.shape[0] != attention_mask.shape[0]:
         raise ValueError("lengths must be an int32 tensor with one entry per sequence of the mask")
     if lengths.device != attention_mask.device:
@@ -180,9 +180,9 @@ def _packing_of(info, batch, seqlen, device):
     if torch.jit.is_tracing():
         valid = torch.arange(seqlen, device=device)[None, :] < info.lengths[:, None]
         return torch.nonzero(valid.flatten()).flatten(), cu
-    seq = torch.repeat_interleave(torch.arange(batch, device=device), info.lengths.long(), output_size=info.total)
-    indices = torch.arange(info.total, device=device) - cu[:-1].long()[seq] + seq * seqlen
-    return indices, cu
+    token, starts = torch.arange(info.total, device=device), cu.long()
+    seq = torch.searchsorted(starts[1:], token, right=True).clamp_(max=batch - 1)
+    return (token - starts[seq] + seq * seqlen).clamp_(0, batch * seqlen - 1), cu     # (a caller's lengths may not fit)
 
 
 class FlashDisentangledSelfAttention(DisentangledSelfAttention):
