@@ -11,7 +11,7 @@
 //   * keys, position products and values pass through one scratch area of the wave, one after the other.
 // Measured, persistent kernel before (12 heads, bf16): 1 x 29 8.1 -> 4.5 us, 1 x 128 9.8 -> 9.3, 32 x 64 12.7 -> 7.0,
 // 128 x 96 42 -> 28, 128 x 128 43 -> 37; packed 64 of 4..32 tokens 21 -> 9, 64 of 32..128 28.6 -> 21.9, 300 of 4..96
-// 120 -> 40 (of which 6 are the zero fill of the output).  What bounds it now: a small call, the instructions and memory
+// 120 -> 34.7.  What bounds it now: a small call, the instructions and memory
 // round trips in front of its one step; a large one, LDS instructions (some 700 clk per CU and wave step) under two waves
 // per SIMD.  160 tokens are the limit because the tables of 320 relative positions and seven waves' scratch fill the LDS; many_tiles
 // below says from where they pay.
