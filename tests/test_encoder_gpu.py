@@ -211,15 +211,21 @@ def test_ids_outside_the_vocabulary(bad, id_type, dtype):
         assert out[1].isnan().all() and not out[0].isnan().any() and not out[2].isnan().any()
 
 
-@pytest.mark.parametrize("packed", [False, True])
-def test_nothing_computed_under_capture_is_kept(packed):
+@pytest.mark.parametrize("kind", ["full", "declared", "measured"])
+def test_nothing_computed_under_capture_is_kept(kind):
     """A forward captured before any eager one: the eager ones after it do not find what only a replay computes."""
     model, warm = _model(torch.bfloat16), _model(torch.bfloat16)
-    ids, mask = _ids([30, 7, 12] if packed else [30, 30, 30], 30)
-    fresh = lambda: declare_right_padded(mask.clone(), mask.sum(-1, dtype=torch.int32), int(mask.sum())) if packed else None
+    ids, mask = _ids([30, 30, 30] if kind == "full" else [30, 7, 12], 30)
+    declared = None
+    if kind == "declared":
+        declared = declare_right_padded(mask.clone(), mask.sum(-1, dtype=torch.int32), int(mask.sum()))
+    elif kind == "measured":
+        declared = mask.clone()
     with torch.no_grad():
-        want = warm._forward_native(ids, fresh())                  # (kernels and position tables are there from here on)
-        declared, graph = fresh(), torch.cuda.CUDAGraph()
+        want = warm._forward_native(ids, mask)                     # (kernels and position tables are there from here on)
+        if kind == "measured":
+            warm._forward_native(ids, declared)
+        graph = torch.cuda.CUDAGraph()
         torch.cuda.synchronize()
         with torch.cuda.graph(graph):
             out = model._forward_native(ids, declared)

@@ -111,6 +111,8 @@ def _mask_info(attention_mask, ids=None, vocab=0):
     tracing = torch.jit.is_tracing()
     cached = getattr(attention_mask, "_tdb_info", None)
     if cached is not None and cached[0] == version and (cached[1].declared or not tracing):
+        if not cached[1].declared and attention_mask.is_cuda:        # (they live as long as the mask, whose owner does not know them)
+            cached[1].lengths.record_stream(torch.cuda.current_stream(attention_mask.device))
         return cached[1]
     scan = _lib.host().scan_mask(attention_mask, ids, vocab) if attention_mask.is_cuda and attention_mask.dim() == 2 else None
     if scan is not None:                                             # one kernel, one synchronisation
