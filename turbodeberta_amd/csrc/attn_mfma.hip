@@ -1137,9 +1137,9 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
                 for (int c = 0; c < 2; ++c)
 #pragma unroll
                     for (int dt = 0; dt < 2; ++dt) {
-                        const uint16_t* src = vbase + (32 * jt + 16 * c) * RS + 32 * dt;
+                        const uint16_t* src = vbase + (32 * jt + 8 * c) * RS + 32 * dt;
                         const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(TDB_LDS(s16x4, src));
-                        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(TDB_LDS(s16x4, src + 8 * RS));
+                        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(TDB_LDS(s16x4, src + 16 * RS));
                         const s16x8 both = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
                         vf[jt][c][dt] = __builtin_bit_cast(X8, both);
                     }
@@ -1180,27 +1180,31 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
             m_run = raise ? m_new : m_run;
         }
         const float mc = (m_run - cadd) * c_exp;
-        float psum = 0.f;
+        // Sums and value products in the order of the kernel with resident tables, whose lanes have four keys of sixteen.
+        float psum[2];
 #pragma unroll
         for (int jt = 0; jt < 2; ++jt)
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 uint32_t pw[4];
+                float part = 0.f;
 #pragma unroll
                 for (int h2 = 0; h2 < 4; ++h2) {
-                    const float p0 = __builtin_amdgcn_exp2f(fmaf(s_acc[jt][8 * c + 2 * h2], c_exp, -mc));
-                    const float p1 = __builtin_amdgcn_exp2f(fmaf(s_acc[jt][8 * c + 2 * h2 + 1], c_exp, -mc));
+                    const int e = 4 * c + 8 * (h2 >> 1) + 2 * (h2 & 1);
+                    const float p0 = __builtin_amdgcn_exp2f(fmaf(s_acc[jt][e], c_exp, -mc));
+                    const float p1 = __builtin_amdgcn_exp2f(fmaf(s_acc[jt][e + 1], c_exp, -mc));
                     const X2 pr = {(ET)p0, (ET)p1};
-                    psum += p0 + p1;
+                    part += p0 + p1;
                     pw[h2] = __builtin_bit_cast(uint32_t, pr);
                 }
+                psum[c] = jt == 0 ? part : psum[c] + part;
                 const X8 pb = __builtin_bit_cast(X8, u32x4{pw[0], pw[1], pw[2], pw[3]});
                 // O^T += V^T.P^T
 #pragma unroll
                 for (int dt = 0; dt < 2; ++dt)
                     o_acc[dt] = E::mfma(vf[jt][c][dt], pb, o_acc[dt]);
             }
-        l_run += psum;
+        l_run += psum[0] + psum[1];
         far_cur = far_nxt;
     };
 
@@ -1346,7 +1350,6 @@ namespace {
 // Per-device launch facts, looked up once per device under a lock: CU count (rounded down to the 8 XCDs the block
 // ids are dealt over) and, per kernel instance, whether its dynamic-LDS limit has been raised on that device.
 constexpr int kMaxDevices = 64;
-constexpr int FAR_MIN_LEN = 1536;
 constexpr int kInstances = 64;      // 32 for tables (layout, far, type, c2p, p2c), the strip instances above them
 std::mutex g_dev_mutex;
 bool g_attr_set[kMaxDevices][kInstances] = {{false}};
@@ -1359,6 +1362,8 @@ int tdb_mfma_set_workgroup_limit(int workgroups) {
     g_workgroup_limit.store(cap, std::memory_order_relaxed);
     return cap;
 }
+
+int tdb_mfma_workgroup_limit() { return g_workgroup_limit.load(std::memory_order_relaxed); }
 
 hipError_t tdb_launch_mfma(const TdbKernelParams& whole, int dtype, hipStream_t stream) {
     // Packed batches of more than 64 sequences go out as several launches of at most 64 (even parts): the kernel
@@ -1412,7 +1417,7 @@ hipError_t tdb_launch_mfma(const TdbKernelParams& whole, int dtype, hipStream_t 
     // Far key steps only exist in sequences longer than the table's reach; the instance that looks for them carries
     // both step bodies and its near steps take 1.12x the time, a far step 0.65x.  At length 1024 a quarter of the steps
     // are far and the plain instance is 7 % faster; at 1536 the far instance wins by 2 %, at 4096 by 13 %.
-    const bool farz = !strip && (c2p || p2c) && p.L >= FAR_MIN_LEN;
+    const bool farz = !strip && (c2p || p2c) && p.L >= TDB_FAR_MIN_LEN;
     const int64_t round = int64_t(8) << (farz ? XG_LONG : XG_PLAIN);     // the id regrouping is a bijection on multiples of this
     const int nblocks = int((tiles + round - 1) / round * round);
     const int instance = (p.varlen ? 16 : 0) + (farz ? 8 : 0) + (dtype == TDB_F16 ? 4 : 0) + (c2p ? 2 : 0) + (p2c ? 1 : 0) +

@@ -508,9 +508,9 @@ __global__ __launch_bounds__((STRIP ? STRIP_WAVES : MAX_WAVES) * 64) void attn_s
                     for (int c = 0; c < 2; ++c)
 #pragma unroll
                         for (int dt = 0; dt < 2; ++dt) {
-                            const uint16_t* src = vbase + (32 * jt + 16 * c) * RS + 32 * dt;
+                            const uint16_t* src = vbase + (32 * jt + 8 * c) * RS + 32 * dt;
                             const s16x4 lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(TDB_LDS(s16x4, src));
-                            const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(TDB_LDS(s16x4, src + 8 * RS));
+                            const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(TDB_LDS(s16x4, src + 16 * RS));
                             const s16x8 both = {lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], hi4[3]};
                             vf[jt][c][dt] = __builtin_bit_cast(X8, both);
                         }
@@ -540,24 +540,27 @@ __global__ __launch_bounds__((STRIP ? STRIP_WAVES : MAX_WAVES) * 64) void attn_s
                 m_run = m_new;
             }
             const float mc = m_run * c_exp;
-            float psum = 0.f;
+            float psum[2];                  // (sums and value products in the order of the kernel with resident tables)
 #pragma unroll
             for (int jt = 0; jt < JT; ++jt)
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
                     uint32_t pw[4];
+                    float part = 0.f;
 #pragma unroll
                     for (int h2 = 0; h2 < 4; ++h2) {
-                        const float p0 = __builtin_amdgcn_exp2f(fmaf(s[jt][8 * c + 2 * h2], c_exp, -mc));
-                        const float p1 = __builtin_amdgcn_exp2f(fmaf(s[jt][8 * c + 2 * h2 + 1], c_exp, -mc));
-                        psum += p0 + p1;
+                        const int e = 4 * c + 8 * (h2 >> 1) + 2 * (h2 & 1);
+                        const float p0 = __builtin_amdgcn_exp2f(fmaf(s[jt][e], c_exp, -mc));
+                        const float p1 = __builtin_amdgcn_exp2f(fmaf(s[jt][e + 1], c_exp, -mc));
+                        part += p0 + p1;
                         pw[h2] = pack2<E>(p0, p1);
                     }
+                    psum[c] = jt == 0 ? part : psum[c] + part;
                     const X8 pb = __builtin_bit_cast(X8, u32x4{pw[0], pw[1], pw[2], pw[3]});
 #pragma unroll
                     for (int dt = 0; dt < 2; ++dt) oacc[dt] = E::mfma(vf[jt][c][dt], pb, oacc[dt]);
                 }
-            l_run += psum;
+            l_run += psum[0] + psum[1];
             wave_fence();                   // the next step's keys reuse the scratch
         };
         int k0 = 0;

@@ -93,6 +93,8 @@ int dispatch(const TdbKernelParams& kp, int dtype, int flags, void* stream) {
     const bool any = !(flags & TDB_FLAG_FORCE_GENERIC);
     if (any && tdb_short_supported(kp, dtype)) {
         e = tdb_launch_short(kp, dtype, s);
+    } else if (any && tdb_resident_supported(kp, dtype) && (tdb_resident_pays(kp) || !tdb_mfma_supported(kp, dtype))) {
+        e = tdb_launch_resident(kp, dtype, s);
     } else if (any && tdb_mfma_supported(kp, dtype)) {
         e = tdb_launch_mfma(kp, dtype, s);
     } else if (any && tdb_f32_supported(kp, dtype)) {

@@ -50,14 +50,21 @@ bool tdb_mfma_supported(const TdbKernelParams& p, int dtype);
 // true when the 16-bit kernel for short sequences can take this launch
 bool tdb_short_supported(const TdbKernelParams& p, int dtype);
 
+// true when the 16-bit kernel with position tables resident in LDS can take this launch
+bool tdb_resident_supported(const TdbKernelParams& p, int dtype);
+
 // launchers; return hipError_t of the launch
 hipError_t tdb_launch_generic(const TdbKernelParams& p, int dtype, hipStream_t stream);
 hipError_t tdb_zero_gaps(const TdbKernelParams& p, int dtype, hipStream_t stream);     // a launch of its own
 hipError_t tdb_launch_short(const TdbKernelParams& p, int dtype, hipStream_t stream);
 hipError_t tdb_launch_f32(const TdbKernelParams& p, hipStream_t stream);
 hipError_t tdb_launch_mfma(const TdbKernelParams& p, int dtype, hipStream_t stream);
+bool tdb_resident_pays(const TdbKernelParams& p);
+hipError_t tdb_launch_resident(const TdbKernelParams& p, int dtype, hipStream_t stream);
 // Cap on the persistent workgroups of a launch (multiple of 8, 0 = none); returns the cap in force.
 int tdb_mfma_set_workgroup_limit(int workgroups);
+int tdb_mfma_workgroup_limit();
+constexpr int TDB_FAR_MIN_LEN = 1536;   // 16-bit launches of longer maxima keep the position terms of far steps in 32 bits
 
 // Maps blockIdx.x to (sequence, first row of the tile, valid length).  Returns false when the
 // block has no tile (packed launches are sized by an upper bound on the tile count).  Must be
