@@ -10,7 +10,7 @@
 // through a wave's own LDS scratch with plain 4-byte reads, and no wave waits for another until the end.
 //
 // Measured (vector-ALU kernel before): 1 x 20 x 12 heads 24 -> 5.6 us; 2 x 128 84 -> 8.9; 8 x 12 heads, lengths 96..384, 660 -> 68 us; 8 x 512
-// full 160 us = 81 TFLOP/s without credit for the half-used outer tiles, 101 with (matrix pipe busy 65 % of the time; what is
+// full 157 us = 83 TFLOP/s without credit for the half-used outer tiles, 103 with (matrix pipe busy 65 % of the time; what is
 // left is the start and end of a workgroup, a tenth, and L2 latency that two waves per SIMD do not quite cover).
 //
 // One workgroup = QT*16 query rows of one (sequence, head); its four waves share out the KEYS (blocks of two
@@ -127,10 +127,13 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
     auto delta_of = [&](int r) { return p.lut[min(max(r + p.lut_half, 0), lut_max)]; };
 
     // This wave's key tiles: blocks of KT, dealt to the waves in turn (the position rows of neighbouring blocks overlap
-    // by half, and waves that work on neighbours at the same time find them in L1), or single tiles where there are few.
-    const int ntiles = (len + 15) >> 4, per = (ntiles + WAVES - 1) / WAVES;
-    const bool few = KT > 1 && per < KT;
-    const int first = wave * (few ? 1 : KT), last = few ? min(first + 1, ntiles) : ntiles, stride = WAVES * KT;
+    // by half, and waves that work on neighbours at the same time find them in L1); of the last, incomplete round single tiles, if it has
+    // no more than one for each wave.  (Pairs there gave 12 tiles to the waves as 4, 4, 2, 2 instead of 3 each.)
+    const int ntiles = (len + 15) >> 4, rest = ntiles % (WAVES * KT), behind = ntiles - rest, in_rest = rest > WAVES ? KT * wave : wave;
+    const bool pair_in_rest = rest > WAVES && in_rest + 1 < rest;
+    const int pairs = KT > 1 ? ntiles / (WAVES * KT) + (pair_in_rest ? 1 : 0) : 0;      // then a single tile, if it exists (KT = 1: one after the other)
+    const int single = KT > 1 ? (!pair_in_rest && in_rest < rest ? behind + in_rest : ntiles) : wave;
+    const int first = pairs > 0 ? KT * wave : single;
 
     // Table rows of position tile x of the block that starts at key tile bt: r = row0 - 16 bt + 16 (x - KT) + c.
     int dl[QT + KT];
@@ -138,7 +141,7 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
 #pragma unroll
         for (int x = 0; x < QT + KT; ++x) dl[x] = delta_of(row0 - 16 * bt + 16 * (x - KT) + c);
     };
-    if (!STRIP && (C2P || P2C) && first < last) read_deltas(first);
+    if (!STRIP && (C2P || P2C) && first < ntiles) read_deltas(first);
 
     f32x4 qf[QT][4];
 #pragma unroll
@@ -156,37 +159,46 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
     // Operands are requested one use ahead: a fragment of position rows while the one before it is contracted, the
     // values under the score products, the next block's keys and first position rows under the softmax.
     f32x4 kf[KT][4], pf[2][4];              // keys; position rows of this phase and the next
-    auto load_keys = [&](int bt) {
+    auto load_keys = [&](int bt, bool pair) {
 #pragma unroll
-        for (int bi = 0; bi < KT; ++bi) load_frag(kf[bi], K + int64_t(min(16 * (bt + bi) + c, len - 1)) * p.ks_l, g);
+        for (int bi = 0; bi < KT; ++bi)
+            if (bi == 0 || pair) load_frag(kf[bi], K + int64_t(min(16 * (bt + bi) + c, len - 1)) * p.ks_l, g);
     };
     // phases of a block: position tile x = ph / TERMS, one term after the other (c2p first)
     constexpr int TERMS = int(C2P) + int(P2C), PHASES = STRIP ? 0 : TERMS * (QT + KT);
-    auto load_pos = [&](int ph) {
+    auto load_pos = [&](int ph, int slot) {
         const int x = ph / (TERMS > 0 ? TERMS : 1);
-        if (C2P && (!P2C || ph % 2 == 0)) load_frag(pf[ph & 1], C + int64_t(dl[x]) * p.pks_r, g);
-        else load_frag(pf[ph & 1], P + int64_t(dl[x]) * p.pqs_r, g);
+        if (C2P && (!P2C || ph % 2 == 0)) load_frag(pf[slot], C + int64_t(dl[x]) * p.pks_r, g);
+        else load_frag(pf[slot], P + int64_t(dl[x]) * p.pqs_r, g);
     };
     // Nothing moves across: left alone, the scheduler sinks every load to just before its use (one exposed L2 round
     // trip per 16 bytes: 190 us instead of 138 at batch 8 x 512).
     auto issued = [] { __builtin_amdgcn_sched_barrier(0); };
-    if (first < last) {
-        load_keys(first);
-        if (PHASES) load_pos(0);
-    }
-    for (int bt = first; bt < last; bt += stride) {
-        const bool two = KT > 1 && bt + 1 < last;     // whether the block's second key tile exists
-        f32x4 s[QT][KT];
+    // Keys and first position rows of a block (one of a single tile has no use for the lowest position tile).
+    auto load_first = [&](int bt, bool pair) {
+        load_keys(bt, pair);
+        if (!PHASES) return;
+        if (KT > 1 && pair) load_pos(0, 0);
+        else load_pos(TERMS * (KT - 1), 0);
+    };
+    if (first < ntiles) load_first(first, pairs > 0);
+    auto block = [&](int bt, int after, bool after_pair, auto pair_tag) {    // after: the block that this wave has next
+        constexpr bool PAIR = decltype(pair_tag)::value;
+        constexpr int TILES = PAIR ? KT : 1, LOWEST = KT - TILES;
+        int c_ = c, g_ = g;                 // (opaque for the last tile: address terms that both blocks share would not leave the registers)
+        if (!PAIR) asm volatile("" : "+v"(c_), "+v"(g_));
+        const int c = c_, g = g_;
+        f32x4 s[QT][TILES];
 #pragma unroll
         for (int a = 0; a < QT; ++a)
 #pragma unroll
-            for (int bi = 0; bi < KT; ++bi) s[a][bi] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int bi = 0; bi < TILES; ++bi) s[a][bi] = f32x4{0.f, 0.f, 0.f, 0.f};
 
         if (STRIP) {
 #pragma unroll
             for (int a = 0; a < QT; ++a)
 #pragma unroll
-                for (int bi = 0; bi < KT; ++bi)
+                for (int bi = 0; bi < TILES; ++bi)
 #pragma unroll
                     for (int t = 0; t < 4; ++t) {
                         const int i = min(row0 + 16 * a + c, len - 1), j = min(16 * (bt + bi) + 4 * g + t, len - 1);
@@ -198,13 +210,14 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
             // c2p: query tile a reaches position tiles a .. a+KT; p2c: key tile bi reaches KT-1-bi .. QT+KT-1-bi.
             // (A product with a single tile is summed in two halves: a dependent MFMA waits longer than the pipe is busy.)
 #pragma unroll
-            for (int ph = 0; ph < PHASES; ++ph) {
+            for (int ph = LOWEST * TERMS; ph < PHASES; ++ph) {
                 const int x = ph / TERMS;
-                if (ph + 1 < PHASES) load_pos(ph + 1);
+                const int slot = (ph - LOWEST * TERMS) & 1;
+                if (ph + 1 < PHASES) load_pos(ph + 1, slot ^ 1);
                 issued();
-                const f32x4(&f)[4] = pf[ph & 1];
+                const f32x4(&f)[4] = pf[slot];
                 if (C2P && (!P2C || ph % 2 == 0)) {
-                    constexpr int HALVES = QT * KT == 1 ? 2 : 1;
+                    constexpr int HALVES = QT * TILES == 1 ? 2 : 1;
                     f32x4 acc[QT][HALVES];
 #pragma unroll
                     for (int a = 0; a < QT; ++a)
@@ -214,34 +227,34 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
                     for (int te = 0; te < 16; ++te)
 #pragma unroll
                         for (int a = 0; a < QT; ++a)
-                            if (x >= a && x <= a + KT) acc[a][te % HALVES] = mfma(f[te >> 2][te & 3], qf[a][te >> 2][te & 3], acc[a][te % HALVES]);
+                            if (x >= a + LOWEST && x <= a + KT) acc[a][te % HALVES] = mfma(f[te >> 2][te & 3], qf[a][te >> 2][te & 3], acc[a][te % HALVES]);
 #pragma unroll
                     for (int a = 0; a < QT; ++a)
-                        if (x >= a && x <= a + KT)
+                        if (x >= a + LOWEST && x <= a + KT)
                             *reinterpret_cast<f32x4*>(&sC[(16 * a + c) * CST + 16 * (x - a) + 4 * g]) = HALVES > 1 ? acc[a][0] + acc[a][HALVES - 1] : acc[a][0];
                 } else {
-                    constexpr int HALVES = KT == 1 ? 2 : 1;
-                    f32x4 acc[KT][HALVES];
+                    constexpr int HALVES = TILES == 1 ? 2 : 1;
+                    f32x4 acc[TILES][HALVES];
 #pragma unroll
-                    for (int bi = 0; bi < KT; ++bi)
+                    for (int bi = 0; bi < TILES; ++bi)
 #pragma unroll
                         for (int n = 0; n < HALVES; ++n) acc[bi][n] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int te = 0; te < 16; ++te)
 #pragma unroll
-                        for (int bi = 0; bi < KT; ++bi)
+                        for (int bi = 0; bi < TILES; ++bi)
                             if (x >= KT - 1 - bi && x <= QT + KT - 1 - bi) acc[bi][te % HALVES] = mfma(f[te >> 2][te & 3], kf[bi][te >> 2][te & 3], acc[bi][te % HALVES]);
 #pragma unroll
-                    for (int bi = 0; bi < KT; ++bi)
+                    for (int bi = 0; bi < TILES; ++bi)
                         if (x >= KT - 1 - bi && x <= QT + KT - 1 - bi)
                             *reinterpret_cast<f32x4*>(&sP[(16 * bi + c) * PST + 16 * (x + bi - (KT - 1)) + 4 * g]) = HALVES > 1 ? acc[bi][0] + acc[bi][HALVES - 1] : acc[bi][0];
                 }
             }
-            if (bt + stride < last) read_deltas(bt + stride);
+            if (after < ntiles) read_deltas(after);
             wave_fence();
             // query 16a + c, key 16bi + jl: position i - j sits at 16 (KT - bi) + c - jl of C's row and at 16 (a + 1) + c - jl of P's
 #pragma unroll
-            for (int bi = 0; bi < KT; ++bi)
+            for (int bi = 0; bi < TILES; ++bi)
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const int jl = 4 * g + t;
@@ -255,14 +268,14 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
                 }
             wave_fence();
         }
-        f32x4 vf[KT][4];                    // V[key 4g + t][4c .. 4c+3]
+        f32x4 vf[TILES][4];                 // V[key 4g + t][4c .. 4c+3]
 #pragma unroll
-        for (int bi = 0; bi < KT; ++bi)
+        for (int bi = 0; bi < TILES; ++bi)
 #pragma unroll
             for (int t = 0; t < 4; ++t) vf[bi][t] = *reinterpret_cast<const f32x4*>(V + int64_t(min(16 * (bt + bi) + 4 * g + t, len - 1)) * p.vs_l + 4 * c);
         issued();
         auto score = [&](int bi) {
-            constexpr int HALVES = QT * KT == 1 ? 2 : 1;
+            constexpr int HALVES = QT * TILES == 1 ? 2 : 1;
             f32x4 rest = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int te = 0; te < 16; ++te)
@@ -274,16 +287,13 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
             if (HALVES > 1) s[0][0] += rest;
         };
         score(0);
-        if (two) score(KT - 1);
-        if (bt + stride < last) {
-            load_keys(bt + stride);
-            if (PHASES) load_pos(0);
-        }
+        if (TILES > 1) score(TILES - 1);
+        if (after < ntiles) load_first(after, after_pair);
         issued();
         // Values past the end are zeros, not the last row again: that may be infinite, and its probability there is 0.
-        if (16 * (bt + KT) > len) {
+        if (16 * (bt + TILES) > len) {
 #pragma unroll
-            for (int bi = 0; bi < KT; ++bi)
+            for (int bi = 0; bi < TILES; ++bi)
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
                     if (16 * (bt + bi) + 4 * g + t >= len) vf[bi][t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -293,10 +303,10 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
         for (int a = 0; a < QT; ++a) {
             float mx = -INFINITY;
 #pragma unroll
-            for (int bi = 0; bi < KT; ++bi)
+            for (int bi = 0; bi < TILES; ++bi)
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    const bool in = (bi == 0 || two) && 16 * (bt + bi) + 4 * g + t < len;
+                    const bool in = 16 * (bt + bi) + 4 * g + t < len;
                     s[a][bi][t] = in ? s[a][bi][t] * p.scale : -INFINITY;
                     mx = fmaxf(mx, s[a][bi][t]);        // (NaN scores pass it by and meet exp_neg)
                 }
@@ -304,7 +314,7 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
             const float alpha = exp_neg(m_run[a] - mn);            // (0 on the first block)
             float sum = 0.f;
 #pragma unroll
-            for (int bi = 0; bi < KT; ++bi)
+            for (int bi = 0; bi < TILES; ++bi)
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     s[a][bi][t] = exp_neg(s[a][bi][t] - mn);
@@ -325,7 +335,16 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
                     for (int u = 0; u < 4; ++u) oacc[a][u] = mfma(vf[bi][t][u], s[a][bi][t], oacc[a][u]);
         };
         pv(0);
-        if (two) pv(KT - 1);
+        if (TILES > 1) pv(TILES - 1);
+    };
+    if constexpr (KT > 1) {
+        for (int i = 0; i < pairs; ++i) {
+            const bool more = i + 1 < pairs;
+            block(KT * (WAVES * i + wave), more ? KT * (WAVES * (i + 1) + wave) : single, more, std::true_type{});
+        }
+        if (single < ntiles) block(single, ntiles, false, std::false_type{});
+    } else {
+        for (int bt = single; bt < ntiles; bt += WAVES) block(bt, bt + WAVES, false, std::true_type{});
     }
 
     // Merge of the four waves: partial sums [QT][4][64 lanes] x 16 B, then maxima and denominators of the queries.
@@ -379,8 +398,9 @@ hipError_t tdb_launch_f32(const TdbKernelParams& p, hipStream_t stream) {
     const int64_t blocks = (int64_t((tiles + 3) / 4) * p.H + 7) / 8 * 32 + (p.gap_cu ? GAP_WGS : 0);      // groups of 4 tiles, rounded up to 8 XCDs
     if (blocks > INT32_MAX) return hipErrorInvalidValue;
     // Up to 64 tokens a wave has a single key tile: blocks of two would spend a third of their loads and products on a
-    // second one that is not there (1 x 64 8.2 -> 6.8 us).
-    const bool single = p.L <= 16 * WAVES;
+    // second one that is not there (1 x 64 8.2 -> 6.8 us).  With five tiles, two waves of which would have a pair, single ones pay in large
+    // launches (32 x 80 40.8 -> 39.9, 24 of 40..80 29.4 -> 23.8) and not in small ones (2 x 80 7.9 against 8.8).
+    const bool single = p.L <= 16 * WAVES || (wide && p.L <= 16 * (WAVES + 1));
     const dim3 grid{unsigned(blocks)}, block(WAVES * 64);
     const size_t smem = sizeof(float) * WAVES * wave_floats(wide ? 2 : 1, single ? 1 : 2);
     const bool c2p = strip ? p.c2p != nullptr : p.pk != nullptr, p2c = strip ? p.p2c != nullptr : p.pq != nullptr;
