@@ -332,6 +332,24 @@ def test_product_tiles(tile, dtype, code):
 
 
 @pytest.mark.parametrize("dtype,code", [(torch.bfloat16, 1), (torch.float16, 2)])
+@pytest.mark.parametrize("tile,M,N", [(5, 4229, 2056), (5, 257 * 128, 256), (5, 8192, 3080), (6, 4229, 4104)])
+@pytest.mark.parametrize("K", [192, 256, 320, 448])
+def test_tile_after_tile(tile, M, N, K, dtype, code):
+    """More large tiles than compute units: one more, some workgroups with one more than others, ends inside the output; steps of the
+    contraction one to four more than stages, and as many (which one workgroup a tile takes)."""
+    lib, ptr = _lib.load(), lambda t: C.c_void_p(t.data_ptr())
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn(M, K, device="cuda", generator=g).to(dtype)
+    w, b = (torch.randn(N, K, device="cuda", generator=g) / K ** 0.5).to(dtype), torch.randn(N, device="cuda", generator=g).to(dtype)
+    ref, eps = x.double() @ w.double().t() + b.double(), torch.finfo(dtype).eps
+    for flags in (0, 4):
+        y = torch.full((M, N), 7., device="cuda", dtype=dtype)
+        assert lib.tdb_enc_gemm(ptr(x), ptr(w), ptr(b), flags | tile << 8, 1, M, N, K, code, ptr(y), stream) == 0
+        torch.testing.assert_close(y.double(), torch.nn.functional.gelu(ref) if flags else ref, rtol=eps, atol=eps)
+
+
+@pytest.mark.parametrize("dtype,code", [(torch.bfloat16, 1), (torch.float16, 2)])
 def test_gelu_over_its_range(dtype, code):
     """GELU of the products' epilogue, through a product with a unit vector: half a unit in the last place of the result, the
     fit's 6e-6 and, below -5, its 3e-10."""

@@ -11,6 +11,9 @@
 //   * the tile comes from a small cost model, the contraction is split where the output has too few tiles; the reader of the
 //     output (residual + LayerNorm) adds up the parts.
 //   * bias and GELU are applied to the float32 sums; results leave through LDS in whole rows.
+//   * with more large tiles than compute units, a workgroup takes one after another, and the first stages of the next are on their
+//     way while the last products of this one are made: a tile of 12 to 16 steps otherwise spends a third of its time on its start
+//     and end (8190 x 3072 x 1024, weights in HBM, 53.4 -> 48.4 us; 8192 x 2304 x 768 40.1 -> 35.0; 8192 x 3072 x 768 with GELU 55.5 -> 50.1).
 // A layer's four products and GELU (768 wide, library against these): 128 rows 39 / 23 us, 512 47 / 31, 1024 54 / 40, 4352
 // 109 / 88, 8192 169 / 147; 1024 wide, 5000 rows 174 / 153.
 #include <atomic>
@@ -63,7 +66,8 @@ __device__ __forceinline__ void wait_loads() {
 }
 __device__ __forceinline__ void barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-template <int DT, int BM, int BN, int WM, int WN, int NS, bool GELU, bool PART>
+// LOOP: as many workgroups as compute units, each takes tile after tile.
+template <int DT, int BM, int BN, int WM, int WN, int NS, bool GELU, bool PART, bool LOOP>
 __global__ __launch_bounds__(WM* WN * 64, 2) void gemm_kernel(GemmArgs p) {
     using E = Elem<DT>;
     using T = typename E::T;
@@ -83,8 +87,7 @@ __global__ __launch_bounds__(WM* WN * 64, 2) void gemm_kernel(GemmArgs p) {
     // tile: blocks of one XCD (ids equal mod 8) take neighbouring ones, eight rows of tiles at a time
     const int mt = (p.M + BM - 1) / BM, nt = (p.N + BN - 1) / BN, tiles = mt * nt;
     int m0, n0, split = 0;
-    {
-        int b = blockIdx.x;
+    auto locate = [&](int b) {
         const int all = tiles * (PART ? p.splits : 1), q = all >> 3, r = all & 7, xcd = b & 7;
         b = xcd * q + min(xcd, r) + (b >> 3);
         if (PART) {
@@ -95,23 +98,28 @@ __global__ __launch_bounds__(WM* WN * 64, 2) void gemm_kernel(GemmArgs p) {
         const int n = in / rows;
         m0 = (group * 8 + in - n * rows) * BM;
         n0 = n * BN;
-    }
+    };
+    int number = blockIdx.x;
+    locate(number);
     const int steps_all = p.K / BK;
     const int k0 = PART ? steps_all * split / p.splits : 0, k1 = PART ? steps_all * (split + 1) / p.splits : steps_all, steps = k1 - k0;
 
     // A row is 8 chunks of 16 bytes; chunk c of row r lies at c ^ (r / 2 % 8): fragment reads (16 rows, one chunk) are free of
     // bank conflicts, and a load still covers whole rows.
     uint32_t xo[JX], wo[JW];
+    auto rows_of = [&](int m, int n) {      // where the loads of the tile at row m and column n start
 #pragma unroll
-    for (int j = 0; j < JX; ++j) {
-        const int row = (wave * JX + j) * 8 + (l >> 3);
-        xo[j] = uint32_t(min(m0 + row, p.M - 1)) * uint32_t(p.K * 2) + (((l & 7) ^ ((row >> 1) & 7)) << 4);
-    }
+        for (int j = 0; j < JX; ++j) {
+            const int row = (wave * JX + j) * 8 + (l >> 3);
+            xo[j] = uint32_t(min(m + row, p.M - 1)) * uint32_t(p.K * 2) + (((l & 7) ^ ((row >> 1) & 7)) << 4);
+        }
 #pragma unroll
-    for (int j = 0; j < JW; ++j) {
-        const int row = (wave * JW + j) * 8 + (l >> 3);
-        wo[j] = uint32_t(min(n0 + row, p.N - 1)) * uint32_t(p.K * 2) + (((l & 7) ^ ((row >> 1) & 7)) << 4);
-    }
+        for (int j = 0; j < JW; ++j) {
+            const int row = (wave * JW + j) * 8 + (l >> 3);
+            wo[j] = uint32_t(min(n + row, p.N - 1)) * uint32_t(p.K * 2) + (((l & 7) ^ ((row >> 1) & 7)) << 4);
+        }
+    };
+    rows_of(m0, n0);
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)smem)));
     constexpr int L = JX + JW;
     auto load = [&](int step, int stage, int lo, int hi) {              // loads lo .. hi - 1 of the L of a stage
@@ -126,12 +134,15 @@ __global__ __launch_bounds__(WM* WN * 64, 2) void gemm_kernel(GemmArgs p) {
             }
     };
     f32x16 acc[TM][TN];
+    auto clear = [&]() {
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    };
+    clear();
     const int h = l >> 5;
     int frag[4];                            // chunk 2 kk + h of row l % 32
 #pragma unroll
@@ -196,8 +207,65 @@ __global__ __launch_bounds__(WM* WN * 64, 2) void gemm_kernel(GemmArgs p) {
         stage = stage == NS - 1 ? 0 : stage + 1;
         multiply(3, MORE, stage, NEXT, s + NS, before, 0);
     };
+    // The finished tile, by way of the weights' part of stage `at` that this wave itself loads: rows of COLS columns, their 16-byte chunks
+    // exchanged by the row's middle bits and, in the upper half of the rows, the chunks' halves too, so that writes of 8 bytes to 32 rows
+    // meet every bank once.  (Everybody has read that stage.)
+    auto finish = [&](int m, int n0, int at) {
+        T4 bias[TN][4];
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                bias[j][g] = *reinterpret_cast<const T4*>(static_cast<const T*>(p.bias) + min(n0 + (wn * TN + j) * 32 + 8 * g + 4 * h, p.N - 4));
+        constexpr int COLS = TN * 32, LANES = COLS / 8, LOW = LANES == 8 ? 1 : 2;       // lanes per row of the way out
+        static_assert(32 * COLS * 2 <= JW * 1024 && (LANES == 8 || LANES == 4), "");
+        char* const mine = smem + at * STAGE + BM * 128 + wave * (JW * 1024);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    T4 out;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float v = acc[i][j][4 * g + e] + float(bias[j][g][e]);
+                        if (GELU) v = tdb_gelu(v);
+                        out[e] = T(v);
+                    }
+                    *reinterpret_cast<T4*>(mine + (l & 31) * (COLS * 2) + (((j * 4 + g) ^ (l >> LOW & (LANES - 1))) << 4) + 8 * (h ^ (l >> 4 & 1))) = out;
+                }
+#pragma unroll
+            for (int r = 0; r < 32 * LANES / 64; ++r) {
+                const int row = r * (64 / LANES) + l / LANES, c = l % LANES;
+                uint4 v = *reinterpret_cast<const uint4*>(mine + row * (COLS * 2) + ((c ^ (row >> LOW & (LANES - 1))) << 4));
+                if (row & 16) v = uint4{v.z, v.w, v.x, v.y};
+                const int to = m + (wm * TM + i) * 32 + row, n = n0 + wn * COLS + c * 8;
+                if (to < p.M && n < p.N) *reinterpret_cast<uint4*>(static_cast<T*>(p.y) + int64_t(to) * p.N + n) = v;
+            }
+        }
+    };
+
     int s = 0;
-    for (; s < steps - NS; ++s) step(s, yes, yes, yes);
+    if constexpr (LOOP) {
+        // The stages of the next tile follow those of this one as if they were its next steps; only the last part of the way, behind the last
+        // products, waits for the tile to leave through its stage.  (steps > NS)
+        while (number + int(gridDim.x) < tiles) {
+            const int m = m0, n = n0;
+            for (s = 0; s < steps - NS; ++s) step(s, yes, yes, yes);
+            number += gridDim.x;
+            locate(number);
+            step(s++, yes, no, yes);        // its last loads
+            rows_of(m0, n0);
+            load(0, before, 0, from(1));
+            for (; s < steps - 1; ++s) step(s - steps, yes, yes, yes);
+            step(s - steps, yes, no, yes);
+            finish(m, n, before);
+            load(NS - 1, before, 0, from(1));
+            clear();
+        }
+    }
+    for (s = 0; s < steps - NS; ++s) step(s, yes, yes, yes);
     if (s == steps - NS && s < steps - 1) step(s++, yes, no, yes);
     for (; s < steps - 1; ++s) step(s, no, no, yes);
     step(s, no, no, no);
@@ -220,38 +288,8 @@ __global__ __launch_bounds__(WM* WN * 64, 2) void gemm_kernel(GemmArgs p) {
         }
         return;
     }
-    T4 bias[TN][4];
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-            bias[j][g] = *reinterpret_cast<const T4*>(static_cast<const T*>(p.bias) + min(n0 + (wn * TN + j) * 32 + 8 * g + 4 * h, p.N - 4));
-    constexpr int COLS = TN * 32, STRIDE = COLS * 2 + 16, LANES = COLS / 8;  // lanes per row of the way out
     barrier();
-    char* const mine = smem + wave * (32 * STRIDE);
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                T4 out;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float v = acc[i][j][4 * g + e] + float(bias[j][g][e]);
-                    if (GELU) v = tdb_gelu(v);
-                    out[e] = T(v);
-                }
-                *reinterpret_cast<T4*>(mine + (l & 31) * STRIDE + (j * 32 + 8 * g + 4 * h) * 2) = out;
-            }
-#pragma unroll
-        for (int r = 0; r < 32 * LANES / 64; ++r) {
-            const int row = r * (64 / LANES) + l / LANES, c = l % LANES;
-            const uint4 v = *reinterpret_cast<const uint4*>(mine + row * STRIDE + c * 16);
-            const int m = m0 + (wm * TM + i) * 32 + row, n = n0 + wn * COLS + c * 8;
-            if (m < p.M && n < p.N) *reinterpret_cast<uint4*>(static_cast<T*>(p.y) + int64_t(m) * p.N + n) = v;
-        }
-    }
+    finish(m0, n0, before);
 }
 
 // What a launch of each tile takes, in us:
@@ -264,12 +302,14 @@ struct Cost {
 };
 constexpr Cost COST[] = {{32, 64, 2.96f, 0.62f, 0.148f, 0.07f},  {64, 64, 2.86f, 0.76f, 0.205f, 0.f},   {128, 64, 3.22f, 1.37f, 0.29f, 0.11f},
                          {128, 128, 2.59f, 4.38f, 0.402f, 0.93f}, {128, 256, 2.67f, 7.89f, 0.601f, 2.59f}, {256, 256, 3.55f, 3.7f, 1.195f, 11.09f}};
+// 128 x 256 where workgroups take one tile after another.
+constexpr Cost LOOP_COST = {128, 256, 3.5f, 3.9f, 0.65f, 3.6f};
 constexpr int TILES = 6;
 constexpr int SPLITS[] = {1, 2, 3, 4, 6, 8};
 
 float cost(int tile, int splits, int M, int N, int K, bool gelu, int cus) {
-    const Cost& c = COST[tile];
-    const int64_t blocks = int64_t((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * splits;
+    const int64_t blocks = int64_t((M + COST[tile].bm - 1) / COST[tile].bm) * ((N + COST[tile].bn - 1) / COST[tile].bn) * splits;
+    const Cost& c = tile == 4 && splits == 1 && blocks > cus ? LOOP_COST : COST[tile];
     const float steps = float(K / BK) / float(splits), n = float((blocks + cus - 1) / cus), fill = float(blocks) / float(cus);
     // Partial sums are written, and read by the kernel after this one, at some 5 bytes per ns.
     const float parts = splits > 1 ? float(splits * 8 - 4) * float(M) * float(N) / 5e6f : 0.f;
@@ -298,8 +338,8 @@ bool takes(int M, int N, int K, int dtype) {
 template <int DT, int BM, int BN, int WM, int WN, int NS>
 int launch(const GemmArgs& a, bool gelu, hipStream_t s) {
     constexpr int smem = NS * (BM + BN) * BK * 2 + 256;
-    const int grid = (a.M + BM - 1) / BM * ((a.N + BN - 1) / BN) * a.splits;
-    auto go = [&](auto kernel, std::atomic<uint64_t>& raised) {
+    const int blocks = (a.M + BM - 1) / BM * ((a.N + BN - 1) / BN) * a.splits, cus = tdb_compute_units(-1) & -8;
+    auto go = [&](auto kernel, std::atomic<uint64_t>& raised, int grid) {
         int dev = 0;
         if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return int(e);
         if (!(raised.load(std::memory_order_acquire) >> dev & 1)) {     // (twice does no harm)
@@ -309,10 +349,13 @@ int launch(const GemmArgs& a, bool gelu, hipStream_t s) {
         hipLaunchKernelGGL(kernel, dim3(grid), dim3(WM * WN * 64), smem, s, a);
         return int(hipGetLastError());
     };
-    static std::atomic<uint64_t> raised[3];
-    if (a.splits > 1) return go(gemm_kernel<DT, BM, BN, WM, WN, NS, false, true>, raised[0]);
-    if (gelu) return go(gemm_kernel<DT, BM, BN, WM, WN, NS, true, false>, raised[1]);
-    return go(gemm_kernel<DT, BM, BN, WM, WN, NS, false, false>, raised[2]);
+    static std::atomic<uint64_t> raised[5];
+    if (a.splits > 1) return go(gemm_kernel<DT, BM, BN, WM, WN, NS, false, true, false>, raised[0], blocks);
+    if constexpr (BM * BN >= 128 * 256)
+        if (blocks > cus && cus >= 8 && a.K / BK > NS)
+            return gelu ? go(gemm_kernel<DT, BM, BN, WM, WN, NS, true, false, true>, raised[3], cus) : go(gemm_kernel<DT, BM, BN, WM, WN, NS, false, false, true>, raised[4], cus);
+    if (gelu) return go(gemm_kernel<DT, BM, BN, WM, WN, NS, true, false, false>, raised[1], blocks);
+    return go(gemm_kernel<DT, BM, BN, WM, WN, NS, false, false, false>, raised[2], blocks);
 }
 
 template <int DT>
