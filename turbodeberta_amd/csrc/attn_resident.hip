@@ -388,7 +388,7 @@ bool tdb_resident_supported(const TdbKernelParams& p, int dtype) {
 
 // The persistent kernel (attn_mfma.hip) has tiles of 128 rows only and loads no whole tables: it is ahead where those tiles nearly fill
 // one round of workgroups, and where few rounds leave many workgroups with less than the longest share.  Measured over 716 launches of
-// 180 to 4096 keys: by this rule 1.073x as fast as that kernel alone (always this one: 1.062x, whichever is faster: 1.083x).
+// 180 to 4096 keys: by this rule 1.067x as fast as that kernel alone (always this one: 1.054x, whichever is faster: 1.079x).
 bool tdb_resident_pays(const TdbKernelParams& p) {
     const Grid g = grid_of(-1, p.H, 0);
     const int64_t B = sequences_of(p), seqs = g.heads * B;
@@ -397,7 +397,9 @@ bool tdb_resident_pays(const TdbKernelParams& p) {
         return std::min(equal_cost<1>(seqs, p.L, g.per_group), equal_cost<2>(seqs, p.L, g.per_group)) * 10 <= 52 * rounds;
     }
     const double rounds = ragged_rounds(p, g) * B / p.B;
-    return p.L <= 4 * BN || rounds <= 0.45 || rounds * p.L >= 3000;
+    if (p.L <= 4 * BN || rounds <= 0.45) return true;
+    // (Of few rounds of very different lengths the longest alone decide: 2 of 650 and 2600 0.82x.  With a mask the lengths are only bounded.)
+    return rounds * p.L >= (rounds >= (p.varlen ? 1.4 : 1.75) ? 3000 : 3400);
 }
 
 hipError_t tdb_launch_resident(const TdbKernelParams& whole, int dtype, hipStream_t stream) {
