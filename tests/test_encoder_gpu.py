@@ -332,11 +332,11 @@ def test_product_tiles(tile, dtype, code):
 
 
 @pytest.mark.parametrize("dtype,code", [(torch.bfloat16, 1), (torch.float16, 2)])
-@pytest.mark.parametrize("tile,M,N", [(5, 4229, 2056), (5, 257 * 128, 256), (5, 8192, 3080), (6, 4229, 4104)])
+@pytest.mark.parametrize("tile,M,N", [(5, 4229, 2056), (5, 257 * 128, 256), (5, 8192, 3080), (6, 4229, 4104), (7, 577, 392), (7, 7000, 1032)])
 @pytest.mark.parametrize("K", [192, 256, 320, 448])
 def test_tile_after_tile(tile, M, N, K, dtype, code):
     """More large tiles than compute units: one more, some workgroups with one more than others, ends inside the output; steps of the
-    contraction one to four more than stages, and as many (which one workgroup a tile takes)."""
+    contraction one to four more than stages, and as many (which one workgroup a tile takes); and the tile of 192 rows."""
     lib, ptr = _lib.load(), lambda t: C.c_void_p(t.data_ptr())
     stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
     g = torch.Generator(device="cuda").manual_seed(K)
