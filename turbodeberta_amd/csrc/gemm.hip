@@ -304,15 +304,15 @@ struct Cost {
 // 4608 x 1024 x 4096 44.5 -> 39.4 us, 4100 x 1024 x 1024 14.3 -> 12.6.)
 constexpr Cost COST[] = {{32, 64, 2.96f, 0.62f, 0.148f, 0.07f},  {64, 64, 2.86f, 0.76f, 0.205f, 0.f},   {128, 64, 3.22f, 1.37f, 0.29f, 0.11f},
                          {128, 128, 2.59f, 4.38f, 0.402f, 0.93f}, {128, 256, 2.67f, 7.89f, 0.601f, 2.59f}, {256, 256, 3.55f, 3.7f, 1.195f, 11.09f},
-                         {192, 128, 2.7f, 6.f, 0.47f, 1.9f}};
-// 128 x 256 where workgroups take one tile after another.
-constexpr Cost LOOP_COST = {128, 256, 3.5f, 3.9f, 0.65f, 3.6f};
+                         {192, 128, 3.3f, 6.f, 0.47f, 1.9f}};
+// 128 x 256 and 192 x 128 where workgroups take one tile after another.
+constexpr Cost LOOP_COST[] = {{128, 256, 3.5f, 3.9f, 0.65f, 3.6f}, {192, 128, 2.35f, 5.f, 0.45f, 2.2f}};
 constexpr int TILES = 7;
 constexpr int SPLITS[] = {1, 2, 3, 4, 6, 8};
 
 float cost(int tile, int splits, int M, int N, int K, bool gelu, int cus) {
     const int64_t blocks = int64_t((M + COST[tile].bm - 1) / COST[tile].bm) * ((N + COST[tile].bn - 1) / COST[tile].bn) * splits;
-    const Cost& c = tile == 4 && splits == 1 && blocks > cus ? LOOP_COST : COST[tile];
+    const Cost& c = (tile == 4 || tile == 6) && splits == 1 && blocks > cus ? LOOP_COST[tile / 6] : COST[tile];
     const float steps = float(K / BK) / float(splits), n = float((blocks + cus - 1) / cus), fill = float(blocks) / float(cus);
     // Partial sums are written, and read by the kernel after this one, at some 5 bytes per ns.
     const float parts = splits > 1 ? float(splits * 8 - 4) * float(M) * float(N) / 5e6f : 0.f;
@@ -354,7 +354,7 @@ int launch(const GemmArgs& a, bool gelu, hipStream_t s) {
     };
     static std::atomic<uint64_t> raised[5];
     if (a.splits > 1) return go(gemm_kernel<DT, BM, BN, WM, WN, NS, false, true, false>, raised[0], blocks);
-    if constexpr (BM * BN >= 128 * 256)
+    if constexpr (BM * BN >= 192 * 128)
         if (blocks > cus && cus >= 8 && a.K / BK > NS)
             return gelu ? go(gemm_kernel<DT, BM, BN, WM, WN, NS, true, false, true>, raised[3], cus) : go(gemm_kernel<DT, BM, BN, WM, WN, NS, false, false, true>, raised[4], cus);
     if (gelu) return go(gemm_kernel<DT, BM, BN, WM, WN, NS, true, false, false>, raised[1], blocks);
