@@ -83,6 +83,33 @@ __device__ __forceinline__ void run(const ResidentArgs& p, const int s_at, const
     // readlanes away, and its divisions are done once and for all lanes together.
     const int per_xcd = gridDim.x >> 3, number = int(blockIdx.x & 7) * per_xcd + int(blockIdx.x >> 3);      // neighbours share an XCD
     const int group = number / p.per_group, mine = number - group * p.per_group;
+    // Sequences of different lengths: how many of them end at or before tile k of their kind.
+    const int wholes = EQUAL ? 0 : __builtin_amdgcn_readlane(s_upto.whole, 63), all = EQUAL ? 0 : wholes + __builtin_amdgcn_readlane(s_upto.half, 63);
+    auto before = [&](int k) {
+        const bool whole = k < wholes;
+        const int among = whole ? k : k - wholes;
+        int from = 0;
+#pragma unroll
+        for (int step = 32; step > 0; step >>= 1) {         // (reads of other lanes, by all lanes)
+            const int a = __builtin_amdgcn_ds_bpermute((from + step - 1) * 4, s_upto.whole), b = __builtin_amdgcn_ds_bpermute((from + step - 1) * 4, s_upto.half);
+            if ((whole ? a : b) <= among) from += step;
+        }
+        return from;
+    };
+    // The last, incomplete round goes to the least loaded workgroup first.  After one or two rounds that is reckoned (32 padded texts of
+    // 64 to 512 57.2 -> 53.7 us; it takes a microsecond, too much for texts up to 320); later, and in groups of more workgroups than
+    // lanes, whoever had the cheaper tile of the round before.
+    const int full = all - all % p.per_group, rounds = full / p.per_group;
+    int last = (rounds & 1) ? p.per_group - 1 - mine : mine;
+    if (!EQUAL && (rounds == 1 || rounds == 2) && full < all && p.per_group <= 64 && __builtin_amdgcn_readlane(s_n, 0) > 5 * BN) {
+        int load = lane < p.per_group ? 0 : 1 << 30;
+        for (int j = 0; j < rounds; ++j) {
+            const int k = j * p.per_group + (j ? p.per_group - 1 - lane : lane), n = __builtin_amdgcn_ds_bpermute(before(k) * 4, s_n);
+            if (lane < p.per_group) load += ((n + BN - 1) / BN + 1) * (k < wholes ? StepCost<QG>::whole : StepCost<QG>::half);
+        }
+        const int own = __builtin_amdgcn_readlane(load, mine);
+        last = __builtin_popcountll(__builtin_amdgcn_ballot_w64(load < own || (load == own && lane < mine)));
+    }
     int t_head, t_at, t_len, t_first, t_units, listed = 0;          // t_len = 0: no tile
     auto list_tiles = [&]() {
         const int j = listed + lane;
@@ -108,20 +135,13 @@ __device__ __forceinline__ void run(const ResidentArgs& p, const int s_at, const
             units_to = units_from + HALF * min(2, end - k);
         } else {
             // Whole tiles by decreasing length of their sequence, then the ends by decreasing length, dealt back and forth: whoever got
-            // the costlier tile of one round gets the cheaper one of the next, and the last, incomplete round goes to the least loaded: by
-            // halves if it is less than half a round.
-            const int wholes = __builtin_amdgcn_readlane(s_upto.whole, 63), all = wholes + __builtin_amdgcn_readlane(s_upto.half, 63);
-            const int full = all - all % p.per_group;
+            // the costlier tile of one round gets the cheaper one of the next.  The last, incomplete round goes by halves if it is less than
+            // half a round.
             const bool split = 2 * (all - full) <= p.per_group;
-            const int d = j * p.per_group + ((j & 1) ? p.per_group - 1 - mine : mine), k = split && d >= full ? full + ((d - full) >> 1) : d;
+            const int d = j < rounds ? j * p.per_group + ((j & 1) ? p.per_group - 1 - mine : mine) : j == rounds ? full + last : all + p.per_group;
+            const int k = split && d >= full ? full + ((d - full) >> 1) : d;
             const bool whole = k < wholes;
-            const int among = whole ? k : k - wholes;
-            int from = 0;                   // how many sequences end at or before that tile
-#pragma unroll
-            for (int step = 32; step > 0; step >>= 1) {     // (reads of other lanes, by all lanes)
-                const int a = __builtin_amdgcn_ds_bpermute((from + step - 1) * 4, s_upto.whole), b = __builtin_amdgcn_ds_bpermute((from + step - 1) * 4, s_upto.half);
-                if ((whole ? a : b) <= among) from += step;
-            }
+            const int among = whole ? k : k - wholes, from = before(k);
             const int n = __builtin_amdgcn_ds_bpermute(from * 4, s_n), upto = __builtin_amdgcn_ds_bpermute(from * 4, s_upto.whole),
                       upto_half = __builtin_amdgcn_ds_bpermute(from * 4, s_upto.half);
             t_at = __builtin_amdgcn_ds_bpermute(from * 4, s_at);
