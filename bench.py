@@ -53,18 +53,18 @@ PEAK_FP32_TFLOPS = 157.3        # MI355X fp32, vector and matrix alike, AMD publ
 # commit and a digest of the kernel source they were taken at are recorded in the files named here; `roofline.traffic`
 # repeats them with that source, and `roofline.traffic_stale` is true when the kernel source has changed since.
 RECORDED_TRAFFIC = {
-    "fixed": "profiles/attn_mfma_kernel_fixed_b32xL512.md",
-    "varlen": "profiles/attn_mfma_kernel_varlen_64seq.md",
-    "long": "profiles/attn_mfma_kernel_long_b4xL4096.md",
-    "long_varlen": "profiles/attn_mfma_kernel_long_b4xL4096.md",
+    "fixed": "profiles/attn_resident_kernel.md",
+    "varlen": "profiles/attn_resident_kernel.md",
+    "long": "profiles/attn_resident_kernel.md",
+    "long_varlen": "profiles/attn_resident_kernel.md",
     "strips_b32xL512": "profiles/attn_mfma_kernel_strips_b32xL512.md",
     "strips_b8xL256": "profiles/attn_mfma_kernel_strips_b32xL512.md",
 }
-KERNEL_SOURCES = ("turbodeberta_amd/csrc/attn_mfma.hip", "turbodeberta_amd/csrc/tdb_internal.h")
+KERNEL_SOURCES = tuple("turbodeberta_amd/csrc/" + f for f in ("attn_mfma.hip", "attn_resident.hip", "attn_step.h", "tdb_internal.h"))
 
 
 def kernel_source_digest():
-    """First 16 hex digits of the SHA-256 over the matrix-core kernel's source files, in the order of KERNEL_SOURCES:
+    """First 16 hex digits of the SHA-256 over the matrix-core kernels' source files, in the order of KERNEL_SOURCES:
     what a profile summary records as `kernel_source_sha256:` when its counters are taken."""
     import hashlib
     h = hashlib.sha256()
@@ -447,26 +447,26 @@ def main():
     tensors = lengths_f = None
     if args.workload in ("all", "both", "fixed"):
         plan, lengths_f, tensors = build_fixed(dev)
-        res_fixed = measure(plan, lengths_f, "fixed", "attn_mfma_kernel<c2p,p2c>")
+        res_fixed = measure(plan, lengths_f, "fixed", "attn_resident_kernel<c2p,p2c>")
     if args.workload in ("all", "both", "varlen"):
         plan_v, lengths_v = build_varlen(dev)
-        res_var = measure(plan_v, lengths_v, "varlen", "attn_mfma_kernel<c2p,p2c>")
+        res_var = measure(plan_v, lengths_v, "varlen", "attn_resident_kernel<c2p,p2c>")
     extra = {}
     if args.workload == "all":
         plan_w, lengths_w, _ = build_fixed(dev, shortest=64)
         extra["fixed_wide"] = {"workload": "fixed b32xL512, valid lengths U[64,512] seed 0 (%d valid tokens), 12 heads x 64, c2p|p2c"
                                            % int(lengths_w.sum()),
-                               **measure(plan_w, lengths_w, "fixed_wide", "attn_mfma_kernel<c2p,p2c>")}
+                               **measure(plan_w, lengths_w, "fixed_wide", "attn_resident_kernel<c2p,p2c>")}
         del plan_w
     if args.workload in ("all", "long"):
         few = max(5, min(args.steps, 40))                      # a launch takes ~1 ms: fewer steps keep the run short
         plan_l, lengths_l = build_long(dev)
         extra["long"] = {"workload": "fixed b4xL4096, full mask, 12 heads x 64, buckets 256, max_rel 512, c2p|p2c",
-                         **measure(plan_l, lengths_l, "long", "attn_mfma_kernel<c2p,p2c>", steps=few)}
+                         **measure(plan_l, lengths_l, "long", "attn_resident_kernel<c2p,p2c>", steps=few)}
         del plan_l
         plan_lv, lengths_lv = build_varlen(dev, n_seq=8, lo=1024, hi=4096)
         extra["long_varlen"] = {"workload": "8 packed sequences, lengths U[1024,4096] seed 0, total tokens %d" % int(lengths_lv.sum()),
-                                **measure(plan_lv, lengths_lv, "long_varlen", "attn_mfma_kernel<c2p,p2c>", steps=few)}
+                                **measure(plan_lv, lengths_lv, "long_varlen", "attn_resident_kernel<c2p,p2c>", steps=few)}
         del plan_lv
     if args.workload in ("all", "strips"):
         extra["strips"] = {}
