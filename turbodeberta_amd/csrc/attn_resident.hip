@@ -96,19 +96,40 @@ __device__ __forceinline__ void run(const ResidentArgs& p, const int s_at, const
         }
         return from;
     };
-    // The last, incomplete round goes to the least loaded workgroup first.  After one or two rounds that is reckoned (32 padded texts of
-    // 64 to 512 57.2 -> 53.7 us; it takes a microsecond, too much for texts up to 320); later, and in groups of more workgroups than
-    // lanes, whoever had the cheaper tile of the round before.
-    const int full = all - all % p.per_group, rounds = full / p.per_group;
+    // The last, incomplete round: whole tiles go by halves if there are workgroups for that, also only the longest of them where the next is
+    // clearly shorter, and the costliest to the least loaded workgroup.  Without: 7 packed texts of 1100 89 -> 103 us, 32 padded ones of 64 to
+    // 512 53.7 -> 57.  What workgroups have is reckoned after one or two rounds; it takes a microsecond or two, too much for texts up to 320,
+    // and a lane per workgroup.  Else the order stays, and whoever had the cheaper tile of the round before gets the costlier one.
+    const int full = all - all % p.per_group, rounds = full / p.per_group, rest = all - full;
+    const bool reckon = !EQUAL && (rounds == 1 || rounds == 2) && rest > 0 && p.per_group <= 64 && __builtin_amdgcn_readlane(s_n, 0) > 5 * BN;
+    int halved = EQUAL ? 0 : max(wholes - full, 0);
+    if (rest + halved > p.per_group) {
+        halved = p.per_group - rest;
+        if (reckon) {
+            const int n = __builtin_amdgcn_ds_bpermute(before(full + (lane ? halved : 0)) * 4, s_n);
+            if (10 * __builtin_amdgcn_readlane(n, 1) > 9 * __builtin_amdgcn_readlane(n, 0)) halved = 0;
+        } else if (rounds > 0) halved = 0;
+    }
+    auto last_tile = [&](int i) { return full + (i < 2 * halved ? i >> 1 : i - halved); };
+    auto cost = [&](int n, bool half) { return ((n + BN - 1) / BN + 1) * (half ? StepCost<QG>::half : StepCost<QG>::whole); };
     int last = (rounds & 1) ? p.per_group - 1 - mine : mine;
-    if (!EQUAL && (rounds == 1 || rounds == 2) && full < all && p.per_group <= 64 && __builtin_amdgcn_readlane(s_n, 0) > 5 * BN) {
+    if (reckon) {
         int load = lane < p.per_group ? 0 : 1 << 30;
         for (int j = 0; j < rounds; ++j) {
             const int k = j * p.per_group + (j ? p.per_group - 1 - lane : lane), n = __builtin_amdgcn_ds_bpermute(before(k) * 4, s_n);
-            if (lane < p.per_group) load += ((n + BN - 1) / BN + 1) * (k < wholes ? StepCost<QG>::whole : StepCost<QG>::half);
+            if (lane < p.per_group) load += cost(n, k >= wholes);
         }
         const int own = __builtin_amdgcn_readlane(load, mine);
         last = __builtin_popcountll(__builtin_amdgcn_ballot_w64(load < own || (load == own && lane < mine)));
+        if (halved > 0) {                   // (without halves the order of the costs is that of the tiles, or nearly)
+            const int k = last_tile(lane), n = __builtin_amdgcn_ds_bpermute(before(k) * 4, s_n);
+            const int key = k < all ? cost(n, lane < 2 * halved || k >= wholes) * 64 + 63 - lane : -1;
+            int rank = k < all ? 0 : 64;
+#pragma unroll
+            for (int i = 0; i < 64; ++i) rank += __builtin_amdgcn_readlane(key, i) > key ? 1 : 0;
+            const uint64_t it = __builtin_amdgcn_ballot_w64(rank == last);
+            last = it ? __builtin_ctzll(it) : p.per_group;
+        }
     }
     int t_head, t_at, t_len, t_first, t_units, listed = 0;          // t_len = 0: no tile
     auto list_tiles = [&]() {
@@ -135,11 +156,9 @@ __device__ __forceinline__ void run(const ResidentArgs& p, const int s_at, const
             units_to = units_from + HALF * min(2, end - k);
         } else {
             // Whole tiles by decreasing length of their sequence, then the ends by decreasing length, dealt back and forth: whoever got
-            // the costlier tile of one round gets the cheaper one of the next.  The last, incomplete round goes by halves if it is less than
-            // half a round.
-            const bool split = 2 * (all - full) <= p.per_group;
-            const int d = j < rounds ? j * p.per_group + ((j & 1) ? p.per_group - 1 - mine : mine) : j == rounds ? full + last : all + p.per_group;
-            const int k = split && d >= full ? full + ((d - full) >> 1) : d;
+            // the costlier tile of one round gets the cheaper one of the next.
+            const bool half = j == rounds && last < 2 * halved;
+            const int k = j < rounds ? j * p.per_group + ((j & 1) ? p.per_group - 1 - mine : mine) : j == rounds ? last_tile(last) : all;
             const bool whole = k < wholes;
             const int among = whole ? k : k - wholes, from = before(k);
             const int n = __builtin_amdgcn_ds_bpermute(from * 4, s_n), upto = __builtin_amdgcn_ds_bpermute(from * 4, s_upto.whole),
@@ -156,15 +175,14 @@ __device__ __forceinline__ void run(const ResidentArgs& p, const int s_at, const
                 units_from = units - end;
             }
             units_to = units_from + WAVES;
-            if (split && d >= full) {
-                if ((d - full) & 1) units_from += HALF;
+            if (half) {
+                if (last & 1) units_from += HALF;
                 else units_to -= HALF;
             }
         }
         t_head = group * p.heads + head;
         t_first = units_from;
         t_units = min(units_to, (t_len + UQ - 1) / UQ) - units_from;
-        if (t_units <= 0) t_len = 0;        // (the second half of an end: the last of its workgroup)
     };
     list_tiles();
 
@@ -407,8 +425,9 @@ bool tdb_resident_supported(const TdbKernelParams& p, int dtype) {
 }
 
 // The persistent kernel (attn_mfma.hip) has tiles of 128 rows only and loads no whole tables: it is ahead where those tiles nearly fill
-// one round of workgroups, and where few rounds leave many workgroups with less than the longest share.  Measured over 716 launches of
-// 180 to 4096 keys: by this rule 1.067x as fast as that kernel alone (always this one: 1.054x, whichever is faster: 1.079x).
+// one round of workgroups, and where few rounds leave many workgroups with less than the longest share.  Measured over 638 launches of
+// 300 to 4096 keys of different lengths: by this rule 1.057x as fast as that kernel alone (always this one: 1.055x, whichever is faster:
+// 1.076x; 48 packed texts of 384 0.89x, four others of less than 0.97x).
 bool tdb_resident_pays(const TdbKernelParams& p) {
     const Grid g = grid_of(-1, p.H, 0);
     const int64_t B = sequences_of(p), seqs = g.heads * B;
@@ -417,7 +436,7 @@ bool tdb_resident_pays(const TdbKernelParams& p) {
         return std::min(equal_cost<1>(seqs, p.L, g.per_group), equal_cost<2>(seqs, p.L, g.per_group)) * 10 <= 52 * rounds;
     }
     const double rounds = ragged_rounds(p, g) * B / p.B;
-    if (p.L <= 4 * BN || rounds <= 0.45) return true;
+    if (p.L <= 4 * BN || rounds <= (p.L <= 900 ? 0.6 : 0.45)) return true;
     // (Of few rounds of very different lengths the longest alone decide: 2 of 650 and 2600 0.82x.  With a mask the lengths are only bounded.)
     return rounds * p.L >= (rounds >= (p.varlen ? 1.4 : 1.75) ? 3000 : 3400);
 }
