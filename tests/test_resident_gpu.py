@@ -50,6 +50,7 @@ LENS = {
     "few": [256, 1, 0, 130], "rounds_of_halves": [511, 64, 300] * 3, "64": list(range(4, 516, 8)), "65_in_two": [500] * 60 + [1, 33, 0, 129, 256],
     "last_round_split": [512] * 43 + [129] * 3, "ends": [289] * 50, "long": [1600, 900, 64, 1537, 1, 1300, 2000, 1100],
     "wholes_by_halves": [1100] * 7, "longest_by_halves": [2000, 1732, 1464, 1196, 928, 660], "less_than_a_round": [800, 532, 264],
+    "rounds_far_apart": list(range(640, 210, -11)),
 }
 
 

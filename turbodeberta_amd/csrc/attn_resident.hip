@@ -96,12 +96,16 @@ __device__ __forceinline__ void run(const ResidentArgs& p, const int s_at, const
         }
         return from;
     };
-    // The last, incomplete round: whole tiles go by halves if there are workgroups for that, also only the longest of them where the next is
-    // clearly shorter, and the costliest to the least loaded workgroup.  Without: 7 packed texts of 1100 89 -> 103 us, 32 padded ones of 64 to
-    // 512 53.7 -> 57.  What workgroups have is reckoned after one or two rounds; it takes a microsecond or two, too much for texts up to 320,
-    // and a lane per workgroup.  Else the order stays, and whoever had the cheaper tile of the round before gets the costlier one.
+    // The last, incomplete round: whole tiles go by halves if there are workgroups for that, also only the longest of them where the next
+    // is clearly shorter, and the costliest to the least loaded workgroup.  Without: 7 packed texts of 1100 89 -> 103 us, 32 padded ones
+    // of 64 to 512 53.7 -> 57.  What workgroups have is reckoned after one or two rounds, and after up to five where lengths of more than
+    // 512 are far apart and at most half a round is left (19 packed texts of 450 to 1800 6 % faster; with more left, 8 of 1024 to 4096 2 %
+    // slower).  It takes a microsecond or two, too much for texts up to 320 and elsewhere (39 texts of 384 to 512 2 % slower), and a lane
+    // per workgroup.  Otherwise the order stays, and whoever had the cheaper tile of the round before gets the costlier one.
     const int full = all - all % p.per_group, rounds = full / p.per_group, rest = all - full;
-    const bool reckon = !EQUAL && (rounds == 1 || rounds == 2) && rest > 0 && p.per_group <= 64 && __builtin_amdgcn_readlane(s_n, 0) > 5 * BN;
+    const int longest = EQUAL ? 0 : __builtin_amdgcn_readlane(s_n, 0), shortest = EQUAL ? 0 : __builtin_amdgcn_readlane(s_n, p.B - 1);
+    const bool far_apart = longest > 8 * BN && 2 * shortest < longest && 2 * rest <= p.per_group;
+    const bool reckon = longest > 5 * BN && rest > 0 && p.per_group <= 64 && rounds > 0 && rounds <= (far_apart ? 5 : 2);
     int halved = EQUAL ? 0 : max(wholes - full, 0);
     if (rest + halved > p.per_group) {
         halved = p.per_group - rest;
@@ -116,7 +120,7 @@ __device__ __forceinline__ void run(const ResidentArgs& p, const int s_at, const
     if (reckon) {
         int load = lane < p.per_group ? 0 : 1 << 30;
         for (int j = 0; j < rounds; ++j) {
-            const int k = j * p.per_group + (j ? p.per_group - 1 - lane : lane), n = __builtin_amdgcn_ds_bpermute(before(k) * 4, s_n);
+            const int k = j * p.per_group + ((j & 1) ? p.per_group - 1 - lane : lane), n = __builtin_amdgcn_ds_bpermute(before(k) * 4, s_n);
             if (lane < p.per_group) load += cost(n, k >= wholes);
         }
         const int own = __builtin_amdgcn_readlane(load, mine);
@@ -426,8 +430,8 @@ bool tdb_resident_supported(const TdbKernelParams& p, int dtype) {
 
 // The persistent kernel (attn_mfma.hip) has tiles of 128 rows only and loads no whole tables: it is ahead where those tiles nearly fill
 // one round of workgroups, and where few rounds leave many workgroups with less than the longest share.  Measured over 638 launches of
-// 300 to 4096 keys of different lengths: by this rule 1.057x as fast as that kernel alone (always this one: 1.055x, whichever is faster:
-// 1.076x; 48 packed texts of 384 0.89x, four others of less than 0.97x).
+// 300 to 4096 keys of different lengths: by this rule 1.059x as fast as that kernel alone (always this one: 1.057x, whichever is faster:
+// 1.078x; 48 packed texts of 384 0.91x, three others less than 0.97x).
 bool tdb_resident_pays(const TdbKernelParams& p) {
     const Grid g = grid_of(-1, p.H, 0);
     const int64_t B = sequences_of(p), seqs = g.heads * B;
