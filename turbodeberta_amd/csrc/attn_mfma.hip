@@ -332,8 +332,22 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
         }
         return t;
     };
+    // What only the change of a tile needs is read from the argument segment there (a scalar read that hits the cache; opaque, or it
+    // would be read once at the start).  Kept in scalar registers, blocks of 16 arguments were spilled into vector lanes and reloaded in
+    // every key step, in most instances; which ones changed with every unrelated edit.  (2 padded texts of 840 and 2100: 59.6 -> 56.1 us;
+    // 8 x 250 with 16 heads 14.1 -> 13.8; strips 32 x 512 133.8 -> 130.7.)
+    auto args = [&]() {
+        auto* a = (const __attribute__((address_space(4))) TdbKernelParams*)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(a));
+        return a;
+    };
     auto k_of = [&](const Tile& t) {
-        return static_cast<const uint16_t*>(p.k) + (packed_rows ? t.tok0 * p.ks_l : int64_t(t.b) * p.ks_b) + int64_t(t.head) * p.ks_h;
+        const auto* a = args();
+        return static_cast<const uint16_t*>(a->k) + (packed_rows ? t.tok0 * a->ks_l : int64_t(t.b) * a->ks_b) + int64_t(t.head) * a->ks_h;
+    };
+    auto v_of = [&](const Tile& t) {
+        const auto* a = args();
+        return static_cast<const uint16_t*>(a->v) + (packed_rows ? t.tok0 * a->vs_l : int64_t(t.b) * a->vs_b) + int64_t(t.head) * a->vs_h;
     };
     auto pk_of = [&](const Tile& t) { return HAS_C2P && !STRIP ? static_cast<const uint16_t*>(p.pk) + int64_t(t.head) * p.pks_h : nullptr; };
     auto pq_of = [&](const Tile& t) { return HAS_P2C && !STRIP ? static_cast<const uint16_t*>(p.pq) + int64_t(t.head) * p.pqs_h : nullptr; };
@@ -412,7 +426,7 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
         rows_here = min(BM, (packed_rows ? len : p.L) - row0);   // rows of this tile that exist in memory
         Q = static_cast<const uint16_t*>(p.q) + (packed_rows ? t.tok0 * p.qs_l : int64_t(t.b) * p.qs_b) + int64_t(t.head) * p.qs_h;
         K = k_of(t);
-        V = static_cast<const uint16_t*>(p.v) + (packed_rows ? t.tok0 * p.vs_l : int64_t(t.b) * p.vs_b) + int64_t(t.head) * p.vs_h;
+        V = v_of(t);
         O = static_cast<uint16_t*>(p.o) + (packed_rows ? t.tok0 * p.os_l : int64_t(t.b) * p.os_b) + int64_t(t.head) * p.os_h;
         PK = pk_of(t);
         PQ = pq_of(t);
@@ -427,9 +441,10 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, rows > 0 ? (rows - 1) * stride_b + 128 : 0, RSRC_FLAGS);
     };
     auto load_q = [&](X8 (&dst)[4], const Tile& t) {
-        const uint16_t* Qt = static_cast<const uint16_t*>(p.q) + (packed_rows ? t.tok0 * p.qs_l : int64_t(t.b) * p.qs_b) + int64_t(t.head) * p.qs_h +
-                             int64_t(t.row0) * p.qs_l;
-        const int qs_b = int(p.qs_l) * 2;
+        const auto* a = args();
+        const uint16_t* Qt = static_cast<const uint16_t*>(a->q) + (packed_rows ? t.tok0 * a->qs_l : int64_t(t.b) * a->qs_b) + int64_t(t.head) * a->qs_h +
+                             int64_t(t.row0) * a->qs_l;
+        const int qs_b = int(a->qs_l) * 2;
         const __amdgpu_buffer_rsrc_t rsrc = rows_of(Qt, t.vb >= 0 ? t.len - t.row0 : 0, qs_b);
         int lane = l;                     // opaque, here and below: offsets are redone where they are used instead of
         asm volatile("" : "+v"(lane));    // occupying a register through the key steps
@@ -987,7 +1002,8 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
     // Keys and values travel global -> registers -> LDS through the score waves: thread tid stages chunk sch of rows
     // srow and srow + 32 of a 64-row step.  Buffer loads: the buffer of a step starts at its first row and ends with
     // the last row of the sequence, so rows past the end come back as zeros (hardware range check) with no lane
-    // predicated off, and the per-load address arithmetic is scalar.
+    // predicated off, and the per-load address arithmetic is scalar.  (Offsets inside a sequence fit 31 bits; a step past its end may
+    // wrap, its buffer is empty.)
     const int srow = tid >> 3, sch = tid & 7;
     const int ks_b = int(p.ks_l) * 2, vs_b = int(p.vs_l) * 2;
     int kvoff[2], vvoff[2];
@@ -1000,9 +1016,9 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
     auto fetch_kv_from = [&](const uint16_t* Kt, const uint16_t* Vt, int tlen, int sk, int sv) {
         const int kleft = tlen - BN * sk, vleft = tlen - BN * sv;
         const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint16_t*>(Kt) + int64_t(BN * sk) * p.ks_l, 0, kleft > 0 ? (kleft - 1) * ks_b + 128 : 0, RSRC_FLAGS);
+            const_cast<char*>(reinterpret_cast<const char*>(Kt)) + uint32_t(BN * sk) * uint32_t(ks_b), 0, kleft > 0 ? (kleft - 1) * ks_b + 128 : 0, RSRC_FLAGS);
         const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint16_t*>(Vt) + int64_t(BN * sv) * p.vs_l, 0, vleft > 0 ? (vleft - 1) * vs_b + 128 : 0, RSRC_FLAGS);
+            const_cast<char*>(reinterpret_cast<const char*>(Vt)) + uint32_t(BN * sv) * uint32_t(vs_b), 0, vleft > 0 ? (vleft - 1) * vs_b + 128 : 0, RSRC_FLAGS);
 #pragma unroll
         for (int n = 0; n < 2; ++n) {
             pre_k[n] = __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, kvoff[n], 0, 0);
@@ -1122,8 +1138,7 @@ __global__ __launch_bounds__(NTHREADS) void attn_mfma_kernel(const TdbKernelPara
             // keys of step 2 and values of step 0 of the next tile: its first half A stores them, and a first touch of
             // a new sequence takes longer than the opening of a tile lasts
             if (nxt.vb >= 0)
-                fetch_kv_from(k_of(nxt), static_cast<const uint16_t*>(p.v) + (packed_rows ? nxt.tok0 * p.vs_l : int64_t(nxt.b) * p.vs_b) + int64_t(nxt.head) * p.vs_h,
-                              nxt.len, 2, 0);
+                fetch_kv_from(k_of(nxt), v_of(nxt), nxt.len, 2, 0);
         }
         if (s + 1 < nsteps) fetch_kv(s + 3, s + 1);   // for the next half A (nothing left to fetch in the last step)
         // V^T fragments through the transposing LDS read: the lane provides the address of 4 dims of one key
