@@ -44,6 +44,10 @@ extern "C" {
 #define TDB_FLAG_FORCE_GENERIC 1  /* run the vector-ALU kernel even where the matrix-core kernel applies */
 #define TDB_FLAG_ZERO_UNCOVERED 2 /* packed calls: rows of o that belong to no sequence (or lie beyond max_seqlen) are
                                      written as zeros; without it they are left as they are */
+/* for tests and measurements: of the kernels for 16-bit types and head_dim 64, which give the same bits and are otherwise chosen by
+ * speed, this one wherever it can take the call */
+#define TDB_FLAG_PERSISTENT 4     /* tiles of 128 query rows, position windows computed by waves of their own */
+#define TDB_FLAG_RESIDENT 8       /* position tables resident in LDS */
 
 /*
  * Position inputs shared by both entry points.  Two modes, chosen per term:

@@ -18,6 +18,18 @@ def golden_dir():
     return os.path.join(ROOT, "tests", "golden")
 
 
+@pytest.fixture(params=["chosen", "persistent", "resident"])
+def each_kernel(request):
+    """The test in the 16-bit kernel that the library chooses, then in each of the two for texts of any length."""
+    if request.param == "chosen":
+        yield
+        return
+    from helpers import in_kernel
+    from turbodeberta_amd import _lib
+    with in_kernel(_lib.TDB_FLAG_PERSISTENT if request.param == "persistent" else _lib.TDB_FLAG_RESIDENT):
+        yield
+
+
 def pytest_collection_modifyitems(config, items):
     """Operator parity first, whole-model tests last: the runs that stop at the first failure (`-x`) then report on
     the kernels before a failure of the much larger model tests (several GB of weights, Hugging Face's own eager

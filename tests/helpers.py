@@ -1,10 +1,16 @@
 """Shared builders for the parity tests: seeded inputs, oracle evaluation, comparison rules."""
 from __future__ import annotations
 
+from contextlib import contextmanager
+from types import SimpleNamespace
+from unittest import mock
+
 import numpy as np
 import torch
 
 from oracle import hf_eager as O
+from turbodeberta_amd import _lib
+from turbodeberta_amd.ops import _launch
 
 # Tolerances of the parity bar: float32 outputs within 1e-4 relative, bfloat16 within 2e-2 max-abs.
 FP32_REL = 1e-4
@@ -57,3 +63,17 @@ def pack(inp, lengths):
     for nm in ("q", "k", "v"):
         out[nm] = torch.cat([inp[nm][b, :, :n].transpose(0, 1) for b, n in enumerate(lengths)], 0).contiguous()
     return out, cu
+
+
+@contextmanager
+def in_kernel(flag):
+    """Operator calls inside run in this one of the 16-bit kernels where it can take them (_lib.TDB_FLAG_PERSISTENT or
+    TDB_FLAG_RESIDENT; 0: in the one that the library chooses), through the operators' Python front, which holds the flags."""
+    launch, none = _launch.PreparedLaunch.launch, lambda *args: None
+
+    def flagged(self):
+        self.args.flags |= flag
+        return launch(self)
+    with mock.patch.object(_lib, "host", lambda front=_lib.host(): SimpleNamespace(fixed=none, varlen=none, add_lut=front.add_lut)), \
+            mock.patch.object(_launch.PreparedLaunch, "launch", flagged):
+        yield

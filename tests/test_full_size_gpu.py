@@ -44,6 +44,7 @@ def _oracle_rows(q, k, v, pk, pq, b, n):
                        position_buckets=BUCKETS, max_relative_positions=MAX_REL)[0]
 
 
+@pytest.mark.usefixtures("each_kernel")
 def test_config2_fixed_b32_l512():
     B, L = 32, 512
     lengths = np.random.RandomState(0).randint(384, 513, size=B)
@@ -112,6 +113,7 @@ def test_config2_strip_signature_b32_l512():
     assert torch.equal(outv, pack(out))
 
 
+@pytest.mark.usefixtures("each_kernel")
 def test_config3_varlen_64_sequences():
     lengths = np.random.RandomState(0).randint(16, 513, size=64)
     T = int(lengths.sum())
@@ -170,6 +172,7 @@ def test_config5_long_context_l4096():
     assert_close_bf16(outv[s:e].permute(1, 0, 2), ref1, "config 5 packed", tol=1e-2)
 
 
+@pytest.mark.usefixtures("each_kernel")
 def test_config5_stated_shape_b4_h12_l4096():
     """BASELINE config 5 at its stated shape (batch 4 x 12 heads x seq 4096, full mask): every workgroup walks many
     tiles of 64 key steps, most of them far beyond max_relative_positions.  Whole tensor: the packed run of the same
@@ -201,6 +204,7 @@ def test_config5_stated_shape_b4_h12_l4096():
     assert_close_bf16(out[1:2, hs], ref, "config 5 stated shape vs oracle", tol=1e-2)
 
 
+@pytest.mark.usefixtures("each_kernel")
 def test_config5_packed_variant_8_sequences():
     """BASELINE config 5, packed variant: 8 sequences with lengths uniform in [1024, 4096] (seed 0), 12 heads.  Every
     sequence of 1536 tokens or more on its own through the fixed-length operator is bit-identical (shorter ones take
@@ -249,6 +253,7 @@ def _rows_in_float64(q, k, v, pk, pq, n, rows):
     return torch.stack(out)                                                                           # [rows, H, D]
 
 
+@pytest.mark.usefixtures("each_kernel")
 def test_packed_sequence_of_131072_tokens():
     """One sequence of 2^17 tokens packed with a short one (2 heads): 1024 query tiles of 2048 key steps each, dealt
     by cost over all workgroups -- the tile walk's cost coordinates pass 2^31 / 64 here -- and almost every key step
@@ -282,6 +287,7 @@ def test_packed_sequence_of_131072_tokens():
     assert (mine.float().cpu() - ref[few]).abs().max().item() <= 1e-4
 
 
+@pytest.mark.usefixtures("each_kernel")
 def test_persistent_tile_walk_mixed_lengths():
     """More tiles than workgroups, with everything a persistent workgroup can meet on its list: single-step tiles
     (length <= 64), tiles with only padded rows (in the middle and at the end of a list), a sequence of length 0,

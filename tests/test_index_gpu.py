@@ -90,6 +90,7 @@ def _check(got, want, dtype, what):
 CASES = [(300, [300, 129, 1, 64]), (640, [640, 300]), (4096, [4096, 700])]
 
 
+@pytest.mark.usefixtures("each_kernel")
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("buckets,max_rel", [(256, 512), (-1, 512)], ids=["bucketed", "unbucketed"])
 @pytest.mark.parametrize("L,lengths", CASES, ids=[f"L{c[0]}" for c in CASES])

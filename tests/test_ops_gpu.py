@@ -263,6 +263,7 @@ def test_bf16_varlen_more_than_64_sequences(force_generic):
             assert torch.equal(part, out[lo:hi]), f"sequences {first}..{first + 49}"
 
 
+@pytest.mark.usefixtures("each_kernel")
 def test_repeated_launches_are_bit_identical():
     """The kernels have no atomics and no order-dependent reduction: the same launch must give the same bits every
     time.  A difference between repetitions would mean a race between the waves of a workgroup (a missing barrier,
@@ -296,6 +297,7 @@ def test_repeated_launches_are_bit_identical():
             assert torch.equal(run(), first), f"{name}: launch {rep + 2} differs from the first"
 
 
+@pytest.mark.usefixtures("each_kernel")
 def test_packed_tile_deal_at_other_grid_sizes():
     """The packed launch deals its tiles to the persistent workgroups inside the kernel.  Grids of 8, 24 and 40
     workgroups and the full device must all produce every tile:
@@ -348,6 +350,7 @@ def test_fp16_fixed_vs_oracle(B, H, L, buckets, max_rel, lengths, force_generic)
     assert_close_bf16(out, ref32, "fp16 vs fp32 oracle on rounded inputs", tol=2e-3)
 
 
+@pytest.mark.usefixtures("each_kernel")
 def test_fp16_varlen_matrix_core_equals_vector_alu():
     H, D, buckets, max_rel = 4, 64, 256, 512
     rs = np.random.RandomState(2)
@@ -375,6 +378,7 @@ def _as_projection_output(t):
     return t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)
 
 
+@pytest.mark.usefixtures("each_kernel")
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,H,L,lengths", [
     (5, 3, 400, (400, 1, 129, 256, 37)),        # whole tiles of padding (zeros from the up-front fill) and partial ones
@@ -405,6 +409,7 @@ def test_padded_projection_layout_equals_head_major_layout(B, H, L, lengths, dty
         assert_close_bf16(row_major, ref, "padded projection layout vs fp32 oracle", tol=1e-2 if dtype == torch.bfloat16 else 2e-3)
 
 
+@pytest.mark.usefixtures("each_kernel")
 def test_padded_batch_at_other_grid_sizes():
     """A padded batch with whole tiles of padding at grids of 8, 40 and 248 workgroups: the deal and the up-front fill of
     the padded tiles are both strided over the grid, and every grid must give the full-grid result bit for bit (the

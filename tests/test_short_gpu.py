@@ -1,11 +1,12 @@
 """The 16-bit kernel for short sequences (up to 128 tokens, 160 in large launches) at the edges of its units (32 query rows a wave, 64 keys a
-step), against the vector-ALU kernel and bit for bit against the persistent kernel, which a longer maximum selects."""
+step), against the vector-ALU kernel and bit for bit against the kernels for texts of any length."""
 import math
 
 import pytest
 import torch
 
-from helpers import assert_close_bf16, make_inputs, oracle_fixed
+from helpers import assert_close_bf16, in_kernel, make_inputs, oracle_fixed
+from turbodeberta_amd import _lib
 from turbodeberta_amd.ops.flash_attention import flash_attention_with_disentangled
 from turbodeberta_amd.ops.flash_attention_varlen import flash_attention_with_disentangled_varlen
 
@@ -25,6 +26,12 @@ def _packed(lens, dtype, terms=("c2p", "p2c"), H=3, seed=0):
     return run
 
 
+def _same_in_the_others(got, run, *args):
+    for flag in (_lib.TDB_FLAG_PERSISTENT, _lib.TDB_FLAG_RESIDENT):
+        with in_kernel(flag):
+            assert torch.equal(got, run(*args)), flag
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("L", [1, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128])
 def test_fixed_edges(L, dtype):
@@ -37,10 +44,10 @@ def test_fixed_edges(L, dtype):
 @pytest.mark.parametrize("terms", [("c2p", "p2c"), ("c2p",), ("p2c",), ()])
 @pytest.mark.parametrize("lens", [[1], [30, 2, 33, 64], [16, 40] * 32, [5, 0, 96, 31, 70] * 20, [128, 1, 65, 100] * 25, [3, 9, 17] * 60],
                          ids=["one", "four", "64_with_single_tiles", "100", "100_to_128", "180_tiny"])
-def test_packed_same_bits_as_the_persistent_kernel(lens, terms):
+def test_packed_same_bits_as_the_other_kernels(lens, terms):
     run = _packed(lens, torch.bfloat16, terms)
     got = run(max(lens))
-    assert torch.equal(got, run(161))
+    _same_in_the_others(got, run, 161)      # (a maximum that the short kernel does not take)
     assert_close_bf16(got, run(max(lens), force_generic=True), str(terms))
 
 
@@ -96,7 +103,7 @@ def test_nan_and_infinity_reach_what_they_belong_to(where, L, dtype):
 
 
 def test_rows_follow_their_own_maximum():
-    # scores that grow along the keys raise the running maximum of some rows only: same bits in both kernels
+    # scores that grow along the keys raise the running maximum of some rows only: same bits in all kernels
     d = {n: t.cuda() for n, t in make_inputs(1, 2, 3, 128, 64, 256, 512, torch.bfloat16).items()}
     d["k"] *= torch.linspace(0.1, 12, 128, device="cuda")[None, None, :, None]
     d["q"] *= torch.linspace(0.1, 3, 128, device="cuda")[None, None, :, None]
@@ -104,8 +111,7 @@ def test_rows_follow_their_own_maximum():
     got = flash_attention_with_disentangled(d["q"], d["k"], d["v"], None, None, False, SCALE, 256, 512, **pos)
     wide = [torch.cat([d[n], d[n][:, :, :1]], 2) for n in "qkv"]                   # one row more, masked by its length
     lens = torch.tensor([128, 128], dtype=torch.int32, device="cuda")
-    ref = flash_attention_with_disentangled(*wide, None, None, False, SCALE, 256, 512, seqlens_k=lens, **pos)
-    assert torch.equal(got, ref[:, :, :128])
+    _same_in_the_others(got, lambda: flash_attention_with_disentangled(*wide, None, None, False, SCALE, 256, 512, seqlens_k=lens, **pos)[:, :, :128])
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
@@ -156,7 +162,7 @@ def test_strips(B, L, buckets, dtype, terms):
 def test_five_query_tiles(lens, terms):
     run = _packed(lens, torch.bfloat16, terms)
     got = run(max(lens))
-    assert torch.equal(got, run(161))
+    _same_in_the_others(got, run, 161)      # (a maximum that the short kernel does not take)
     assert_close_bf16(got, run(max(lens), force_generic=True), str(terms))
 
 

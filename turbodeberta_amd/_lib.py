@@ -16,6 +16,7 @@ LIB_PATH = os.path.join(PKG, "libtdb_attn.so")
 TDB_F32, TDB_BF16, TDB_F16 = 0, 1, 2
 TDB_FLAG_FORCE_GENERIC = 1
 TDB_FLAG_ZERO_UNCOVERED = 2
+TDB_FLAG_PERSISTENT, TDB_FLAG_RESIDENT = 4, 8
 ABI_VERSION = 2
 
 ERROR_NAMES = {

@@ -90,10 +90,10 @@ void fill_pos(TdbKernelParams& kp, const tdb_pos_args& ps) {
 int dispatch(const TdbKernelParams& kp, int dtype, int flags, void* stream) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     hipError_t e = hipSuccess;
-    const bool any = !(flags & TDB_FLAG_FORCE_GENERIC);
-    if (any && tdb_short_supported(kp, dtype)) {
+    const bool any = !(flags & TDB_FLAG_FORCE_GENERIC), persistent = flags & TDB_FLAG_PERSISTENT, resident = flags & TDB_FLAG_RESIDENT;
+    if (any && !persistent && !resident && tdb_short_supported(kp, dtype)) {
         e = tdb_launch_short(kp, dtype, s);
-    } else if (any && tdb_resident_supported(kp, dtype) && (tdb_resident_pays(kp) || !tdb_mfma_supported(kp, dtype))) {
+    } else if (any && tdb_resident_supported(kp, dtype) && (resident || (!persistent && tdb_resident_pays(kp)) || !tdb_mfma_supported(kp, dtype))) {
         e = tdb_launch_resident(kp, dtype, s);
     } else if (any && tdb_mfma_supported(kp, dtype)) {
         e = tdb_launch_mfma(kp, dtype, s);
