@@ -1,0 +1,67 @@
+"""The rules by which a 16-bit launch is given to the persistent kernel or to the one with resident tables, and to units of 16 or 32 query
+rows there (turbodeberta_amd/csrc/attn_resident.hip), at launches that were measured.  Without a device they count with 256 compute units."""
+import ctypes as C
+import os
+import re
+
+import pytest
+
+from turbodeberta_amd import _lib
+
+CSRC = os.path.join(os.path.dirname(_lib.PKG), "turbodeberta_amd", "csrc")
+TYPES = {"const void": C.c_void_p, "void": C.c_void_p, "const int32_t": C.c_void_p, "int64_t": C.c_int64, "int32_t": C.c_int32, "float": C.c_float}
+
+
+def _params():
+    """TdbKernelParams, as tdb_internal.h declares it."""
+    body = re.search(r"struct TdbKernelParams \{(.*?)\n\};", open(os.path.join(CSRC, "tdb_internal.h")).read(), re.S).group(1)
+    fields = []
+    for decl in re.sub(r"//.*", "", body).split(";"):
+        m = re.match(r"\s*((?:const )?\w+)\s*(.*)", decl, re.S)
+        if m:
+            fields += [(n.strip(" *\n"), TYPES[m[1]]) for n in m[2].split(",")]
+    return type("TdbKernelParams", (C.Structure,), {"_fields_": fields})
+
+
+def _rule(name):
+    fn = getattr(_lib.load(), f"_Z17tdb_resident_{name}RK15TdbKernelParams")
+    fn.argtypes, fn.restype = [C.c_void_p], C.c_bool
+    return fn
+
+
+def _launch(kind, lens, heads=12, terms=2):
+    p = _params()()
+    p.B, p.H, p.D, p.L, p.span, p.lut_half = len(lens), heads, 64, max(lens), 256, 511
+    p.pk, p.pq = (1 if terms > 0 else None), (1 if terms > 1 else None)
+    if kind == "packed":
+        p.varlen, p.total, p.cu_seqlens = 1, sum(lens), 1
+    elif kind == "padded":
+        p.seqlens = 1
+    return C.byref(p)
+
+
+def _even(n, lo, hi):
+    return [lo + (hi - lo) * i // max(n - 1, 1) for i in range(n)]
+
+
+SHORT_ONES = [10] * 20 + [100] * 10 + [190] * 13 + [233]               # 83 tokens in the mean
+
+
+@pytest.mark.parametrize("kind,lens,heads,terms,resident", [
+    ("packed", _even(64, 16, 512), 12, 2, True), ("padded", _even(32, 384, 512), 12, 2, True), ("equal", [4096] * 4, 12, 2, True),
+    ("packed", _even(8, 1024, 4096), 12, 2, True), ("equal", [250] * 8, 16, 2, False), ("padded", [840, 2100], 12, 2, False),
+    ("packed", _even(35, 384, 384), 8, 0, True), ("packed", [298, 1494], 24, 0, True), ("equal", [2048], 8, 0, True),       # no terms: always
+])
+def test_which_kernel(kind, lens, heads, terms, resident):
+    assert _rule("pays")(_launch(kind, lens, heads, terms)) == resident
+
+
+@pytest.mark.parametrize("kind,lens,heads,wide", [
+    ("packed", _even(64, 16, 512), 12, True), ("padded", _even(32, 384, 512), 12, True), ("packed", _even(8, 1024, 4096), 12, True),
+    ("equal", [512] * 64, 12, True), ("equal", [180], 12, False), ("packed", [300, 200], 12, False),
+    ("packed", SHORT_ONES, 12, False), ("packed", _even(32, 19, 195), 8, False), ("packed", [233] * 44, 12, True),          # short texts among longer ones
+    ("packed", [1835, 3059], 8, True), ("packed", [100] * 5 + [3059], 8, False),                                            # long ones of similar lengths
+    ("packed", _even(66, 22, 222), 8, False),           # a part has half of the tokens
+])
+def test_which_units(kind, lens, heads, wide):
+    assert _rule("wide")(_launch(kind, lens, heads)) == wide

@@ -388,15 +388,32 @@ Grid grid_of(int device, int H, int limit) {
     const int groups = std::gcd(wgs, H);
     return {wgs, wgs / groups, H / groups};
 }
-// Sequences of different lengths: rounds of tiles of 128 rows, as far as the host can tell.
-double ragged_rounds(const TdbKernelParams& p, const Grid& g) {
-    return (p.varlen ? p.total / 128.0 + 0.5 * p.B : double(p.B) * ((p.L + 127) / 128)) * g.heads / g.per_group;
-}
 
 constexpr int MAX_SEQS = 64;                // of different lengths in a launch: one per lane
 int sequences_of(const TdbKernelParams& p) {
     const int parts = p.varlen || p.seqlens ? (p.B + MAX_SEQS - 1) / MAX_SEQS : 1;
     return (p.B + parts - 1) / parts;
+}
+// Sequences of different lengths: rounds of tiles of 128 rows of a launch, as far as the host can tell (p: the whole batch).
+double ragged_rounds(const TdbKernelParams& p, const Grid& g) {
+    return (p.varlen ? p.total / 128.0 / p.B + 0.5 : double((p.L + 127) / 128)) * sequences_of(p) * g.heads / g.per_group;
+}
+// Whether a unit has 32 rows, which read keys and values once where units of 16 read them twice but fill a round or two better.  In packed
+// batches the mean length tells how the sequences end: short ones far below the longest leave units of 32 rows mostly idle (44 of 10 to 233
+// tokens, 83 in the mean: 30.1 -> 24.4 us with 16), long ones of similar lengths end in few half tiles (2 of 1835 and 3059 with 8 heads:
+// 105 -> 78 with 32).  With a mask the host knows the longest possible length only.
+bool wide_units(const TdbKernelParams& p, const Grid& g) {
+    if (!p.varlen && !p.seqlens) {
+        const int64_t seqs = int64_t(g.heads) * p.B;
+        return equal_cost<2>(seqs, p.L, g.per_group) <= equal_cost<1>(seqs, p.L, g.per_group);
+    }
+    double from = 1.25;
+    if (p.varlen) {
+        const double mean = double(p.total) / p.B / p.L;
+        if (p.L <= 4 * BN) from = mean < 0.5 ? 3.2 : mean < 0.65 ? 1.8 : 1.25;
+        else if (p.L >= TDB_FAR_MIN_LEN && mean > 0.65) from = 1.1;
+    }
+    return ragged_rounds(p, g) > from;
 }
 
 constexpr int kMaxDevices = 64;
@@ -428,52 +445,30 @@ bool tdb_resident_supported(const TdbKernelParams& p, int dtype) {
     return (p.pks_r + p.pqs_r) * 2 * (MAX_ROWS + 256) < lim && int64_t(p.B) * p.H * (p.L / 64 + 1) < lim;
 }
 
+bool tdb_resident_wide(const TdbKernelParams& p) { return wide_units(p, grid_of(-1, p.H, 0)); }
+
 // The persistent kernel (attn_mfma.hip) has tiles of 128 rows only and loads no whole tables: it is ahead where those tiles nearly fill
-// one round of workgroups, and where few rounds leave many workgroups with less than the longest share.  Measured over 638 launches of
-// 300 to 4096 keys of different lengths: by this rule 1.059x as fast as that kernel alone (always this one: 1.057x, whichever is faster:
-// 1.078x; 48 packed texts of 384 0.91x, three others less than 0.97x).
+// one round of workgroups, and where few rounds leave many workgroups with less than the longest share.  Measured against that kernel as it
+// was when it took every launch, over 5000 random ones of 161 to 4096 keys (6 to 24 heads; both terms, one or none; equal lengths, evenly
+// spread ones and such as texts have): 1.09x by this rule, 1.115x if the fastest of the two kernels and both heights of units were known.
+// Equal lengths 0.984x at worst; packed 2.5 % of the launches below 0.97x, 0.78x at worst; padded, of which the host knows the longest
+// possible length only, 4.9 %, 0.79x (18 texts, most of them short, 12 heads: 15.7 -> 19.9 us).
 bool tdb_resident_pays(const TdbKernelParams& p) {
+    if (!p.pk && !p.pq) return true;        // (no tables to load: 1.21x over 708 such launches, 1.12x before this line)
     const Grid g = grid_of(-1, p.H, 0);
     const int64_t B = sequences_of(p), seqs = g.heads * B;
     if (!p.varlen && !p.seqlens) {          // (5.2: a step of the persistent kernel's tile in units of StepCost)
         const int64_t rounds = (seqs * ((p.L + 127) / 128) + g.per_group - 1) / g.per_group;
         return std::min(equal_cost<1>(seqs, p.L, g.per_group), equal_cost<2>(seqs, p.L, g.per_group)) * 10 <= 52 * rounds;
     }
-    const double rounds = ragged_rounds(p, g) * B / p.B;
+    const double rounds = ragged_rounds(p, g);
     if (p.L <= 4 * BN || rounds <= (p.L <= 900 ? 0.6 : 0.45)) return true;
     // (Of few rounds of very different lengths the longest alone decide: 2 of 650 and 2600 0.82x.  With a mask the lengths are only bounded.)
     return rounds * p.L >= (rounds >= (p.varlen ? 1.4 : 1.75) ? 3000 : 3400);
 }
 
-hipError_t tdb_launch_resident(const TdbKernelParams& whole, int dtype, hipStream_t stream) {
-    const int per = sequences_of(whole);
-    if (per < whole.B) {                    // in even parts
-        for (int first = 0; first < whole.B; first += per) {
-            TdbKernelParams part = whole;
-            if (first > 0) part.gap_cu = nullptr;
-            part.B = std::min(per, whole.B - first);
-            if (whole.varlen) {
-                part.cu_seqlens = whole.cu_seqlens + first;
-            } else {
-                auto at = [first](const void* base, int64_t stride_b) { return static_cast<const uint16_t*>(base) + first * stride_b; };
-                part.seqlens = whole.seqlens + first;
-                part.q = at(whole.q, whole.qs_b);
-                part.k = at(whole.k, whole.ks_b);
-                part.v = at(whole.v, whole.vs_b);
-                part.o = const_cast<uint16_t*>(at(whole.o, whole.os_b));
-            }
-            const hipError_t e = tdb_launch_resident(part, dtype, stream);
-            if (e != hipSuccess) return e;
-        }
-        return hipSuccess;
-    }
-    const TdbKernelParams& p = whole;
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
-    const Grid g = grid_of(dev, p.H, tdb_mfma_workgroup_limit());
-
+// All sequences of one length, or up to MAX_SEQS of different ones.
+static hipError_t launch_part(const TdbKernelParams& p, bool wide, const Grid& g, int dev, int dtype, hipStream_t stream) {
     ResidentArgs a;
     a.q = static_cast<const char*>(p.q), a.k = static_cast<const char*>(p.k), a.v = static_cast<const char*>(p.v), a.o = static_cast<char*>(p.o);
     a.pk = static_cast<const char*>(p.pk), a.pq = static_cast<const char*>(p.pq);
@@ -492,14 +487,13 @@ hipError_t tdb_launch_resident(const TdbKernelParams& whole, int dtype, hipStrea
     a.exact_far = p.L >= TDB_FAR_MIN_LEN;
     a.c_exp = p.scale * 1.4426950408889634f;
     a.per_group = g.per_group, a.heads = g.heads;
-    const int64_t seqs = int64_t(g.heads) * p.B;
-    const bool equal = a.mode == FIXED, wide = equal ? equal_cost<2>(seqs, p.L, g.per_group) <= equal_cost<1>(seqs, p.L, g.per_group) : ragged_rounds(p, g) > 1.25;
+    const bool equal = a.mode == FIXED;
     const void* fn = dtype == TDB_F16 ? kernel_of<TDB_F16>(c2p, p2c, wide, equal) : kernel_of<TDB_BF16>(c2p, p2c, wide, equal);
     {
         std::lock_guard<std::mutex> lock(g_mutex);
         bool& set = g_attr_set[dev][(wide ? 16 : 0) + (equal ? 8 : 0) + (dtype == TDB_F16 ? 4 : 0) + (c2p ? 2 : 0) + (p2c ? 1 : 0)];
         if (!set) {
-            e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
             if (e != hipSuccess) return e;
             set = true;
         }
@@ -507,4 +501,33 @@ hipError_t tdb_launch_resident(const TdbKernelParams& whole, int dtype, hipStrea
     const size_t lds = (int(c2p) + int(p2c)) * size_t(a.rows) * ROW + 4 * BLOCK;
     void* args[] = {&a};
     return hipLaunchKernel(fn, dim3(unsigned(g.wgs)), dim3(NTHREADS), args, lds, stream);
+}
+
+hipError_t tdb_launch_resident(const TdbKernelParams& whole, int dtype, hipStream_t stream) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
+    const Grid g = grid_of(dev, whole.H, tdb_mfma_workgroup_limit());
+    const bool wide = wide_units(whole, g);
+    const int per = sequences_of(whole);
+    if (per == whole.B) return launch_part(whole, wide, g, dev, dtype, stream);
+    for (int first = 0; first < whole.B; first += per) {        // in even parts
+        TdbKernelParams part = whole;
+        if (first > 0) part.gap_cu = nullptr;
+        part.B = std::min(per, whole.B - first);
+        if (whole.varlen) {
+            part.cu_seqlens = whole.cu_seqlens + first;
+        } else {
+            auto at = [first](const void* base, int64_t stride_b) { return static_cast<const uint16_t*>(base) + first * stride_b; };
+            part.seqlens = whole.seqlens + first;
+            part.q = at(whole.q, whole.qs_b);
+            part.k = at(whole.k, whole.ks_b);
+            part.v = at(whole.v, whole.vs_b);
+            part.o = const_cast<uint16_t*>(at(whole.o, whole.os_b));
+        }
+        e = launch_part(part, wide, g, dev, dtype, stream);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }

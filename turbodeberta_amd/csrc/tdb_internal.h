@@ -59,7 +59,9 @@ hipError_t tdb_zero_gaps(const TdbKernelParams& p, int dtype, hipStream_t stream
 hipError_t tdb_launch_short(const TdbKernelParams& p, int dtype, hipStream_t stream);
 hipError_t tdb_launch_f32(const TdbKernelParams& p, hipStream_t stream);
 hipError_t tdb_launch_mfma(const TdbKernelParams& p, int dtype, hipStream_t stream);
+// what the rules say of a launch on the current device: whether that kernel is the faster one, and whether its units have 32 query rows
 bool tdb_resident_pays(const TdbKernelParams& p);
+bool tdb_resident_wide(const TdbKernelParams& p);
 hipError_t tdb_launch_resident(const TdbKernelParams& p, int dtype, hipStream_t stream);
 // Cap on the persistent workgroups of a launch (multiple of 8, 0 = none); returns the cap in force.
 int tdb_mfma_set_workgroup_limit(int workgroups);
