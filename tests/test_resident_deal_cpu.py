@@ -30,7 +30,7 @@ class Ragged:
         self.full = self.all - self.rest
         self.rounds = self.full // per_group
         longest, shortest = self.lens[0], self.lens[-1]
-        far_apart = longest > 8 * BN and 2 * shortest < longest and 2 * self.rest <= per_group
+        far_apart = longest > 8 * BN and 2 * shortest < longest and 8 * self.rest < 7 * per_group
         self.reckon = longest > 5 * BN and self.rest > 0 and per_group <= 64 and 0 < self.rounds <= (5 if far_apart else 2)
         self.halved = max(self.wholes - self.full, 0)
         if self.rest + self.halved > per_group:

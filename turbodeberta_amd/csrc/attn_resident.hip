@@ -99,12 +99,13 @@ __device__ __forceinline__ void run(const ResidentArgs& p, const int s_at, const
     // The last, incomplete round: whole tiles go by halves if there are workgroups for that, also only the longest of them where the next
     // is clearly shorter, and the costliest to the least loaded workgroup.  Without: 7 packed texts of 1100 89 -> 103 us, 32 padded ones
     // of 64 to 512 53.7 -> 57.  What workgroups have is reckoned after one or two rounds, and after up to five where lengths of more than
-    // 512 are far apart and at most half a round is left (19 packed texts of 450 to 1800 6 % faster; with more left, 8 of 1024 to 4096 2 %
-    // slower).  It takes a microsecond or two, too much for texts up to 320 and elsewhere (39 texts of 384 to 512 2 % slower), and a lane
-    // per workgroup.  Otherwise the order stays, and whoever had the cheaper tile of the round before gets the costlier one.
+    // 512 are far apart and less than seven eighths of a round are left (900 launches of 8 to 24 heads: 1.025x there, 0.96 to 1.17x; with more
+    // left a quarter of them are slower).  It takes a microsecond or two, too much for texts up to 320 and elsewhere (39 texts of 384 to 512
+    // 2 % slower), and a lane per workgroup.  Otherwise the order stays, and whoever had the cheaper tile of the round before gets the
+    // costlier one.
     const int full = all - all % p.per_group, rounds = full / p.per_group, rest = all - full;
     const int longest = EQUAL ? 0 : __builtin_amdgcn_readlane(s_n, 0), shortest = EQUAL ? 0 : __builtin_amdgcn_readlane(s_n, p.B - 1);
-    const bool far_apart = longest > 8 * BN && 2 * shortest < longest && 2 * rest <= p.per_group;
+    const bool far_apart = longest > 8 * BN && 2 * shortest < longest && 8 * rest < 7 * p.per_group;
     const bool reckon = longest > 5 * BN && rest > 0 && p.per_group <= 64 && rounds > 0 && rounds <= (far_apart ? 5 : 2);
     int halved = EQUAL ? 0 : max(wholes - full, 0);
     if (rest + halved > p.per_group) {
