@@ -268,7 +268,8 @@ def test_repeated_launches_are_bit_identical():
     """The kernels have no atomics and no order-dependent reduction: the same launch must give the same bits every
     time.  A difference between repetitions would mean a race between the waves of a workgroup (a missing barrier,
     an LDS slot overwritten early) that the parity tolerances could hide.  Fixed layout with ragged lengths, packed
-    batch, and a sequence long enough for the instances with far key steps, 100 launches each."""
+    batch, equal lengths (several tiles and heads a workgroup), and a sequence long enough for the instances with far key
+    steps, 100 launches each."""
     H, D, buckets, max_rel = 12, 64, 256, 512
     rs = np.random.RandomState(5)
     lengths = [int(x) for x in rs.randint(16, 513, size=24)]
@@ -280,6 +281,8 @@ def test_repeated_launches_are_bit_identical():
     cud = cu.to(DEV)
     long_inp = make_inputs(32, 1, 2, 2304, D, buckets, max_rel, dtype=torch.bfloat16)
     ldev = {k: long_inp[k].to(DEV) for k in ("q", "k", "v", "pk", "pq")}
+    equal_inp = make_inputs(33, 40, H, 400, D, buckets, max_rel, dtype=torch.bfloat16)
+    edev = {k: equal_inp[k].to(DEV) for k in ("q", "k", "v", "pk", "pq")}
     scale = 1 / math.sqrt(3 * D)
     runs = {
         "fixed": lambda: flash_attention_with_disentangled(dev["q"], dev["k"], dev["v"], None, None, False, scale, buckets, max_rel,
@@ -287,6 +290,8 @@ def test_repeated_launches_are_bit_identical():
         "packed": lambda: flash_attention_with_disentangled_varlen(pdev["q"], pdev["k"], pdev["v"], None, None, cud, cud, 512, 512,
                                                                    False, scale, buckets, max_rel, pos_key_layer=dev["pk"],
                                                                    pos_query_layer=dev["pq"]),
+        "equal": lambda: flash_attention_with_disentangled(edev["q"], edev["k"], edev["v"], None, None, False, scale, buckets,
+                                                           max_rel, pos_key_layer=edev["pk"], pos_query_layer=edev["pq"]),
         "long": lambda: flash_attention_with_disentangled(ldev["q"], ldev["k"], ldev["v"], None, None, False, scale, buckets,
                                                           max_rel, pos_key_layer=ldev["pk"], pos_query_layer=ldev["pq"]),
     }
