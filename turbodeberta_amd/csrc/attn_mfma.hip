@@ -1430,8 +1430,9 @@ hipError_t tdb_launch_mfma(const TdbKernelParams& whole, int dtype, hipStream_t 
     const bool strip = p.c2p != nullptr || p.p2c != nullptr;
     const bool c2p = strip ? p.c2p != nullptr : p.pk != nullptr, p2c = strip ? p.p2c != nullptr : p.pq != nullptr;
     // Far key steps only exist in sequences longer than the table's reach; the instance that looks for them carries
-    // both step bodies and its near steps take 1.12x the time, a far step 0.65x.  At length 1024 a quarter of the steps
-    // are far and the plain instance is 7 % faster; at 1536 the far instance wins by 2 %, at 4096 by 13 %.
+    // both step bodies, and its near steps take longer.  It keeps the position terms of far steps in 32 bits, which texts of
+    // this length get in either 16-bit kernel: the limit is one of results.  For speed alone it would lie near 2048 (12 heads,
+    // plain against far: 8 x 1024 82.5 / 94.4 us, 8 x 1536 183 / 187, 8 x 2048 292 / 289, 8 x 4096 1140 / 995).
     const bool farz = !strip && (c2p || p2c) && p.L >= TDB_FAR_MIN_LEN;
     const int64_t round = int64_t(8) << (farz ? XG_LONG : XG_PLAIN);     // the id regrouping is a bijection on multiples of this
     const int nblocks = int((tiles + round - 1) / round * round);

@@ -452,8 +452,10 @@ bool tdb_resident_wide(const TdbKernelParams& p) { return wide_units(p, grid_of(
 // one round of workgroups, and where few rounds leave many workgroups with less than the longest share.  Measured against that kernel as it
 // was when it took every launch, over 5000 random ones of 161 to 4096 keys (6 to 24 heads; both terms, one or none; equal lengths, evenly
 // spread ones and such as texts have): 1.09x by this rule, 1.115x if the fastest of the two kernels and both heights of units were known.
-// Equal lengths 0.984x at worst; packed 2.5 % of the launches below 0.97x, 0.78x at worst; padded, of which the host knows the longest
-// possible length only, 4.9 %, 0.79x (18 texts, most of them short, 12 heads: 15.7 -> 19.9 us).
+// Equal lengths 0.978x at worst; packed 2.5 % of the launches below 0.97x, 0.73x at worst (one of 3619 among 4 texts, 6 heads: 82 -> 113 us);
+// padded, of which the host knows the longest possible length only, 2 % if lengths are evenly spread and 9 % if most are far below it, 0.73x
+// (18 of up to 974, 359 in the mean, 8 heads: 37.5 -> 51).  No limit in L and rounds tells these from padded batches of nearly full texts, which
+// would lose as much (1250 launches: limits of 3400 to 5000, 16-row units up to 2 to 4 rounds, the other kernel below 2.2 to 3.5 of them).
 bool tdb_resident_pays(const TdbKernelParams& p) {
     if (!p.pk && !p.pq) return true;        // (no tables to load: 1.21x over 708 such launches, 1.12x before this line)
     const Grid g = grid_of(-1, p.H, 0);

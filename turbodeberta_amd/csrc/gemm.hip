@@ -13,7 +13,7 @@
 //   * bias and GELU are applied to the float32 sums; results leave through LDS in whole rows.
 //   * with more large tiles than compute units, a workgroup takes one after another, and the first stages of the next are on their
 //     way while the last products of this one are made: a tile of 12 to 16 steps otherwise spends a third of its time on its start
-//     and end (8190 x 3072 x 1024, weights in HBM, 53.4 -> 48.4 us; 8192 x 2304 x 768 40.1 -> 35.0; 8192 x 3072 x 768 with GELU 55.5 -> 50.1).
+//     and end (8190 x 3072 x 1024, weights in HBM, 53.1 -> 47.4 us; 8190 x 2304 x 768 39.3 -> 33.1; 8190 x 3072 x 768 with GELU 53.7 -> 49.5).
 // A layer's four products and GELU (768 wide, library against these): 128 rows 39 / 23 us, 512 47 / 31, 1024 54 / 40, 4352
 // 109 / 88, 8192 169 / 147; 1024 wide, 5000 rows 174 / 153.
 #include <atomic>
@@ -300,8 +300,10 @@ struct Cost {
     int bm, bn;
     float base, round, step, gelu;
 };
-// (192 x 128 is for a thousand columns or so and some 4000 to 7000 rows, where 128 x 256 leaves half the chip without a tile:
-// 4608 x 1024 x 4096 44.5 -> 39.4 us, 4100 x 1024 x 1024 14.3 -> 12.6.)
+// (192 x 128 is for outputs that give the other large tiles a nearly empty last round.  Of 144 products of 1200 to 9000 rows, 512 to 1536 wide,
+// 43 take it, 1.093x as fast as what they took before: 1900 x 2304 x 768 11.7 -> 10.3 us, 5800 x 768 x 3072 32.4 -> 29.6, 4100 x 1024 x 1024
+// 13.6 -> 12.2, 7500 x 2304 x 768 40.4 -> 29.8.  3700 x 3072 x 768 with GELU 28.3 -> 29.8 and 2600 x 1024 x 4096 28.1 -> 29.1 are the two
+// below 0.97x; the other 101 products 1.016x.)
 constexpr Cost COST[] = {{32, 64, 2.96f, 0.62f, 0.148f, 0.07f},  {64, 64, 2.86f, 0.76f, 0.205f, 0.f},   {128, 64, 3.22f, 1.37f, 0.29f, 0.11f},
                          {128, 128, 2.59f, 4.38f, 0.402f, 0.93f}, {128, 256, 2.67f, 7.89f, 0.601f, 2.59f}, {256, 256, 3.55f, 3.7f, 1.195f, 11.09f},
                          {192, 128, 3.3f, 6.f, 0.47f, 1.9f}};
