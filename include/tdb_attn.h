@@ -48,6 +48,8 @@ extern "C" {
  * speed, this one wherever it can take the call */
 #define TDB_FLAG_PERSISTENT 4     /* tiles of 128 query rows, position windows computed by waves of their own */
 #define TDB_FLAG_RESIDENT 8       /* position tables resident in LDS */
+/* the same bits for float32 (whose kernels differ in the order of their sums): 4 each wave reads its own operands, 8 a workgroup's waves
+ * share them through LDS, 12 the same with two sets of waves */
 
 /*
  * Position inputs shared by both entry points.  Two modes, chosen per term:

@@ -1,0 +1,112 @@
+"""The float32 kernel whose products are products of bf16 parts (64 query rows a workgroup, steps of one 16-key tile, one or two sets of
+waves that share out the keys), where its tiles, sets and rings of position rows can go wrong; and the other float32 kernel at the sizes that
+the library no longer gives it."""
+import math
+
+import pytest
+import torch
+
+import test_f32_gpu as f32
+from helpers import in_kernel, make_inputs
+from turbodeberta_amd import _lib
+from turbodeberta_amd.ops.flash_attention import flash_attention_with_disentangled
+from turbodeberta_amd.ops.flash_attention_varlen import flash_attention_with_disentangled_varlen
+
+pytestmark = pytest.mark.gpu
+DIRECT, ONE_SET, TWO_SETS = _lib.TDB_FLAG_PERSISTENT, _lib.TDB_FLAG_RESIDENT, _lib.TDB_FLAG_PERSISTENT | _lib.TDB_FLAG_RESIDENT
+# Products and sums of 32 bits on both sides, in other orders: a few units of 2^-24 of values of order 1 for each of some 64 to 300 terms.
+BOUND = 2e-5
+
+
+def _in_and_generic(flag, call):
+    with in_kernel(flag):
+        got = call(False)
+    return got, call(True)
+
+
+@pytest.mark.parametrize("flag", [ONE_SET, TWO_SETS])
+@pytest.mark.parametrize("terms", [("pk", "pq"), ("pk",), ("pq",), ()])
+@pytest.mark.parametrize("L", [1, 16, 17, 63, 64, 65, 96, 128, 129, 200, 273])      # one tile to 18: odd and even, rings once and three times around
+def test_tiles_and_terms(flag, terms, L):
+    d = {n: t.cuda() for n, t in make_inputs(L, 3, 2, L, 64, 32, 128).items()}
+    lens = torch.tensor([L, max(1, L - 17), max(1, L // 3)], dtype=torch.int32, device="cuda")
+    got, ref = _in_and_generic(flag, lambda g: flash_attention_with_disentangled(
+        d["q"], d["k"], d["v"], None, None, False, f32.SCALE, 32, 128, seqlens_k=lens, force_generic=g, **{
+            "pos_key_layer": d["pk"] if "pk" in terms else None, "pos_query_layer": d["pq"] if "pq" in terms else None}))
+    assert (got - ref).abs().max() < BOUND
+    assert all(not got[b, :, n:].any() for b, n in enumerate(lens.tolist()))
+
+
+@pytest.mark.parametrize("flag", [DIRECT, ONE_SET, TWO_SETS])
+@pytest.mark.parametrize("B", [7, 70])                                               # sorted by length up to 64 sequences
+def test_packed_with_gaps(flag, B):
+    lens = torch.randint(0, 150, (B,), generator=torch.Generator().manual_seed(B))
+    cu = torch.cat([torch.zeros(1, dtype=torch.long), lens.cumsum(0)]).int()
+    T = int(cu[-1]) + 40
+    d = {n: t.cuda() for n, t in make_inputs(6, 1, 4, T, 64, 256, 512).items()}
+    q, k, v = (d[n][0].transpose(0, 1).contiguous() for n in "qkv")
+    cu = (cu + 20).cuda()                                                            # 20 rows before the first and behind the last
+    got, ref = _in_and_generic(flag, lambda g: flash_attention_with_disentangled_varlen(
+        q, k, v, None, None, cu, cu, 150, 150, False, f32.SCALE, 256, 512, pos_key_layer=d["pk"], pos_query_layer=d["pq"], force_generic=g))
+    assert (got - ref).abs().max() < BOUND and not got[:20].any() and not got[T - 20:].any()
+
+
+@pytest.mark.parametrize("flag", [DIRECT, ONE_SET, TWO_SETS])
+@pytest.mark.parametrize("where", ["query", "key", "value", "last_value", "c2p_row", "p2c_row", "score", "low_scores", "padding"])
+def test_nan_and_infinity(flag, where):
+    with in_kernel(flag):
+        f32.test_nan_and_infinity_reach_what_they_belong_to(where, 2, 2, 130)
+
+
+@pytest.mark.parametrize("flag", [ONE_SET, TWO_SETS])
+@pytest.mark.parametrize("scale", [0.0, -0.3, 40.0])
+def test_any_scale(flag, scale):
+    """A score is scaled before its maximum is taken, and rounded as the maximum is: no scale makes a probability larger than 1."""
+    d = {n: t.cuda() for n, t in make_inputs(1, 2, 2, 100, 64, 256, 512).items()}
+    got, ref = _in_and_generic(flag, lambda g: flash_attention_with_disentangled(
+        d["q"], d["k"], d["v"], None, None, False, scale, 256, 512, pos_key_layer=d["pk"], pos_query_layer=d["pq"], force_generic=g))
+    # scores of some 25 |scale|, each off by a few units of 2^-24 of itself in either kernel
+    assert (got - ref).abs().max() < BOUND * (1 + 25 * abs(scale))
+
+
+@pytest.mark.parametrize("flag", [ONE_SET, TWO_SETS])
+@pytest.mark.parametrize("size", [1e-25, 1e30])
+def test_size_of_values(flag, size):
+    """Parts keep the exponent: small and large values are as exact as others."""
+    d = {n: t.cuda() for n, t in make_inputs(2, 1, 2, 90, 64, 256, 512).items()}
+    d["v"] *= size
+    got, ref = _in_and_generic(flag, lambda g: flash_attention_with_disentangled(
+        d["q"], d["k"], d["v"], None, None, False, f32.SCALE, 256, 512, pos_key_layer=d["pk"], pos_query_layer=d["pq"], force_generic=g))
+    assert (got - ref).abs().max() < BOUND * size
+
+
+@pytest.mark.parametrize("flag", [ONE_SET, TWO_SETS])
+def test_strided_rows_and_shared_tables(flag):
+    """Rows of a wider array, and a table of equal rows (stride 0) as an expanded tensor has it."""
+    d = {n: t.cuda() for n, t in make_inputs(3, 2, 3, 80, 64, 256, 512).items()}
+    wide = torch.zeros(2, 80, 3, 5, 64, device="cuda")
+    for i, n in enumerate("qkv"):
+        wide[:, :, :, i] = d[n].permute(0, 2, 1, 3)
+    q, k, v = (wide[:, :, :, i].permute(0, 2, 1, 3) for i in range(3))
+    pk = d["pk"][:, :1].expand(-1, 512, -1)
+    got, ref = _in_and_generic(flag, lambda g: flash_attention_with_disentangled(
+        q, k, v, None, None, False, f32.SCALE, 256, 512, pos_key_layer=pk, pos_query_layer=d["pq"], force_generic=g))
+    assert (got - ref).abs().max() < BOUND
+
+
+def test_error_against_64_bits_is_no_larger():
+    """Small products first: sums of parts are more exact than float32 products one after another."""
+    d = {n: t.cuda() for n, t in make_inputs(4, 2, 4, 300, 64, 256, 512).items()}
+    x = {n: t.double() for n, t in d.items()}
+    delta = torch.from_numpy(_lib.delta_table(300, 256, 512).astype("int64")).cuda()
+    at = delta[(torch.arange(300)[:, None] - torch.arange(300)[None] + 299).cuda()].expand(2, 4, 300, 300)
+    s = x["q"] @ x["k"].transpose(-1, -2).contiguous() + (x["q"] @ x["pk"].transpose(-1, -2).contiguous()[None]).gather(3, at)
+    s = s + (x["k"] @ x["pq"].transpose(-1, -2).contiguous()[None]).gather(3, at.transpose(-1, -2)).transpose(-1, -2)
+    exact = torch.softmax(s * f32.SCALE, -1) @ x["v"]
+    err = {}
+    for flag in (DIRECT, ONE_SET, TWO_SETS):
+        with in_kernel(flag):
+            out = flash_attention_with_disentangled(d["q"], d["k"], d["v"], None, None, False, f32.SCALE, 256, 512, pos_key_layer=d["pk"], pos_query_layer=d["pq"])
+        err[flag] = float((out.double() - exact).norm() / exact.norm())
+    assert err[ONE_SET] <= err[DIRECT] and err[TWO_SETS] <= err[DIRECT] and err[DIRECT] < 1e-6, err
+    assert math.isfinite(err[ONE_SET])

@@ -65,3 +65,15 @@ def test_which_kernel(kind, lens, heads, terms, resident):
 ])
 def test_which_units(kind, lens, heads, wide):
     assert _rule("wide")(_launch(kind, lens, heads)) == wide
+
+
+@pytest.mark.parametrize("kind,lens,heads,terms,sets", [
+    ("padded", _even(8, 96, 384), 12, 2, 1), ("equal", [128] * 32, 12, 2, 1), ("packed", _even(12, 209, 209), 12, 2, 1),
+    ("equal", [512] * 2, 12, 2, 2), ("equal", [256] * 4, 12, 2, 2), ("equal", [190] * 3, 16, 2, 2), ("padded", _even(3, 151, 460), 12, 2, 2),
+    ("equal", [128] * 2, 12, 2, 0), ("equal", [512], 12, 2, 0), ("equal", [21] * 44, 12, 2, 0), ("packed", _even(58, 17, 30), 16, 2, 0),
+    ("packed", [134] * 7, 12, 1, 0), ("equal", [59] * 8, 16, 1, 0),
+])
+def test_which_float32_kernel(kind, lens, heads, terms, sets):
+    fn = _lib.load()._Z18tdb_f32_split_setsRK15TdbKernelParams
+    fn.argtypes, fn.restype = [C.c_void_p], C.c_int
+    assert fn(_launch(kind, lens, heads, terms)) == sets

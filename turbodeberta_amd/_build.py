@@ -13,7 +13,7 @@ ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 LIB_PATH = os.path.join(PKG, "libtdb_attn.so")
 HOST_PATH = os.path.join(PKG, "_host.so")
-SOURCES = ("capi.hip", "attn_generic.hip", "attn_f32.hip", "attn_short.hip", "encoder.hip", "gemm.hip", "attn_mfma.hip", "attn_resident.hip")
+SOURCES = ("capi.hip", "attn_generic.hip", "attn_f32.hip", "attn_f32_split.hip", "attn_short.hip", "encoder.hip", "gemm.hip", "attn_mfma.hip", "attn_resident.hip")
 
 # packed-fp32 VALU forms are switched off for every device compile
 HIPCC_FLAGS = [

@@ -1,8 +1,8 @@
 // Matrix-core disentangled-attention forward for float32, head_dim 64 (gfx950, wave64, MFMA 16x16x4 f32).
 //
-// float32 is the type checkpoints load in, and its 1e-4 bar leaves no room for split or reduced operands: products and
-// sums are float32 FMAs, on the matrix cores (152 TFLOP/s measured for a large product; the packed vector forms that
-// would reach that rate are not used here).
+// float32 is the type checkpoints load in.  Products and sums are float32 FMAs, on the matrix cores (152 TFLOP/s measured for a large
+// product; the packed vector forms that would reach that rate are not used here).  Larger launches with tables are attn_f32_split.hip's: here
+// a wave reads its own operands, and taking them apart for bf16 products would cost it what those products save.
 //
 // What bounds it: the matrix pipe.  A 16 x 16 x 64 tile product takes 16 MFMAs = 512 clk, sixteen times a bf16 one, so
 // everything else is chosen to be simple rather than cheap: operands go straight from global memory to registers (a

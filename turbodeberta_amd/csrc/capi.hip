@@ -97,6 +97,8 @@ int dispatch(const TdbKernelParams& kp, int dtype, int flags, void* stream) {
         e = tdb_launch_resident(kp, dtype, s);
     } else if (any && tdb_mfma_supported(kp, dtype)) {
         e = tdb_launch_mfma(kp, dtype, s);
+    } else if (const int sets = resident ? 1 + persistent : persistent ? 0 : tdb_f32_split_sets(kp); any && sets > 0 && tdb_f32_split_supported(kp, dtype)) {
+        e = tdb_launch_f32_split(kp, sets, s);
     } else if (any && tdb_f32_supported(kp, dtype)) {
         e = tdb_launch_f32(kp, s);
     } else {

@@ -44,6 +44,10 @@ constexpr int TDB_SHORT_TILE = 32;     // per wave
 
 // true when the float32 matrix-core kernel can take this launch
 bool tdb_f32_supported(const TdbKernelParams& p, int dtype);
+// true when the float32 kernel that takes its operands apart once per workgroup can, and with how many sets of waves it is the
+// faster one on the current device (0: it is not)
+bool tdb_f32_split_supported(const TdbKernelParams& p, int dtype);
+int tdb_f32_split_sets(const TdbKernelParams& p);
 // true when the 16-bit matrix-core kernel can take this launch
 bool tdb_mfma_supported(const TdbKernelParams& p, int dtype);
 
@@ -58,6 +62,7 @@ hipError_t tdb_launch_generic(const TdbKernelParams& p, int dtype, hipStream_t s
 hipError_t tdb_zero_gaps(const TdbKernelParams& p, int dtype, hipStream_t stream);     // a launch of its own
 hipError_t tdb_launch_short(const TdbKernelParams& p, int dtype, hipStream_t stream);
 hipError_t tdb_launch_f32(const TdbKernelParams& p, hipStream_t stream);
+hipError_t tdb_launch_f32_split(const TdbKernelParams& p, int sets, hipStream_t stream);
 hipError_t tdb_launch_mfma(const TdbKernelParams& p, int dtype, hipStream_t stream);
 // what the rules say of a launch on the current device: whether that kernel is the faster one, and whether its units have 32 query rows
 bool tdb_resident_pays(const TdbKernelParams& p);
