@@ -186,6 +186,24 @@ __global__ __launch_bounds__(256) void add_norm_kernel(const void* x, int splits
     norm_row<DT, CH>(v, w, b, chunks, hidden, eps, out, t, mt_out);
 }
 
+// Fragments of 16 rows x 32 columns whose rows lie apart (weights): a load in operand order, consecutive lanes in different rows, occupies the
+// CU's load path for 54 clk; here four lanes share a row (16 clk), and the wave's own LDS brings the chunks to their lanes.  (Replayed as a graph, operand order ->
+// this: 12 layers of 768, 48 rows 357 -> 351 us, 24 of 1024 862 -> 848, 8 of 1536 451 -> 433.)
+__device__ __forceinline__ int row_chunk(int l) { return (l & 3) ^ ((l >> 4) & 3); }       // lane l loads this chunk of eight of row l >> 2
+// N fragments at once (slots: 64 N of the wave's own), so that one waits for LDS under the next.
+template <int N, typename X8>
+__device__ __forceinline__ void to_operands(X8* slots, X8 (&x)[N]) {
+    const int l = threadIdx.x & 63, c = l & 15, g = l >> 4;
+#pragma unroll
+    for (int i = 0; i < N; ++i) slots[64 * i + l] = x[i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");          // (a wave's LDS accesses are in order: only the compiler is held back)
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = slots[64 * i + 4 * c + (g ^ ((c >> 2) & 3))];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // One workgroup: 16 columns of the output, a share of the contraction given by blockIdx.y and, inside it, by the wave.
 // MT: token tiles of 16.  Lane (c, g) has 16 bytes of weight row n0 + c and of token row 16 m + c: columns 32 k + 8 g .. +7.
 // IN / OUT: x / y in the order of row_at.
@@ -195,14 +213,15 @@ __global__ __launch_bounds__(512) void small_gemm_kernel(const void* xv, const v
     using X8 = typename E::X8;
     using T = typename E::T;
     extern __shared__ __attribute__((aligned(16))) float red[];
+    __shared__ X8 s_w[8 * 4 * 64];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6, l = threadIdx.x & 63;
     const int c = l & 15, g = l >> 4, n0 = blockIdx.x * 16, steps = K / 32;
     const int parts = splits * waves, part = blockIdx.y * waves + wave;
     const int k0 = steps * part / parts, k1 = steps * (part + 1) / parts;
-    const T* const w = static_cast<const T*>(wv) + int64_t(n0 + c) * K + 8 * g;
+    const T* const w = static_cast<const T*>(wv) + int64_t(n0 + (l >> 2)) * K + 8 * row_chunk(l);
     const T* x[MT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) x[m] = static_cast<const T*>(xv) + (IN ? m * 512 + l * 8 : min(16 * m + c, M - 1) * K + 8 * g);
+    for (int m = 0; m < MT; ++m) x[m] = static_cast<const T*>(xv) + (IN ? m * 512 + l * 8 : min(16 * m + (l >> 2), M - 1) * K + 8 * row_chunk(l));
     typedef __attribute__((ext_vector_type(4))) T T4;
     const int col = n0 + 4 * g;             // (of every element this thread sums up below)
     T4 b4;
@@ -220,6 +239,11 @@ __global__ __launch_bounds__(512) void small_gemm_kernel(const void* xv, const v
             for (int m = 0; m < MT; ++m) b[u][m] = *reinterpret_cast<const X8*>(x[m] + (k + u) * (IN ? MT * 512 : 32));
         }
         __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if constexpr (!IN) to_operands(s_w + wave * 256, b[u]);
+        }
+        to_operands(s_w + wave * 256, a);
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
