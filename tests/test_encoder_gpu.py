@@ -73,6 +73,14 @@ def test_widths(hidden, heads, inner, lens, L):
     _check(*_both(_model(torch.bfloat16, hidden, heads, 1, inner), ids, mask), mask, torch.bfloat16)
 
 
+@pytest.mark.parametrize("hidden,heads,inner,L", [(704, 11, 3104, 50), (768, 12, 4096, 64), (768, 12, 3072, 17), (128, 2, 4128, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_few_rows_with_the_normalisation_in_the_products(hidden, heads, inner, L, dtype):
+    """Workgroups of one to four column blocks, the last of them short; contractions that the waves share unevenly."""
+    ids, mask = _ids([L], L)
+    _check(*_both(_model(dtype, hidden, heads, 2, inner), ids, mask), mask, dtype)
+
+
 @pytest.fixture(scope="module")
 def base_width():
     """Three base-sized layers: Hugging Face's model with weights as a 16-bit model holds them, in float32 and in the type."""

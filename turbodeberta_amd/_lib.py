@@ -123,7 +123,8 @@ def host():
             raise RuntimeError(f"{PKG}/_host.so is missing or does not load ({e}): build it with "
                                "`python -m turbodeberta_amd._build`") from e
         address = lambda n: C.cast(getattr(lib, n), C.c_void_p).value
-        module.bind_encoder(*(address("tdb_enc_" + n) for n in ("scan_mask", "embed", "add_norm", "small_gemm", "small_tiles", "small_splits", "unpack", "gemm", "gemm_splits")))
+        module.bind_encoder(*(address("tdb_enc_" + n) for n in ("scan_mask", "embed", "add_norm", "small_gemm", "small_tiles", "small_splits", "unpack", "gemm", "gemm_splits",
+                                                                                "rows_fused", "embed_rows", "norm_gemm", "gemm_add", "norm_rows")))
         module.bind(address("tdb_attn_fwd_fixed"), address("tdb_attn_fwd_varlen"))
         _host = module
     return _host

@@ -115,10 +115,14 @@ __device__ __forceinline__ void norm_row(float (&v)[CH][8], const float (&w)[CH]
         }
 }
 
-template <int DT, int CH>
+// Row t, columns 4 c4 .. + 3 of rows in float32 (see norm_gemm_kernel), in the order in which the products load them: 1 KB in one piece for a load instruction.
+__device__ __forceinline__ int64_t x_at(int t, int c4, int mt) { return int64_t((((c4 >> 3) * mt + (t >> 4)) * 2 + (c4 & 1)) * 64 + ((c4 >> 1) & 3) * 16 + (t & 15)) * 4; }
+
+// ROWS: the row before its LayerNorm (`out`, `stats`) for the products that normalise what they load.
+template <int DT, int CH, bool ROWS>
 __global__ __launch_bounds__(256) void embed_kernel(const void* ids, int ids64, const void* table, int64_t vocab, const void* gamma,
                                                     const void* beta, float eps, const int32_t* cu, int B, int L, int T, int hidden,
-                                                    int mt, void* out) {
+                                                    int mt, void* out, float2* stats) {
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63, chunks = hidden / 8;
     if (t >= T) return;
     int64_t at = t;
@@ -134,7 +138,7 @@ __global__ __launch_bounds__(256) void embed_kernel(const void* ids, int ids64, 
     const int64_t id = ids64 ? static_cast<const int64_t*>(ids)[at] : static_cast<const int32_t*>(ids)[at];
     const bool ok = id >= 0 && id < vocab;
     float v[CH][8], w[CH][8], b[CH][8];
-    load_affine<DT, CH>(w, b, chunks, gamma, beta);
+    if constexpr (!ROWS) load_affine<DT, CH>(w, b, chunks, gamma, beta);
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
 #pragma unroll
@@ -144,7 +148,27 @@ __global__ __launch_bounds__(256) void embed_kernel(const void* ids, int ids64, 
             else v[c][0] = __builtin_nanf("");          // an id outside the table: the row says so
         }
     }
-    norm_row<DT, CH>(v, w, b, chunks, hidden, eps, out, t, mt);
+    if constexpr (ROWS) {
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            float sum = 0.f, dev = 0.f;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sum += v[c][i];
+            const float mid = (sum + __shfl_xor(sum, 1)) * (1.f / 16.f);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) dev += (v[c][i] - mid) * (v[c][i] - mid);
+            dev += __shfl_xor(dev, 1);
+            const int chunk = l + 64 * c;
+            if (chunk < chunks) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    *reinterpret_cast<f32x4*>(static_cast<float*>(out) + x_at(t, 2 * chunk + h, mt)) = f32x4{v[c][4 * h], v[c][4 * h + 1], v[c][4 * h + 2], v[c][4 * h + 3]};
+                if (!(l & 1)) stats[(chunk >> 1) * 16 * mt + t] = float2{mid, dev};
+            }
+        }
+    } else {
+        norm_row<DT, CH>(v, w, b, chunks, hidden, eps, out, t, mt);
+    }
 }
 
 template <int DT, int CH, int PARTS>      // PARTS: 0, or the most partial sums
@@ -276,6 +300,278 @@ __global__ __launch_bounds__(512) void small_gemm_kernel(const void* xv, const v
     }
 }
 
+// The two kinds of products of a short request, where a launch costs as much as what it does: the residual + LayerNorm between them
+// is no launch of its own.  A product with a hidden-sized output adds the residual in its epilogue and writes the row before its LayerNorm in
+// float32, with the mean and the sum of squared deviations of each 16 columns (`x`, `stats`); whoever reads the row joins these and normalises
+// what it loads.  A workgroup takes 16 rows and 16 columns of the output, its waves share out the contraction.
+// What bounds them: a launch (1.6 us even in a graph), one round trip for what the kernel before wrote, and what a CU reads, at some 30 bytes a clk: hence
+// workgroups of few rows and as many columns as leave one workgroup to a CU.  12 layers of 768 as a graph, 7 launches a layer -> 5: 48 rows
+// 351 -> 338 us, 64 rows 366 -> 346; as launches 13 % where the host is slow.  See FUSED_WIDTH.
+
+// Sums of a row's blocks of 16 columns around the mean of the first one.
+struct Moments {
+    float shift, d, dd, q;                  // sums of (mean - shift), its square, and squared deviations
+    __device__ __forceinline__ void join(float& mean, float& rstd, int hidden, float eps) const {
+        const float blocks = float(hidden / 16);
+        mean = shift + d / blocks;
+        rstd = rsqrtf((q + 16.f * (dd - d * d / blocks)) / float(hidden) + eps);
+    }
+};
+// This thread's share of row 16 m + (thread & 15), whose blocks the groups of 16 threads share out: requested, then summed up over the wave.
+template <int GROUPS>
+struct MomentLoads {
+    static constexpr int AT_ONCE = 64 / GROUPS < 2 ? 2 : 64 / GROUPS;   // (all of a row of 1024)
+    const float2* at;
+    float2 first, v[AT_ONCE];
+    int blocks, rows;
+    __device__ __forceinline__ void request(const float2* stats, int hidden, int mt, int m) {
+        blocks = hidden / 16, rows = 16 * mt, at = stats + 16 * m + (threadIdx.x & 15);
+        first = at[0];
+        more(0);
+    }
+    __device__ __forceinline__ void more(int from) {
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i) v[i] = at[min(from + i * GROUPS + int(threadIdx.x >> 4), blocks - 1) * rows];
+    }
+    __device__ __forceinline__ Moments sums() {
+        Moments s = {first.x, 0.f, 0.f, 0.f};
+        for (int from = 0;;) {
+#pragma unroll
+            for (int i = 0; i < AT_ONCE; ++i)
+                if (from + i * GROUPS + int(threadIdx.x >> 4) < blocks) {
+                    const float d = v[i].x - s.shift;
+                    s.d += d, s.dd += d * d, s.q += v[i].y;
+                }
+            from += AT_ONCE * GROUPS;
+            if (from >= blocks) break;
+            more(from);
+        }
+#pragma unroll
+        for (int o = 16; o < 64; o <<= 1) s.d += __shfl_xor(s.d, o), s.dd += __shfl_xor(s.dd, o), s.q += __shfl_xor(s.q, o);
+        return s;
+    }
+};
+// (LDS: [wave][row] of three sums)
+__device__ __forceinline__ void put_moments(float4* lds, const Moments& s) {
+    if ((threadIdx.x & 63) < 16) lds[(threadIdx.x >> 6) * 16 + (threadIdx.x & 15)] = float4{s.d, s.dd, s.q, 0.f};
+}
+__device__ __forceinline__ void get_moments(const float4* lds, int waves, Moments s, int hidden, float eps, float& mean, float& rstd) {
+    s.d = s.dd = s.q = 0.f;
+    for (int w = 0; w < waves; ++w) {
+        const float4 v = lds[w * 16 + (threadIdx.x & 15)];
+        s.d += v.x, s.dd += v.y, s.q += v.z;
+    }
+    s.join(mean, rstd, hidden, eps);
+}
+
+// f(how many of the steps that are left come next, at most MOST)
+template <int MOST, typename F>
+__device__ __forceinline__ void with_steps(int left, F f) {
+    if (left >= MOST) f(std::integral_constant<int, MOST>{});
+    else if constexpr (MOST > 1) with_steps<MOST - 1>(left, f);
+}
+
+// Weights of the products to come, brought into the L2 of the XCD that will read them by workgroups of their own (blockIdx.y >= mt) beside the present
+// product: chunk i, the rows of one workgroup of that product, by blocks whose number is i modulo 8, which go to the same XCD.  (12 layers of 768, 48 rows, weights in HBM: 414 -> 380 us; weights in the last-level cache 348 -> 343.
+// The attention's table rows as well: no change.)
+struct Ahead {
+    static constexpr int MOST = 2;
+    const char* w[MOST];
+    int lines[MOST], chunks[MOST];          // 128-byte lines of a chunk
+    __device__ __forceinline__ void fetch(int mt) const {
+        const int id = blockIdx.y * gridDim.x + blockIdx.x, xcd = id & 7;
+        const int thread = ((id - mt * gridDim.x) >> 3) * blockDim.x + threadIdx.x, threads = max((int(gridDim.y - mt) * int(gridDim.x)) >> 3, 1) * blockDim.x;
+        uint32_t any = 0;
+#pragma unroll
+        for (int i = 0; i < MOST; ++i) {
+            const int mine = (chunks[i] - xcd + 7) >> 3;        // chunks of this XCD
+            for (int at = thread; at < mine * lines[i]; at += threads) {
+                const int chunk = at / lines[i];
+                any |= *reinterpret_cast<const uint32_t*>(w[i] + (int64_t(8 * chunk + xcd) * lines[i] + (at - chunk * lines[i])) * 128);
+            }
+        }
+        asm volatile("" ::"v"(any));        // (loaded, though nobody wants to know)
+    }
+};
+
+struct NormRows {                           // rows before their LayerNorm, and what it needs
+    const float* x;
+    const float2* stats;
+    const void *gamma, *beta;
+    float eps;
+};
+
+// y = LayerNorm(rows) w^T + bias; GELU: of that, and y in the order of row_at.  K: the rows' width; NB: blocks of 16 columns a workgroup.
+template <int DT, int NB, bool GELU>
+__global__ __launch_bounds__(512) void norm_gemm_kernel(NormRows in, const void* wv, const void* bias, void* y, int M, int N, int K, int mt, Ahead next) {
+    if (int(blockIdx.y) >= mt) return next.fetch(mt);
+    using E = Elem<DT>;
+    using X8 = typename E::X8;
+    using T = typename E::T;
+    typedef __attribute__((ext_vector_type(4))) T T4;
+    constexpr int WAVES = 8, U = 4;         // steps at a time
+    __shared__ float4 s_moments[WAVES * 16];
+    __shared__ f32x4 s_sum[WAVES * NB * 64];
+    __shared__ X8 s_w[WAVES * NB * 64];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+    const int c = l & 15, g = l >> 4, n0 = blockIdx.x * 16 * NB, m = blockIdx.y, steps = K / 32;
+    const int k0 = steps * wave / WAVES, k1 = steps * (wave + 1) / WAVES;
+    const T* w[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) w[j] = static_cast<const T*>(wv) + int64_t(min(n0 + 16 * j, N - 16) + (l >> 2)) * K + 8 * row_chunk(l);
+    const float* const x = in.x + (m * 2 * 64 + l) * 4;
+    X8 a[U][NB], gamma[U], beta[U];
+    f32x4 lo[U], hi[U];
+    auto load = [&](int k, auto count) {
+#pragma unroll
+        for (int u = 0; u < decltype(count)::value; ++u) {
+#pragma unroll
+            for (int j = 0; j < NB; ++j) a[u][j] = *reinterpret_cast<const X8*>(w[j] + 32 * (k + u));
+            lo[u] = *reinterpret_cast<const f32x4*>(x + int64_t(k + u) * mt * 512);
+            hi[u] = *reinterpret_cast<const f32x4*>(x + int64_t(k + u) * mt * 512 + 256);
+            gamma[u] = *reinterpret_cast<const X8*>(static_cast<const T*>(in.gamma) + 32 * (k + u) + 8 * g);
+            beta[u] = *reinterpret_cast<const X8*>(static_cast<const T*>(in.beta) + 32 * (k + u) + 8 * g);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    float mean, rstd;
+    f32x4 acc[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto use = [&](auto count) {
+#pragma unroll
+        for (int u = 0; u < decltype(count)::value; ++u) {
+            to_operands(s_w + wave * NB * 64, a[u]);
+            X8 b;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) b[i] = T(((i < 4 ? lo[u][i & 3] : hi[u][i & 3]) - mean) * rstd * float(gamma[u][i]) + float(beta[u][i]));
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[j] = E::mfma(a[u][j], b, acc[j]);
+        }
+    };
+    MomentLoads<WAVES * 4> moments;
+    moments.request(in.stats, K, mt, m);
+    with_steps<U>(k1 - k0, [&](auto count) { load(k0, count); });
+    const Moments part = moments.sums();
+    put_moments(s_moments, part);
+    __syncthreads();
+    get_moments(s_moments, WAVES, part, K, in.eps, mean, rstd);
+    with_steps<U>(k1 - k0, use);
+    for (int k = k0 + U; k < k1; k += U)
+        with_steps<U>(k1 - k, [&](auto count) {
+            load(k, count);
+            use(count);
+        });
+#pragma unroll
+    for (int j = 0; j < NB; ++j) s_sum[(wave * NB + j) * 64 + l] = acc[j];
+    __syncthreads();
+    const int row = 16 * m + c, col = n0 + 16 * wave + 4 * g;          // (a wave for each block)
+    if (wave >= NB || col >= N || row >= M) return;
+    const T4 b4 = *reinterpret_cast<const T4*>(static_cast<const T*>(bias) + col);
+    f32x4 sum = s_sum[wave * 64 + l];
+#pragma unroll
+    for (int v = 1; v < WAVES; ++v) sum += s_sum[(v * NB + wave) * 64 + l];
+    T4 out;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float v = sum[i] + float(b4[i]);
+        if (GELU) v = tdb_gelu(v);
+        out[i] = T(v);
+    }
+    *reinterpret_cast<T4*>(static_cast<T*>(y) + row_at(row, col >> 3, N, GELU ? mt : 0) + (col & 7)) = out;
+}
+
+// rows (x, stats) = in w^T + bias + LayerNorm(residual), the latter rounded to the type as a product reads it.  IN: in the order of row_at.
+template <int DT, int WAVES, bool IN>
+__global__ __launch_bounds__(WAVES * 64) void gemm_add_kernel(const void* inv, const void* wv, const void* bias, NormRows residual, float* x, float2* stats, int M,
+                                                              int N, int K, int mt, Ahead next) {
+    if (int(blockIdx.y) >= mt) return next.fetch(mt);
+    using E = Elem<DT>;
+    using X8 = typename E::X8;
+    using T = typename E::T;
+    typedef __attribute__((ext_vector_type(4))) T T4;
+    __shared__ float4 s_moments[WAVES * 16];
+    __shared__ f32x4 s_sum[WAVES * 64];
+    __shared__ X8 s_w[WAVES * 8 * 64];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
+    const int c = l & 15, g = l >> 4, n0 = blockIdx.x * 16, m = blockIdx.y, steps = K / 32;
+    const int k0 = steps * wave / WAVES, k1 = steps * (wave + 1) / WAVES;
+    const T* const w = static_cast<const T*>(wv) + int64_t(n0 + (l >> 2)) * K + 8 * row_chunk(l);
+    const T* const in = static_cast<const T*>(inv) + (IN ? (m * 64 + l) * 8 : int64_t(min(16 * m + (l >> 2), M - 1)) * K + 8 * row_chunk(l));
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    auto run = [&](int k, auto count) {     // `count` steps from k: all requested before the first is used
+        constexpr int U = decltype(count)::value;
+        X8 a[U], b[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            a[u] = *reinterpret_cast<const X8*>(w + 32 * (k + u));
+            b[u] = *reinterpret_cast<const X8*>(in + int64_t(k + u) * (IN ? mt * 512 : 32));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        to_operands(s_w + wave * 512, a);
+        if constexpr (!IN) to_operands(s_w + wave * 512, b);
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc = E::mfma(a[u], b[u], acc);
+    };
+    const int row = 16 * m + c, col = n0 + 4 * g;
+    MomentLoads<WAVES * 4> moments;
+    moments.request(residual.stats, N, mt, m);
+    f32x4 old;
+    T4 b4, g4, s4;
+    if (wave == 0) {                        // (what the epilogue needs: not another round trip behind the sums)
+        old = *reinterpret_cast<const f32x4*>(residual.x + x_at(row, col >> 2, mt));
+        b4 = *reinterpret_cast<const T4*>(static_cast<const T*>(bias) + col);
+        g4 = *reinterpret_cast<const T4*>(static_cast<const T*>(residual.gamma) + col);
+        s4 = *reinterpret_cast<const T4*>(static_cast<const T*>(residual.beta) + col);
+    }
+    for (int k = k0; k < k1; k += 8) with_steps<8>(k1 - k, [&](auto count) { run(k, count); });
+    const Moments part = moments.sums();
+    put_moments(s_moments, part);
+    s_sum[wave * 64 + l] = acc;
+    __syncthreads();
+    if (wave > 0) return;
+    float mean, rstd;
+    get_moments(s_moments, WAVES, part, N, residual.eps, mean, rstd);
+    f32x4 sum = acc;
+#pragma unroll
+    for (int v = 1; v < WAVES; ++v) sum += s_sum[v * 64 + l];
+    float s1 = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        sum[i] += float(b4[i]);
+        sum[i] += float(T((old[i] - mean) * rstd * float(g4[i]) + float(s4[i])));
+        s1 += sum[i];
+    }
+    s1 += __shfl_xor(s1, 16);
+    s1 += __shfl_xor(s1, 32);
+    const float mid = s1 * (1.f / 16.f);
+    float dev = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dev += (sum[i] - mid) * (sum[i] - mid);
+    dev += __shfl_xor(dev, 16);
+    dev += __shfl_xor(dev, 32);
+    *reinterpret_cast<f32x4*>(x + x_at(row, col >> 2, mt)) = sum;       // (rows past M: there is room, and nothing looks at them)
+    if (g == 0) stats[blockIdx.x * 16 * mt + row] = float2{mid, dev};
+}
+
+// out = LayerNorm(rows), row after row.
+template <int DT, int CH>
+__global__ __launch_bounds__(64) void norm_rows_kernel(NormRows in, int hidden, int mt, void* out) {
+    const int t = blockIdx.x, l = threadIdx.x, chunks = hidden / 8;
+    float v[CH][8], w[CH][8], b[CH][8];
+    load_affine<DT, CH>(w, b, chunks, in.gamma, in.beta);
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            f32x4 x = {0.f, 0.f, 0.f, 0.f};
+            if (l + 64 * c < chunks) x = *reinterpret_cast<const f32x4*>(in.x + x_at(t, 2 * (l + 64 * c) + h, mt));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[c][4 * h + i] = x[i];
+        }
+    norm_row<DT, CH>(v, w, b, chunks, hidden, in.eps, out, t, 0);
+}
+
 struct ScanIds {
     const void* ids;                        // of the row, or nullptr
     int ids64;
@@ -389,6 +685,29 @@ void with_type(int dtype, F f) {
 // Up to here a layer's four products take less here than in the tiles of gemm.hip (768 wide: 16.5 against 18.5 us at 64 rows,
 // 20.2 against 19.1 at 80).
 constexpr int SMALL_ROWS = 64;
+// Each of the column blocks reads and normalises its rows anew, 64 bytes of float32 for each column of them: 24 layers of 1024 take 927 us that way and 848 with
+// launches for residual + LayerNorm.
+constexpr int FUSED_WIDTH = 768;
+
+// Blocks of 16 columns that a workgroup of norm_gemm_kernel takes: as few as give each compute unit one workgroup.
+int norm_blocks(int N, int mt) {
+    const int blocks = N / 16, units = tdb_compute_units(-1);
+    int n = 1;
+    while (n < 4 && (blocks + n - 1) / n * mt > units) ++n;
+    return n;
+}
+Ahead ahead_of(const tdb_enc_next* next, int nexts, int mt) {
+    Ahead a{};
+    int n = 0;
+    for (int i = 0; i < nexts; ++i) {
+        const int rows = 16 * (next[i].norm ? norm_blocks(next[i].N, mt) : 1);
+        const int64_t bytes = int64_t(rows) * next[i].K * 2;
+        if (!next[i].w || bytes % 128 || next[i].N % rows) continue;
+        a.w[n] = static_cast<const char*>(next[i].w), a.lines[n] = int(bytes / 128), a.chunks[n] = next[i].N / rows;
+        ++n;
+    }
+    return a;
+}
 
 bool hidden_ok(int hidden) { return hidden > 0 && hidden % 8 == 0 && hidden <= 4096; }
 
@@ -409,8 +728,8 @@ int tdb_enc_embed(const void* ids, int ids64, const void* table, int64_t vocab, 
     if (!hidden_ok(hidden) || T < 1) return int(hipErrorInvalidValue);
     with_type(dtype, [&](auto dt) {
         with_chunks(hidden, [&](auto ch) {
-            hipLaunchKernelGGL((embed_kernel<decltype(dt)::value, decltype(ch)::value>), dim3((T + 3) / 4), dim3(256), 0, static_cast<hipStream_t>(stream),
-                               ids, ids64, table, vocab, gamma, beta, eps, cu, B, L, T, hidden, mt, out);
+            hipLaunchKernelGGL((embed_kernel<decltype(dt)::value, decltype(ch)::value, false>), dim3((T + 3) / 4), dim3(256), 0, static_cast<hipStream_t>(stream),
+                               ids, ids64, table, vocab, gamma, beta, eps, cu, B, L, T, hidden, mt, out, nullptr);
         });
     });
     return int(hipGetLastError());
@@ -477,6 +796,83 @@ int tdb_enc_small_gemm(const void* x, const void* w, const void* bias, int flags
     if (dtype == TDB_BF16) rows(std::integral_constant<int, TDB_BF16>{});
     else rows(std::integral_constant<int, TDB_F16>{});
     return known ? int(hipGetLastError()) : int(hipErrorInvalidValue);
+}
+
+int tdb_enc_rows_fused(int M, int hidden, int inner, int dtype) {
+    return hidden % 32 == 0 && hidden <= FUSED_WIDTH && tdb_enc_small_tiles(M, 3 * hidden, hidden, dtype) && tdb_enc_small_tiles(M, inner, hidden, dtype)
+               ? tdb_enc_small_tiles(M, hidden, inner, dtype)
+               : 0;
+}
+
+int tdb_enc_embed_rows(const void* ids, int ids64, const void* table, int64_t vocab, const int32_t* cu, int B, int L, int T, int hidden, int dtype, int mt,
+                       float* x, float* stats, void* stream) {
+    if (!hidden_ok(hidden) || hidden % 32 || T < 1 || T > 16 * mt || dtype == TDB_F32) return int(hipErrorInvalidValue);
+    auto go = [&](auto dt) {
+        with_chunks(hidden, [&](auto ch) {
+            hipLaunchKernelGGL((embed_kernel<decltype(dt)::value, decltype(ch)::value, true>), dim3((T + 3) / 4), dim3(256), 0, static_cast<hipStream_t>(stream),
+                               ids, ids64, table, vocab, nullptr, nullptr, 0.f, cu, B, L, T, hidden, mt, x, reinterpret_cast<float2*>(stats));
+        });
+    };
+    if (dtype == TDB_BF16) go(std::integral_constant<int, TDB_BF16>{});
+    else go(std::integral_constant<int, TDB_F16>{});
+    return int(hipGetLastError());
+}
+
+int tdb_enc_norm_gemm(const tdb_enc_rows* in, const void* w, const void* bias, int gelu, int M, int N, int K, int dtype, const tdb_enc_next* next,
+                      int nexts, void* y, void* stream) {
+    const int mt = tdb_enc_small_tiles(M, N, K, dtype);
+    if (!mt || K % 32 || nexts < 0 || nexts > Ahead::MOST) return int(hipErrorInvalidValue);
+    const Ahead ahead = ahead_of(next, nexts, mt);
+    const int extra = ahead.chunks[0] > 0;
+    const NormRows r{in->x, reinterpret_cast<const float2*>(in->stats), in->gamma, in->beta, in->eps};
+    const int blocks = N / 16;
+    auto wide = [&](auto nb) {
+        constexpr int NB = decltype(nb)::value;
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((blocks + NB - 1) / NB, mt + extra), dim3(512), 0, static_cast<hipStream_t>(stream), r, w, bias, y, M, N, K, mt, ahead); };
+        if (dtype == TDB_BF16) gelu ? go(norm_gemm_kernel<TDB_BF16, NB, true>) : go(norm_gemm_kernel<TDB_BF16, NB, false>);
+        else gelu ? go(norm_gemm_kernel<TDB_F16, NB, true>) : go(norm_gemm_kernel<TDB_F16, NB, false>);
+    };
+    const int nb = norm_blocks(N, mt);
+    if (nb == 1) wide(std::integral_constant<int, 1>{});
+    else if (nb == 2) wide(std::integral_constant<int, 2>{});
+    else if (nb == 3) wide(std::integral_constant<int, 3>{});
+    else wide(std::integral_constant<int, 4>{});
+    return int(hipGetLastError());
+}
+
+int tdb_enc_gemm_add(const void* in, int ordered, const void* w, const void* bias, const tdb_enc_rows* residual, int M, int N, int K, int dtype, const tdb_enc_next* next,
+                     int nexts, float* x, float* stats, void* stream) {
+    const int mt = tdb_enc_small_tiles(M, N, K, dtype);
+    if (!mt || N % 32 || nexts < 0 || nexts > Ahead::MOST) return int(hipErrorInvalidValue);
+    const Ahead ahead = ahead_of(next, nexts, mt);
+    const int extra = ahead.chunks[0] > 0 ? 2 : 0;     // (96 workgroups of 768 columns' product)
+    const NormRows r{residual->x, reinterpret_cast<const float2*>(residual->stats), residual->gamma, residual->beta, residual->eps};
+    auto go = [&](auto kernel, int waves) {
+        hipLaunchKernelGGL(kernel, dim3(N / 16, mt + extra), dim3(waves * 64), 0, static_cast<hipStream_t>(stream), in, w, bias, r, x,
+                           reinterpret_cast<float2*>(stats), M, N, K, mt, ahead);
+    };
+    auto typed = [&](auto dt) {
+        constexpr int DT = decltype(dt)::value;
+        if (K > 1536) ordered ? go(gemm_add_kernel<DT, 16, true>, 16) : go(gemm_add_kernel<DT, 16, false>, 16);
+        else ordered ? go(gemm_add_kernel<DT, 8, true>, 8) : go(gemm_add_kernel<DT, 8, false>, 8);
+    };
+    if (dtype == TDB_BF16) typed(std::integral_constant<int, TDB_BF16>{});
+    else typed(std::integral_constant<int, TDB_F16>{});
+    return int(hipGetLastError());
+}
+
+int tdb_enc_norm_rows(const tdb_enc_rows* in, int T, int hidden, int dtype, void* out, void* stream) {
+    const int mt = (T + 15) / 16;
+    if (!hidden_ok(hidden) || hidden % 32 || T < 1 || dtype == TDB_F32) return int(hipErrorInvalidValue);
+    const NormRows r{in->x, reinterpret_cast<const float2*>(in->stats), in->gamma, in->beta, in->eps};
+    auto go = [&](auto dt) {
+        with_chunks(hidden, [&](auto ch) {
+            hipLaunchKernelGGL((norm_rows_kernel<decltype(dt)::value, decltype(ch)::value>), dim3(T), dim3(64), 0, static_cast<hipStream_t>(stream), r, hidden, mt, out);
+        });
+    };
+    if (dtype == TDB_BF16) go(std::integral_constant<int, TDB_BF16>{});
+    else go(std::integral_constant<int, TDB_F16>{});
+    return int(hipGetLastError());
 }
 
 int tdb_enc_unpack(const void* x, const int32_t* cu, int B, int L, int T, int hidden, int dtype, void* out, void* stream) {

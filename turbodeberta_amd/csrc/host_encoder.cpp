@@ -40,6 +40,11 @@ struct Enc {
     decltype(&tdb_enc_unpack) unpack;
     decltype(&tdb_enc_gemm) gemm;
     decltype(&tdb_enc_gemm_splits) gemm_splits;
+    decltype(&tdb_enc_rows_fused) rows_fused;
+    decltype(&tdb_enc_embed_rows) embed_rows;
+    decltype(&tdb_enc_norm_gemm) norm_gemm;
+    decltype(&tdb_enc_gemm_add) gemm_add;
+    decltype(&tdb_enc_norm_rows) norm_rows;
 } g_enc = {};
 
 struct Decref {
@@ -303,6 +308,7 @@ at::Tensor encode(const Plan& p, const at::Tensor& ids, const at::Tensor* cu, in
                          g_enc.small_tiles(int(T), int(inner), int(hidden), dt)};
     const bool small = tiles[0] && tiles[1] && tiles[2];
     const int mt = small ? tiles[0] : 0;    // (the same for all three)
+    const bool fused = small && g_enc.rows_fused(int(T), int(hidden), int(inner), dt);
     const int64_t rows = small ? 16 * mt : T;
     // Contractions with hidden-sized outputs are split where the output alone gives the CUs too little to do; the add + norm
     // behind them adds the parts up.
@@ -310,20 +316,42 @@ at::Tensor encode(const Plan& p, const at::Tensor& ids, const at::Tensor* cu, in
     const int splits_o = small ? few : g_enc.gemm_splits(int(T), int(hidden), int(hidden), dt);
     const int splits_f = small ? few : g_enc.gemm_splits(int(T), int(hidden), int(inner), dt);
     const bool own = !small && splits_o && splits_f && g_enc.gemm_splits(int(T), int(3 * hidden), int(hidden), dt) && g_enc.gemm_splits(int(T), int(inner), int(hidden), dt);
-    at::Tensor x = empty({rows, hidden}, type), y = empty({rows, hidden}, type), attended = empty({T, hidden}, type);
-    at::Tensor last = small ? empty({T, hidden}, type) : x;             // the last layer's output, row after row
-    at::Tensor qkv, ff, part, proj;
+    at::Tensor attended = empty({T, hidden}, type);
+    at::Tensor x, y, last, qkv, ff, part, proj;
+    // Rows before their LayerNorm: those that a layer starts from, and those between its attention and its feed-forward products.
+    at::Tensor wide[2];
+    tdb_enc_rows from{}, between{};
+    if (fused) {
+        const int64_t sums = hidden / 8;    // (floats of a row)
+        for (at::Tensor& w : wide) w = empty({rows, hidden + sums}, at::kFloat);
+        auto rows_in = [&](const at::Tensor& w) {
+            const float* const at = static_cast<const float*>(w.data_ptr());
+            return tdb_enc_rows{at, at + rows * hidden, p.emb_g.data_ptr(), p.emb_b.data_ptr(), float(p.emb_eps)};
+        };
+        from = rows_in(wide[0]), between = rows_in(wide[1]);
+    } else {
+        x = empty({rows, hidden}, type), y = empty({rows, hidden}, type);
+    }
+    last = small ? empty({T, hidden}, type) : x;                        // the last layer's output, row after row
     if (small || own) qkv = empty({T, 3 * hidden}, type), ff = empty({rows, inner}, type);
-    if (small || (own && std::max(splits_o, splits_f) > 1)) part = empty({std::max(splits_o, splits_f), T, hidden}, at::kFloat);
+    if ((small && !fused) || (own && std::max(splits_o, splits_f) > 1)) part = empty({std::max(splits_o, splits_f), T, hidden}, at::kFloat);
     if (own && std::min(splits_o, splits_f) == 1) proj = empty({T, hidden}, type);
-    must(g_enc.embed(ids.data_ptr(), ids.scalar_type() == at::kLong, p.emb.data_ptr(), p.emb.size(0), p.emb_g.data_ptr(), p.emb_b.data_ptr(),
+    auto writable = [](const float* rows) { return const_cast<float*>(rows); };
+    if (fused)
+        must(g_enc.embed_rows(ids.data_ptr(), ids.scalar_type() == at::kLong, p.emb.data_ptr(), p.emb.size(0), bounds, int(B), int(L), int(T), int(hidden), dt, mt,
+                              writable(from.x), writable(from.stats), s));
+    else
+        must(g_enc.embed(ids.data_ptr(), ids.scalar_type() == at::kLong, p.emb.data_ptr(), p.emb.size(0), p.emb_g.data_ptr(), p.emb_b.data_ptr(),
                      float(p.emb_eps), bounds, int(B), int(L), int(T), int(hidden), dt, mt, x.data_ptr(), s));
     auto ptr = [](const at::Tensor& t) { return t.data_ptr(); };
     auto norm = [&](const at::Tensor& d, int splits, const at::Tensor& bias, const at::Tensor& res, const at::Tensor& g, const at::Tensor& b, double eps, at::Tensor& out, int mt_out) {
         must(g_enc.add_norm(ptr(d), splits, ptr(bias), ptr(res), ptr(g), ptr(b), float(eps), int(T), int(hidden), dt, mt, mt_out, ptr(out), s));
     };
     for (const Layer& w : p.layers) {
-        if (small) must(g_enc.small_gemm(ptr(x), ptr(w.wqkv), ptr(w.bqkv), TDB_ENC_IN, 0, int(T), int(3 * hidden), int(hidden), dt, ptr(qkv), s));
+        auto weight = [&](const at::Tensor& t, int norm) { return tdb_enc_next{t.data_ptr(), int(t.size(0)), int(t.size(1)), norm}; };
+        const tdb_enc_next next[] = {weight(w.wo, 0), weight(w.wi, 1), weight(w.wf, 0), &w != &p.layers.back() ? weight((&w + 1)->wqkv, 1) : tdb_enc_next{}};
+        if (fused) must(g_enc.norm_gemm(&from, ptr(w.wqkv), ptr(w.bqkv), 0, int(T), int(3 * hidden), int(hidden), dt, next, 1, ptr(qkv), s));
+        else if (small) must(g_enc.small_gemm(ptr(x), ptr(w.wqkv), ptr(w.bqkv), TDB_ENC_IN, 0, int(T), int(3 * hidden), int(hidden), dt, ptr(qkv), s));
         else if (own) must(g_enc.gemm(ptr(x), ptr(w.wqkv), ptr(w.bqkv), 0, 1, int(T), int(3 * hidden), int(hidden), dt, ptr(qkv), s));
         else qkv = at::addmm(w.bqkv, x, w.wqkv.t());
         tdb_pos_args pos;
@@ -357,7 +385,13 @@ at::Tensor encode(const Plan& p, const at::Tensor& ids, const at::Tensor* cu, in
         if (rc != TDB_OK) return at::Tensor();
         at::Tensor& out = &w == &p.layers.back() ? last : x;
         const int mt_out = &w == &p.layers.back() ? 0 : mt;
-        if (small) {
+        if (fused) {
+            must(g_enc.gemm_add(ptr(attended), 0, ptr(w.wo), ptr(w.bo), &from, int(T), int(hidden), int(hidden), dt, next + 1, 2, writable(between.x), writable(between.stats), s));
+            between.gamma = ptr(w.g1), between.beta = ptr(w.b1), between.eps = float(w.eps1);
+            must(g_enc.norm_gemm(&between, ptr(w.wi), ptr(w.bi), 1, int(T), int(inner), int(hidden), dt, nullptr, 0, ptr(ff), s));
+            must(g_enc.gemm_add(ptr(ff), 1, ptr(w.wf), ptr(w.bf), &between, int(T), int(hidden), int(inner), dt, next + 3, 1, writable(from.x), writable(from.stats), s));
+            from.gamma = ptr(w.g2), from.beta = ptr(w.b2), from.eps = float(w.eps2);
+        } else if (small) {
             must(g_enc.small_gemm(ptr(attended), ptr(w.wo), nullptr, 0, few, int(T), int(hidden), int(hidden), dt, ptr(part), s));
             norm(part, few, w.bo, x, w.g1, w.b1, w.eps1, y, mt);
             must(g_enc.small_gemm(ptr(y), ptr(w.wi), ptr(w.bi), TDB_ENC_IN | TDB_ENC_OUT | TDB_ENC_GELU, 0, int(T), int(inner), int(hidden), dt, ptr(ff), s));
@@ -379,6 +413,7 @@ at::Tensor encode(const Plan& p, const at::Tensor& ids, const at::Tensor* cu, in
             norm(at::addmm(w.bf, f, w.wf.t()), 0, w.bf, y, w.g2, w.b2, w.eps2, out, 0);
         }
     }
+    if (fused) must(g_enc.norm_rows(&from, int(T), int(hidden), dt, ptr(last), s));
     if (!cu) return last.view({B, L, hidden});
     at::Tensor out = empty({B, L, hidden}, type);
     must(g_enc.unpack(ptr(last), bounds, int(B), int(L), int(T), int(hidden), dt, ptr(out), s));
@@ -561,8 +596,8 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 // bind_encoder(addresses of the tdb_enc_* functions in the order of Enc)
 PyObject* py_bind_encoder(PyObject*, PyObject* args) {
-    unsigned long long f[9];
-    if (!PyArg_ParseTuple(args, "KKKKKKKKK", f, f + 1, f + 2, f + 3, f + 4, f + 5, f + 6, f + 7, f + 8)) return nullptr;
+    unsigned long long f[14];
+    if (!PyArg_ParseTuple(args, "KKKKKKKKKKKKKK", f, f + 1, f + 2, f + 3, f + 4, f + 5, f + 6, f + 7, f + 8, f + 9, f + 10, f + 11, f + 12, f + 13)) return nullptr;
     g_enc.scan_mask = reinterpret_cast<decltype(g_enc.scan_mask)>(f[0]);
     g_enc.embed = reinterpret_cast<decltype(g_enc.embed)>(f[1]);
     g_enc.add_norm = reinterpret_cast<decltype(g_enc.add_norm)>(f[2]);
@@ -572,6 +607,11 @@ PyObject* py_bind_encoder(PyObject*, PyObject* args) {
     g_enc.unpack = reinterpret_cast<decltype(g_enc.unpack)>(f[6]);
     g_enc.gemm = reinterpret_cast<decltype(g_enc.gemm)>(f[7]);
     g_enc.gemm_splits = reinterpret_cast<decltype(g_enc.gemm_splits)>(f[8]);
+    g_enc.rows_fused = reinterpret_cast<decltype(g_enc.rows_fused)>(f[9]);
+    g_enc.embed_rows = reinterpret_cast<decltype(g_enc.embed_rows)>(f[10]);
+    g_enc.norm_gemm = reinterpret_cast<decltype(g_enc.norm_gemm)>(f[11]);
+    g_enc.gemm_add = reinterpret_cast<decltype(g_enc.gemm_add)>(f[12]);
+    g_enc.norm_rows = reinterpret_cast<decltype(g_enc.norm_rows)>(f[13]);
     Py_RETURN_NONE;
 }
 

@@ -41,6 +41,33 @@ int tdb_enc_small_tiles(int M, int N, int K, int dtype);
 // the number of partial sums of a product with N columns whose reader adds them up
 int tdb_enc_small_splits(int N);
 
+// The same products with the residual + LayerNorm between them in their own launches, 16-bit, up to 64 rows.  Rows before their LayerNorm are float32 in
+// an order of their own ([16 mt, hidden] floats, mt = tdb_enc_rows_fused) with the mean and sum of squared deviations of each 16
+// columns ([hidden / 16, 16 mt, 2] floats).
+typedef struct tdb_enc_rows {
+    const float *x, *stats;
+    const void *gamma, *beta;               // of the LayerNorm
+    float eps;
+} tdb_enc_rows;
+// A weight [N, K] that a product to come will read, a tdb_enc_norm_gemm (norm) or a tdb_enc_gemm_add: brought nearer meanwhile (w may be NULL).
+typedef struct tdb_enc_next {
+    const void* w;
+    int N, K, norm;
+} tdb_enc_next;
+// mt where the four products of a layer are taken this way, else 0
+int tdb_enc_rows_fused(int M, int hidden, int inner, int dtype);
+// rows = table[ids of token t], NaN for an id outside the table; cu as above
+int tdb_enc_embed_rows(const void* ids, int ids64, const void* table, int64_t vocab, const int32_t* cu, int B, int L, int T, int hidden, int dtype,
+                       int mt, float* x, float* stats, void* stream);
+// y[M, N] = LayerNorm(in)[M, K] w[N, K]^T + bias, row after row; gelu: GELU of that, in the small products' order.  next: up to 2.
+int tdb_enc_norm_gemm(const tdb_enc_rows* in, const void* w, const void* bias, int gelu, int M, int N, int K, int dtype, const tdb_enc_next* next,
+                      int nexts, void* y, void* stream);
+// rows (x, stats) = in[M, K] w[N, K]^T + bias + LayerNorm(residual); ordered: `in` is in the small products' order.  Not in place.
+int tdb_enc_gemm_add(const void* in, int ordered, const void* w, const void* bias, const tdb_enc_rows* residual, int M, int N, int K, int dtype,
+                     const tdb_enc_next* next, int nexts, float* x, float* stats, void* stream);
+// out[T, hidden] = LayerNorm(in), row after row
+int tdb_enc_norm_rows(const tdb_enc_rows* in, int T, int hidden, int dtype, void* out, void* stream);
+
 // Products of any size, 16-bit, rows in order: y[M, N] = x[M, K] w[N, K]^T + bias (flags: 0 or TDB_ENC_GELU), or (splits > 1)
 // float32 partial sums [splits, M, N] without bias.  K a multiple of 64, N of 8; pointers 16-byte aligned.
 // flags >> TDB_ENC_TILE_SHIFT: 1 + the number of a tile, for tests; 0: the kernel's choice.
