@@ -59,6 +59,20 @@ def test_equal_lengths(B, H, L, dtype, buckets, terms):
                 _lib.set_workgroup_limit(0)
 
 
+@pytest.mark.parametrize("terms", [BOTH, ("pk",), ("pq",)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,L,buckets,max_rel", [
+    (1, 2, 1536, 8, 4096), (8, 12, 1537, 16, 4096), (2, 12, 2500, 8, 2048),        # wide buckets: far steps of one table row after another
+    (1, 3, 1700, 16, 64), (9, 12, 1536, 4, 16),                                     # one run of near steps, also within a single step
+])
+def test_far_and_near_steps_in_turn(B, H, L, buckets, max_rel, dtype, terms):
+    d = {n: t.cuda() for n, t in make_inputs(L + buckets, B, H, L, 64, buckets, max_rel, dtype).items()}
+    kw = {"pos_key_layer": d["pk"] if "pk" in terms else None, "pos_query_layer": d["pq"] if "pq" in terms else None}
+    print(f"[case] {B} x {H} x {L}, {buckets} buckets to {max_rel}", flush=True)
+    run = lambda **more: flash_attention_with_disentangled(d["q"], d["k"], d["v"], None, None, False, SCALE, buckets, max_rel, **kw, **more)
+    assert_close_bf16(_same_in_each(run, "far and near"), run(force_generic=True), f"{L}, {buckets} buckets")
+
+
 LENS = {
     "few": [256, 1, 0, 130], "rounds_of_halves": [511, 64, 300] * 3, "64": list(range(4, 516, 8)), "65_in_two": [500] * 60 + [1, 33, 0, 129, 256],
     "last_round_split": [512] * 43 + [129] * 3, "ends": [289] * 50, "long": [1600, 900, 64, 1537, 1, 1300, 2000, 1100],

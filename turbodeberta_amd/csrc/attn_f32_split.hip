@@ -77,14 +77,6 @@ __device__ __forceinline__ f32x4 dot(const Parts (&x)[2], const Parts (&y)[2]) {
     return acc;
 }
 
-// The compiler does not count the wait states between a product and a branch behind which a vector instruction reads its result
-// (seen: the first of four scores was that of the step before).
-__device__ __forceinline__ void settled(f32x4& x) {
-    float a = x[0], b = x[1], c = x[2], d = x[3];
-    asm volatile("s_nop 7\n\ts_nop 7" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
-    x = f32x4{a, b, c, d};
-}
-
 __device__ __forceinline__ float fold_max(float x) {
     x = fmaxf(x, __shfl_xor(x, 16));
     return fmaxf(x, __shfl_xor(x, 32));

@@ -6,7 +6,7 @@
 // a compute unit, and tiles are dealt so that it mostly keeps its head: the tables are read once for many tiles.
 //
 // Microseconds at 12 heads, both terms, bf16, against the persistent kernel of attn_mfma.hip, whose waves compute windows of positions
-// for each other through LDS: 64 x 512 keys 187 -> 166, 32 x 1024 315 -> 264, 8 x 4096 977 -> 770; c2p alone 64 x 512 131 -> 117, p2c
+// for each other through LDS: 64 x 512 keys 187 -> 166, 32 x 1024 315 -> 264, 8 x 4096 977 -> 700; c2p alone 64 x 512 131 -> 117, p2c
 // alone 138 -> 120, neither 104 -> 77.  1 x 512 18.2 -> 16, 1 x 180 11.8 -> 10.
 #include <algorithm>
 #include <mutex>
@@ -34,7 +34,6 @@ struct ResidentArgs {
     int32_t mode, gap_B;
     int32_t B, H, L, total, lut_half, rows; // rows: of a table
     float c_exp;
-    int32_t exact_far;
     int32_t per_group, heads;               // workgroups and heads of a group that deals its tiles among itself
 };
 enum { FIXED = 0, LENGTHS = 1, PACKED = 2 };
@@ -66,10 +65,10 @@ __device__ __forceinline__ Upto tiles_upto(int n, int heads) {
 }
 // One workgroup's tiles.  s_at, s_n, s_upto: of the sequence of this lane, in order of decreasing length: what the batch strides are
 // multiplied with, its length, its tiles.
-template <bool C2P, bool P2C, int DT, int QG, bool EQUAL>
+template <bool C2P, bool P2C, int DT, int QG, bool EQUAL, bool LONG>
 __device__ __forceinline__ void run(const ResidentArgs& p, const int s_at, const int s_n, const Upto s_upto) {
 #pragma clang fp contract(off)
-    using W = Wave<C2P, P2C, DT, QG>;
+    using W = Wave<C2P, P2C, DT, QG, LONG>;
     using X8 = typename W::X8;
     constexpr int UQ = W::UQ, NT = W::NT;
     constexpr bool POS = W::POS;
@@ -243,7 +242,7 @@ __device__ __forceinline__ void run(const ResidentArgs& p, const int s_at, const
     // A step is far if its relative positions have one table row (delta is monotone: the two ends decide), in long sequences those of the
     // whole block of 128 rows, as in the persistent kernel: its far steps keep the position terms in 32 bits.
     auto ends_of = [&](int q0, int k0) {
-        const int from = p.exact_far ? q0 & -128 : q0, to = p.exact_far ? from + 127 : from + UQ - 1;
+        const int from = LONG ? q0 & -128 : q0, to = LONG ? from + 127 : from + UQ - 1;
         return delta(min(max((lane & 1 ? to : from - (BN - 1)) - k0, -p.lut_half), p.lut_half));
     };
     auto load_tables = [&](int head) {
@@ -281,11 +280,12 @@ __device__ __forceinline__ void run(const ResidentArgs& p, const int s_at, const
         if (len <= 0) break;
         const int head = __builtin_amdgcn_readlane(t_head, j - listed);
         const int q0 = UQ * (__builtin_amdgcn_readlane(t_first, j - listed) + wave);
-        const bool busy = wave < __builtin_amdgcn_readlane(t_units, j - listed);
-        int ends = 0;                       // even lanes: table row at the lower end of the step's window, odd lanes: at the upper end
-        if (busy) {
+        const int units = __builtin_amdgcn_readlane(t_units, j - listed);      // wave < units: this wave has one
+        int ends = 0, ends_next = 0;        // even lanes: table row at the lower end of the step's window, odd lanes: at the upper end
+        if (wave < units) {
             w.open();
             if (POS) ends = ends_of(q0, 0);
+            if (POS && LONG) ends_next = ends_of(q0, BN);
             const char* const qt = p.q + int64_t(__builtin_amdgcn_readlane(t_at, j - listed)) * p.qb + uint64_t(head) * p.qh + uint64_t(q0) * p.ql;
             const auto rsrc = rows_from(qt, p.ql, len - q0);
 #pragma unroll
@@ -308,31 +308,48 @@ __device__ __forceinline__ void run(const ResidentArgs& p, const int s_at, const
             stage(0);
             fetch();
         }
+        // Where L allows runs of far steps (LONG), a step knows two ahead whether there is one table row, so that far steps need neither the
+        // rows of the tiles of the next (all of them are read anew before a near one) nor their addresses: with the c2p values kept from one
+        // far step to the next 195 -> 163 vector instructions and 44 -> 40 products a step:
+        // 4 x 4096 keys (12 heads) 390 -> 355 us, 2 x 8192 711 -> 621, 8 x 1536 177 -> 173.  The loads for the next steps stand behind those of
+        // keys and values (before them each step waited for what it had just asked for: 370).  Scores of a step beside the softmax of the one
+        // before in one wave (448, registers spilled) or half a step between the two waves of a SIMD, by barriers (374): slower.
+        int low = __builtin_amdgcn_readlane(ends, 0), high = __builtin_amdgcn_readlane(ends, 1);
+        int low_next = __builtin_amdgcn_readlane(ends_next, 0), high_next = __builtin_amdgcn_readlane(ends_next, 1);
         for (int k0 = 0; k0 < len; k0 += BN) {
             __syncthreads();                // step k0 is in LDS, and nobody reads the other buffer any more
             stage(buf ^ 1);
             fetch();
-            if (busy) {
-                int raw[4] = {0, 0, 0, 0};  // the position rows of the next step, whose lowest four tiles are new
-                if (POS) {
+            if (wave < units) {
+                const uint32_t at = kv_base + buf * 2 * BLOCK;
+                int raw[NT];                // the position rows of the next step, whose lowest four tiles are new
+                if (POS && (!LONG || low_next != high_next)) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) raw[i] = delta(q0 - k0 - BN + 16 * (i - 4) + w.n);
+                    if (LONG && low == high) {
+#pragma unroll
+                        for (int i = 4; i < NT; ++i) raw[i] = delta(q0 - k0 - BN + 16 * (i - 4) + w.n);
+                    }
                 }
-                const uint32_t at = kv_base + buf * 2 * BLOCK;
-                const bool far = POS && __builtin_amdgcn_readlane(ends, 0) == __builtin_amdgcn_readlane(ends, 1);
-                const uint32_t row = POS ? w.row_at(__builtin_amdgcn_readfirstlane(ends)) ^ (w.g << 4) : 0;
-                if (POS) ends = ends_of(q0, k0 + BN);
-                w.step(at, at + BLOCK, len - k0, p.c_exp, k0 == 0, far, p.exact_far, row);
-                if (POS) {
+                if (POS) ends = ends_of(q0, k0 + (LONG ? 2 : 1) * BN);
+                w.step(at, at + BLOCK, len - k0, p.c_exp, k0 == 0, POS && low == high, (uint32_t(low) << 7) ^ ((uint32_t(low) << 3) & 0x70));
+                if (POS && (!LONG || low_next != high_next)) {
 #pragma unroll
                     for (int i = 0; i < QG; ++i) w.a[4 + i] = w.a[i];
+                    if (LONG && low == high) {
+#pragma unroll
+                        for (int i = 4; i < NT; ++i) w.a[i] = w.row_at(raw[i]);
+                    }
 #pragma unroll
                     for (int i = 0; i < 4; ++i) w.a[i] = w.row_at(raw[i]);
                 }
+                if (LONG) low = low_next, high = high_next;
+                (LONG ? low_next : low) = __builtin_amdgcn_readlane(ends, 0);
+                (LONG ? high_next : high) = __builtin_amdgcn_readlane(ends, 1);
             }
             buf ^= 1;
         }
-        if (busy) {
+        if (wave < units) {
             char* const ot = p.o + int64_t(__builtin_amdgcn_readlane(t_at, j - listed)) * p.ob + uint64_t(head) * p.oh + uint64_t(q0) * p.ol;
             w.store(ot, p.ol, (p.mode == PACKED ? len : p.L) - q0, len - q0);
         }
@@ -340,10 +357,10 @@ __device__ __forceinline__ void run(const ResidentArgs& p, const int s_at, const
 }
 
 // Units of 16 QG query rows; sequences that are all equal, or up to 64 of different lengths, which the device alone may know.
-template <bool C2P, bool P2C, int DT, int QG, bool EQUAL>
+template <bool C2P, bool P2C, int DT, int QG, bool EQUAL, bool LONG>
 __global__ __launch_bounds__(NTHREADS) void attn_resident_kernel(const ResidentArgs p) {
     if constexpr (EQUAL) {
-        run<C2P, P2C, DT, QG, true>(p, 0, 0, Upto{0, 0});
+        run<C2P, P2C, DT, QG, true, LONG>(p, 0, 0, Upto{0, 0});
         return;
     }
     const int lane = threadIdx.x & 63;
@@ -365,7 +382,7 @@ __global__ __launch_bounds__(NTHREADS) void attn_resident_kernel(const ResidentA
     }
     at = __builtin_amdgcn_ds_permute(rank * 4, at);
     n = __builtin_amdgcn_ds_permute(rank * 4, n);
-    run<C2P, P2C, DT, QG, false>(p, at, n, tiles_upto<QG>(n, p.heads));
+    run<C2P, P2C, DT, QG, false, LONG>(p, at, n, tiles_upto<QG>(n, p.heads));
 }
 
 // What equal sequences cost: see how run() deals them.
@@ -419,17 +436,23 @@ bool wide_units(const TdbKernelParams& p, const Grid& g) {
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mutex;
-bool g_attr_set[kMaxDevices][32] = {{false}};
+bool g_attr_set[kMaxDevices][64] = {{false}};
 
+template <bool C2P, bool P2C, int DT, int QG, bool LONG>
+const void* kernel_of(bool equal) {
+    return equal ? reinterpret_cast<const void*>(&attn_resident_kernel<C2P, P2C, DT, QG, true, LONG>)
+                 : reinterpret_cast<const void*>(&attn_resident_kernel<C2P, P2C, DT, QG, false, LONG>);
+}
 template <bool C2P, bool P2C, int DT>
-const void* kernel_of(bool wide, bool equal) {
-    return wide ? (equal ? reinterpret_cast<const void*>(&attn_resident_kernel<C2P, P2C, DT, 2, true>) : reinterpret_cast<const void*>(&attn_resident_kernel<C2P, P2C, DT, 2, false>))
-                : (equal ? reinterpret_cast<const void*>(&attn_resident_kernel<C2P, P2C, DT, 1, true>) : reinterpret_cast<const void*>(&attn_resident_kernel<C2P, P2C, DT, 1, false>));
+const void* kernel_of(bool wide, bool equal, bool far) {
+    if constexpr (C2P || P2C)
+        if (far) return wide ? kernel_of<C2P, P2C, DT, 2, true>(equal) : kernel_of<C2P, P2C, DT, 1, true>(equal);
+    return wide ? kernel_of<C2P, P2C, DT, 2, false>(equal) : kernel_of<C2P, P2C, DT, 1, false>(equal);
 }
 template <int DT>
-const void* kernel_of(bool c2p, bool p2c, bool wide, bool equal) {
-    return c2p ? (p2c ? kernel_of<true, true, DT>(wide, equal) : kernel_of<true, false, DT>(wide, equal))
-               : (p2c ? kernel_of<false, true, DT>(wide, equal) : kernel_of<false, false, DT>(wide, equal));
+const void* kernel_of(bool c2p, bool p2c, bool wide, bool equal, bool far) {
+    return c2p ? (p2c ? kernel_of<true, true, DT>(wide, equal, far) : kernel_of<true, false, DT>(wide, equal, far))
+               : (p2c ? kernel_of<false, true, DT>(wide, equal, far) : kernel_of<false, false, DT>(wide, equal, far));
 }
 
 }  // namespace
@@ -487,14 +510,13 @@ static hipError_t launch_part(const TdbKernelParams& p, bool wide, const Grid& g
     a.B = p.B, a.H = p.H, a.L = p.L, a.total = p.total, a.lut_half = p.lut_half;
     const bool c2p = p.pk != nullptr, p2c = p.pq != nullptr;
     a.rows = c2p || p2c ? 2 * p.span : 0;
-    a.exact_far = p.L >= TDB_FAR_MIN_LEN;
     a.c_exp = p.scale * 1.4426950408889634f;
     a.per_group = g.per_group, a.heads = g.heads;
-    const bool equal = a.mode == FIXED;
-    const void* fn = dtype == TDB_F16 ? kernel_of<TDB_F16>(c2p, p2c, wide, equal) : kernel_of<TDB_BF16>(c2p, p2c, wide, equal);
+    const bool equal = a.mode == FIXED, far = p.L >= TDB_FAR_MIN_LEN;
+    const void* fn = dtype == TDB_F16 ? kernel_of<TDB_F16>(c2p, p2c, wide, equal, far) : kernel_of<TDB_BF16>(c2p, p2c, wide, equal, far);
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        bool& set = g_attr_set[dev][(wide ? 16 : 0) + (equal ? 8 : 0) + (dtype == TDB_F16 ? 4 : 0) + (c2p ? 2 : 0) + (p2c ? 1 : 0)];
+        bool& set = g_attr_set[dev][(far ? 32 : 0) + (wide ? 16 : 0) + (equal ? 8 : 0) + (dtype == TDB_F16 ? 4 : 0) + (c2p ? 2 : 0) + (p2c ? 1 : 0)];
         if (!set) {
             const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
             if (e != hipSuccess) return e;

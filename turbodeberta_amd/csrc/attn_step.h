@@ -158,7 +158,16 @@ __device__ __forceinline__ float rows_sum(float x) {
     return __builtin_bit_cast(float, uint32_t(r[0])) + __builtin_bit_cast(float, uint32_t(r[1]));
 }
 
-template <bool C2P, bool P2C, int DT, int QG>
+// The compiler does not count the wait states between a product and a branch behind which a vector instruction reads its result
+// (seen: the first of four scores was that of the step before).
+__device__ __forceinline__ void settled(f32x4& x) {
+    float a = x[0], b = x[1], c = x[2], d = x[3];
+    asm volatile("s_nop 7\n\ts_nop 7" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
+    x = f32x4{a, b, c, d};
+}
+
+// EXACT: steps whose relative positions all have one table row keep their position terms in 32 bits.
+template <bool C2P, bool P2C, int DT, int QG, bool EXACT>
 struct Wave {
     using E = Elem<DT>;
     using X8 = typename E::X8;
@@ -178,6 +187,7 @@ struct Wave {
     // c2p of the highest tile of each query group, which is the lowest of the step before: packed (QG = 2) or as it is (QG = 1)
     u32x4 carry;
     bool carried;
+    uint32_t far_row;                       // EXACT: the row whose c2p values are in `carry` instead
 
     __device__ __forceinline__ void init(int lane, uint32_t kr_base_) {
         n = lane & 15, g = lane >> 4;
@@ -194,7 +204,7 @@ struct Wave {
         }
     }
     __device__ __forceinline__ void open() {
-        carried = false;
+        carried = false, far_row = ~0u;
 #pragma unroll
         for (int x = 0; x < QG; ++x) {
             m[x] = -INFINITY, l[x] = 0.f;
@@ -411,8 +421,9 @@ struct Wave {
     }
 
     // Scores of a step all of whose relative positions have one table row (at LDS offset `row`, chunk 0): a c2p value per query and a
-    // p2c value per key.  exact: both stay in 32 bits, c2p is returned in `add`; otherwise the bits are those of scores().
-    __device__ __forceinline__ void far_scores(f32x4 (&s)[4][QG], float (&add)[QG], uint32_t k_at, uint32_t row, bool exact) const {
+    // p2c value per key.  EXACT: both stay in 32 bits, c2p is returned in `add` and kept for the next step of this row; otherwise the bits
+    // are those of scores().
+    __device__ __forceinline__ void far_scores(f32x4 (&s)[4][QG], float (&add)[QG], uint32_t k_at, uint32_t row) {
         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
         X8 kf[4][2];
         keys(kf, k_at);
@@ -425,7 +436,7 @@ struct Wave {
             plain(r, at);
 #pragma unroll
             for (int kg = 0; kg < 4; ++kg) p[kg] = dot(kf[kg], r, zero);
-            if (!exact) {
+            if constexpr (!EXACT) {
 #pragma unroll
                 for (int kg = 0; kg < 4; ++kg) {
                     const uint32_t w0 = pack2<E>(p[kg][0], p[kg][1]), w1 = pack2<E>(p[kg][2], p[kg][3]);
@@ -438,11 +449,24 @@ struct Wave {
 #pragma unroll
             for (int x = 0; x < QG; ++x) s[kg][x] = dot(kf[kg], q[x], p[kg]);
         if constexpr (C2P) {
-            plain(r, at + kr_base);
-            if (exact) {
+            if constexpr (EXACT) {
+                if (row != far_row) {
+                    plain(r, at + kr_base);
 #pragma unroll
-                for (int x = 0; x < QG; ++x) add[x] = dot(r, q[x], zero)[0];
+                    for (int x = 0; x < QG; ++x) {
+                        f32x4 c = dot(r, q[x], zero);
+                        settled(c);
+                        carry[x] = bits(c[0]);
+                    }
+                    far_row = row;
+                }
+#pragma unroll
+                for (int x = 0; x < QG; ++x) {
+                    const uint32_t kept = carry[x];     // (the cast of the element itself is that of element 0)
+                    add[x] = __builtin_bit_cast(float, kept);
+                }
             } else {
+                plain(r, at + kr_base);
                 f32x4 c[QG];
                 u32x4 w;
 #pragma unroll
@@ -486,12 +510,11 @@ struct Wave {
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 uint32_t w[4];
-                total[c] = 0.f;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const f32x4& v = s[2 * c + (e >> 1)][x];
                     const float p0 = __builtin_amdgcn_exp2f(fmaf(v[2 * (e & 1)], c_exp, -mc)), p1 = __builtin_amdgcn_exp2f(fmaf(v[2 * (e & 1) + 1], c_exp, -mc));
-                    total[c] += p0 + p1;
+                    total[c] = e ? total[c] + (p0 + p1) : p0 + p1;
                     w[e] = pack2<E>(p0, p1);
                 }
                 pb[x][c] = __builtin_bit_cast(X8, u32x4{w[0], w[1], w[2], w[3]});
@@ -501,8 +524,8 @@ struct Wave {
     }
 
     // One step: keys at LDS offset k_at, values at v_at, `left` keys from its first one to the end of the sequence.  far: all its relative
-    // positions have the table row at LDS offset `row`; exact: see far_scores().
-    __device__ __forceinline__ void step(uint32_t k_at, uint32_t v_at, int left, float c_exp, bool first, bool far, bool exact, uint32_t row) {
+    // positions have the table row at LDS offset `row`.
+    __device__ __forceinline__ void step(uint32_t k_at, uint32_t v_at, int left, float c_exp, bool first, bool far, uint32_t row) {
         f32x4 s[4][QG];
         float add[QG], sum[QG];
         X8 pb[QG][2];
@@ -512,20 +535,27 @@ struct Wave {
         // other way about 64 x 512 keys take 5 % more).
         __builtin_amdgcn_s_setprio(1);
         if (far) {
-            far_scores(s, add, k_at, row, exact);
+            far_scores(s, add, k_at, row);
             carried = false;
         } else {
+            far_row = ~0u;
             scores<false>(s, k_at);
         }
         if (left < BN) mask(s, left);
         __builtin_amdgcn_s_setprio(0);
         // V^T through the transposing read: the lane provides the address of four columns of one key.
         s16x8 vf[2][4];
+        uint32_t v_from[4];
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+            v_from[dt] = v_at + (v_lane ^ (32 * dt));
+            asm("" : "+v"(v_from[dt]));     // (or every read has an addition of its own, instead of an offset)
+        }
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) {
-                const uint32_t at = v_at + (v_lane ^ (32 * dt)) + 32 * ROW * c;
+                const uint32_t at = v_from[dt] + 32 * ROW * c;
                 const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)at);
                 const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(at + 16 * ROW));
                 vf[c][dt] = s16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
@@ -551,7 +581,7 @@ struct Wave {
 #pragma unroll
                 for (int x = 0; x < QG; ++x) nan = nan || mx[x] != mx[x];
                 if (__builtin_expect(__builtin_amdgcn_ballot_w64(nan) != 0, 0)) {
-                    if (!far || !exact) {
+                    if (!far || !EXACT) {
                         scores<true>(s, k_at);
                         if (left < BN) mask(s, left);
                     }
