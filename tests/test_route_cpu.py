@@ -56,6 +56,15 @@ def test_which_kernel(kind, lens, heads, terms, resident):
     assert _rule("pays")(_launch(kind, lens, heads, terms)) == resident
 
 
+@pytest.mark.parametrize("kind,lens,heads,resident", [
+    ("equal", [1535] * 6, 12, False), ("equal", [1536] * 6, 12, True), ("equal", [1990], 16, False),        # 5.25 and 6 units a round
+    ("packed", [2269], 16, True), ("packed", [1717, 1717], 6, False), ("packed", [500, 1700, 1100, 2290], 6, False), ("packed", [1024, 1000, 4000], 8, True),
+    ("padded", [900, 1935], 12, False), ("padded", [1935], 12, True), ("padded", [1000, 1700, 400], 12, True),
+])
+def test_which_kernel_of_long_launches(kind, lens, heads, resident):
+    assert _rule("pays")(_launch(kind, lens, heads)) == resident
+
+
 @pytest.mark.parametrize("kind,lens,heads,wide", [
     ("packed", _even(64, 16, 512), 12, True), ("padded", _even(32, 384, 512), 12, True), ("packed", _even(8, 1024, 4096), 12, True),
     ("equal", [512] * 64, 12, True), ("equal", [180], 12, False), ("packed", [300, 200], 12, False),

@@ -479,15 +479,25 @@ bool tdb_resident_wide(const TdbKernelParams& p) { return wide_units(p, grid_of(
 // padded, of which the host knows the longest possible length only, 2 % if lengths are evenly spread and 9 % if most are far below it, 0.73x
 // (18 of up to 974, 359 in the mean, 8 heads: 37.5 -> 51).  No limit in L and rounds tells these from padded batches of nearly full texts, which
 // would lose as much (1250 launches: limits of 3400 to 5000, 16-row units up to 2 to 4 rounds, the other kernel below 2.2 to 3.5 of them).
+// From TDB_FAR_MIN_LEN on the far steps here take less time than there, and limits of their own hold, from 23 000 random launches of up to
+// 3.2 rounds: equal lengths all but one round of whole tiles (0.97x; two of them at 12 to 2: 1.05x); packed ones all but nearly a round, or
+// a little more of lengths far apart (of 11 400 31 % change, by 1.14x; 2.2 % of these are below 0.97x, 0.76x at worst); padded ones all but
+// 1.2 to 1.75 rounds (27 % change, by 1.08x; 3.7 % of these below 0.97x, 0.93x at worst; in between 1.05x, but 12 % below 0.97x).
 bool tdb_resident_pays(const TdbKernelParams& p) {
     if (!p.pk && !p.pq) return true;        // (no tables to load: 1.21x over 708 such launches, 1.12x before this line)
     const Grid g = grid_of(-1, p.H, 0);
     const int64_t B = sequences_of(p), seqs = g.heads * B;
-    if (!p.varlen && !p.seqlens) {          // (5.2: a step of the persistent kernel's tile in units of StepCost)
+    const bool far = p.L >= TDB_FAR_MIN_LEN;
+    if (!p.varlen && !p.seqlens) {          // (5.2, 5.8: a step of the persistent kernel's tile in units of StepCost)
         const int64_t rounds = (seqs * ((p.L + 127) / 128) + g.per_group - 1) / g.per_group;
-        return std::min(equal_cost<1>(seqs, p.L, g.per_group), equal_cost<2>(seqs, p.L, g.per_group)) * 10 <= 52 * rounds;
+        return std::min(equal_cost<1>(seqs, p.L, g.per_group), equal_cost<2>(seqs, p.L, g.per_group)) * 10 <= (far ? 58 : 52) * rounds;
     }
     const double rounds = ragged_rounds(p, g);
+    if (far) {
+        if (!p.varlen) return rounds <= 1.2 || rounds >= 1.75 || rounds * p.L >= 3400;
+        const double mean = double(p.total) / p.B / p.L;
+        return rounds <= (mean > 0.9 ? 0.6 : 0.8) || rounds > (mean > 0.65 ? 1.0 : 1.3);
+    }
     if (p.L <= 4 * BN || rounds <= (p.L <= 900 ? 0.6 : 0.45)) return true;
     // (Of few rounds of very different lengths the longest alone decide: 2 of 650 and 2600 0.82x.  With a mask the lengths are only bounded.)
     return rounds * p.L >= (rounds >= (p.varlen ? 1.4 : 1.75) ? 3000 : 3400);
