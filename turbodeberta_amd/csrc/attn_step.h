@@ -13,14 +13,16 @@
 //     two more by 4 and 8 under row masks (row g turns by 4 g) bring it to the lanes of its queries.
 //   * C'[query][r] = Q_query . K_r[delta(r)], its columns in the opposite order, turns into C[query][key], lanes along the keys, in the
 //     same way; the product that adds it to S^T transposes it.
-//   * a dword holds two values (16 bits, as the model rounds these terms) of two key groups / query groups that turn alike.  p2c is
-//     where the score products start from; c2p is added to them by products with an identity (exact: one addend each).
+//   * a dword holds two values (16 bits, as the model rounds these terms) that turn alike: p2c of two key groups, c2p of two query groups
+//     (one query group: of two key groups).  p2c is where the score products start from; c2p is added to them by products with an identity (exact: one addend each).
 // Against a scratch in LDS (results stored, read back element by element or through a ring, as in attn_mfma.hip) this costs three
 // vector instructions per dword and a product, and saves the stores, the reads, their waits and the barriers between the waves that
 // compute positions and those that compute scores: here every wave does the same, with one barrier a step for the keys.
 //
-// A near step is bound by the issue of its instructions, about 440 vector ones and 80 matrix ones of a wave of 32 rows; two waves of a
-// SIMD keep it busy for 82 to 90 % of the time.
+// A near step is bound by its SIMD: about 430 vector instructions and 80 matrix ones of a wave of 32 rows.  Measured there: a matrix
+// instruction of this shape takes 16.5 clk; conversions, selects, lane moves and shifts 4.3; exponentials 8.5; additions, products and
+// masks 4.3 too, but those of the two waves at the same time.  Vector instructions beside a stream of matrix instructions go at half their
+// rate, so the two together take about the sum of their times.
 //
 // Such a product multiplies every element of a row with a zero but one, so an infinity or a NaN among the c2p terms spoils its
 // neighbours' scores.  The maximum of a row tells: if a score is not a number, the step's scores are computed again, the finite terms
@@ -292,20 +294,21 @@ struct Wave {
         auto p_turn = [&](auto cc) {
             constexpr int first = decltype(cc)::value;
             if constexpr (P2C) {
+                // A word has two key groups, so that a tile is packed once for both query groups that take it (of one key group and two
+                // query groups it was 32 conversions a step for 24: 1.0 to 1.6 %).  To add the words by products with an identity instead
+                // of unpacking them saves 32 instructions for 8 products and is not faster: of either there is as much to do.
+                uint32_t w[QG + 1][4];
 #pragma unroll
-                for (int k = 0; k < QG; ++k) {          // QG = 2: a word of both query groups; QG = 1: of two key groups
-                    const int k0 = QG == 2 ? first + k : first, k1 = QG == 2 ? first + k : first + 1;
-                    uint32_t on[4], before[4];
+                for (int y = 0; y <= QG; ++y)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) w[y][t] = packed2<E>(p[first][y][t], p[first + 1][y][t]);
+#pragma unroll
+                for (int x = 0; x < QG; ++x) {
+                    const u32x4 to = turned<0>(in, w[QG - 1 - x], w[QG - x]);
 #pragma unroll
                     for (int t = 0; t < 4; ++t) {
-                        on[t] = packed2<E>(p[k0][QG - 1][t], p[k1][0][t]);
-                        before[t] = packed2<E>(p[k0][QG][t], p[k1][1][t]);
-                    }
-                    const u32x4 w = turned<0>(in, on, before);
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        s[k0][0][t] = E::low(w[t]);
-                        s[k1][QG - 1][t] = E::high(w[t]);
+                        s[first][x][t] = E::low(to[t]);
+                        s[first + 1][x][t] = E::high(to[t]);
                     }
                 }
             }
