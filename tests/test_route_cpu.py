@@ -65,6 +65,14 @@ def test_which_kernel_of_long_launches(kind, lens, heads, resident):
     assert _rule("pays")(_launch(kind, lens, heads)) == resident
 
 
+@pytest.mark.parametrize("kind,lens,heads,resident", [
+    ("padded", _even(16, 64, 512), 16, True), ("padded", _even(13, 64, 512), 16, False), ("padded", _even(16, 64, 512), 12, False),
+    ("packed", _even(15, 200, 512), 16, True), ("packed", _even(10, 200, 512), 16, False),
+])
+def test_which_kernel_of_workgroups_that_keep_one_head(kind, lens, heads, resident):
+    assert _rule("pays")(_launch(kind, lens, heads)) == resident
+
+
 @pytest.mark.parametrize("kind,lens,heads,wide", [
     ("packed", _even(64, 16, 512), 12, True), ("padded", _even(32, 384, 512), 12, True), ("packed", _even(8, 1024, 4096), 12, True),
     ("equal", [512] * 64, 12, True), ("equal", [180], 12, False), ("packed", [300, 200], 12, False),

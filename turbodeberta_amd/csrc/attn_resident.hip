@@ -499,6 +499,10 @@ bool tdb_resident_pays(const TdbKernelParams& p) {
         return rounds <= (mean > 0.9 ? 0.6 : 0.8) || rounds > (mean > 0.65 ? 1.0 : 1.3);
     }
     if (p.L <= 4 * BN || rounds <= (p.L <= 900 ? 0.6 : 0.45)) return true;
+    // Workgroups that keep one head load its tables once: 2700 such launches of 257 to 1535 keys below the limits of the next line, 1.06x
+    // packed (below 2.25 rounds 0.98x) and 1.085x padded (3 to 3.5 rounds 1.02x, and a quarter of them slower); 0.9 % are below 0.97x,
+    // 0.92x at worst.  With three heads 1.02x and 1.035x, but up to an eighth of them slower.
+    if (g.heads == 1 && rounds >= (p.varlen ? 2.25 : 3.5)) return true;
     // (Of few rounds of very different lengths the longest alone decide: 2 of 650 and 2600 0.82x.  With a mask the lengths are only bounded.)
     return rounds * p.L >= (rounds >= (p.varlen ? 1.4 : 1.75) ? 3000 : 3400);
 }
