@@ -285,6 +285,7 @@ __global__ __launch_bounds__(WAVES * 64, STRIP || QT > 1 ? 2 : 3) void attn_f32_
                     sum = mfma(kf[bi][te >> 2][te & 3], qf[a][te >> 2][te & 3], sum);
                 }
             if (HALVES > 1) s[0][0] += rest;
+            if (STRIP) asm volatile("" : "+v"(s[0][bi]));      // (added up ahead of the conditions below: see tdb_settled)
         };
         score(0);
         if (TILES > 1) score(TILES - 1);

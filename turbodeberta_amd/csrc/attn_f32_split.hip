@@ -334,8 +334,8 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
                 const uint32_t on[4] = {bits(ph[0]), bits(ph[1]), bits(ph[2]), bits(ph[3])}, before[4] = {bits(pl[0]), bits(pl[1]), bits(pl[2]), bits(pl[3])};
                 s += __builtin_bit_cast(f32x4, turned<0>(in, on, before));
             }
-            settled(s);
             s *= c_exp;
+            asm volatile("" : "+v"(s));     // (read ahead of the condition below: see tdb_settled)
             if (SETS > 1) __builtin_amdgcn_s_setprio(0);
             if (16 * (bt + 1) > len) {
 #pragma unroll
@@ -384,8 +384,7 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
 
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
-        settled(low[dt]);
-        o[dt] += low[dt];
+        o[dt] += tdb_settled(low[dt]);
     }
     if constexpr (SETS > 1) {               // the second set's sums to the first one
         __syncthreads();

@@ -37,7 +37,7 @@
 
 #include <type_traits>
 
-#include "tdb_attn.h"
+#include "tdb_internal.h"
 
 namespace tdb_step {
 
@@ -158,14 +158,6 @@ __device__ __forceinline__ float rows_sum(float x) {
     const uint32_t u = __builtin_bit_cast(uint32_t, x);
     const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
     return __builtin_bit_cast(float, uint32_t(r[0])) + __builtin_bit_cast(float, uint32_t(r[1]));
-}
-
-// The compiler does not count the wait states between a product and a branch behind which a vector instruction reads its result
-// (seen: the first of four scores was that of the step before).
-__device__ __forceinline__ void settled(f32x4& x) {
-    float a = x[0], b = x[1], c = x[2], d = x[3];
-    asm volatile("s_nop 7\n\ts_nop 7" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
-    x = f32x4{a, b, c, d};
 }
 
 // EXACT: steps whose relative positions all have one table row keep their position terms in 32 bits.
@@ -457,8 +449,7 @@ struct Wave {
                     plain(r, at + kr_base);
 #pragma unroll
                     for (int x = 0; x < QG; ++x) {
-                        f32x4 c = dot(r, q[x], zero);
-                        settled(c);
+                        const f32x4 c = tdb_settled(dot(r, q[x], zero));
                         carry[x] = bits(c[0]);
                     }
                     far_row = row;

@@ -461,6 +461,8 @@ __global__ __launch_bounds__(512) void norm_gemm_kernel(NormRows in, const void*
         with_steps<U>(k1 - k, [&](auto count) {
             load(k, count);
             use(count);
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[j] = tdb_settled(acc[j]);
         });
 #pragma unroll
     for (int j = 0; j < NB; ++j) s_sum[(wave * NB + j) * 64 + l] = acc[j];

@@ -182,6 +182,16 @@ __device__ __forceinline__ bool tdb_locate_tile_sorted(const TdbKernelParams& p,
     return true;
 }
 
+// A product's result as it is behind all wait states that a matrix instruction may need (12; 16 of them).  The compiler counts them, but where
+// paths join behind a condition it follows one of them back to the product: on another, which jumps over what lies between, the result
+// may be read, or its registers reused, too early (seen: 1 state of 8, and the score of the step before).  Not needed where a vector
+// instruction reads the result ahead of the condition.  tests/test_wait_states_cpu.py follows every path of the built kernels.
+template <typename T>
+__device__ __forceinline__ T tdb_settled(T x) {
+    asm volatile("s_nop 7\n\ts_nop 7" : "+v"(x));
+    return x;
+}
+
 // v Phi(v) as v / (1 + 2^-(v r(v^2))), r a polynomial fitted here to the logarithm of Phi(v) / Phi(-v).  Error against 64 bits,
 // evaluated in 32 (in brackets that of v (1 + erf) / 2 in 32 bits, which cancels below): relative 2.4e-6 on [-1, 0] and 3.1e-6
 // (2.6e-6) on [-2.5, 0], 3.6e-6 (4.6e-4) to -4, 4.4e-6 (4.3e-3) to -4.5, 6e-6 (4.7e-2) to -5; below, where the result is under
