@@ -59,6 +59,29 @@ def test_nan_and_infinity(flag, where):
 
 
 @pytest.mark.parametrize("flag", [ONE_SET, TWO_SETS])
+@pytest.mark.parametrize("L", [65, 273])                                             # a wave without queries, and the second set's keys
+@pytest.mark.parametrize("where", ["value", "last_value", "c2p_row", "p2c_row", "score"])
+def test_rows_computed_again(flag, where, L):
+    with in_kernel(flag):
+        f32.test_nan_and_infinity_reach_what_they_belong_to(where, 2, 2, L)
+
+
+@pytest.mark.parametrize("flag", [ONE_SET, TWO_SETS])
+def test_results_beside_an_infinity_keep_their_bits(flag):
+    """A query that is NaN and values that are infinite change their own row and column, also in the tile that is computed again."""
+    d = {n: t.cuda() for n, t in make_inputs(7, 1, 2, 150, 64, 256, 512).items()}
+    run = lambda: flash_attention_with_disentangled(d["q"], d["k"], d["v"], None, None, False, f32.SCALE, 256, 512, pos_key_layer=d["pk"], pos_query_layer=d["pq"])
+    with in_kernel(flag):
+        clean = run()
+        d["q"][0, 0, 37, 5], d["v"][0, 1, 20, 9] = math.nan, math.inf
+        got = run()
+    own = torch.zeros_like(clean, dtype=torch.bool)
+    own[0, 0, 37], own[0, 1, :, 9] = True, True
+    assert got[0, 0, 37].isnan().all() and (got[0, 1, :, 9] == math.inf).all()
+    assert torch.equal(got[~own], clean[~own])
+
+
+@pytest.mark.parametrize("flag", [ONE_SET, TWO_SETS])
 @pytest.mark.parametrize("scale", [0.0, -0.3, 40.0])
 def test_any_scale(flag, scale):
     """A score is scaled before its maximum is taken, and rounded as the maximum is: no scale makes a probability larger than 1."""

@@ -24,7 +24,9 @@
 // for themselves only (5 % slower), the next rows' parts shared out over both stages of products (5 % slower).
 //
 // An infinity has no parts (its rest is NaN), nor has what rounds to one: a wave whose results are not all finite computes its rows
-// again from the float32 operands (`again`), one key after another.  Values below about 1e-33 lose bits of their third part.
+// again from the float32 operands and takes what was not finite from there.  A NaN or an infinity in each sequence costs that for all its rows: 8 x 512
+// 121 -> 338 us, 2 x 4096 1.5 -> 4.3 ms (one key after another 1950 us and 14.2 ms; attn_f32.hip, which needs nothing of the kind, 160 us
+// and 2.2 ms).  Values below about 1e-33 lose bits of their third part.
 // (Same definition as the other kernels: modeling_deberta_v2.py:243, :317-324, :337-343.)
 #include <algorithm>
 #include <atomic>
@@ -214,15 +216,29 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
             }
     }
     Parts q[2];
+    bool plain = true;                      // this lane's query is finite.  (Another one takes part as zeros: its c2p terms would reach its neighbours.)
     {
         const float* const row = Q + int64_t(min(row0 + 16 * a + n, len - 1)) * p.qs_l + 8 * g;
+        f32x4 x[4];
+        bool ok = true;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            x[i] = *reinterpret_cast<const f32x4*>(row + 32 * (i >> 1) + 4 * (i & 1));
+#pragma unroll
+            for (int t = 0; t < 4; ++t) ok = ok && fabsf(x[i][t]) <= FLT_MAX;
+        }
+        const uint64_t other = __builtin_amdgcn_ballot_w64(!ok);
+        plain = !((other >> n | other >> (n + 16) | other >> (n + 32) | other >> (n + 48)) & 1);
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
-            const f32x4 x = *reinterpret_cast<const f32x4*>(row + 32 * half), y = *reinterpret_cast<const f32x4*>(row + 32 * half + 4);
             uint32_t w[4][3];
-            split2(x[0], x[1], w[0]), split2(x[2], x[3], w[1]), split2(y[0], y[1], w[2]), split2(y[2], y[3], w[3]);
 #pragma unroll
-            for (int i = 0; i < 3; ++i) q[half].p[i] = __builtin_bit_cast(bf16x8, u32x4{w[0][i], w[1][i], w[2][i], w[3][i]});
+            for (int i = 0; i < 4; ++i) {
+                const f32x4& y = x[2 * half + (i >> 1)];
+                split2(y[2 * (i & 1)], y[2 * (i & 1) + 1], w[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < 3; ++i) q[half].p[i] = __builtin_bit_cast(bf16x8, plain ? u32x4{w[0][i], w[1][i], w[2][i], w[3][i]} : u32x4{0, 0, 0, 0});
         }
     }
     const uint32_t frag_lane = operand_at(n, g), mirror_lane = operand_at(15 - n, g), v_lane = value_at(4 * g + (n >> 2), 0) + 8 * (n & 3);
@@ -403,7 +419,7 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
     }
     const int row_mine = row0 + 16 * a + n;
     const float inv = 1.f / fold_sum(sum);
-    bool finite = true;
+    bool finite = plain;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
@@ -411,47 +427,98 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
             o[dt][t] *= inv;
             finite = finite && fabsf(o[dt][t]) <= FLT_MAX;
         }
+    if constexpr (SETS == 1) __syncthreads();       // (the other waves' last step: its LDS is written below)
     if (__builtin_expect(live && __builtin_amdgcn_ballot_w64(!finite && row_mine < len) != 0, 0)) {
-#pragma clang fp contract(off)
-        // again: lane (n, g) has the columns 16 dt + 4 g .. + 3 of query n
-        const int i = min(row_mine, len - 1);
-        f32x4 qv[4];
+        // Again, as in attn_f32.hip: tiles of 16 keys, the position products through this wave's own LDS.  The results' layout is that of `o`.
+        constexpr int CS = 36;
+        float* const sC = reinterpret_cast<float*>(smem) + a * (2 * 16 * CS);
+        float* const sP = sC + 16 * CS;
+        auto fence = [] {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        };
+        auto row_of = [&](f32x4 (&f)[4], const float* row) {
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt) {
-            qv[dt] = *reinterpret_cast<const f32x4*>(Q + int64_t(i) * p.qs_l + 16 * dt + 4 * g);
-            o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
+            for (int dt = 0; dt < 4; ++dt) f[dt] = *reinterpret_cast<const f32x4*>(row + 16 * dt + 4 * g);
+        };
+        auto product = [&](const f32x4 (&x)[4], const f32x4 (&y)[4], f32x4 acc) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i >> 2][i & 3], y[i >> 2][i & 3], acc, 0, 0, 0);
+            return acc;
+        };
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        f32x4 qf[4], kr[4], qr[2][4], c[2] = {zero, zero}, res[4];      // [0]: the step's lower position tile, [1]: its upper one, the lower one of the step before
+        row_of(qf, Q + int64_t(min(row_mine, len - 1)) * p.qs_l);
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) res[dt] = zero;
         float top = -FLT_MAX, all = 0.f;
-        for (int j = 0; j < len; ++j) {
-            const float* const kj = K + int64_t(j) * p.ks_l + 4 * g;
-            const float* const vj = V + int64_t(j) * p.vs_l + 4 * g;
-            const int64_t d = C2P || P2C ? delta_of(i - j) : 0;
-            float s = 0.f, c = 0.f, r = 0.f;
+        int64_t d = 0;
+        if (C2P || P2C) {
+            d = delta_of(16 * (a0 + a) + n);
+            if (C2P) row_of(kr, KR + d * p.pks_r), c[1] = product(kr, qf, zero);
+            if (P2C) row_of(qr[1], QR + d * p.pqs_r);
+            d = delta_of(16 * (a0 + a - 1) + n);
+        }
+        for (int b = 0; b < ntiles; ++b) {
+            f32x4 kf[4], s = zero;
+            float v[4][4];
+            row_of(kf, K + int64_t(min(16 * b + n, len - 1)) * p.ks_l);
+            if (C2P) row_of(kr, KR + d * p.pks_r);
+            if (P2C) row_of(qr[0], QR + d * p.pqs_r);
 #pragma unroll
-            for (int dt = 0; dt < 4; ++dt) {
-                const f32x4 kv = *reinterpret_cast<const f32x4*>(kj + 16 * dt);
-                f32x4 cv = {0.f, 0.f, 0.f, 0.f}, rv = cv;
-                if (C2P) cv = *reinterpret_cast<const f32x4*>(KR + d * p.pks_r + 16 * dt + 4 * g);
-                if (P2C) rv = *reinterpret_cast<const f32x4*>(QR + d * p.pqs_r + 16 * dt + 4 * g);
+            for (int t = 0; t < 4; ++t) {
+                const int key = 16 * b + 4 * g + t;
+                const float* const row = V + int64_t(min(key, len - 1)) * p.vs_l + n;
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt) v[dt][t] = key < len ? row[16 * dt] : 0.f;
+            }
+            if (C2P || P2C) {
+                d = delta_of(16 * (a0 + a - b - 2) + n);
+                if (C2P) {
+                    c[0] = product(kr, qf, zero);
+#pragma unroll
+                    for (int x = 0; x < 2; ++x) *reinterpret_cast<f32x4*>(&sC[n * CS + 16 * x + 4 * g]) = c[x];
+                    c[1] = c[0];
+                }
+                if (P2C) {
+#pragma unroll
+                    for (int x = 0; x < 2; ++x) *reinterpret_cast<f32x4*>(&sP[n * CS + 16 * x + 4 * g]) = product(qr[x], kf, zero);
+#pragma unroll
+                    for (int dt = 0; dt < 4; ++dt) qr[1][dt] = qr[0][dt];
+                }
+                fence();
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    s = fmaf(qv[dt][t], kv[t], s);
-                    if (C2P) c = fmaf(qv[dt][t], cv[t], c);
-                    if (P2C) r = fmaf(kv[t], rv[t], r);
+                    const int r = 16 + n - (4 * g + t);
+                    if (C2P) s[t] = sC[n * CS + r];
+                    if (P2C) s[t] += sP[(4 * g + t) * CS + r];
                 }
+                fence();
             }
-            s = fold_sum(s);
-            if (C2P) s += fold_sum(c);
-            if (P2C) s += fold_sum(r);
-            s *= p.scale;
-            const float up = fmaxf(top, s), alpha = expf(top - up), e = expf(s - up);
-            top = up, all = all * alpha + e;
+            s = tdb_settled(product(kf, qf, s));
+            float most = -INFINITY;
 #pragma unroll
-            for (int dt = 0; dt < 4; ++dt) o[dt] = o[dt] * alpha + *reinterpret_cast<const f32x4*>(vj + 16 * dt) * e;
+            for (int t = 0; t < 4; ++t) {
+                s[t] = 16 * b + 4 * g + t < len ? s[t] * p.scale : -INFINITY;
+                most = fmaxf(most, s[t]);               // (NaN scores pass it by and meet expf)
+            }
+            const float up = fmaxf(top, fold_max(most)), alpha = expf(top - up);
+            top = up, all *= alpha;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) s[t] = expf(s[t] - up), all += s[t];
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) {
+                res[dt] *= alpha;
+#pragma unroll
+                for (int t = 0; t < 4; ++t) res[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[dt][t], s[t], res[dt], 0, 0, 0);
+                res[dt] = tdb_settled(res[dt]);
+            }
         }
-        const float div = 1.f / all;
+        const float div = 1.f / fold_sum(all);
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt) o[dt] *= div;
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) o[dt][t] = plain && fabsf(o[dt][t]) <= FLT_MAX ? o[dt][t] : res[dt][t] * div;
     }
     if (row_mine < row0 + rows_here) {
 #pragma unroll
