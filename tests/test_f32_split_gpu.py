@@ -103,6 +103,36 @@ def test_size_of_values(flag, size):
     assert (got - ref).abs().max() < BOUND * size
 
 
+def _exact(d, L, scale):
+    """The definition in 64 bits."""
+    x = {n: t.double() for n, t in d.items()}
+    delta = torch.from_numpy(_lib.delta_table(L, 256, 512).astype("int64")).cuda()
+    at = delta[(torch.arange(L)[:, None] - torch.arange(L)[None] + L - 1).cuda()].expand(*x["q"].shape[:2], L, L)
+    s = x["q"] @ x["k"].transpose(-1, -2).contiguous() + (x["q"] @ x["pk"].transpose(-1, -2).contiguous()[None]).gather(3, at)
+    s = s + (x["k"] @ x["pq"].transpose(-1, -2).contiguous()[None]).gather(3, at.transpose(-1, -2)).transpose(-1, -2)
+    return torch.softmax(s * scale, -1) @ x["v"]
+
+
+@pytest.mark.parametrize("flag", [DIRECT, ONE_SET, TWO_SETS])
+@pytest.mark.parametrize("sizes", [dict(v=1e-33), dict(v=1e-36), dict(v=2e-38), dict(v=1e36), dict(q=1e-36, k=1e36, pk=1e36, pq=1e-36), dict(q=1e36, k=1e-36, pk=1e-36, pq=1e36),
+                                   dict(k=1e-36, pq=1e36, pk=0), dict(q=1e-36, pk=1e36, k=1), dict(q=1e-18, k=1e-18, pk=1e-18, pq=1e-18, scale=1e36)],
+                         ids=lambda s: "-".join(f"{n}={x:g}" for n, x in s.items()))
+def test_error_at_any_size(flag, sizes):
+    """Where the last part of an operand is too small for its type, the result is as exact as elsewhere: sums of 64 products and 150 weighted
+    values in 32 bits, 1.2e-7 to 2.4e-7 of their size for values of order 1."""
+    d = {n: t.cuda() for n, t in make_inputs(8, 1, 2, 150, 64, 256, 512).items()}
+    for n in d:
+        d[n] *= sizes.get(n, 1)
+    d["v"][..., 60:] = 0
+    scale = f32.SCALE * sizes.get("scale", 1)
+    exact = _exact(d, 150, scale)
+    with in_kernel(flag):
+        out = flash_attention_with_disentangled(d["q"], d["k"], d["v"], None, None, False, scale, 256, 512, pos_key_layer=d["pk"], pos_query_layer=d["pq"])
+    err = float((out.double() - exact).norm() / exact.norm())
+    print(f"{sizes}: {err:.2e}")
+    assert err < 1e-6 and not out[..., 60:].any()
+
+
 @pytest.mark.parametrize("flag", [ONE_SET, TWO_SETS])
 def test_strided_rows_and_shared_tables(flag):
     """Rows of a wider array, and a table of equal rows (stride 0) as an expanded tensor has it."""
@@ -120,12 +150,7 @@ def test_strided_rows_and_shared_tables(flag):
 def test_error_against_64_bits_is_no_larger():
     """Small products first: sums of parts are more exact than float32 products one after another."""
     d = {n: t.cuda() for n, t in make_inputs(4, 2, 4, 300, 64, 256, 512).items()}
-    x = {n: t.double() for n, t in d.items()}
-    delta = torch.from_numpy(_lib.delta_table(300, 256, 512).astype("int64")).cuda()
-    at = delta[(torch.arange(300)[:, None] - torch.arange(300)[None] + 299).cuda()].expand(2, 4, 300, 300)
-    s = x["q"] @ x["k"].transpose(-1, -2).contiguous() + (x["q"] @ x["pk"].transpose(-1, -2).contiguous()[None]).gather(3, at)
-    s = s + (x["k"] @ x["pq"].transpose(-1, -2).contiguous()[None]).gather(3, at.transpose(-1, -2)).transpose(-1, -2)
-    exact = torch.softmax(s * f32.SCALE, -1) @ x["v"]
+    exact = _exact(d, 300, f32.SCALE)
     err = {}
     for flag in (DIRECT, ONE_SET, TWO_SETS):
         with in_kernel(flag):

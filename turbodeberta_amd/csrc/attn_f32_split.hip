@@ -26,7 +26,11 @@
 // An infinity has no parts (its rest is NaN), nor has what rounds to one: a wave whose results are not all finite computes its rows
 // again from the float32 operands and takes what was not finite from there.  A NaN or an infinity in each sequence costs that for all its rows: 8 x 512
 // 121 -> 338 us, 2 x 4096 1.5 -> 4.3 ms (one key after another 1950 us and 14.2 ms; attn_f32.hip, which needs nothing of the kind, 160 us
-// and 2.2 ms).  Values below about 1e-33 lose bits of their third part.
+// and 2.2 ms).
+// Operands below about 1e-33 lose bits of their third part, at most TINY each (bf16 has the exponents of float32).  In a score that is nothing
+// unless what it is multiplied with is beyond LARGE; in a result it is unless the result is as small.  Both are looked for, and such results
+// are computed again too.  (Against no such look 8 of 96..384 50.6 -> 51.2 us, 8 x 512 118.3 -> 120, 32 x 128 38.9 -> 40.1, 2 x 512 40.2 -> 40.8; errors of
+// 150 keys whose values are 1e-36 2.5e-5 -> 1.8e-7, whose keys are 1e36 and queries 1e-36 2.6e-5 -> 1.8e-7; attn_f32.hip 3.9e-7.)
 // (Same definition as the other kernels: modeling_deberta_v2.py:243, :317-324, :337-343.)
 #include <algorithm>
 #include <atomic>
@@ -46,11 +50,22 @@ constexpr int ROWS = 64;                    // query rows of a workgroup
 constexpr int PLANE = 16 * ROW, TILE = 3 * PLANE;       // bytes of 16 rows x 64: one part, all three
 constexpr int RING = 5;
 constexpr int GAP_WGS = 64;                 // workgroups that look for packed rows outside every sequence
-constexpr int set_bytes(bool c2p, bool p2c) { return TILE * (3 + RING * (int(c2p) + int(p2c))); }
+constexpr int tiles_bytes(bool c2p, bool p2c) { return TILE * (3 + RING * (int(c2p) + int(p2c))); }
+constexpr int MAGS = 5 * D;                 // floats: largest magnitudes that each wave of a set has passed on, and the second one when it opened
+constexpr int smem_bytes(bool c2p, bool p2c, int sets) { return sets * (tiles_bytes(c2p, p2c) + 4 * MAGS); }
+
+// What the parts of an operand may miss: half of the least subnormal bf16 (the products take them as they are).  128 products of TINY and LARGE
+// are 2^-63 of a score; a scale (up to LARGE_SCALE) makes 2^-33 of that.
+constexpr float TINY = 0x1p-134f, LARGE = 0x1p64f, LARGE_SCALE = 0x1p30f;
 
 struct Parts {                              // of eight elements
     bf16x8 p[3];
 };
+
+__device__ __forceinline__ float largest(float mag, float x, float y) {
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(mag) : "v"(x), "v"(y));      // (fmaxf of what was loaded has an instruction more for each of them)
+    return mag;
+}
 
 // The three parts of two values, packed.
 __device__ __forceinline__ void split2(float x, float y, uint32_t (&w)[3]) {
@@ -83,6 +98,14 @@ __device__ __forceinline__ float fold_max(float x) {
     x = fmaxf(x, __shfl_xor(x, 16));
     return fmaxf(x, __shfl_xor(x, 32));
 }
+// Of the lanes that have the same columns, without LDS.
+__device__ __forceinline__ float rows_max(float x) {
+    const uint32_t u = bits(x);
+    const auto h = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    const uint32_t v = bits(fmaxf(__builtin_bit_cast(float, uint32_t(h[0])), __builtin_bit_cast(float, uint32_t(h[1]))));
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return fmaxf(__builtin_bit_cast(float, uint32_t(r[0])), __builtin_bit_cast(float, uint32_t(r[1])));
+}
 __device__ __forceinline__ float fold_sum(float x) {
     x += __shfl_xor(x, 16);
     return x + __shfl_xor(x, 32);
@@ -91,7 +114,7 @@ __device__ __forceinline__ float fold_sum(float x) {
 template <bool C2P, bool P2C, int SETS>
 __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const TdbKernelParams p, const int tiles_x) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    constexpr int SET = set_bytes(C2P, P2C);
+    constexpr int SET = tiles_bytes(C2P, P2C);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63;
     const int a = wave & 3, set = SETS > 1 ? wave >> 2 : 0;
     const int n = l & 15, g = l >> 4;
@@ -177,6 +200,14 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
             for (int i = 0; i < 3; ++i) *(__attribute__((address_space(3))) u32x2*)(to + PLANE * i) = w[t][i];
         }
     };
+    // Largest magnitudes, of each column that this lane passes on.  (NaN passes by: it shows in the results.)
+    auto look = [&](const f32x4 (&x)[4], f32x4& mag) {
+#pragma unroll
+        for (int t = 0; t < 4; t += 2)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) mag[c] = largest(mag[c], x[t][c], x[t + 1][c]);
+    };
+    f32x4 mag = {0.f, 0.f, 0.f, 0.f}, mag_first = mag;      // (mag_first: of the tables' rows in the opening, whichever wave has them)
     // Opening: the first keys and values, and five tiles of each table.
     {
         int d[3][4];
@@ -210,13 +241,14 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
             if (a + 4 * i < ITEMS) {
                 int kind, e;
                 item(i, kind, e);
+                look(x[i], i ? mag_first : mag);
                 u32x2 w[4][3];
                 take_apart(x[i], w, Int<0>{}, Int<4>{});
                 put(kind, tile_at(kind, e), w);
             }
     }
     Parts q[2];
-    bool plain = true;                      // this lane's query is finite.  (Another one takes part as zeros: its c2p terms would reach its neighbours.)
+    bool plain = true;                      // this lane's query is finite and not LARGE.  (Another one takes part as zeros: infinite c2p terms would reach its neighbours.)
     {
         const float* const row = Q + int64_t(min(row0 + 16 * a + n, len - 1)) * p.qs_l + 8 * g;
         f32x4 x[4];
@@ -225,7 +257,7 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
         for (int i = 0; i < 4; ++i) {
             x[i] = *reinterpret_cast<const f32x4*>(row + 32 * (i >> 1) + 4 * (i & 1));
 #pragma unroll
-            for (int t = 0; t < 4; ++t) ok = ok && fabsf(x[i][t]) <= FLT_MAX;
+            for (int t = 0; t < 4; ++t) ok = ok && fabsf(x[i][t]) <= LARGE;
         }
         const uint64_t other = __builtin_amdgcn_ballot_w64(!ok);
         plain = !((other >> n | other >> (n + 16) | other >> (n + 32) | other >> (n + 48)) & 1);
@@ -315,6 +347,7 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
                     if (o < 5) s = E::mfma(kf[half].p[u], q[half].p[v], s);
                 }
             take_apart(x, w, Int<0>{}, Int<4>{});
+            look(x, mag);
             stage_end<10 + 12 * int(C2P), 3>();
             if constexpr (P2C) {
 #pragma unroll
@@ -402,6 +435,16 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
     for (int dt = 0; dt < 4; ++dt) {
         o[dt] += tdb_settled(low[dt]);
     }
+    {
+        float* const mine = reinterpret_cast<float*>(smem + SETS * SET) + set * MAGS;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (a != 1) mag[c] = fmaxf(mag[c], mag_first[c]);
+            mag[c] = rows_max(mag[c]);
+        }
+        if (g == 0) *reinterpret_cast<f32x4*>(&mine[D * a + 4 * n]) = mag;
+        if (a == 1) mine[4 * D + l] = fmaxf(fmaxf(mag_first[0], mag_first[1]), fmaxf(mag_first[2], mag_first[3]));
+    }
     if constexpr (SETS > 1) {               // the second set's sums to the first one
         __syncthreads();
         float* const mine = reinterpret_cast<float*>(smem) + a * (64 * 18);
@@ -418,17 +461,42 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
         for (int dt = 0; dt < 4; ++dt) o[dt] = o[dt] * f0 + *reinterpret_cast<const f32x4*>(&mine[(dt * 64 + l) * 4]) * f1;
     }
     const int row_mine = row0 + 16 * a + n;
+    if constexpr (SETS == 1) __syncthreads();       // (the magnitudes are there; the other waves' last step is over: its LDS is written below)
+    const float* const seen = reinterpret_cast<const float*>(smem + SETS * SET);
+    float of_kr = 0.f, of_v = 0.f;
+#pragma unroll
+    for (int i = 0; i < 5 * SETS; ++i) (i % 5 == 1 ? of_v : of_kr) = fmaxf(i % 5 == 1 ? of_v : of_kr, seen[D * i + l]);
+    // A value misses up to TINY, a probability (of up to 4096 keys) too: a result has to exceed what that makes by 2^26.
+    constexpr float LEAST = 0x1p26f * TINY, LEAST_BY = 0x1p38f * TINY, ORDINARY = 0x1p40f;
+    const bool sound = __builtin_amdgcn_ballot_w64(of_kr > LARGE && of_kr <= FLT_MAX) == 0;
+    const bool ordinary = sound && __builtin_amdgcn_ballot_w64(of_v > ORDINARY) == 0;
     const float inv = 1.f / fold_sum(sum);
-    bool finite = plain;
+    float total = 0.f, least = FLT_MAX;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             o[dt][t] *= inv;
-            finite = finite && fabsf(o[dt][t]) <= FLT_MAX;
+            total += fabsf(o[dt][t]);       // (neither NaN nor an infinity passes by)
+            least = fminf(least, fabsf(o[dt][t]));
         }
-    if constexpr (SETS == 1) __syncthreads();       // (the other waves' last step: its LDS is written below)
-    if (__builtin_expect(live && __builtin_amdgcn_ballot_w64(!finite && row_mine < len) != 0, 0)) {
+    uint32_t keep = plain && ordinary && total <= FLT_MAX && least >= LEAST_BY * ORDINARY ? 0xffff : 0;      // results that stay
+    if (__builtin_expect(live && __builtin_amdgcn_ballot_w64(keep == 0 && row_mine < len) != 0, 0)) {
+        keep = 0;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+            f32x4 v = *reinterpret_cast<const f32x4*>(&seen[D + 16 * dt + 4 * g]);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                if (SETS > 1) v[t] = fmaxf(v[t], seen[MAGS + D + 16 * dt + 4 * g + t]);
+                const float x = fabsf(o[dt][t]);
+                // (Zeros are ordinary results, but not of tiny values.)
+                const bool enough = x >= fmaxf(LEAST, v[t] * LEAST_BY) || (x == 0.f && (v[t] == 0.f || v[t] > 0x1p16f * TINY));
+                if (plain && sound && x <= FLT_MAX && enough) keep |= 1u << (4 * dt + t);
+            }
+        }
+    }
+    if (__builtin_expect(live && __builtin_amdgcn_ballot_w64(keep != 0xffff && row_mine < len) != 0, 0)) {
         // Again, as in attn_f32.hip: tiles of 16 keys, the position products through this wave's own LDS.  The results' layout is that of `o`.
         constexpr int CS = 36;
         float* const sC = reinterpret_cast<float*>(smem) + a * (2 * 16 * CS);
@@ -441,12 +509,15 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) f[dt] = *reinterpret_cast<const f32x4*>(row + 16 * dt + 4 * g);
         };
-        auto product = [&](const f32x4 (&x)[4], const f32x4 (&y)[4], f32x4 acc) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i >> 2][i & 3], y[i >> 2][i & 3], acc, 0, 0, 0);
-            return acc;
-        };
         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        auto product = [&](const f32x4 (&x)[4], const f32x4 (&y)[4]) {      // (four sums of 16: rounded at its full size two times for sixteen)
+            f32x4 acc[4];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[i & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i >> 2][i & 3], y[i >> 2][i & 3], i < 4 ? zero : acc[i & 3], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] = tdb_settled(acc[i]);
+            return (acc[0] + acc[1]) + (acc[2] + acc[3]);
+        };
         f32x4 qf[4], kr[4], qr[2][4], c[2] = {zero, zero}, res[4];      // [0]: the step's lower position tile, [1]: its upper one, the lower one of the step before
         row_of(qf, Q + int64_t(min(row_mine, len - 1)) * p.qs_l);
 #pragma unroll
@@ -455,7 +526,7 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
         int64_t d = 0;
         if (C2P || P2C) {
             d = delta_of(16 * (a0 + a) + n);
-            if (C2P) row_of(kr, KR + d * p.pks_r), c[1] = product(kr, qf, zero);
+            if (C2P) row_of(kr, KR + d * p.pks_r), c[1] = product(kr, qf);
             if (P2C) row_of(qr[1], QR + d * p.pqs_r);
             d = delta_of(16 * (a0 + a - 1) + n);
         }
@@ -475,14 +546,14 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
             if (C2P || P2C) {
                 d = delta_of(16 * (a0 + a - b - 2) + n);
                 if (C2P) {
-                    c[0] = product(kr, qf, zero);
+                    c[0] = product(kr, qf);
 #pragma unroll
                     for (int x = 0; x < 2; ++x) *reinterpret_cast<f32x4*>(&sC[n * CS + 16 * x + 4 * g]) = c[x];
                     c[1] = c[0];
                 }
                 if (P2C) {
 #pragma unroll
-                    for (int x = 0; x < 2; ++x) *reinterpret_cast<f32x4*>(&sP[n * CS + 16 * x + 4 * g]) = product(qr[x], kf, zero);
+                    for (int x = 0; x < 2; ++x) *reinterpret_cast<f32x4*>(&sP[n * CS + 16 * x + 4 * g]) = product(qr[x], kf);
 #pragma unroll
                     for (int dt = 0; dt < 4; ++dt) qr[1][dt] = qr[0][dt];
                 }
@@ -495,7 +566,7 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
                 }
                 fence();
             }
-            s = tdb_settled(product(kf, qf, s));
+            s += product(kf, qf);
             float most = -INFINITY;
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
@@ -508,17 +579,17 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
             for (int t = 0; t < 4; ++t) s[t] = expf(s[t] - up), all += s[t];
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) {
-                res[dt] *= alpha;
+                f32x4 add = zero;           // (the tile's own sum first)
 #pragma unroll
-                for (int t = 0; t < 4; ++t) res[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[dt][t], s[t], res[dt], 0, 0, 0);
-                res[dt] = tdb_settled(res[dt]);
+                for (int t = 0; t < 4; ++t) add = __builtin_amdgcn_mfma_f32_16x16x4f32(v[dt][t], s[t], add, 0, 0, 0);
+                res[dt] = res[dt] * alpha + tdb_settled(add);
             }
         }
         const float div = 1.f / fold_sum(all);
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) o[dt][t] = plain && fabsf(o[dt][t]) <= FLT_MAX ? o[dt][t] : res[dt][t] * div;
+            for (int t = 0; t < 4; ++t) o[dt][t] = keep >> (4 * dt + t) & 1 ? o[dt][t] : res[dt][t] * div;
     }
     if (row_mine < row0 + rows_here) {
 #pragma unroll
@@ -532,7 +603,7 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
 // (Offsets inside a sequence and a table are 32-bit numbers here.)
 bool tdb_f32_split_supported(const TdbKernelParams& p, int dtype) {
     auto fits = [](int64_t rows, int64_t stride) { return stride <= (int64_t(INT32_MAX) / 4 - 1024) / std::max<int64_t>(rows, 1); };
-    return dtype == TDB_F32 && p.D == D && !p.c2p && !p.p2c && fits(int64_t(p.L) + 16, std::max(p.ks_l, p.vs_l)) &&
+    return dtype == TDB_F32 && p.D == D && fabsf(p.scale) <= LARGE_SCALE && !p.c2p && !p.p2c && fits(int64_t(p.L) + 16, std::max(p.ks_l, p.vs_l)) &&
            (!p.pk || fits(2 * int64_t(p.span), p.pks_r)) && (!p.pq || fits(2 * int64_t(p.span), p.pqs_r));
 }
 
@@ -569,7 +640,7 @@ hipError_t tdb_launch_f32_split(const TdbKernelParams& p, int sets, hipStream_t 
         constexpr bool C2P = decltype(c)::value, P2C = decltype(x)::value;
         constexpr int SETS = decltype(s)::value;
         const auto kernel = attn_f32_split_kernel<C2P, P2C, SETS>;
-        constexpr int smem = SETS * set_bytes(C2P, P2C);
+        constexpr int smem = smem_bytes(C2P, P2C, SETS);
         static std::atomic<uint64_t> raised{0};     // devices whose limit for this instance is raised (twice does no harm)
         const uint64_t bit = uint64_t(1) << (dev & 63);
         if (dev >= 64 || !(raised.load(std::memory_order_relaxed) & bit)) {
