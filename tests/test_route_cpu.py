@@ -60,6 +60,8 @@ def test_which_kernel(kind, lens, heads, terms, resident):
     ("equal", [1535] * 6, 12, False), ("equal", [1536] * 6, 12, True), ("equal", [1990], 16, False),        # 5.25 and 6 units a round
     ("packed", [2269], 16, True), ("packed", [1717, 1717], 6, False), ("packed", [500, 1700, 1100, 2290], 6, False), ("packed", [1024, 1000, 4000], 8, True),
     ("padded", [900, 1935], 12, False), ("padded", [1935], 12, True), ("padded", [1000, 1700, 400], 12, True),
+    # the longest decides alone (52 us there, 69 here), or has far steps enough (118 here, 160 there)
+    ("packed", [343, 234, 843, 265, 204, 1064, 259, 74, 2322, 910, 279], 6, False), ("packed", [4603, 509], 8, True), ("packed", [1835, 3059], 12, True),
 ])
 def test_which_kernel_of_long_launches(kind, lens, heads, resident):
     assert _rule("pays")(_launch(kind, lens, heads)) == resident
@@ -68,6 +70,7 @@ def test_which_kernel_of_long_launches(kind, lens, heads, resident):
 @pytest.mark.parametrize("kind,lens,heads,resident", [
     ("padded", _even(16, 64, 512), 16, True), ("padded", _even(13, 64, 512), 16, False), ("padded", _even(16, 64, 512), 12, False),
     ("packed", _even(15, 200, 512), 16, True), ("packed", _even(10, 200, 512), 16, False),
+    ("packed", [562] + [48] * 39, 16, False), ("packed", [562] + [200] * 39, 16, True),         # a tenth and a third of the longest in the mean
 ])
 def test_which_kernel_of_workgroups_that_keep_one_head(kind, lens, heads, resident):
     assert _rule("pays")(_launch(kind, lens, heads)) == resident

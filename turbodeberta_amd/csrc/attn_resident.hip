@@ -479,10 +479,12 @@ bool tdb_resident_wide(const TdbKernelParams& p) { return wide_units(p, grid_of(
 // padded, of which the host knows the longest possible length only, 2 % if lengths are evenly spread and 9 % if most are far below it, 0.73x
 // (18 of up to 974, 359 in the mean, 8 heads: 37.5 -> 51).  No limit in L and rounds tells these from padded batches of nearly full texts, which
 // would lose as much (1250 launches: limits of 3400 to 5000, 16-row units up to 2 to 4 rounds, the other kernel below 2.2 to 3.5 of them).
-// From TDB_FAR_MIN_LEN on the far steps here take less time than there, and limits of their own hold, from 23 000 random launches of up to
-// 3.2 rounds: equal lengths all but one round of whole tiles (0.97x; two of them at 12 to 2: 1.05x); packed ones all but nearly a round, or
-// a little more of lengths far apart (of 11 400 31 % change, by 1.14x; 2.2 % of these are below 0.97x, 0.76x at worst); padded ones all but
-// 1.2 to 1.75 rounds (27 % change, by 1.08x; 3.7 % of these below 0.97x, 0.93x at worst; in between 1.05x, but 12 % below 0.97x).
+// From TDB_FAR_MIN_LEN on the far steps here take less time than there, and limits of their own hold, from random launches of up to
+// 3.6 rounds: equal lengths all but one round of whole tiles (0.97x; two of them at 12 to 2: 1.05x); packed ones all but nearly a round, and
+// what the limits at the end leave to the other kernel of lengths far apart (of 3000, evenly spread and such as texts have, 404 change, by 1.11x; 23 of these are
+// below 0.97x, 0.845x at worst: 5 of 559 to 1700, 6 heads, 54 -> 64 us.  All of more than 1.3 rounds: 0.72x where the mean is below half of the
+// longest, one of 2322 among 11, 370 in the mean, 52 -> 69); padded ones all but 1.2 to 1.75 rounds (of 3000 503 change, by 1.06x; 30 of these below
+// 0.97x, 0.895x at worst; in between 1.05x, but 12 % below 0.97x).
 bool tdb_resident_pays(const TdbKernelParams& p) {
     if (!p.pk && !p.pq) return true;        // (no tables to load: 1.21x over 708 such launches, 1.12x before this line)
     const Grid g = grid_of(-1, p.H, 0);
@@ -492,17 +494,21 @@ bool tdb_resident_pays(const TdbKernelParams& p) {
         const int64_t rounds = (seqs * ((p.L + 127) / 128) + g.per_group - 1) / g.per_group;
         return std::min(equal_cost<1>(seqs, p.L, g.per_group), equal_cost<2>(seqs, p.L, g.per_group)) * 10 <= (far ? 58 : 52) * rounds;
     }
-    const double rounds = ragged_rounds(p, g);
+    const double rounds = ragged_rounds(p, g), mean = p.varlen ? double(p.total) / p.B / p.L : 1.0;
     if (far) {
         if (!p.varlen) return rounds <= 1.2 || rounds >= 1.75 || rounds * p.L >= 3400;
-        const double mean = double(p.total) / p.B / p.L;
-        return rounds <= (mean > 0.9 ? 0.6 : 0.8) || rounds > (mean > 0.65 ? 1.0 : 1.3);
+        if (rounds <= (mean > 0.9 ? 0.6 : 0.8)) return true;
+        if (rounds <= 1.0) return false;
+        if (mean > 0.65 || (mean >= 0.5 && rounds > 1.3)) return true;
+    } else {
+        if (p.L <= 4 * BN || rounds <= (p.L <= 900 ? 0.6 : 0.45)) return true;
+        // Workgroups that keep one head load its tables once: launches of 257 to 1535 keys below the limits of the next line.  Packed, from a third of
+        // the longest in the mean on, 785 of 3000 change, by 1.077x (below 2.25 rounds 0.98x); 24 of these are below 0.97x, 0.926x at worst (shorter
+        // ones 0.78 to 1.02x: 53 of up to 1092, 120 in the mean, 51 -> 61 us).  Padded 1.085x if lengths are evenly spread, 0.95x at worst (3 to
+        // 3.5 rounds 1.02x, and a quarter of them slower); such as texts have 1.02x, but 0.72x where most of a batch is padding (14 of up to 605, 145 in the
+        // mean, 27 -> 37 us), which the host does not know.  With three heads 1.02x and 1.035x, but up to an eighth of them slower.
+        if (g.heads == 1 && (p.varlen ? rounds >= 2.25 && mean >= 0.35 : rounds >= 3.5)) return true;
     }
-    if (p.L <= 4 * BN || rounds <= (p.L <= 900 ? 0.6 : 0.45)) return true;
-    // Workgroups that keep one head load its tables once: 2700 such launches of 257 to 1535 keys below the limits of the next line, 1.06x
-    // packed (below 2.25 rounds 0.98x) and 1.085x padded (3 to 3.5 rounds 1.02x, and a quarter of them slower); 0.9 % are below 0.97x,
-    // 0.92x at worst.  With three heads 1.02x and 1.035x, but up to an eighth of them slower.
-    if (g.heads == 1 && rounds >= (p.varlen ? 2.25 : 3.5)) return true;
     // (Of few rounds of very different lengths the longest alone decide: 2 of 650 and 2600 0.82x.  With a mask the lengths are only bounded.)
     return rounds * p.L >= (rounds >= (p.varlen ? 1.4 : 1.75) ? 3000 : 3400);
 }
