@@ -92,6 +92,8 @@ def test_which_units(kind, lens, heads, wide):
     ("equal", [512] * 2, 12, 2, 2), ("equal", [256] * 4, 12, 2, 2), ("equal", [190] * 3, 16, 2, 2), ("padded", _even(3, 151, 460), 12, 2, 2),
     ("equal", [128] * 2, 12, 2, 0), ("equal", [512], 12, 2, 0), ("equal", [21] * 44, 12, 2, 0), ("packed", _even(58, 17, 30), 16, 2, 0),
     ("packed", [134] * 7, 12, 1, 0), ("equal", [59] * 8, 16, 1, 0),
+    ("packed", [126] + [23] * 12, 12, 2, 0), ("packed", [247] + [32] * 19, 8, 2, 0), ("packed", [247] + [150] * 9, 8, 2, 1),    # a long one among short ones
+    ("equal", [68] * 9, 16, 2, 0), ("equal", [120] * 9, 16, 2, 1), ("padded", [139] * 6, 16, 2, 0),
 ])
 def test_which_float32_kernel(kind, lens, heads, terms, sets):
     fn = _lib.load()._Z18tdb_f32_split_setsRK15TdbKernelParams

@@ -612,22 +612,31 @@ int tiles_of(const TdbKernelParams& p) { return p.varlen ? p.total / ROWS + p.B 
 int64_t blocks_of(const TdbKernelParams& p) { return (int64_t((tiles_of(p) + 3) / 4) * p.H + 7) / 8 * 32; }      // groups of 4 tiles, rounded up to 8 XCDs
 }  // namespace
 
-// How many sets of waves make a launch faster than attn_f32.hip does, or 0.  Fitted to 368 random launches (16 to 1200 keys, 6 to 16 heads; geometric mean
-// of all 1.10x, 1.11x if the fastest were known; 5 below 0.97x, 0.88 at worst):
+// How many sets of waves make a launch faster than attn_f32.hip does, or 0.  Fitted to 4000 random launches (16 to 1200 keys, 6 to 16 heads, lengths evenly
+// spread and such as texts have).  Equal lengths: 574 taken, 1.214x, 9 of these below 0.97x, 0.86x at worst; packed: 442, 1.176x, 31, 0.84x; padded, of which
+// the host knows the longest possible length only: evenly spread 271, 1.18x, 30, 0.76x; as texts have them 282, 1.09x, 73, and down to 0.58x where
+// most of a batch is padding (10 of up to 248, 45 in the mean, 22 -> 35 us): a limit that spares these would cost full batches as much.
 //   * as many workgroups as compute units: two sets, from three quarters of the units on (4 x 256 32.2 -> 24.0 us, 2 x 512 55.5 -> 39; 4 x 128, half of the
 //     units, 15 either way), earlier for long texts, where the opening of a workgroup (2.5 us) weighs less (3 x 190 26.0 -> 19.7).  Short texts leave the
-//     second set little (9 of 53..66 11.7 -> 14.3).  With lengths, of which the host knows the longest possible, a good half of the workgroups has keys;
-//   * more: one set, two workgroups to a compute unit (8 of 96..384 65.6 -> 45.6, 32 x 128 56.4 -> 36.7), but not for one or two key tiles (44 x 21 12.3 -> 15.9)
-//     nor for one term alone where the units are hardly filled (7 x 134 17.3 -> 20.9).
+//     second set little (9 of 53..66 11.7 -> 14.3), and a long one among them decides alone, which the four waves of the other kernel share (packed, half of the
+//     longest in the mean: below 0.7 to 1.04x, 14 of 36 below 0.97x; above 1.1 to 1.39x).  With lengths, of which the host knows the longest possible, a good
+//     half of the workgroups has keys;
+//   * more: one set, two workgroups to a compute unit (8 of 96..384 65.6 -> 46, 32 x 128 56.4 -> 37), but not for one or two key tiles (44 x 21 12.3 -> 15.9),
+//     nor for one term alone where the units are hardly filled (7 x 134 17.3 -> 20.9), nor up to one and a half workgroups to a unit if lengths are far apart
+//     (packed, mean below 0.55: 0.6 to 1.0x) or the second of two is nearly empty (9 x 68, 16 heads, 18.3 -> 21.8), nor for an eighth more than the units
+//     if they may be padding (0.9x).
 int tdb_f32_split_sets(const TdbKernelParams& p) {
     const int64_t units = tdb_compute_units(-1), wgs = int64_t(tiles_of(p)) * p.H;
     const bool both = p.pk && p.pq, lengths = p.varlen || p.seqlens;
+    const double mean = p.varlen ? double(p.total) / p.B / p.L : 1.0;
     if (blocks_of(p) <= (p.seqlens && p.L > 200 ? units * 25 / 16 : units)) {
         const int64_t least = p.L <= 160 ? units * 3 / 4 : both ? units * 17 / 32 : units * 21 / 32;
-        return p.L > 80 && wgs >= least && (both || p.L >= 300) ? 2 : 0;
+        return p.L > 80 && wgs >= least && (both || p.L >= 300) && mean >= 0.5 ? 2 : 0;
     }
     const int keys = p.varlen ? p.total / p.B : p.L;
-    return keys <= (lengths ? 40 : 32) || (!both && wgs <= units * 17 / 16) ? 0 : 1;
+    if (keys <= (lengths ? 40 : 32) || (!both && wgs <= units * 17 / 16)) return 0;
+    if (wgs <= units * 3 / 2 && (mean < 0.55 || (keys > 64 && keys <= 80))) return 0;
+    return p.seqlens && wgs <= units * 9 / 8 ? 0 : 1;
 }
 
 hipError_t tdb_launch_f32_split(const TdbKernelParams& p, int sets, hipStream_t stream) {
