@@ -25,7 +25,7 @@
 //
 // An infinity has no parts (its rest is NaN), nor has what rounds to one: a wave whose results are not all finite computes its rows
 // again from the float32 operands and takes what was not finite from there.  A NaN or an infinity in each sequence costs that for all its rows: 8 x 512
-// 121 -> 338 us, 2 x 4096 1.5 -> 4.3 ms (one key after another 1950 us and 14.2 ms; attn_f32.hip, which needs nothing of the kind, 160 us
+// 132 -> 345 us, 2 x 4096 1.5 -> 4.4 ms (one key after another 1950 us and 14.2 ms; attn_f32.hip, which needs nothing of the kind, 160 to 170 us
 // and 2.2 ms).
 // Operands below about 1e-33 lose bits of their third part, at most TINY each (bf16 has the exponents of float32).  In a score that is nothing
 // unless what it is multiplied with is beyond LARGE; in a result it is unless the result is as small.  Both are looked for, and such results
@@ -514,8 +514,6 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
             f32x4 acc[4];
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[i & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i >> 2][i & 3], y[i >> 2][i & 3], i < 4 ? zero : acc[i & 3], 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[i] = tdb_settled(acc[i]);
             return (acc[0] + acc[1]) + (acc[2] + acc[3]);
         };
         f32x4 qf[4], kr[4], qr[2][4], c[2] = {zero, zero}, res[4];      // [0]: the step's lower position tile, [1]: its upper one, the lower one of the step before
@@ -582,7 +580,7 @@ __global__ __launch_bounds__(SETS * 256, 2) void attn_f32_split_kernel(const Tdb
                 f32x4 add = zero;           // (the tile's own sum first)
 #pragma unroll
                 for (int t = 0; t < 4; ++t) add = __builtin_amdgcn_mfma_f32_16x16x4f32(v[dt][t], s[t], add, 0, 0, 0);
-                res[dt] = res[dt] * alpha + tdb_settled(add);
+                res[dt] = res[dt] * alpha + add;
             }
         }
         const float div = 1.f / fold_sum(all);
