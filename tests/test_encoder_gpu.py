@@ -81,6 +81,16 @@ def test_few_rows_with_the_normalisation_in_the_products(hidden, heads, inner, L
     _check(*_both(_model(dtype, hidden, heads, 2, inner), ids, mask), mask, dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens,L", [([1], 1), ([15], 15), ([17], 17), ([48], 48), ([49], 49), ([64], 64), ([20, 3, 41], 41)])
+def test_few_rows_of_wider_models(lens, L, dtype):
+    """Products, then residual and LayerNorm in launches of their own: one to four row tiles, and a first layer whose rows the next
+    one's product reads in its own order."""
+    assert _lib.load().tdb_enc_rows_fused(64, 832, 160, _lib.TDB_BF16) == 0
+    ids, mask = _ids(lens, L)
+    _check(*_both(_model(dtype, 832, 13, 2, 160), ids, mask), mask, dtype)
+
+
 @pytest.fixture(scope="module")
 def base_width():
     """Three base-sized layers: Hugging Face's model with weights as a 16-bit model holds them, in float32 and in the type."""

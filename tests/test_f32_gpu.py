@@ -1,5 +1,6 @@
-"""The float32 matrix-core kernel at the edges of its tiles (16 queries or 32 per workgroup, keys dealt to four waves in
-blocks of two 16-key tiles), against the vector-ALU kernel."""
+"""float32 calls at the edges of the matrix-core kernels' tiles, against the vector-ALU kernel, in whichever kernel the library chooses: small
+ones in the one that has 16 queries or 32 per workgroup and deals keys to four waves in blocks of two 16-key tiles, larger ones mostly in the one whose
+products are of bf16 parts (tests/test_f32_split_gpu.py runs both by name)."""
 import math
 
 import pytest
@@ -19,7 +20,7 @@ def _both(d, terms=("c2p", "p2c"), lens=None):
             for f in (False, True)]
 
 
-@pytest.mark.parametrize("B,H", [(1, 2), (40, 16)])          # 16 and 32 query rows per workgroup
+@pytest.mark.parametrize("B,H", [(1, 2), (40, 16)])          # 16 query rows per workgroup, and 32 or bf16 parts
 @pytest.mark.parametrize("L", [1, 15, 16, 17, 33, 64, 127, 129, 161])
 def test_tile_edges(B, H, L):
     d = {n: t.cuda() for n, t in make_inputs(L, B, H, L, 64, 256, 512).items()}

@@ -51,6 +51,25 @@ def test_packed_with_gaps(flag, B):
     assert (got - ref).abs().max() < BOUND and not got[:20].any() and not got[T - 20:].any()
 
 
+@pytest.mark.parametrize("L", [15, 17, 33, 64, 129, 161])
+def test_direct_tile_edges(L):
+    """32 query rows a workgroup."""
+    with in_kernel(DIRECT):
+        f32.test_tile_edges(40, 16, L)
+
+
+@pytest.mark.parametrize("terms", [("c2p",), ("p2c",), ()])
+def test_direct_term_subsets(terms):
+    with in_kernel(DIRECT):
+        f32.test_term_subsets(terms, 40, 16)
+
+
+@pytest.mark.parametrize("where", ["query", "key", "value", "last_value", "c2p_row", "p2c_row", "score", "low_scores", "padding"])
+def test_direct_nan_and_infinity(where):
+    with in_kernel(DIRECT):
+        f32.test_nan_and_infinity_reach_what_they_belong_to(where, 33, 16, 77)
+
+
 @pytest.mark.parametrize("flag", [DIRECT, ONE_SET, TWO_SETS])
 @pytest.mark.parametrize("where", ["query", "key", "value", "last_value", "c2p_row", "p2c_row", "score", "low_scores", "padding"])
 def test_nan_and_infinity(flag, where):
