@@ -9,9 +9,10 @@
 // fragment is four 16-byte loads whose lanes cover 64 contiguous bytes of 16 rows), the two position terms are shifted
 // through a wave's own LDS scratch with plain 4-byte reads, and no wave waits for another until the end.
 //
-// Measured (vector-ALU kernel before): 1 x 20 x 12 heads 24 -> 5.6 us; 2 x 128 84 -> 8.9; 8 x 12 heads, lengths 96..384, 660 -> 66 us; 8 x 512
-// full 157 us = 83 TFLOP/s without credit for the half-used outer tiles, 103 with (matrix pipe busy 65 % of the time; what is
-// left is the start and end of a workgroup, a tenth, and L2 latency that two waves per SIMD do not quite cover).
+// Measured (vector-ALU kernel before): 1 x 20 x 12 heads 24 -> 5.6 us; 2 x 128 84 -> 9.1 (bound by its chain of loads and products, with
+// three waves to a compute unit).  What launches above its present ones took here, before they went to attn_f32_split.hip: 8 x 12 heads, lengths
+// 96..384, 66 us; 8 x 512 full 157 us = 83 TFLOP/s without credit for the half-used outer tiles, 103 with (matrix pipe busy 65 % of the time; what
+// is left is the start and end of a workgroup, a tenth, and L2 latency that two waves per SIMD do not quite cover).
 //
 // One workgroup = QT*16 query rows of one (sequence, head); its four waves share out the KEYS (blocks of two
 // 16-key tiles, in turn) and merge their partial softmax sums through LDS at the end.  Splitting the keys rather than the

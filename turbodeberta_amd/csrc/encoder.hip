@@ -371,8 +371,8 @@ __device__ __forceinline__ void with_steps(int left, F f) {
     else if constexpr (MOST > 1) with_steps<MOST - 1>(left, f);
 }
 
-// Weights of the products to come, brought into the L2 of the XCD that will read them by workgroups of their own (blockIdx.y >= mt) beside the present
-// product: chunk i, the rows of one workgroup of that product, by blocks whose number is i modulo 8, which go to the same XCD.  (12 layers of 768, 48 rows, weights in HBM: 414 -> 380 us; weights in the last-level cache 348 -> 343.
+// Weights of the products to come, brought into the L2 of the XCD that will read them by workgroups of their own (blockIdx.y >= mt), beside the present
+// product as far as there is room: chunk i, the rows of one workgroup of that product, by blocks whose number is i modulo 8, which go to the same XCD.  (12 layers of 768, 48 rows, weights in HBM: 414 -> 380 us; weights in the last-level cache 348 -> 343.
 // The attention's table rows as well: no change.)
 struct Ahead {
     static constexpr int MOST = 2;
@@ -688,7 +688,11 @@ void with_type(int dtype, F f) {
 // 20.2 against 19.1 at 80).
 constexpr int SMALL_ROWS = 64;
 // Each of the column blocks reads and normalises its rows anew, 64 bytes of float32 for each column of them: 24 layers of 1024 take 927 us that way and 848 with
-// launches for residual + LayerNorm.
+// launches for residual + LayerNorm.  12 layers replayed as a graph, with such launches against without, 1, 16, 17..32, 33..48 and 49..64 rows: 128 wide
+// 1.07, 1.12, 1.14, 1.15, 1.17x; 256 1.03, 1.06, 1.09; 384 0.98, 1.01, 1.04, 1.05, 1.06; 512 0.94, 0.97, 1.00, 1.00, 1.03; 640 0.99, 1.03, 1.03, 1.04, 1.00; 768 0.99,
+// 1.02, 1.00, 1.02, 1.03; 832 0.98, 1.00, 0.97, 0.94, 0.98; 896 1.00, 1.02, 1.01, 0.98, 1.06; 960 0.99, 1.01, 0.97, 1.00, 0.95; 1024 0.98, 1.00, 1.01, 0.99, 0.94.
+// At 448 and 512 wide with up to 16 rows the contraction shared out over 8 workgroups there is what is ahead.  That stays as it is: calls from a program are bound by
+// the host's launches, 63 here and 86 there, where it is slow (512 wide, one row: 379 -> 271 us; on a faster host 258 -> 270).
 constexpr int FUSED_WIDTH = 768;
 
 // Blocks of 16 columns that a workgroup of norm_gemm_kernel takes: as few as give each compute unit one workgroup.
@@ -847,7 +851,9 @@ int tdb_enc_gemm_add(const void* in, int ordered, const void* w, const void* bia
     const int mt = tdb_enc_small_tiles(M, N, K, dtype);
     if (!mt || N % 32 || nexts < 0 || nexts > Ahead::MOST) return int(hipErrorInvalidValue);
     const Ahead ahead = ahead_of(next, nexts, mt);
-    const int extra = ahead.chunks[0] > 0 ? 2 : 0;     // (96 workgroups of 768 columns' product)
+    // Two rows of workgroups to fetch ahead.  (12 layers of 768 as a graph, none, one and two: 16 rows 311, 310, 304 us, 32 325, 326, 319, 48 350, 352, 345; also where
+    // they are more than one to a compute unit, 49 rows 358, 360, 356.  640 wide 300, 302, 294 to 358, 354, 355; 384 wide equal.)
+    const int extra = ahead.chunks[0] > 0 ? 2 : 0;
     const NormRows r{residual->x, reinterpret_cast<const float2*>(residual->stats), residual->gamma, residual->beta, residual->eps};
     auto go = [&](auto kernel, int waves) {
         hipLaunchKernelGGL(kernel, dim3(N / 16, mt + extra), dim3(waves * 64), 0, static_cast<hipStream_t>(stream), in, w, bias, r, x,
